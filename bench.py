@@ -375,7 +375,7 @@ def main():
         del pool, bigpool
 
     # ---- roofline of the dominant kernel ------------------------------------------------
-    # Every launch of the timed region is the same kernel (qmv_mfma_kernel); its average launch
+    # Every launch of the timed region is the same kernel (qmv_flow_kernel); its average launch
     # duration is the timed region (events on the launch stream around the graph replay) divided
     # by the launches in it -- back-to-back kernels of one stream, so launch gaps are included.
     avg_launch_us = ms_per_step * 1e3 / launches_per_layer
@@ -551,8 +551,8 @@ def main():
         out["roofline_small_batch"] = {
             "bound": "hbm", "achieved": round(small_bytes / (small_us * 1e-6) / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(small_bytes / (small_us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4), "traffic": None,
-            "kernel": "qmv_flow_kernel_1 (M = 1), qmv_ring_kernel (2..16 rows), qmv_stream_kernel (2..4 rows over "
-                      "5120->151936): the 20 (shape, M) cases of BASELINE config 3, algorithmic bytes of all over "
+            "kernel": "qmv_flow_kernel_1 (M = 1), qmv_batch_kernel (2..16 rows): the "
+                      "20 (shape, M) cases of BASELINE config 3, algorithmic bytes of all over "
                       "the time of all",
             "timing": "per case one HIP graph of 8 x (packs in rotation) calls, median of 5 replays",
             "profile": "profiles/qmv_small_batch_m1_m4_m16.txt (rocprofv3 kernel trace + FETCH_SIZE / WRITE_SIZE)"}

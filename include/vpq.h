@@ -131,19 +131,19 @@ size_t vpq_qmv_workspace_bytes(int K, int N, int M);
 enum {
   VPQ_QMV_AUTO = 0,
   VPQ_QMV_SIMPLE = 1,      /* one wavefront per output row, fp32 VALU */
-  VPQ_QMV_MFMA = 2,        /* LDS-staged codes, bf16 MFMA on the integer codes */
+  VPQ_QMV_MFMA = 2,        /* codes and x staged through LDS, bf16 MFMA on the integer codes; what AUTO takes for 2..16
+                              rows (any K % 64 there), and for one row where FLOW and ROWS do not run */
   /* 3 is unassigned */
   VPQ_QMV_STREAM = 4,      /* M <= 4: persistent workgroups, x staged in LDS, prefetched items */
   VPQ_QMV_RING = 5,        /* x in registers across a workgroup's tiles, codes through a two-slot LDS ring per wavefront */
   VPQ_QMV_ROWS = 6,        /* M <= 2, any K % 64: a wavefront streams whole rows with full-width loads, packed bf16
-                              dot products, no LDS; what AUTO takes for M <= 2 where K is not a multiple of 512 */
+                              dot products, no LDS; what AUTO takes for M = 1 where K is not a multiple of 512 */
   VPQ_QMV_FLOW = 7,        /* M = 1, K % 512 == 0, K >= 2048: one wavefront per (row set, K part), every load of the
                               launch requested up front, x in registers, scales / biases staged in LDS; what AUTO
-                              takes for M = 1 below lm_head-sized packs */
+                              takes for M = 1 */
   VPQ_QMV_RING_SPLITK = 8  /* as 5 with K split across workgroups (up to 4 parts, K >= 1024): fp32 planes in `ws`, added
                               in part order by a fold launch that rounds once -- the deep-K split of
-                              generative-models/shared/mma-splitk.h:30-52.  AUTO takes it by itself for 2..16 rows when
-                              `ws` is given and its cost model says it pays (many rows of x, deep K, narrow N) */
+                              generative-models/shared/mma-splitk.h:30-52 */
 };
 
 /* ---- a6/a7/a8 (+a10): QMM ----------------------------------------------
@@ -239,12 +239,12 @@ int vpq_lora_a_bf16(vpq_stream_t stream, const uint16_t* x, const uint16_t* lora
  * Replaces `MetalQwenModel::qmm_auto_`
  * (generative-models/qwen3/metal-qwen-model.cc:3964-4033) with its ladder
  * (:3839-3962: GEMV, a batched plan that walks M in slabs, the tiled GEMM): up
- * to 64 rows run the QMV arithmetic in slabs of at most 16 rows (one launch per
- * slab), larger M the QMM arithmetic.  (The reference crosses over to the GEMM at
- * M = 8; here the 256-row GEMM tile does not pay below ~64 rows: measured 57 us at
- * 4096->4096 for any M <= 256 against ~10 us per slab.)  Above 32 rows the GEMM
- * splits K (vpq_qmm_splitk_w4g64_bf16) where that pays and `ws` has
- * vpq_qmm_workspace_bytes() bytes (without that room, 33..64 rows stay slabs).  From 8192 rows on, when `ws` holds the
+ * to 64 rows run the QMV arithmetic in one launch, larger M the QMM arithmetic.
+ * (The reference crosses over to the GEMM at M = 8; here the 256-row GEMM tile
+ * does not pay below ~64 rows: measured 57 us at 4096->4096 for any M <= 256
+ * against 9.5 us at 64 rows.)  Above 32 rows over a narrow N, and above 64 rows
+ * where that pays, the GEMM splits K (vpq_qmm_splitk_w4g64_bf16), if `ws` has
+ * vpq_qmm_workspace_bytes() bytes.  From 8192 rows on, when `ws` holds the
  * expanded weight (N*K*2 bytes), the GEMM runs by the dequant-once route
  * (vpq_qmm_dense_route_w4g64_bf16: expansion + dense GEMM, the reference's route
  * for large M, minimax-h3/metal-minimax-h3-transformer.cc:2020-2160), which is the
@@ -267,11 +267,9 @@ int vpq_linear_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t
  * case w[1] = w[0] + q_rows*K/8 words (scales, biases alike); gate|up of an
  * MLP is count = 2.  Arithmetic and requirements are those of
  * vpq_qmv_w4g64_bf16 per pack (no residual); results are bit-identical to
- * `count` separate calls of its VPQ_QMV_FLOW kernel at M = 1 (K % 512 == 0,
- * K >= 2048), of its VPQ_QMV_MFMA kernel at other M where K % 512 == 0, of
- * its VPQ_QMV_ROWS kernel for other K at M <= 2.  The pointer tables are
- * host arrays, read before the call returns.  Shapes neither grouped kernel
- * takes (K % 512 != 0 with M > 2) run as separate launches. */
+ * `count` separate calls of it (VPQ_QMV_AUTO).  The pointer tables are host
+ * arrays, read before the call returns.  Packs whose scales or biases are not
+ * 16-byte aligned run as separate launches at M > 2. */
 int vpq_qmv_group_w4g64_bf16(vpq_stream_t stream, int count, const uint32_t* const* w,
                              const uint16_t* const* scales, const uint16_t* const* biases,
                              const uint16_t* x, uint16_t* const* y, int K, const int* N, int M);
@@ -316,7 +314,7 @@ int vpq_qmm_swiglu_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint
 /* The size-based entrance of the fused MLP first half, as the reference's call
  * sites choose between the two (generative-models/llama3/metal-llama-model.cc:
  * 466-477 decode, 634-650 and 800-812 prefill): up to 64 rows the QMV arithmetic
- * in slabs of 16 rows, larger M the QMM arithmetic (as vpq_linear_w4g64_bf16). */
+ * in one launch, larger M the QMM arithmetic (as vpq_linear_w4g64_bf16). */
 int vpq_linear_swiglu_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
                                  const uint16_t* biases, const uint16_t* x, uint16_t* y,
                                  int K, int N, int M);
@@ -511,7 +509,7 @@ int vpq_qmm_w4g32_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t* s
 int vpq_qmm_tiled_w4g32_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
                              const uint16_t* biases, const uint16_t* x, uint16_t* y,
                              int K, int N, int M, int activation, int tile_n);
-/* The size-based entrance over a group-32 pack: slabs of vpq_qmv_w4g32_bf16 up to 64 rows (at every M where
+/* The size-based entrance over a group-32 pack: the arithmetic of vpq_qmv_w4g32_bf16 up to 64 rows (at every M where
  * K % 64 != 0), vpq_qmm_w4g32_bf16 above. */
 int vpq_linear_w4g32_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales, const uint16_t* biases,
                           const uint16_t* x, uint16_t* y, int K, int N, int M);
@@ -608,8 +606,8 @@ int vpq_qmm_tiled_w8g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint1
                              const uint16_t* biases, const uint16_t* x, uint16_t* y,
                              int K, int N, int M, int activation, int tile_n);
 /* The size-based entrance over an 8-bit pack (qmm_auto_'s ladder, generative-models/qwen3/
- * metal-qwen-model.cc:3964-4033, which takes the width from the layer): slabs of vpq_qmv_w8g64_bf16 up to
- * 64 rows, vpq_qmm_w8g64_bf16 above. */
+ * metal-qwen-model.cc:3964-4033, which takes the width from the layer): the arithmetic of
+ * vpq_qmv_w8g64_bf16 up to 64 rows, vpq_qmm_w8g64_bf16 above. */
 int vpq_linear_w8g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
                           const uint16_t* biases, const uint16_t* x, uint16_t* y, int K, int N, int M);
 /* `affine_requant_w8_to_w4_g64` (affine_dequant.metal:134-186): the half-width copy of an 8-bit pack (the draft

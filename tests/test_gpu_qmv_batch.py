@@ -1,0 +1,85 @@
+"""The batch QMV kernel (vpq_qmv_batch.h) where it can go wrong: K that ends inside a chunk of codes or a piece of x, N
+that ends inside a tile of 16 rows or leaves a partial 16-byte piece of scales, every count of staged rows of x, two
+tiles of rows of x, more chunks than wavefronts -- against the oracle of each format, through the C ABI."""
+import numpy as np
+import pytest
+import torch
+
+from tests import parity
+from tests.test_oracle_pins import f16_pack
+from vpipe_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+# K: below one chunk of 256 (128 for 8-bit codes), one more than a whole number of chunks, K / 64 odd (scales read in
+# 2-byte pieces), more than eight chunks; N: one row, one short of / past a tile, more tiles than CUs
+SHAPES = [(64, 1, 2), (192, 15, 3), (320, 17, 4), (832, 33, 5), (2112, 31, 8), (2304, 4133, 9), (3904, 48, 13), (4096, 65, 16)]
+
+
+@pytest.mark.parametrize("K,N,M", SHAPES)
+@pytest.mark.parametrize("fmt", ["w4g64", "w4g32", "w8g64", "f16"])
+def test_qmv_batch_edges(vpq, oracle, dev, D, fmt, K, N, M):
+    seed = K + 3 * N + M
+    if fmt == "f16":
+        w, s, b = f16_pack(N, K, seed)
+        x = np.random.default_rng(seed).standard_normal((M, K)).astype(np.float16).view(np.uint16)
+        y64, _ = oracle.matmul_f16(w, s, b, x, K, N, M, rounded=False)
+        t16 = [torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).to(dev).view(torch.float16) for a in (s, b, x)]
+        run, args = vpq.qmv_w4g64_f16, (D.u32(w, dev), *t16)
+    else:
+        make = {"w4g64": synth.make_weight, "w4g32": synth.make_weight_g32, "w8g64": synth.make_weight8}[fmt]
+        w, s, b = make(N, K, seed)
+        x = synth.make_act(M, K, seed + 1)
+        if fmt == "w8g64":
+            y64, _ = oracle.matmul8(w, s, b, x, K, N, M, rounded=False)
+        else:
+            y64, _ = (oracle.qmv if fmt == "w4g64" else oracle.qmv_g32)(w, s, b, x, K, N, M)
+        run = {"w4g64": vpq.qmv_w4g64, "w4g32": vpq.qmv_w4g32, "w8g64": vpq.qmv_w8g64}[fmt]
+        args = (D.u32(w, dev), D.bf16(s, dev), D.bf16(b, dev), D.bf16(x, dev))
+    f = run(*args, K, N, M, f32out=True)
+    out = parity.Guarded((M, N), args[3].dtype, dev)
+    run(*args, K, N, M, out=out.view)
+    torch.cuda.synchronize()
+    out.assert_intact()
+    parity.check_f32(f.cpu().numpy(), y64)
+    # the stored element is the fp32 result rounded once
+    assert torch.equal(out.view, f.to(args[3].dtype))
+
+
+@pytest.mark.parametrize("M", [17, 31, 32, 33, 50, 64])
+@pytest.mark.parametrize("K,N", [(960, 80), (4352, 24)])
+def test_a_row_of_x_has_the_same_bits_in_any_batch(vpq, oracle, dev, D, M, K, N):
+    # plain and gated, through the size-based entrances: up to 64 rows in one launch, each row as in a batch of its own
+    w, s, b = synth.make_weight(N, K, 5 + M)
+    x = synth.make_act(M, K, 6 + M)
+    y64, yb = oracle.qmv(w, s, b, x, K, N, M)
+    wd, sd, bd, xd = D.u32(w, dev), D.bf16(s, dev), D.bf16(b, dev), D.bf16(x, dev)
+    out = parity.Guarded((M, N), torch.bfloat16, dev)
+    vpq.linear_w4g64(wd, sd, bd, xd, K, N, M, out=out.view)
+    torch.cuda.synchronize()
+    out.assert_intact()
+    parity.check_bf16(D.bits(out.view), y64, yb)
+    gated = vpq.linear_swiglu_w4g64(wd, sd, bd, xd, K, N, M)
+    for m0 in range(0, M - 2, 13):
+        n = min(13, M - m0)
+        part = xd[m0:m0 + n].contiguous()
+        assert torch.equal(vpq.qmv_w4g64(wd, sd, bd, part, K, N, n), out.view[m0:m0 + n])
+        assert torch.equal(vpq.qmv_swiglu_w4g64(wd, sd, bd, part, K, N, n), gated[m0:m0 + n])
+
+
+@pytest.mark.parametrize("fmt", ["w4g64", "w4g32", "w8g64"])
+def test_grouped_launch_of_the_batch_kernel(vpq, dev, D, fmt):
+    # four packs of different heights, none a multiple of a workgroup's rows: the bits of the separate calls
+    K, M, Ns = 1344, 7, (40, 1, 133, 16)
+    make = {"w4g64": synth.make_weight, "w4g32": synth.make_weight_g32, "w8g64": synth.make_weight8}[fmt]
+    xd = D.bf16(synth.make_act(M, K, 3), dev)
+    packs, outs = [], [parity.Guarded((M, N), torch.bfloat16, dev) for N in Ns]
+    for i, N in enumerate(Ns):
+        w, s, b = make(N, K, 40 + i)
+        packs.append((D.u32(w, dev), D.bf16(s, dev), D.bf16(b, dev), N))
+    {"w4g64": vpq.qmv_group_w4g64, "w4g32": vpq.qmv_group_w4g32, "w8g64": vpq.qmv_group_w8g64}[fmt](
+        packs, xd, K, M, outs=[o.view for o in outs])
+    single = {"w4g64": vpq.qmv_w4g64, "w4g32": vpq.qmv_w4g32, "w8g64": vpq.qmv_w8g64}[fmt]
+    for (w, s, b, N), o in zip(packs, outs):
+        o.assert_intact()
+        assert torch.equal(o.view, single(w, s, b, xd, K, N, M))

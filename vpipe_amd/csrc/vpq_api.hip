@@ -82,6 +82,15 @@ int check_pack(const uint32_t* w, const uint16_t* scales, const uint16_t* biases
 // are even on 4096->12288 and the fused kernel is ahead on the N = 4096 shapes).
 constexpr int kDenseRouteMinRows = 8192;
 
+// The batch kernel over one pack.
+hipError_t launch_batch(hipStream_t hs, const vpq::QmvArgs& a, const vpq::BatchFormat& f)
+{
+  vpq::QmvGroup g;
+  g.count = 1;
+  g.seg[0] = vpq::QmvSeg{a.w, a.scales, a.biases, a.y, a.N};
+  return vpq::launch_qmv_batch(hs, a, g, f);
+}
+
 int qmv_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
                const uint16_t* biases, const uint16_t* x, void* y, bool y_f32, int K, int N, int M,
                const uint16_t* residual, void* ws, size_t ws_bytes, int variant, int gate_act = 0)
@@ -107,7 +116,8 @@ int qmv_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
   a.gate_act = gate_act;
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
 
-  const bool mfma_ok = vpq::qmv_mfma_supports(K, N, M) && aligned(scales, 16) && aligned(biases, 16);
+  const bool batch_ok = vpq::qmv_batch_supports(K, M, vpq::BatchFormat{}) && aligned(scales, 16) && aligned(biases, 16);
+  const bool mfma_ok = batch_ok && (K % 512) == 0;           // what the forced variants of the MFMA kernels take
   const bool flow_ok = vpq::qmv_flow_supports(K, N, M) && aligned(scales, 16) && aligned(biases, 16);
   if (gelu_mul) {        // the two kernels that have this store: the streaming one and the general one
     return finish(flow_ok ? vpq::launch_qmv_flow(hs, a) : vpq::launch_qmv_simple(hs, a));
@@ -133,38 +143,19 @@ int qmv_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
     return finish(vpq::launch_qmv_ring(hs, a, 0, parts));
   }
   if (variant == VPQ_QMV_STREAM) {
-    // handled below, after the shape check of the streaming kernel
-  } else if (variant == VPQ_QMV_MFMA) {
-    if (!mfma_ok) { return VPQ_ERR_BAD_SHAPE; }
-    return finish(vpq::launch_qmv_mfma(hs, a));
-  }
-  const bool stream_ok = mfma_ok && gate_act == 0 && vpq::qmv_stream_supports(K, N, M);
-  if (variant == VPQ_QMV_STREAM) {
-    if (!stream_ok) { return VPQ_ERR_BAD_SHAPE; }
+    if (!mfma_ok || gate_act != 0 || !vpq::qmv_stream_supports(K, N, M)) { return VPQ_ERR_BAD_SHAPE; }
     return finish(vpq::launch_qmv_stream(hs, a));
   }
-  // One row of x: the streaming kernel that requests the whole pack up front (measured, HBM-cold: 4096->12288
-  // 6.8 us against 9.0 for the tile kernel, 4096->2x12288 11.5 against 15.6, the 5120->151936 lm_head 75.6 against
-  // 79.7 for the persistent kernel below).
-  if (flow_ok) { return finish(vpq::launch_qmv_flow(hs, a)); }
-  // Two to four rows over an lm_head-sized pack: persistent workgroups that walk a tile's whole K.
-  const double pack_bytes = (double)N * (double)K * 9.0 / 16.0;
-  if (stream_ok && pack_bytes >= 150e6) { return finish(vpq::launch_qmv_stream(hs, a)); }
-  // Several rows of x: the ring kernel keeps a slice of x in registers for all the tiles of a
-  // workgroup (one workgroup per CU; it chooses its tiles per workgroup so that the launch runs in
-  // few, full generations of workgroups), so x is re-read from L2 once per slice and workgroup instead
-  // of once per item (measured at 16 rows: 117 vs 284 us at 5120->151936, 17.6 vs 39.9 us at
-  // 5120->17408; at 4 rows 8.8 vs 12.0 us at 4096->12288; at 2 rows 15.1 vs 17.1 us at 5120->17408,
-  // 16.0 vs 17.5 at 17408->5120).
-  // (with a workspace the ring kernel splits K across workgroups where its cost model says that pays: many rows
-  // over a deep K and a narrow N)
-  if (mfma_ok && vpq::qmv_ring_supports(K, N, M) && M >= 2) {
-    if (a.ws != nullptr && !aligned(a.ws, 16)) { a.ws = nullptr; a.ws_bytes = 0; }
-    return finish(vpq::launch_qmv_ring(hs, a, 0, 0));
+  if (variant == VPQ_QMV_MFMA) {
+    if (!mfma_ok) { return VPQ_ERR_BAD_SHAPE; }
+    return finish(launch_batch(hs, a, vpq::BatchFormat{}));
   }
-  if (mfma_ok) { return finish(vpq::launch_qmv_mfma(hs, a)); }
-  // K not a multiple of 512, or scales / biases off 16-byte alignment: the row-streaming kernel
-  // for up to two rows of x, the general one above.
+  // One row of x: the streaming kernel that requests the whole pack up front.
+  if (flow_ok) { return finish(vpq::launch_qmv_flow(hs, a)); }
+  // One row over a K that is not a multiple of 512: the row-streaming kernel.
+  if (M == 1 && (K % 512) != 0) { return finish(vpq::launch_qmv_rows(hs, a, 0)); }
+  if (batch_ok) { return finish(launch_batch(hs, a, vpq::BatchFormat{})); }
+  // Scales or biases off 16-byte alignment, or a K too deep for the batch kernel's LDS.
   if (vpq::qmv_rows_supports(K, N, M)) { return finish(vpq::launch_qmv_rows(hs, a, 0)); }
   return finish(vpq::launch_qmv_simple(hs, a));
 }
@@ -246,6 +237,10 @@ static int qmv8_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* s
   a.w = w; a.scales = scales; a.biases = biases; a.x = x; a.y = y; a.residual = residual;
   a.K = K; a.N = N; a.M = M; a.y_f32 = y_f32; a.cu_count = g_dev.cu_count;
   a.gate_act = store;
+  const vpq::BatchFormat f{8, 64, false, false};
+  if (M >= 2 && store == 0 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && aligned(biases, 16)) {
+    return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
+  }
   return finish(vpq::launch_qmv_simple8(reinterpret_cast<hipStream_t>(stream), a));
 }
 
@@ -301,6 +296,11 @@ static int rows8_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* 
   a.w = w; a.scales = scales; a.biases = biases; a.x = x; a.y = y;
   a.K = K; a.N = N; a.M = 1; a.y_f32 = false; a.cu_count = g_dev.cu_count;
   a.gate_act = gate_act;
+  const vpq::BatchFormat f{8, 64, false, false};
+  if (!gathered && rows >= 2 && vpq::qmv_batch_supports(K, rows, f) && aligned(scales, 16) && aligned(biases, 16)) {
+    a.M = rows;
+    return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
+  }
   return finish(vpq::launch_qmv_rows8(reinterpret_cast<hipStream_t>(stream), a, rows, gathered ? pair_eid : nullptr, x_div,
                                       n_experts));
 }
@@ -433,6 +433,10 @@ int vpq_qmv_w8g32_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t* s
   vpq::QmvArgs a{};
   a.w = w; a.scales = scales; a.biases = biases; a.x = x; a.y = y; a.residual = residual;
   a.K = K; a.N = N; a.M = M; a.y_f32 = false; a.cu_count = g_dev.cu_count;
+  const vpq::BatchFormat f{8, 32, false, false};
+  if (M >= 2 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && aligned(biases, 16)) {
+    return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
+  }
   return finish(vpq::launch_qmv_simple8(reinterpret_cast<hipStream_t>(stream), a, 32));
 }
 
@@ -701,14 +705,9 @@ static int qmv_f16_common(vpq_stream_t stream, const uint32_t* w, const uint16_t
   if (vpq::qmv_flow_supports(K, N, M) && aligned(scales, 16) && aligned(biases, 16)) {
     return finish(vpq::launch_qmv_flow_f16(reinterpret_cast<hipStream_t>(stream), a));
   }
-  // several rows (K % 512 == 0): the kernels of the bf16 entry on binary16 arithmetic -- two to four rows over an
-  // lm_head-sized pack the streaming kernel, otherwise the ring kernel
-  const bool tuned = M >= 2 && vpq::qmv_mfma_supports(K, N, M) && aligned(scales, 16) && aligned(biases, 16);
-  if (tuned && gate_act == 0 && vpq::qmv_stream_supports(K, N, M) && (double)N * (double)K * 9.0 / 16.0 >= 150e6) {
-    return finish(vpq::launch_qmv_stream(reinterpret_cast<hipStream_t>(stream), a, true));
-  }
-  if (tuned && vpq::qmv_ring_supports(K, N, M)) {
-    return finish(vpq::launch_qmv_ring(reinterpret_cast<hipStream_t>(stream), a, 0, 0, true));
+  const vpq::BatchFormat f{4, 64, true, false};
+  if (M >= 2 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && aligned(biases, 16)) {
+    return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
   }
   return finish(vpq::launch_qmv_simple_f16(reinterpret_cast<hipStream_t>(stream), a));
 }
@@ -834,26 +833,55 @@ int vpq_qmm_dense_route_w4g64_f16(vpq_stream_t stream, const uint32_t* w, const 
   return VPQ_OK;
 }
 
-// Rows up to which the size-based entrances run the GEMV arithmetic in slabs of 16 rows instead of
-// the 256-row GEMM tile: below it the tile kernel has one row of tiles and N/128 workgroups, and
-// its time is its K loop's latency (57 us at 4096->4096 for any M <= 256) against ~10 us per slab.
+// Rows up to which the size-based entrances run the GEMV arithmetic: one launch of the batch kernel, or slabs of 16
+// rows where it does not run.  The 256-row GEMM tile has one row of tiles and N/128 workgroups there, and its time is
+// its K loop's latency (57 us at 4096->4096 for any M <= 256 against 9.5 us at 64 rows).
 constexpr int kSlabPlanMaxRows = 64;
-constexpr int kSlabPlanSplitRows = 32;   // above: the split-K GEMM instead, when the workspace has the room
+constexpr int kSlabPlanSplitRows = 32;   // above, over a narrow N: the split-K GEMM, when the workspace has the room
+
+namespace {
+
+// Whether the batch kernel takes a call of more than 16 rows (what it does not, runs as slabs of 16, which report it).
+bool batch_takes(const void* w, const void* scales, const void* biases, const void* x, const void* y, int K, int N, int M,
+                 const vpq::BatchFormat& f)
+{
+  return w != nullptr && scales != nullptr && (f.scale_only || biases != nullptr) && N > 0 && K > 0 &&
+         vpq::qmv_batch_supports(K, M, f) && aligned(w, 16) && aligned(scales, 16) && aligned(biases, 16) && aligned(x, 16) &&
+         aligned(y, 2);
+}
+
+int batch_call(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales, const uint16_t* biases, const uint16_t* x,
+               uint16_t* y, int K, int N, int M, int activation, const vpq::BatchFormat& f)
+{
+  const int st = ensure_init();
+  if (st != VPQ_OK) { return st; }
+  vpq::QmvArgs a{};
+  a.w = w; a.scales = scales; a.biases = biases; a.x = x; a.y = y;
+  a.K = K; a.N = N; a.M = M; a.cu_count = g_dev.cu_count;
+  a.gate_act = activation;
+  return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
+}
+
+}  // namespace
 
 int vpq_linear_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
                           const uint16_t* biases, const uint16_t* x, uint16_t* y, int K, int N, int M,
                           void* ws, size_t ws_bytes)
 {
   if (M >= 1 && M <= kSlabPlanMaxRows && x != nullptr && y != nullptr && K > 0 && N > 0) {
-    // Three or four slabs: the GEMM with K split over the workgroups is faster where the workspace lets it
-    // split (measured at 64 rows: 40 / 34 / 21 us against 43 / 68 / 31 us for four slabs at
-    // 4096->12288 / 12288->4096 / 4096->4096; two slabs, 23 / 35 / 16 us, stay ahead of it).
+    // 33..64 rows over a narrow N: where the batch kernel's workgroups would fill less than a quarter of the CUs, the
+    // GEMM with K split over the workgroups, if the workspace lets it split (measured at 48 rows, split GEMM / batch
+    // kernel: 20 / 9.5 us at 4096 -> 4096 and 39 / 23 us at 4096 -> 12288, so not on wider ones).
     bool split_gemm = false;
-    if (M > kSlabPlanSplitRows && ws != nullptr && aligned(ws, 256) && (K % 64) == 0 && ensure_init() == VPQ_OK) {
+    if (M > kSlabPlanSplitRows && ws != nullptr && aligned(ws, 256) && (K % 64) == 0 && ensure_init() == VPQ_OK &&
+        (long)((N + 15) / 16) * ((M + 31) / 32) * 4 < (g_dev.cu_count > 0 ? g_dev.cu_count : 256)) {
       const int splits = vpq::qmm_choose_splits(K, N, M, g_dev.cu_count);
       split_gemm = splits > 1 && ws_bytes >= (size_t)splits * (size_t)M * (size_t)N * sizeof(float);
     }
     if (!split_gemm) {
+      if (M > 16 && batch_takes(w, scales, biases, x, y, K, N, M, vpq::BatchFormat{})) {
+        return batch_call(stream, w, scales, biases, x, y, K, N, M, 0, vpq::BatchFormat{});
+      }
       for (int m0 = 0; m0 < M; m0 += 16) {
         const int rows = M - m0 < 16 ? M - m0 : 16;
         const int st = vpq_qmv_w4g64_bf16(stream, w, scales, biases, x + (size_t)m0 * K, y + (size_t)m0 * N, K, N, rows,
@@ -950,6 +978,10 @@ int vpq_linear_gated_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const ui
                                 int activation)
 {
   if (M >= 1 && M <= kSlabPlanMaxRows && x != nullptr && y != nullptr && K > 0 && N > 0) {
+    if (M > 16 && (N & 1) == 0 && (activation == VPQ_GATE_SWIGLU || activation == VPQ_GATE_GEGLU) &&
+        batch_takes(w, scales, biases, x, y, K, N, M, vpq::BatchFormat{})) {
+      return batch_call(stream, w, scales, biases, x, y, K, N, M, activation, vpq::BatchFormat{});
+    }
     for (int m0 = 0; m0 < M; m0 += 16) {
       const int rows = M - m0 < 16 ? M - m0 : 16;
       const int st = vpq_qmv_gated_w4g64_bf16(stream, w, scales, biases, x + (size_t)m0 * K, y + (size_t)m0 * (N / 2), K, N,
@@ -1313,6 +1345,10 @@ int vpq_linear_w8g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t
                           const uint16_t* x, uint16_t* y, int K, int N, int M)
 {
   if (M >= 1 && M <= kSlabPlanMaxRows && x != nullptr && y != nullptr && K > 0 && N > 0) {
+    const vpq::BatchFormat f{8, 64, false, false};
+    if (M > 16 && batch_takes(w, scales, biases, x, y, K, N, M, f)) {
+      return batch_call(stream, w, scales, biases, x, y, K, N, M, 0, f);
+    }
     for (int m0 = 0; m0 < M; m0 += 16) {
       const int rows = M - m0 < 16 ? M - m0 : 16;
       const int st = vpq_qmv_w8g64_bf16(stream, w, scales, biases, x + (size_t)m0 * K, y + (size_t)m0 * N, K, N, rows,
@@ -1377,7 +1413,11 @@ int qmv_g32_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scale
   a.gate_act = gate_act;
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
   if (gelu_mul) { return finish(vpq::launch_qmv_simple_g32(hs, a, scale_only)); }    // the kernel that has this store
-  // up to two rows of x: the row-streaming kernel; more: one wavefront per weight row
+  // up to two rows of x: the row-streaming kernel; more: the batch kernel
+  const vpq::BatchFormat f{4, 32, false, scale_only};
+  if (M > 2 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && (scale_only || aligned(biases, 16))) {
+    return finish(launch_batch(hs, a, f));
+  }
   if (M <= 2) { return finish(vpq::launch_qmv_rows_g32(hs, a, scale_only)); }
   return finish(vpq::launch_qmv_simple_g32(hs, a, scale_only));
 }
@@ -1470,6 +1510,10 @@ int vpq_linear_w4g32_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t
 {
   // K % 64 != 0 (a group-32 pack may have K % 64 == 32) has no fused GEMM: slabs at every M
   if (M >= 1 && (M <= kSlabPlanMaxRows || (K % 64) != 0) && x != nullptr && y != nullptr && K > 0 && N > 0) {
+    const vpq::BatchFormat f{4, 32, false, false};
+    if (M > 16 && batch_takes(w, scales, biases, x, y, K, N, M, f)) {
+      return batch_call(stream, w, scales, biases, x, y, K, N, M, 0, f);
+    }
     for (int m0 = 0; m0 < M; m0 += 16) {
       const int rows = M - m0 < 16 ? M - m0 : 16;
       const int st = vpq_qmv_w4g32_bf16(stream, w, scales, biases, x + (size_t)m0 * K, y + (size_t)m0 * N, K, N, rows,
@@ -1581,19 +1625,21 @@ int vpq_qmv_group_w4g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
 {
   if (w == nullptr || scales == nullptr || biases == nullptr || y == nullptr || N == nullptr) { return VPQ_ERR_NULL_POINTER; }
   if (count < 1 || count > 4) { return VPQ_ERR_BAD_SHAPE; }
-  // The tile kernel's grouped form where its shapes allow, else the row-streaming kernel's (M <= 2).
-  bool mfma_group = vpq::qmv_mfma_supports(K, 1, M);
+  bool batch = vpq::qmv_batch_supports(K, M, vpq::BatchFormat{});
   for (int i = 0; i < count; ++i) {
     int st = check_pack(w[i], scales[i], biases[i], K, N[i]);
     if (st != VPQ_OK) { return st; }
     if (y[i] == nullptr) { return VPQ_ERR_NULL_POINTER; }
     if (!aligned(y[i], 2)) { return VPQ_ERR_MISALIGNED; }
-    mfma_group = mfma_group && aligned(scales[i], 16) && aligned(biases[i], 16);
+    batch = batch && aligned(scales[i], 16) && aligned(biases[i], 16);
   }
   if (x == nullptr) { return VPQ_ERR_NULL_POINTER; }
   if (M < 1 || M > 16) { return VPQ_ERR_BAD_SHAPE; }
   if (!aligned(x, 16)) { return VPQ_ERR_MISALIGNED; }
-  if (!mfma_group && !vpq::qmv_rows_supports(K, 1, M)) {
+  // The kernels of the single call (qmv_common), each in its grouped form.
+  const bool flow = batch && vpq::qmv_flow_supports(K, 1, M);
+  const bool rows = !flow && vpq::qmv_rows_supports(K, 1, M) && (!batch || (M == 1 && (K % 512) != 0));
+  if (!flow && !rows && !batch) {
     for (int i = 0; i < count; ++i) {
       const int st = vpq_qmv_w4g64_bf16(stream, w[i], scales[i], biases[i], x, y[i], K, N[i], M, nullptr, nullptr, 0,
                                         VPQ_QMV_AUTO);
@@ -1608,11 +1654,10 @@ int vpq_qmv_group_w4g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
   vpq::QmvGroup g;
   g.count = count;
   for (int i = 0; i < count; ++i) { g.seg[i] = vpq::QmvSeg{w[i], scales[i], biases[i], y[i], N[i]}; }
-  if (mfma_group && vpq::qmv_flow_supports(K, 1, M)) {
-    return finish(vpq::launch_qmv_flow_group(reinterpret_cast<hipStream_t>(stream), a, g));
-  }
-  if (!mfma_group) { return finish(vpq::launch_qmv_rows_group(reinterpret_cast<hipStream_t>(stream), a, g)); }
-  return finish(vpq::launch_qmv_mfma_group(reinterpret_cast<hipStream_t>(stream), a, g));
+  hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+  if (flow) { return finish(vpq::launch_qmv_flow_group(hs, a, g)); }
+  if (rows) { return finish(vpq::launch_qmv_rows_group(hs, a, g)); }
+  return finish(vpq::launch_qmv_batch(hs, a, g, vpq::BatchFormat{}));
 }
 
 // The fused-QKV GEMV of the format twins (`affine_qmv_qkv_w4g32`, `affine_qmv_qkv_w8g64`,
@@ -1635,7 +1680,12 @@ int vpq_qmv_group_w4g32_bf16(vpq_stream_t stream, int count, const uint32_t* con
     if (!aligned(y[i], 2)) { return VPQ_ERR_MISALIGNED; }
   }
   if (!aligned(x, 16)) { return VPQ_ERR_MISALIGNED; }
-  if (M > 2) {
+  const vpq::BatchFormat f{4, 32, false, scale_only != 0};
+  bool batch = M > 2 && vpq::qmv_batch_supports(K, M, f);
+  for (int i = 0; i < count; ++i) {
+    batch = batch && aligned(scales[i], 16) && (scale_only != 0 || aligned(biases[i], 16));
+  }
+  if (M > 2 && !batch) {
     for (int i = 0; i < count; ++i) {
       const int st = vpq_qmv_w4g32_bf16(stream, w[i], scales[i], scale_only ? nullptr : biases[i], x, y[i], K, N[i], M,
                                         nullptr, scale_only);
@@ -1650,6 +1700,7 @@ int vpq_qmv_group_w4g32_bf16(vpq_stream_t stream, int count, const uint32_t* con
   vpq::QmvGroup g;
   g.count = count;
   for (int i = 0; i < count; ++i) { g.seg[i] = vpq::QmvSeg{w[i], scales[i], scale_only ? nullptr : biases[i], y[i], N[i]}; }
+  if (batch) { return finish(vpq::launch_qmv_batch(reinterpret_cast<hipStream_t>(stream), a, g, f)); }
   return finish(vpq::launch_qmv_rows_group(reinterpret_cast<hipStream_t>(stream), a, g, 32, scale_only != 0));
 }
 
@@ -1659,6 +1710,23 @@ int vpq_qmv_group_w8g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
 {
   if (w == nullptr || scales == nullptr || biases == nullptr || y == nullptr || N == nullptr) { return VPQ_ERR_NULL_POINTER; }
   if (count < 1 || count > 4) { return VPQ_ERR_BAD_SHAPE; }
+  const vpq::BatchFormat f{8, 64, false, false};
+  bool batch = M >= 2 && M <= 16 && x != nullptr && aligned(x, 16) && vpq::qmv_batch_supports(K, M, f);
+  for (int i = 0; i < count && batch; ++i) {
+    batch = check_pack(w[i], scales[i], biases[i], K, N[i]) == VPQ_OK && y[i] != nullptr && aligned(y[i], 2) &&
+            aligned(scales[i], 16) && aligned(biases[i], 16);
+  }
+  if (batch) {
+    const int st = ensure_init();
+    if (st != VPQ_OK) { return st; }
+    vpq::QmvArgs a{};
+    a.x = x; a.K = K; a.M = M; a.y_f32 = false; a.cu_count = g_dev.cu_count;
+    vpq::QmvGroup g;
+    g.count = count;
+    for (int i = 0; i < count; ++i) { g.seg[i] = vpq::QmvSeg{w[i], scales[i], biases[i], y[i], N[i]}; }
+    return finish(vpq::launch_qmv_batch(reinterpret_cast<hipStream_t>(stream), a, g, f));
+  }
+  // one row, or something to report: the separate calls
   for (int i = 0; i < count; ++i) {
     const int st = vpq_qmv_w8g64_bf16(stream, w[i], scales[i], biases[i], x, y[i], K, N[i], M, nullptr);
     if (st != VPQ_OK) { return st; }
@@ -1704,7 +1772,9 @@ int vpq_qmv_group_w4g64_f16(vpq_stream_t stream, int count, const uint32_t* cons
 {
   if (w == nullptr || scales == nullptr || biases == nullptr || y == nullptr || N == nullptr) { return VPQ_ERR_NULL_POINTER; }
   if (count < 1 || count > 4) { return VPQ_ERR_BAD_SHAPE; }
-  bool one_launch = vpq::qmv_flow_supports(K, 1, M);
+  const vpq::BatchFormat f{4, 64, true, false};
+  const bool flow = vpq::qmv_flow_supports(K, 1, M);
+  bool one_launch = flow || (M >= 2 && vpq::qmv_batch_supports(K, M, f));
   for (int i = 0; i < count; ++i) {
     int st = check_pack(w[i], scales[i], biases[i], K, N[i]);
     if (st != VPQ_OK) { return st; }
@@ -1729,7 +1799,8 @@ int vpq_qmv_group_w4g64_f16(vpq_stream_t stream, int count, const uint32_t* cons
   vpq::QmvGroup g;
   g.count = count;
   for (int i = 0; i < count; ++i) { g.seg[i] = vpq::QmvSeg{w[i], scales[i], biases[i], y[i], N[i]}; }
-  return finish(vpq::launch_qmv_flow_group(reinterpret_cast<hipStream_t>(stream), a, g, true));
+  hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+  return finish(flow ? vpq::launch_qmv_flow_group(hs, a, g, true) : vpq::launch_qmv_batch(hs, a, g, f));
 }
 
 int vpq_quantize_w4g64(vpq_stream_t stream, const uint16_t* src, uint32_t* w, uint16_t* scales_f16,

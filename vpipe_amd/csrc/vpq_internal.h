@@ -161,10 +161,6 @@ hipError_t launch_qmv_rows8(hipStream_t st, const QmvArgs& a, int rows, const in
 // Two-slot expert-sorted GEMV over a batched 8-bit pack (a.gate_act != 0: x rows gathered through srow).
 hipError_t launch_qmv_rows8_sorted(hipStream_t st, const QmvArgs& a, const int* tile2e, const int* srow, int tiles,
                                    int n_experts);
-// Returns hipErrorInvalidValue if the shape is outside what the MFMA kernel
-// handles (the caller then falls back to the simple kernel).
-bool qmv_mfma_supports(int K, int N, int M);
-hipError_t launch_qmv_mfma(hipStream_t st, const QmvArgs& a);
 // Up to four projections that share x, K and M in ONE launch (q|k|v, gate|up): a.w/scales/
 // biases/y/N/residual/ws are ignored, the segments give them.
 struct QmvSeg {
@@ -178,7 +174,14 @@ struct QmvGroup {
   int count;
   QmvSeg seg[4];
 };
-hipError_t launch_qmv_mfma_group(hipStream_t st, const QmvArgs& a, const QmvGroup& g);
+// QMV for a batch of rows (vpq_qmv_batch.h): any M >= 1 (built for 2..64), any K that is a multiple of the group, up to
+// four packs that share x; 16-byte aligned packs, scales and biases.  A result's bits depend on K and the format alone.
+struct BatchFormat {
+  int bits = 4, group = 64;
+  bool f16 = false, scale_only = false;    // scale_only: groups of 32, bias = -8 * scale
+};
+bool qmv_batch_supports(int K, int M, const BatchFormat& f);
+hipError_t launch_qmv_batch(hipStream_t st, const QmvArgs& a, const QmvGroup& g, const BatchFormat& f);
 // Streaming kernel for M = 1 (K % 512 == 0, K >= 2048, 16-byte aligned scales / biases): one wavefront per
 // (row set, K part), every load requested up front; also as one launch over up to four packs that share x.
 bool qmv_flow_supports(int K, int N, int M);

@@ -1,0 +1,575 @@
+// QMV for a batch of rows (2..64 rows of x; one row where the one-row kernel does not run), any K that is a multiple
+// of 64 (of 32 for groups of 32): the kernel template of vpq_qmv_batch*.hip.
+//
+// What bounds it: HBM for the pack at few rows, issue of vector instructions from 16 rows on (unpacking costs 14 per
+// 16 x 64 codes, every 16 x 16 outputs 8 multiply-adds per group; the vector ALU is 60-72 % busy at 16..48 rows, the
+// matrix pipe a quarter of that).  Measured (us; before: one-item and ring kernels where K % 512 == 0, one wavefront
+// per weight row elsewhere, slabs of 16 rows above 16): 4096 -> 4096 at 16 / 48 rows 9.3 / 20.4 -> 6.0 / 9.5;
+// 4096 -> 12288 13.3 / 38.6 -> 11.8 / 22.6; 5120 -> 151936 at 8 / 16 rows 102 / 124 -> 97 / 114; 3840 -> 19328 at
+// 4 / 16 rows 51 / 156 -> 13.4 / 16.4.
+//
+// Split.  A workgroup of eight wavefronts owns T tiles of 16 weight rows and up to 32 rows of x.  K is cut into chunks
+// of 128 bytes of codes per row (256 values of 4 bits, 128 of 8 bits); chunk c belongs to wavefront c % 8, which
+// contracts it for all T tiles and all rows of x.  The eight partial results meet in LDS once, at the end, in
+// wavefront order.  So a result depends on K and the format alone -- not on M, N, T or the launch it is part of: a row
+// of x has the same bits in a batch of any size, and a grouped launch the bits of separate ones.
+//
+// Loads.  Codes and x arrive by 128-bit direct-to-LDS loads into one slot per wavefront, laid out so that eight
+// consecutive lanes cover one 128-byte line (an L1 has about 72 requests in flight, so what counts is bytes per
+// request).  A slot is copied to registers (codes, x as MFMA operands, scales, biases), re-requested for the
+// wavefront's next chunk, and only then the copy is contracted: one chunk per wavefront is always in flight and no
+// wait has to be counted.  The 16-byte pieces of a row are XOR-swizzled so that the operand reads do not collide on
+// banks.  The scales and biases of the workgroup's rows are two contiguous blocks of the pack and are brought in whole,
+// before anything else.
+//
+// Math.  4-bit codes become (128 + q) in bf16 (16 + q in binary16) by one v_and_or_b32 per pair, against an
+// accumulator seeded with -128 * sum(x) of the group; 8-bit codes become q itself (exact in bf16).  The result of a
+// group is sum(x q) exactly to fp32 accumulation, then y += scale * sum(x q) + bias * sum(x) in fp32 -- the factored
+// form of gpu-kernels/metal/quant/affine_qmv.metal:151-174.  The weight is never rounded.
+//
+// No inline-assembly VALU instruction may sit near the MFMAs (the compiler's hazard recogniser cannot see what such a
+// statement writes); the asm here is waits only.
+#pragma once
+
+#include <atomic>
+#include <cstddef>
+#include <type_traits>
+
+#include "vpq_device.h"
+#include "vpq_internal.h"
+
+namespace vpq {
+
+constexpr int kBatchWaves = 8;
+
+struct BatchParams {
+  const uint32_t* w;
+  const uint16_t* scales;
+  const uint16_t* biases;
+  const uint16_t* x;
+  int K, N, M;
+  int blocks;           // workgroups along N, all packs together
+  int m_tiles;          // workgroups along M
+  int rows;             // rows of x per workgroup
+  // ---- not preloaded ----
+  void* y;
+  const uint16_t* residual;
+  int gate_act;         // rows are interleaved gate|up; y is [M, N/2] = act(gate) * up (1 SwiGLU, 2 GEGLU)
+  int y_f32;
+  int nseg;             // packs that share x; the first is (w, scales, biases, N, y)
+  QmvSeg seg[3];        // the others
+  int seg_first[3];     // their first workgroup
+};
+static_assert(offsetof(BatchParams, y) == kPreloadWords * 4, "y starts the part that is not preloaded");
+
+// BITS: 4 or 8.  GROUP: 64 or 32.
+template <int T, int MR, int BITS, int GROUP>
+struct BatchShape {
+  static constexpr int CK = 128 * 8 / BITS;                       // values of K per chunk
+  static constexpr int AT = MR == 8 ? 2 : 1;                      // MFMA tiles of 16 rows of x
+  static constexpr int RA = MR == 8 ? 4 : MR;                     // accumulator registers of one
+  // x of a chunk comes in pieces of at most 4 KB: 16 registers of operands per lane, and two workgroups fit a CU
+  static constexpr int XS = MR * 4 * CK * 2 > 4096 ? MR * 4 * CK * 2 / 4096 : 1;
+  static constexpr int SK = CK / XS;                              // values of K per piece
+  static constexpr int XROWB = SK * 2;
+  static constexpr int XLOADS = MR * 4 * XROWB / 1024;            // direct-to-LDS loads per piece
+  static constexpr int CLOADS = T * 2;                            // ... and per chunk of codes
+  static constexpr int SLOT = (CLOADS + XLOADS) * 1024;
+  static constexpr int SG = CK / GROUP;                           // groups per chunk
+  static constexpr int SGW = SG / 2;                              // their scales of one row, in words
+  static constexpr int MPG = GROUP / 32;                          // MFMAs per group
+};
+
+// Whether two workgroups may share a CU: at most 128 registers per lane (the build refuses a spill).
+constexpr bool batch_two_per_cu(int t, int mr, int group) { return !(t == 2 && group == 32 && mr == 8); }
+
+inline int batch_scale_bytes(int tiles, int K, int group) { return (tiles * 16 * (K / group) * 2 + 1023) / 1024 * 1024; }
+
+namespace {
+
+template <bool F16>
+__device__ __forceinline__ floatx4 batch_mfma(u32x4 a, u32x4 b, floatx4 c)
+{
+  if constexpr (F16) {
+    typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
+  } else {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+}
+
+// Eight nibbles of a word -> eight elements 128+q (bf16) or 16+q (binary16), order [k0,k4,k1,k5,k2,k6,k3,k7].
+template <bool F16>
+__device__ __forceinline__ u32x4 batch_nibbles(uint32_t word, uint32_t mask, uint32_t magic)
+{
+  u32x4 v;
+  if constexpr (F16) {
+    v[0] = ((word << 6) & mask) | magic;
+    v[1] = ((word << 2) & mask) | magic;
+    v[2] = ((word >> 2) & mask) | magic;
+    v[3] = ((word >> 6) & mask) | magic;
+  } else {
+    v[0] = (word & mask) | magic;
+    v[1] = ((word >> 4) & mask) | magic;
+    v[2] = ((word >> 8) & mask) | magic;
+    v[3] = ((word >> 12) & mask) | magic;
+  }
+  return v;
+}
+
+// Eight bytes of two words -> eight bf16 values q, in order (0..255 has at most eight significant bits: the upper
+// half of the fp32 value is exact).
+__device__ __forceinline__ u32x4 batch_bytes(uint32_t w0, uint32_t w1)
+{
+  auto pair = [](uint32_t lo, uint32_t hi) {
+    return __builtin_amdgcn_perm(__float_as_uint((float)hi), __float_as_uint((float)lo), 0x07060302u);
+  };
+  u32x4 v;
+  v[0] = pair(w0 & 0xffu, (w0 >> 8) & 0xffu);
+  v[1] = pair((w0 >> 16) & 0xffu, w0 >> 24);
+  v[2] = pair(w1 & 0xffu, (w1 >> 8) & 0xffu);
+  v[3] = pair((w1 >> 16) & 0xffu, w1 >> 24);
+  return v;
+}
+
+// Eight consecutive elements of x -> the order batch_nibbles produces.
+__device__ __forceinline__ u32x4 batch_permute_x(u32x4 d)
+{
+  u32x4 v;
+  v[0] = __builtin_amdgcn_perm(d[2], d[0], 0x05040100u);
+  v[1] = __builtin_amdgcn_perm(d[2], d[0], 0x07060302u);
+  v[2] = __builtin_amdgcn_perm(d[3], d[1], 0x05040100u);
+  v[3] = __builtin_amdgcn_perm(d[3], d[1], 0x07060302u);
+  return v;
+}
+
+__device__ __forceinline__ void batch_to_lds(const void* src, void* lds_dst)
+{
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)lds_dst, 16, 0, 0);
+}
+
+}  // namespace
+
+// MR: accumulator registers per lane and tile, 1 / 2 / 4 / 8 for up to 4 / 8 / 16 / 32 rows of x.  Row m of an MFMA
+// tile of x sits in MFMA row 4*(m%4) + m/4, so that output row m is register m/4 of lane group m%4 and up to four rows
+// need one register.
+template <int T, int MR, int BITS, int GROUP, bool F16, bool SONLY>
+__global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 4 : 2) void qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
+{
+  using S = BatchShape<T, MR, BITS, GROUP>;
+  const BatchParams p = preload_assemble<BatchParams>(VPQ_PRELOADED_WORD_LIST, tail);
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int fr = lane & 15;                 // MFMA row (A) / column (B, D) of this lane
+  const int g = lane >> 4;                  // k sub-block of this lane
+
+  // Workgroups go to the XCDs round robin: the workgroups of one block of weight rows (one per tile of rows of x) are
+  // eight apart, so that the second reads the codes from its XCD's L2.
+  int nb = blockIdx.x, mt = 0;
+  if (p.m_tiles > 1) {
+    const int span = 8 * p.m_tiles;
+    const int q = nb / span, r = nb - q * span;
+    nb = q * 8 + (r & 7);
+    mt = r >> 3;
+  }
+  if (nb >= p.blocks) { return; }
+  const int m0 = mt * p.rows;
+  const int rows = (p.M - m0) < p.rows ? (p.M - m0) : p.rows;
+  if (rows <= 0) { return; }
+
+  const uint32_t* w_ = p.w;
+  const uint16_t* scales_ = p.scales;
+  const uint16_t* biases_ = p.biases;
+  void* y_ = p.y;
+  int N_ = p.N;
+  if (p.nseg > 1 && nb >= p.seg_first[0]) {                 // (constant indexes: a variable one would put p into scratch)
+    int first = p.seg_first[0];
+    QmvSeg seg = p.seg[0];
+    if (p.nseg > 2 && nb >= p.seg_first[1]) { first = p.seg_first[1]; seg = p.seg[1]; }
+    if (p.nseg > 3 && nb >= p.seg_first[2]) { first = p.seg_first[2]; seg = p.seg[2]; }
+    w_ = seg.w; scales_ = seg.scales; biases_ = seg.biases; y_ = seg.y; N_ = seg.N;
+    nb -= first;
+  }
+  const int n0 = nb * (T * 16);
+  const int n_live = (N_ - n0) < T * 16 ? (N_ - n0) : T * 16;
+  const int Kg = p.K / GROUP;
+  const uint32_t row_bytes = (uint32_t)p.K * BITS / 8;
+  const int chunks = (p.K + S::CK - 1) / S::CK;
+
+  uint8_t* slot = lds + wave * S::SLOT;
+  uint8_t* xbuf = slot + S::CLOADS * 1024;
+  uint8_t* sblk = lds + kBatchWaves * S::SLOT;
+  const int sb_bytes = n_live * Kg * 2;
+  const int sb_loads = (sb_bytes + 1023) >> 10;
+  uint8_t* bblk = sblk + sb_loads * 1024;
+
+  // ---- requests ----
+  const uint8_t* wtile = reinterpret_cast<const uint8_t*>(w_) + (size_t)n0 * row_bytes;
+  const uint8_t* xtile = reinterpret_cast<const uint8_t*>(p.x) + (size_t)m0 * p.K * 2;
+  // Load i of a chunk's codes covers rows 8i..8i+7: lane l takes row 8i + l/8, LDS piece l%8 of its 128 bytes; the
+  // swizzle key (row/2)%8 is l/16 with bit 2 flipped in every second load.  A load's offset is one v_xad from two
+  // registers (kept opaque, or the compiler would hold one register per load over the loop); rows past the last one
+  // repeat it.
+  uint32_t code_piece = (uint32_t)(((lane & 7) ^ (lane >> 4)) * 16);
+  uint32_t code_row = __umul24((uint32_t)(lane >> 3), row_bytes);
+  auto request_codes = [&](int c) {
+    const uint8_t* base = wtile + (size_t)c * 128;
+    const int left = (int)row_bytes - c * 128;              // bytes of a row from here on
+    uint32_t rb = row_bytes;
+    asm volatile("" : "+v"(code_piece), "+s"(rb));
+    if (left >= 128 && n_live == T * 16) {
+#pragma unroll
+      for (int i = 0; i < S::CLOADS; ++i) {
+        batch_to_lds(base + ((code_piece ^ ((i & 1) * 64)) + code_row), slot + i * 1024);
+        base += 8 * (size_t)rb;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < S::CLOADS; ++i) {
+        const int row = i * 8 + (lane >> 3);
+        const uint32_t at = code_piece ^ ((i & 1) * 64);
+        batch_to_lds(base + (__umul24((uint32_t)(row < n_live ? row : n_live - 1), rb) + ((int)at < left ? at : 0)),
+                     slot + i * 1024);
+      }
+    }
+  };
+  // Lane l of load i of x takes 16 bytes of row (i*1024 + l*16) / XROWB; swizzle key row % 16
+  // ((row/2) % 8 in rows of 128 bytes).  Rows past the live ones
+  // are not staged: their MFMA rows are computed from what the slot holds and not stored.
+  constexpr int kXPieces = S::XROWB / 16, kRowsPerLoad = 1024 / S::XROWB;
+  const uint32_t x_bytes = (uint32_t)p.K * 2u;
+  uint32_t x_piece = (uint32_t)(((lane & (kXPieces - 1)) ^ (kXPieces >= 16 ? lane / kXPieces : lane >> 4)) * 16);
+  uint32_t x_row = __umul24((uint32_t)(lane / kXPieces), x_bytes);
+  auto request_x = [&](int c, int sub) {
+    const int k0 = c * S::CK + sub * S::SK;
+    const int left = (p.K - k0) * 2;
+    const uint8_t* base = xtile + (size_t)k0 * 2;
+    uint32_t xb = x_bytes;
+    asm volatile("" : "+v"(x_piece), "+s"(xb));
+#pragma unroll
+    for (int i = 0; i < S::XLOADS; ++i) {
+      const uint32_t at = x_piece ^ (uint32_t)(kXPieces >= 16 ? ((i * kRowsPerLoad) & 15) * 16 : (i & 1) * 64);
+      if (left >= S::XROWB && (i + 1) * kRowsPerLoad <= rows) {
+        batch_to_lds(base + (at + x_row), xbuf + i * 1024);
+      } else if (i * kRowsPerLoad < rows) {
+        const int row = lane / kXPieces;
+        const int last = rows - 1 - i * kRowsPerLoad;
+        batch_to_lds(base + (__umul24((uint32_t)(row < last ? row : last), xb) + ((int)at < left ? at : 0)), xbuf + i * 1024);
+      }
+      base += kRowsPerLoad * (size_t)xb;
+    }
+  };
+  // One block of scales (biases): whole 16-byte pieces here, a last partial piece after the wait below.
+  auto request_block = [&](const uint16_t* src, uint8_t* dst) {
+    const int last = (sb_bytes >> 4) - 1;
+    if (last >= 0) {
+      for (int i = wave; i < sb_loads; i += kBatchWaves) {
+        int piece = i * 64 + lane;
+        if (piece > last) { piece = last; }
+        batch_to_lds(reinterpret_cast<const uint8_t*>(src) + (size_t)piece * 16, dst + i * 1024);
+      }
+    }
+  };
+  const uint16_t* sc_src = scales_ + (size_t)n0 * Kg;
+  const uint16_t* bi_src = SONLY ? nullptr : biases_ + (size_t)n0 * Kg;
+  request_block(sc_src, sblk);
+  if (!SONLY) { request_block(bi_src, bblk); }
+  if (wave < chunks) {
+    request_x(wave, 0);
+    request_codes(wave);
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(S::CLOADS) : "memory");
+  } else {
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+  }
+  asm volatile("s_barrier" : : : "memory");                 // (__syncthreads would wait for the chunks as well)
+  if ((sb_bytes & 15) != 0) {                               // the last rows of an N that is not a multiple of 8
+    const int at = (sb_bytes >> 4) * 8 + (int)threadIdx.x;
+    if (at < (sb_bytes >> 1)) {
+      reinterpret_cast<uint16_t*>(sblk)[at] = sc_src[at];
+      if (!SONLY) { reinterpret_cast<uint16_t*>(bblk)[at] = bi_src[at]; }
+    }
+    __syncthreads();
+  }
+
+  uint32_t magic = F16 ? 0x4c004c00u : 0x43004300u;         // 16.0 (binary16) or 128.0 (bf16) in both halves
+  uint32_t mask = F16 ? 0x03c003c0u : 0x000f000fu;
+  asm volatile("" : "+v"(magic));                           // no instruction: only hides the constants
+  asm volatile("" : "+s"(mask));                            // from constant folding
+  // What x is contracted with for sum(x) of a group: the negated offset of the codes (4 bits), or one.
+  u32x4 unit;
+  unit[0] = unit[1] = unit[2] = unit[3] = BITS == 8 ? 0x3f803f80u : F16 ? 0xcc00cc00u : 0xc300c300u;
+  asm volatile("" : "+v"(unit));
+  constexpr float kBiasOverUnit = BITS == 8 ? 1.0f : F16 ? -0.0625f : -0.0078125f;
+
+  float acc[T][S::AT][S::RA];
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+#pragma unroll
+    for (int a = 0; a < S::AT; ++a) {
+#pragma unroll
+      for (int q = 0; q < S::RA; ++q) { acc[t][a][q] = 0.0f; }
+    }
+  }
+
+  // A lane's operands of a chunk.  MFMA j takes from lane (fr, g) the eight values at k = 32j + 8g (groups of 32) or
+  // at k = 64(j/2) + 16g + 8(j%2) (groups of 64): any order inside a group is right as long as codes and x agree.
+  constexpr int kMfmas = S::CK / 32;
+  constexpr int kPieceMfmas = S::SK / 32;
+  uint32_t cw[T][8];
+  u32x4 xq[S::AT][kPieceMfmas];
+  uint32_t sw[T][S::SGW], bw[T][S::SGW];
+
+  auto take_codes = [&](int c) {
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int row = t * 16 + fr;
+      const uint8_t* rp = slot + row * 128;
+      const int key = (row >> 1) & 7;
+      if constexpr (BITS == 4 && GROUP == 64) {
+#pragma unroll
+        for (int grp = 0; grp < 4; ++grp) {
+          const u32x2 v = *reinterpret_cast<const u32x2*>(rp + (((2 * grp + (g >> 1)) ^ key) * 16) + (g & 1) * 8);
+          cw[t][2 * grp] = v[0];
+          cw[t][2 * grp + 1] = v[1];
+        }
+      } else if constexpr (BITS == 4) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) { cw[t][j] = *reinterpret_cast<const uint32_t*>(rp + ((j ^ key) * 16) + g * 4); }
+      } else if constexpr (GROUP == 64) {
+#pragma unroll
+        for (int grp = 0; grp < 2; ++grp) {
+          const u32x4 v = *reinterpret_cast<const u32x4*>(rp + (((4 * grp + g) ^ key) * 16));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) { cw[t][4 * grp + i] = v[i]; }
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const u32x2 v = *reinterpret_cast<const u32x2*>(rp + (((2 * j + (g >> 1)) ^ key) * 16) + (g & 1) * 8);
+          cw[t][2 * j] = v[0];
+          cw[t][2 * j + 1] = v[1];
+        }
+      }
+      // scales and biases of the chunk's groups (past the row's end: neighbours, never used)
+      const int at = row * Kg + c * S::SG;
+      const uint16_t* sp = reinterpret_cast<const uint16_t*>(sblk) + at;
+      const uint16_t* bp = reinterpret_cast<const uint16_t*>(bblk) + at;
+      if ((Kg & (S::SG - 1)) == 0) {
+        __builtin_memcpy(sw[t], __builtin_assume_aligned(sp, S::SG * 2), S::SG * 2);
+        if (!SONLY) { __builtin_memcpy(bw[t], __builtin_assume_aligned(bp, S::SG * 2), S::SG * 2); }
+      } else {
+#pragma unroll
+        for (int i = 0; i < S::SGW; ++i) {
+          sw[t][i] = (uint32_t)sp[2 * i] | ((uint32_t)sp[2 * i + 1] << 16);
+          if (!SONLY) { bw[t][i] = (uint32_t)bp[2 * i] | ((uint32_t)bp[2 * i + 1] << 16); }
+        }
+      }
+    }
+  };
+  auto take_x = [&]() {
+#pragma unroll
+    for (int a = 0; a < S::AT; ++a) {
+      const int m_real = a * 16 + 4 * (fr & 3) + (fr >> 2);
+      const int row = m_real < MR * 4 ? m_real : MR * 4 - 1;   // (MFMA rows past the slot's repeat its last)
+      const uint8_t* rp = xbuf + row * S::XROWB;
+      const int key = kXPieces >= 16 ? row & 15 : (row >> 1) & 7;
+#pragma unroll
+      for (int j = 0; j < kPieceMfmas; ++j) {
+        // (the upper bits of the piece are above the key: an offset instead of another address)
+        const int piece = GROUP == 64 ? 8 * (j >> 1) + 2 * g + (j & 1) : 4 * j + g;
+        xq[a][j] = *reinterpret_cast<const u32x4*>(rp + (((piece & 15) ^ key) * 16) + (j >> 2) * 256);
+      }
+    }
+  };
+
+  // Contracts piece `sub` of the taken chunk; PART: only its first `live` groups are inside K.
+  auto contract_as = [&](auto sub_c, auto part_c, int live) {
+    constexpr int kGroups = S::SK / GROUP, kG0 = decltype(sub_c)::value * kGroups;
+    if constexpr (BITS == 4) {
+#pragma unroll
+      for (int a = 0; a < S::AT; ++a) {
+#pragma unroll
+        for (int j = 0; j < kPieceMfmas; ++j) { xq[a][j] = batch_permute_x(xq[a][j]); }
+      }
+    }
+#pragma unroll
+    for (int grp = 0; grp < kGroups; ++grp) {
+      if (decltype(part_c)::value && grp >= live) { break; }
+      floatx4 xs[S::AT];
+#pragma unroll
+      for (int a = 0; a < S::AT; ++a) {
+        xs[a] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < S::MPG; ++j) { xs[a] = batch_mfma<F16>(xq[a][grp * S::MPG + j], unit, xs[a]); }
+      }
+      const int gc = kG0 + grp;                              // group of the chunk
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        floatx4 s4[S::AT];
+#pragma unroll
+        for (int a = 0; a < S::AT; ++a) { s4[a] = BITS == 4 ? xs[a] : floatx4{0.f, 0.f, 0.f, 0.f}; }
+#pragma unroll
+        for (int j = 0; j < S::MPG; ++j) {
+          const int jc = gc * S::MPG + j;                    // MFMA of the chunk
+          u32x4 b;
+          if constexpr (BITS == 4) {
+            b = batch_nibbles<F16>(cw[t][jc], mask, magic);
+          } else {
+            b = batch_bytes(cw[t][2 * jc], cw[t][2 * jc + 1]);
+          }
+#pragma unroll
+          for (int a = 0; a < S::AT; ++a) { s4[a] = batch_mfma<F16>(xq[a][grp * S::MPG + j], b, s4[a]); }
+        }
+        const float s = (gc & 1) ? elt_hi_to_f32<F16>(sw[t][gc >> 1]) : elt_lo_to_f32<F16>(sw[t][gc >> 1]);
+        float b2;
+        if constexpr (SONLY) {
+          b2 = s * (-8.0f * kBiasOverUnit);
+        } else {
+          b2 = ((gc & 1) ? elt_hi_to_f32<F16>(bw[t][gc >> 1]) : elt_lo_to_f32<F16>(bw[t][gc >> 1])) * kBiasOverUnit;
+        }
+#pragma unroll
+        for (int a = 0; a < S::AT; ++a) {
+#pragma unroll
+          for (int q = 0; q < S::RA; ++q) {
+            acc[t][a][q] = fmaf(s, s4[a][q], acc[t][a][q]);
+            acc[t][a][q] = fmaf(b2, xs[a][q], acc[t][a][q]);
+          }
+        }
+      }
+    }
+  };
+  auto contract = [&](auto sub_c, int live) {
+    if (live >= S::SK / GROUP) {
+      contract_as(sub_c, std::false_type(), live);
+    } else {
+      contract_as(sub_c, std::true_type(), live);
+    }
+  };
+
+  // The next chunk's codes are requested behind the piece of x after which they have the longest time that does not
+  // make a later piece wait for them (loads return in order).
+  constexpr int kCodesAt = S::XS >= 2 ? S::XS - 2 : 0;
+  for (int c = wave; c < chunks; c += kBatchWaves) {
+    const int nxt = c + kBatchWaves;
+    const bool more = nxt < chunks;                          // (a chunk that ends past K is its wavefront's last)
+    auto piece = [&](auto s_c) {
+      constexpr int s = decltype(s_c)::value;
+      const int left = p.K - c * S::CK - s * S::SK;
+      if (s > 0 && left <= 0) { return; }
+      if (s > 0 && s == kCodesAt + 1 && more) {
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(S::CLOADS) : "memory");
+      } else {
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+      }
+      if (s == 0) { take_codes(c); }
+      take_x();
+      asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+      if (s + 1 < S::XS) {
+        if (left > S::SK) { request_x(c, s + 1); }
+      } else if (more) {
+        request_x(nxt, 0);
+      }
+      if (s == kCodesAt && more) { request_codes(nxt); }
+      contract(s_c, left / GROUP);
+    };
+    piece(std::integral_constant<int, 0>());
+    if constexpr (S::XS > 1) { piece(std::integral_constant<int, 1>()); }
+    if constexpr (S::XS > 2) {
+      piece(std::integral_constant<int, 2>());
+      piece(std::integral_constant<int, 3>());
+    }
+  }
+  __syncthreads();
+
+  // ---- the wavefronts' partial results: sums[tile][a][register][wave][lane], over the slots ----
+  float* sums = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+#pragma unroll
+    for (int a = 0; a < S::AT; ++a) {
+#pragma unroll
+      for (int q = 0; q < S::RA; ++q) {
+        sums[(((t * S::AT + a) * S::RA + q) * kBatchWaves + wave) * kWave + lane] = acc[t][a][q];
+      }
+    }
+  }
+  __syncthreads();
+  const int live_waves = chunks < kBatchWaves ? chunks : kBatchWaves;
+  constexpr int kOuts = T * S::AT * S::RA * kWave;
+  for (int o_idx = threadIdx.x; o_idx < kOuts; o_idx += kBatchWaves * kWave) {
+    const int l = o_idx & 63;
+    const int r = o_idx >> 6;                                // (t * AT + a) * RA + q
+    const float* sp = sums + (size_t)r * kBatchWaves * kWave + l;
+    float total = 0.0f;
+    for (int wv = 0; wv < live_waves; ++wv) { total += sp[wv * kWave]; }
+    const int q = r % S::RA;
+    const int a = (r / S::RA) % S::AT;
+    const int t = r / (S::RA * S::AT);
+    const int m_loc = a * 16 + 4 * q + (l >> 4);
+    const int n_loc = t * 16 + (l & 15);
+    const bool ok = m_loc < rows && n_loc < n_live;
+    const int m = m0 + m_loc, n = n0 + n_loc;
+    if (p.gate_act) {
+      // Lanes 2j and 2j+1 hold the gate and the up sum of one feature (N is even).
+      const float up = from_neighbour_lane(total);
+      if (ok && (l & 1) == 0) {
+        const float v = gated_f32(p.gate_act, total, up);
+        const size_t o = (size_t)m * (N_ >> 1) + (n >> 1);
+        if (p.y_f32) {
+          reinterpret_cast<float*>(y_)[o] = v;
+        } else {
+          reinterpret_cast<uint16_t*>(y_)[o] = (uint16_t)f32_to_elt_bits<F16>(v);
+        }
+      }
+    } else if (ok) {
+      const size_t o = (size_t)m * N_ + n;
+      if (p.y_f32) {
+        reinterpret_cast<float*>(y_)[o] = total;
+      } else {
+        uint32_t v = f32_to_elt_bits<F16>(total);
+        if (p.residual != nullptr) {
+          v = f32_to_elt_bits<F16>(elt_bits_to_f32<F16>(v) + elt_bits_to_f32<F16>(p.residual[o]));
+        }
+        reinterpret_cast<uint16_t*>(y_)[o] = (uint16_t)v;
+      }
+    }
+  }
+}
+
+constexpr int kLdsOfCu = 160 * 1024;
+
+// One instantiation's launch; the attribute is set once per kernel, whichever thread comes first (two may both set it,
+// which is harmless; neither launches before its own call has returned).
+template <int T, int MR, int BITS, int GROUP, bool F16, bool SONLY>
+hipError_t batch_launch_one(hipStream_t st, const BatchParams& p, size_t lds_bytes, int grid)
+{
+  static std::atomic<bool> ready{false};
+  auto kern = qmv_batch_kernel<T, MR, BITS, GROUP, F16, SONLY>;
+  if (!ready.load(std::memory_order_acquire)) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, kLdsOfCu);
+    if (e != hipSuccess) { return e; }
+    ready.store(true, std::memory_order_release);
+  }
+  return launch_preloaded(kern, dim3((unsigned)grid), dim3(kBatchWaves * kWave), lds_bytes, st, p);
+}
+
+template <int BITS, int GROUP, bool F16, bool SONLY = false>
+hipError_t batch_launch(hipStream_t st, const BatchParams& p, int tiles, int mr, size_t lds_bytes, int grid)
+{
+#define VPQ_BATCH(T_, MR_) \
+  if (tiles == T_ && mr == MR_) { return batch_launch_one<T_, MR_, BITS, GROUP, F16, SONLY>(st, p, lds_bytes, grid); }
+  VPQ_BATCH(1, 1) VPQ_BATCH(1, 2) VPQ_BATCH(1, 4) VPQ_BATCH(1, 8)
+  VPQ_BATCH(2, 1) VPQ_BATCH(2, 2) VPQ_BATCH(2, 4) VPQ_BATCH(2, 8)
+#undef VPQ_BATCH
+  return hipErrorInvalidValue;
+}
+
+// The instantiations of the other formats (vpq_qmv_batch_twins.hip).
+hipError_t launch_qmv_batch_twin(hipStream_t st, const BatchParams& p, int tiles, int mr, size_t lds_bytes, int grid,
+                                 const BatchFormat& f);
+
+}  // namespace vpq
