@@ -186,10 +186,10 @@ int vpq_qmm_tiled_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint1
                              uint16_t* lora_t_ws, int tile_n);
 
 /* Split-K form of the fused kernel for GEMMs with few output tiles (M of a few
- * hundred rows, or a narrow N, over a long K), where one workgroup per 256 x 128
+ * hundred rows, or a narrow N, over a long K), where one workgroup per output
  * tile leaves most of the chip idle and each walks a long serial K loop: `splits`
- * (2..16; 0 = chosen so that about one workgroup per CU results, at least 512 of K
- * each; 1 = none) shares of K run as separate workgroups into fp32 planes
+ * (2..16; 0 = the count that a model of the kernel's measured times says is least,
+ * at least 256 of K each; 1 = none) shares of K run as separate workgroups into fp32 planes
  * [splits][M][N] in `ws`, and a fold adds the planes in order and rounds once.  The
  * model is the reference's deep-K split (generative-models/shared/mma-splitk.h:
  * 30-52, 66-140: f32 planes + fold, chosen by chunk width); results differ from the

@@ -1,0 +1,79 @@
+"""The GEMM with 128-row weight tiles (vpq_qmm_mid.hip) where it can go wrong: K that ends inside a chunk of codes or
+has an odd number of groups, fewer steps of K than x stages, N and M that end inside a tile, each count of rows of x per
+workgroup, split shares of uneven length -- against the oracle and, bit for bit, the 256 x 128 tile kernel."""
+import numpy as np
+import pytest
+import torch
+
+from tests import parity
+from tests.test_oracle_pins import f16_pack
+from vpipe_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+# (K, N, M): one step; two; an odd group count and a last chunk of one step; 96- and 128-row tiles with remainders
+SHAPES = [(64, 130, 65), (128, 2, 17), (320, 258, 33), (1088, 262, 97), (3840, 200, 129), (2112, 1030, 300)]
+
+
+@pytest.mark.parametrize("K,N,M", SHAPES)
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("fmt", ["w4g64", "w4g32", "w8g64", "f16"])
+def test_qmm_mid_edges(vpq, oracle, dev, D, fmt, act, K, N, M):
+    seed = K + 3 * N + M
+    ms = np.unique(np.r_[0:3, M // 2, M - 3:M])
+    if fmt == "f16":
+        w, s, b = f16_pack(N, K, seed)
+        x = np.random.default_rng(seed).standard_normal((M, K)).astype(np.float16).view(np.uint16)
+        args = (D.u32(w, dev), *(torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).to(dev).view(torch.float16) for a in (s, b, x)))
+        y64, yb = oracle.matmul_f16(w, s, b, x[ms], K, N, len(ms), rounded=True)
+        run = vpq.qmm_w4g64_f16
+    else:
+        make = {"w4g64": synth.make_weight, "w4g32": synth.make_weight_g32, "w8g64": synth.make_weight8}[fmt]
+        w, s, b = make(N, K, seed)
+        x = synth.make_act(M, K, seed + 1)
+        args = (D.u32(w, dev), D.bf16(s, dev), D.bf16(b, dev), D.bf16(x, dev))
+        if fmt == "w8g64":
+            y64, yb = oracle.matmul8(w, s, b, x[ms], K, N, len(ms), rounded=True)
+        elif fmt == "w4g32":
+            y64 = synth.bf16_bits_to_f32(x[ms]).astype(np.float64) @ synth.bf16_bits_to_f32(oracle.dequant_g32_bf16(w, s, b, K, N)).astype(np.float64).T
+            yb = None
+        else:
+            y64, yb = oracle.qmm(w, s, b, x[ms], K, N, len(ms))
+        run = {"w4g64": vpq.qmm_w4g64, "w4g32": vpq.qmm_w4g32, "w8g64": vpq.qmm_w8g64}[fmt]
+    dt = args[3].dtype
+    out = parity.Guarded((M, N // 2 if act else N), dt, dev)
+    if act and fmt == "w4g64":
+        vpq.qmm_swiglu_w4g64(*args, K, N, M, out=out.view)
+    else:
+        run(*args, K, N, M, out=out.view, **({"activation": 1} if act else {}))
+    torch.cuda.synchronize()
+    out.assert_intact()
+    if act:
+        # the store of the same sums: silu(gate) * up of the plain result's fp32 sums, to the element's rounding
+        g, u = torch.from_numpy(np.asarray(y64)).double()[:, 0::2], torch.from_numpy(np.asarray(y64)).double()[:, 1::2]
+        want = g / (1 + torch.exp(-g)) * u
+        got = out.view.cpu()[torch.from_numpy(ms)].double()
+        # sums differ by fp32 accumulation over K, the result by its own rounding (2^-9; 2^-11 in binary16)
+        assert ((got - want).norm() / want.norm()).item() < 2.0 ** -8
+        return
+    got = out.view[torch.from_numpy(ms).to(dev)]
+    if fmt == "f16":
+        # binary16 rounding (2^-11 relative) and fp32 accumulation over K
+        y = torch.from_numpy(np.asarray(y64)).reshape(len(ms), N).double()
+        assert ((got.cpu().double() - y).norm() / y.norm()).item() < 2.0 ** -10
+        return
+    parity.check_bf16(D.bits(got), y64, yb)
+    assert torch.equal(out.view, run(*args, K, N, M, tile_n=128))
+
+
+@pytest.mark.parametrize("K,N,M,splits", [(1088, 131, 97, 3), (1088, 132, 129, 2), (640, 260, 48, 5)])
+def test_qmm_mid_uneven_shares(vpq, oracle, dev, D, K, N, M, splits):
+    # shares that end inside a chunk of codes; a count of outputs that is and is not a multiple of four in the fold
+    w, s, b = synth.make_weight(N, K, 40 + M)
+    x = synth.make_act(M, K, 41 + M)
+    y64, yb = oracle.qmm(w, s, b, x, K, N, M)
+    out = parity.Guarded((M, N), torch.bfloat16, dev)
+    vpq.qmm_splitk_w4g64(D.u32(w, dev), D.bf16(s, dev), D.bf16(b, dev), D.bf16(x, dev), K, N, M, splits=splits, out=out.view)
+    torch.cuda.synchronize()
+    out.assert_intact()
+    parity.check_bf16(D.bits(out.view), y64, yb)

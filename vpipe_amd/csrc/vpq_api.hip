@@ -513,6 +513,16 @@ int vpq_lora_a_bf16(vpq_stream_t stream, const uint16_t* x, const uint16_t* lora
 
 namespace {
 
+// The fused GEMM by size, for every format: the three kernels give the same bits.  The large-tile kernel from one round
+// of its tiles on (1.02-1.16 against 0.83-0.91 PFLOP/s of the 256 x 128 tiles at M = 16320, 0.98 against 0.78 at
+// 4096 -> 12288 and 0.94 against 0.91 at 12288 -> 4096 with M = 2048), unless the 128-row kernel's tiles fit M better.
+int gemm_by_size(hipStream_t hs, const vpq::GemmArgs& g)
+{
+  const vpq::GemmKernel k = vpq::qmm_choose(g);
+  if (k == vpq::GemmKernel::kBig) { return finish(vpq::launch_qmm_big(hs, g, 0)); }
+  return finish(k == vpq::GemmKernel::kMid ? vpq::launch_qmm_mid(hs, g) : vpq::launch_qmm_tile(hs, g));
+}
+
 // tile: 0 = by size, 128 = the 256 x 128 tile kernel, 192 / 256 = the large-tile kernel at that width,
 // -128 = the large-tile kernel at width 128
 int qmm_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
@@ -550,15 +560,7 @@ int qmm_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
     if (!vpq::qmm_big_supports(g)) { return VPQ_ERR_BAD_SHAPE; }
     return finish(vpq::launch_qmm_big(hs, g, tile < 0 ? -tile : tile));
   }
-  // The large-tile kernel once its tiles fill the CUs at least once (measured: 1.02-1.16 against
-  // 0.83-0.91 PFLOP/s at M = 16320, 0.98 against 0.78 at 4096 -> 12288 and 0.94 against 0.91 at
-  // 12288 -> 4096 with M = 2048); with fewer tiles the two are equal and the tile kernel has the
-  // split-K form beside it.
-  if (tile == 0 && vpq::qmm_big_supports(g)) {
-    const int bn = vpq::qmm_big_tile_n(N, M, g_dev.cu_count);
-    const long tiles = (long)((M + 255) / 256) * (long)((N + bn - 1) / bn);
-    if (tiles >= (long)(g_dev.cu_count > 0 ? g_dev.cu_count : 256)) { return finish(vpq::launch_qmm_big(hs, g, bn)); }
-  }
+  if (tile == 0) { return gemm_by_size(hs, g); }
   return finish(vpq::launch_qmm_tile(hs, g));
 }
 
@@ -613,9 +615,9 @@ int vpq_qmm_splitk_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint
   g.K = K; g.N = N; g.M = M;
   g.cu_count = g_dev.cu_count;
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
-  if (splits <= 1) { return finish(vpq::launch_qmm_tile(hs, g)); }
+  if (splits <= 1) { return gemm_by_size(hs, g); }
   if (ws == nullptr || ws_bytes < (size_t)splits * (size_t)M * (size_t)N * sizeof(float)) { return VPQ_ERR_WORKSPACE; }
-  return finish(vpq::launch_qmm_tile_splitk(hs, g, splits, static_cast<float*>(ws)));
+  return finish(vpq::launch_qmm_splitk(hs, g, splits, static_cast<float*>(ws)));
 }
 
 int vpq_qmm_dense_route_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
@@ -770,12 +772,7 @@ int qmm_f16_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scale
   g.cu_count = g_dev.cu_count;
   g.gate_act = activation;
   g.f16 = true;
-  if (vpq::qmm_big_supports(g)) {
-    const int bn = vpq::qmm_big_tile_n(N, M, g_dev.cu_count);
-    const long tiles = (long)((M + 255) / 256) * (long)((N + bn - 1) / bn);
-    if (tiles >= (long)(g_dev.cu_count > 0 ? g_dev.cu_count : 256)) { return finish(vpq::launch_qmm_big(hs, g, bn)); }
-  }
-  return finish(vpq::launch_qmm_tile(hs, g));
+  return gemm_by_size(hs, g);
 }
 
 }  // namespace
@@ -962,15 +959,7 @@ int vpq_qmm_gated_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint1
   g.gate_act = activation;
   g.out_stride = out_stride;
   g.out_off = out_off;
-  // as vpq_qmm_w4g64_bf16: the large-tile kernel once its tiles fill the CUs (bit-identical results)
-  if (vpq::qmm_big_supports(g)) {
-    const int bn = vpq::qmm_big_tile_n(N, M, g_dev.cu_count);
-    const long tiles = (long)((M + 255) / 256) * (long)((N + bn - 1) / bn);
-    if (tiles >= (long)(g_dev.cu_count > 0 ? g_dev.cu_count : 256)) {
-      return finish(vpq::launch_qmm_big(reinterpret_cast<hipStream_t>(stream), g, bn));
-    }
-  }
-  return finish(vpq::launch_qmm_tile(reinterpret_cast<hipStream_t>(stream), g));
+  return gemm_by_size(reinterpret_cast<hipStream_t>(stream), g);
 }
 
 int vpq_linear_gated_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
@@ -1277,11 +1266,7 @@ int twin_gemm_launch(vpq_stream_t stream, const vpq::GemmArgs& g, int tile)
     if (!vpq::qmm_big_supports(g) || (tile == 256 && g.bits == 8) || (tile == 192 && g.group == 32)) { return VPQ_ERR_BAD_SHAPE; }
     return finish(vpq::launch_qmm_big(hs, g, tile < 0 ? -tile : tile));
   }
-  if (tile == 0 && vpq::qmm_big_supports(g)) {
-    const int bn = vpq::qmm_big_tile_n(g.N, g.M, g_dev.cu_count, g.bits == 8 ? 192 : 256, g.group != 32);
-    const long tiles = (long)((g.M + 255) / 256) * (long)((g.N + bn - 1) / bn);
-    if (tiles >= (long)(g_dev.cu_count > 0 ? g_dev.cu_count : 256)) { return finish(vpq::launch_qmm_big(hs, g, bn)); }
-  }
+  if (tile == 0) { return gemm_by_size(hs, g); }
   return finish(vpq::launch_qmm_tile(hs, g));
 }
 

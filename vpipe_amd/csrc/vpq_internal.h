@@ -227,6 +227,7 @@ hipError_t launch_lora_a(hipStream_t st, const uint16_t* x, const uint16_t* a, u
                          float alpha, bool f16 = false);
 // 256x128-tile quantized GEMM (+ fused LoRA second factor); a.w must be non-null.
 hipError_t launch_qmm_tile(hipStream_t st, const GemmArgs& a);
+hipError_t launch_qmm_tile_planes(hipStream_t st, const GemmArgs& a, int splits, float* plane);
 // Grouped (expert-sorted) form of the tile kernel at 128 rows per block: a.w/scales/biases are the
 // batched pack [E, N, ...], a.M the padded slot count (a multiple of kGroupedBlockRows); see TileParams.
 constexpr int kGroupedBlockRows = 128;
@@ -247,12 +248,17 @@ hipError_t launch_qmm_grouped(hipStream_t st, const GemmArgs& a, const GroupedAr
 bool qmm_big_supports(const GemmArgs& a);
 int qmm_big_tile_n(int N, int M, int cu_count, int max_width = 256, bool with_192 = true);
 hipError_t launch_qmm_big(hipStream_t st, const GemmArgs& a, int tile_n);
-// Split-K form of the same kernel (no adapter, no gated store): `splits` shares of the K steps,
-// fp32 planes [splits][M][N] in `plane`, then a fold.  qmm_choose_splits() returns 1 where the tiles
-// alone fill the chip.
+// 128 weight rows x {64, 96, 128} rows of x per workgroup, for GEMMs that have few 256-row tiles; every format, gated
+// stores, no adapter; the bits of the other two kernels.
+hipError_t launch_qmm_mid(hipStream_t st, const GemmArgs& a);
+// Which of the three takes least for this call (a rule on sizes, alignment and format).
+enum class GemmKernel { kTile, kBig, kMid };
+GemmKernel qmm_choose(const GemmArgs& a);
+// Split-K (no adapter, no gated store, bf16): `splits` shares of the K steps on that kernel or the 256 x 128 one, fp32
+// planes [splits][M][N] in `plane`, then a fold.  qmm_choose_splits() returns 1 where that does not pay.
 int qmm_choose_splits(int K, int N, int M, int cu_count);
 size_t qmm_splitk_workspace_bytes(int K, int N, int M, int cu_count);
-hipError_t launch_qmm_tile_splitk(hipStream_t st, const GemmArgs& a, int splits, float* plane);
+hipError_t launch_qmm_splitk(hipStream_t st, const GemmArgs& a, int splits, float* plane);
 // y[M,N] = x[M,K] . b[N,K]^T on the large-tile kernel with dense 2-byte weights (bf16, or binary16 with f16;
 // fp32 accumulate, one rounding).  0, or -2 (shape outside the kernel / launch failed) with *why set.
 bool dense_gemm_supports(int M, int N, int K);

@@ -1,0 +1,491 @@
+// QMM for GEMMs whose 256-row tiles would leave CUs idle (a prompt of some hundred rows, the narrow projections of a
+// longer one): y[M,N] = x[M,K] . bf16(W)^T on v_mfma_f32_32x32x16, K in ascending order, fp32 accumulators, one
+// rounding -- the arithmetic and the bits of the 256 x 128 tile kernel.
+//
+// Split.  A workgroup of four wavefronts owns 32 MT rows of x and 128 weight rows; wavefront i holds the weight rows
+// [32 i, 32 (i + 1)) against all rows of x.  So every weight is unpacked once per workgroup, by the wavefront
+// that multiplies it, straight into the MFMA's operand registers: no weight tile in LDS, no producer role, and the
+// only thing the wavefronts share is the x tile.  Two workgroups fit a CU and fill each other's waits.  Unpacking costs
+// about 2.9 vector instructions a weight, so a tile shorter than 96 rows would be bound by it.
+//
+// Loads.  x comes through three LDS stages of 64 values of K (direct-to-LDS, 8 rows x 128 bytes each), requested two
+// steps ahead; one barrier a step.  Codes come 128 bytes per weight row at a time (four steps of 4 bits, two of 8), whole
+// lines into a slot of the wavefront's own, which is copied to registers at the start of those steps and requested
+// again at once.  Scales and biases of those steps are one load of each per lane, a chunk ahead.
+//
+// With K split over workgroups (few tiles over a long K) a share leaves fp32 planes that splitk_fold adds in order.
+//
+// What bounds it: a step's chain (barrier, operand reads, unpacking, MFMAs) for a workgroup alone on its CU, 0.57 us at
+// 96 rows; several to a CU, the LDS reads of x (4 KB a row fragment and wavefront) and the MFMAs together.  Two 32-row
+// fragments of weights a wavefront halve the LDS reads but leave half the workgroups: slower up to 1024 rows (4096 -> 24576
+// at 128 / 333 rows 73 / 114 us against 52 / 99).  Pinning one MFMA between every seven vector instructions: no gain.
+// Measured (us, before: the 256 x 128 tiles, split over K where a workspace allows, and the large tile; after):
+// 4096 -> 24576 gated at 80 / 128 / 333 rows 78 / 78 / 104 -> 44 / 51 / 92; 4096 -> 1024 at 333 rows 22 -> 15;
+// 12288 -> 4096 at 80 / 333 rows 38 / 69 -> 26 / 62; without a workspace 4096 -> 4096 at 80..333 rows 57 -> 37.
+#include <type_traits>
+
+#include "vpq_device.h"
+#include "vpq_internal.h"
+#include "vpq_tile_dequant.h"
+
+namespace vpq {
+
+namespace {
+
+constexpr int kMidWaves = 4;
+constexpr int kMidStages = 3;
+constexpr int kMidTileN = 32 * kMidWaves;     // weight rows per workgroup
+constexpr int kMidRowB = 128;                 // bytes of an LDS row: 64 elements of x, or a chunk of codes
+
+struct MidParams {
+  const uint32_t* w;
+  const uint16_t* scales;
+  const uint16_t* biases;
+  const uint16_t* x;
+  uint16_t* y;
+  int K, N, M;
+  int tiles_m, tiles_n;
+  int gate_act, out_stride, out_off;          // as in the tile kernel
+  int ksplit, steps_per_split;
+  float* plane;                               // ksplit > 1: [ksplit][M][N]
+};
+
+__device__ __forceinline__ uint32_t mid_lds(const uint8_t* q)
+{
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)q;
+}
+
+// 16 bytes per lane, global -> LDS at lds_dst + 16 * lane.  Written out by hand: the compiler orders every later LDS read
+// after a direct-to-LDS load that it knows about, whatever that load fills.  The LDS base travels in M0, bound as an
+// operand (the s_nop is the wait state between that write and the load).
+__device__ __forceinline__ void mid_dma16(uint32_t lds_dst, const uint8_t* base, uint32_t lane_off)
+{
+  const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds_dst);
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(base), "{m0}"(m0v) : "memory");
+}
+
+template <bool F16>
+__device__ __forceinline__ floatx16 mid_mfma(u32x4 a, u32x4 b, floatx16 c)
+{
+  if constexpr (F16) {
+    typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
+  } else {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+}
+
+}  // namespace
+
+template <int MT, int BITS, int GROUP, bool F16>
+__global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidParams p)
+{
+  constexpr int BM = 32 * MT, BN = kMidTileN;
+  constexpr int SPC = 16 / BITS;                    // K steps of 64 per chunk of codes: 4 or 2
+  constexpr int SG = SPC * 64 / GROUP;              // groups per chunk
+  constexpr int SGW = SG / 2;                       // ... in words of two
+  constexpr int XL = MT;                            // loads of x per wavefront and step
+  constexpr int CL = 4;                             // loads of codes per wavefront and chunk
+  constexpr int kXStage = BM * kMidRowB;
+  constexpr int kSlot = 32 * kMidRowB;
+  constexpr int kWords = kMidRowB / 4 / 2;          // words of a weight row's chunk that one lane unpacks
+  __shared__ __attribute__((aligned(16))) uint8_t x_lds[kMidStages * kXStage];
+  __shared__ __attribute__((aligned(16))) uint8_t c_lds[kMidWaves * kSlot];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int frow = lane & 31;                       // row of a 32-row operand
+  const int fkh = lane >> 5;                        // which 8 of its 16 k
+
+  // Workgroups go to the XCDs round robin: those that share a weight tile (one per tile of rows of x) are eight apart,
+  // so that the pack is read from HBM once.
+  const int units = p.tiles_n * p.ksplit;
+  const int span = 8 * p.tiles_m;
+  const int uq = (int)blockIdx.x / span, ur = (int)blockIdx.x - uq * span;
+  const int unit = uq * 8 + (ur & 7);
+  if (unit >= units) { return; }
+  const int ks = unit / p.tiles_n;
+  const int m0 = (ur >> 3) * BM, n0 = (unit - ks * p.tiles_n) * BN;
+  const int k_first = ks * p.steps_per_split;
+  const int k_left = p.K / 64 - k_first;
+  const int steps = k_left < p.steps_per_split ? k_left : p.steps_per_split;
+  const int chunks = (steps + SPC - 1) / SPC;
+
+  // ---- addresses ----
+  const uint8_t* xblk = reinterpret_cast<const uint8_t*>(p.x) + (size_t)m0 * p.K * 2 + (size_t)k_first * 128;
+  uint32_t x_off[XL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int row = (wave * XL + i) * 8 + (lane >> 3);
+    const int rg = m0 + row < p.M ? row : p.M - 1 - m0;
+    x_off[i] = (uint32_t)rg * (uint32_t)p.K * 2u + (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) * 16);
+  }
+  const int nw = n0 + wave * 32;                    // this wavefront's first weight row
+  const uint32_t row_bytes = (uint32_t)p.K * BITS / 8;
+  const int row_left = (int)row_bytes - k_first * (8 * BITS);   // bytes of a row from this share's start on
+  const uint8_t* cblk = reinterpret_cast<const uint8_t*>(p.w) + (size_t)(nw < p.N ? nw : p.N - 1) * row_bytes +
+                        (size_t)k_first * (8 * BITS);
+  const int w_last = nw < p.N ? p.N - 1 - nw : 0;   // rows past the last repeat it
+  uint32_t c_row[CL];
+#pragma unroll
+  for (int i = 0; i < CL; ++i) {
+    const int row = i * 8 + (lane >> 3);
+    c_row[i] = (uint32_t)(row < w_last ? row : w_last) * row_bytes;
+  }
+  const uint32_t c_piece = (uint32_t)(((lane & 7) ^ (lane >> 4)) * 16);   // key (row >> 1) & 7, bit 2 by the load
+  const int Kg = p.K / GROUP;
+  const size_t at = (size_t)((nw < p.N ? nw : p.N - 1) + (frow < w_last ? frow : w_last)) * Kg;
+  const uint16_t* srow = p.scales + at;
+  const uint16_t* brow = p.biases + at;
+  uint8_t* slot = c_lds + wave * kSlot;
+
+  auto request_x = [&](int step, int stage) {
+    const uint8_t* src = xblk + (size_t)step * 128;
+    const uint32_t dst = mid_lds(x_lds) + (uint32_t)(stage * kXStage + wave * (XL * 1024));
+#pragma unroll
+    for (int i = 0; i < XL; ++i) { mid_dma16(dst + i * 1024, src, x_off[i]); }
+  };
+  auto request_codes = [&](int c) {
+    const uint8_t* src = cblk + (size_t)c * 128;
+    const int left = row_left - c * 128;            // a piece past the row's end reads the chunk's first, unused
+    const uint32_t dst = mid_lds(slot);
+#pragma unroll
+    for (int i = 0; i < CL; ++i) {
+      const uint32_t at = c_piece ^ (uint32_t)((i & 1) * 64);
+      mid_dma16(dst + i * 1024, src, c_row[i] + ((int)at < left ? at : 0u));
+    }
+  };
+  uint32_t sn[SGW], bn[SGW];                        // scales and biases of the coming chunk
+  auto request_scales = [&](int c) {
+    const int g0 = k_first * (64 / GROUP) + c * SG;
+    if (g0 + SG <= Kg) {
+      __builtin_memcpy(sn, srow + g0, SG * 2);
+      __builtin_memcpy(bn, brow + g0, SG * 2);
+    } else {
+#pragma unroll
+      for (int i = 0; i < SGW; ++i) {
+        const int a = g0 + 2 * i < Kg ? g0 + 2 * i : Kg - 1, b = g0 + 2 * i + 1 < Kg ? g0 + 2 * i + 1 : Kg - 1;
+        sn[i] = (uint32_t)srow[a] | ((uint32_t)srow[b] << 16);
+        bn[i] = (uint32_t)brow[a] | ((uint32_t)brow[b] << 16);
+      }
+    }
+  };
+
+  floatx16 acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) { acc[i][e] = 0.0f; }
+  }
+  uint32_t cw[kWords], sc[SGW], bi[SGW];
+
+  const uint32_t f_sw = (uint32_t)((frow >> 1) & 7);
+  auto take_codes = [&]() {
+    const uint8_t* rp = slot + frow * kMidRowB;
+    if constexpr (BITS == 4) {
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {                // MFMA q of the chunk: word 2q + fkh
+        cw[q] = *reinterpret_cast<const uint32_t*>(rp + (((uint32_t)(q >> 1) ^ f_sw) * 16) + (q & 1) * 8 + fkh * 4);
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {                 // MFMA q: words 4q + 2 fkh, + 1
+        const u32x2 v = *reinterpret_cast<const u32x2*>(rp + (((uint32_t)q ^ f_sw) * 16) + fkh * 8);
+        cw[2 * q] = v[0];
+        cw[2 * q + 1] = v[1];
+      }
+    }
+  };
+  // Step `sub` of the taken chunk against the x tile of `stage`.
+  auto contract = [&](auto sub_c, int stage) {
+    constexpr int sub = decltype(sub_c)::value;
+    const uint8_t* xb = x_lds + stage * kXStage + frow * kMidRowB;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      u32x4 xf[MT];
+      const uint32_t c = ((uint32_t)(2 * k + fkh) ^ f_sw) * 16;
+#pragma unroll
+      for (int i = 0; i < MT; ++i) { xf[i] = *reinterpret_cast<const u32x4*>(xb + i * (32 * kMidRowB) + c); }
+      constexpr int q0 = sub * 4;
+      const int q = q0 + k;
+      const int g = q * 16 / GROUP;                 // group of the chunk
+      const float s = (g & 1) ? elt_hi_to_f32<F16>(sc[g >> 1]) : elt_lo_to_f32<F16>(sc[g >> 1]);
+      const float b = (g & 1) ? elt_hi_to_f32<F16>(bi[g >> 1]) : elt_lo_to_f32<F16>(bi[g >> 1]);
+      uint4 wv;
+      if constexpr (BITS == 4) {
+        wv = dequant_word<F16>(cw[q], s, b);
+      } else {
+        wv = dequant_bytes(cw[2 * q], cw[2 * q + 1], s, b);
+      }
+      const u32x4 wf = {wv.x, wv.y, wv.z, wv.w};
+#pragma unroll
+      for (int i = 0; i < MT; ++i) { acc[i] = mid_mfma<F16>(wf, xf[i], acc[i]); }
+    }
+  };
+
+  // ---- K loop ----
+  // Loads of step t, in order: x(t + 2) [XL], and at a chunk's first step the next chunk's codes [CL] and scales.  The
+  // first step of a chunk waits for everything (its scales are ordinary loads, whose wait is the compiler's); the third
+  // needs x that has the codes and a step of x behind it, the fourth x that has a step of x behind it.  The last steps
+  // request the last tile again (never read), so that the counts hold to the end.
+  request_codes(0);
+  request_scales(0);
+  request_x(0, 0);
+  request_x(steps > 1 ? 1 : 0, 1);
+  int stage = 0;
+  for (int c = 0; c < chunks; ++c) {
+    const bool more = c + 1 < chunks;
+    auto step = [&](auto sub_c) {
+      constexpr int sub = decltype(sub_c)::value;
+      const int t = c * SPC + sub;
+      if (sub > 0 && t >= steps) { return; }
+      if (sub == 0) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : : : "memory");
+      } else if (sub == 2 && more) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(CL + XL) : "memory");
+      } else if (sub >= 2) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(XL) : "memory");
+      } else {
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+      }
+      __builtin_amdgcn_s_barrier();                 // x(t) is here, and everybody is done with the stage of x(t - 1)
+      asm volatile("" : : : "memory");
+      const int fill = stage == 0 ? 2 : stage - 1;
+      request_x(t + 2 < steps ? t + 2 : steps - 1, fill);
+      if (sub == 0) {
+        take_codes();
+#pragma unroll
+        for (int i = 0; i < SGW; ++i) { sc[i] = sn[i]; bi[i] = bn[i]; }
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+        if (more) {
+          request_codes(c + 1);
+          request_scales(c + 1);
+        }
+      }
+      contract(sub_c, stage);
+      stage = stage == 2 ? 0 : stage + 1;
+    };
+    step(std::integral_constant<int, 0>());
+    step(std::integral_constant<int, 1>());
+    if constexpr (SPC > 2) {
+      step(std::integral_constant<int, 2>());
+      step(std::integral_constant<int, 3>());
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+
+  // ---- store: a lane holds, for row m = lane % 32 of each i, four consecutive n per register quad ----
+  const bool quads = (p.N & 3) == 0;
+  const bool pairs = ((p.out_stride | p.out_off) & 1) == 0;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = m0 + i * 32 + frow;
+    if (m >= p.M) { continue; }
+#pragma unroll
+    for (int rq = 0; rq < 4; ++rq) {
+      const int n = nw + rq * 8 + fkh * 4;
+      if (n >= p.N) { continue; }
+      const float v[4] = {acc[i][rq * 4], acc[i][rq * 4 + 1], acc[i][rq * 4 + 2], acc[i][rq * 4 + 3]};
+      if (p.ksplit > 1) {
+        float* o = p.plane + ((size_t)ks * p.M + m) * p.N + n;
+        if (quads) {
+          *reinterpret_cast<floatx4*>(o) = floatx4{v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (n + e < p.N) { o[e] = v[e]; }
+          }
+        }
+      } else if (p.gate_act) {                    // (gate, up, gate, up)
+        uint16_t* o = p.y + (size_t)m * p.out_stride + p.out_off + (n >> 1);
+        const float f0 = gated_f32(p.gate_act, v[0], v[1]), f1 = gated_f32(p.gate_act, v[2], v[3]);
+        if (pairs && n + 3 < p.N) {
+          *reinterpret_cast<uint32_t*>(o) = pack_elt2<F16>(f0, f1);
+        } else {
+          o[0] = (uint16_t)f32_to_elt_bits<F16>(f0);
+          if (n + 3 < p.N) { o[1] = (uint16_t)f32_to_elt_bits<F16>(f1); }
+        }
+      } else {
+        uint16_t* o = p.y + (size_t)m * p.N + n;
+        if (quads) {
+          *reinterpret_cast<uint2*>(o) = make_uint2(pack_elt2<F16>(v[0], v[1]), pack_elt2<F16>(v[2], v[3]));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (n + e < p.N) { o[e] = (uint16_t)f32_to_elt_bits<F16>(v[e]); }
+          }
+        }
+      }
+    }
+  }
+}
+
+// y[i] = elt(plane[0][i] + plane[1][i] + ...) in that order, four at a time where the count allows.
+template <int VEC>
+__global__ __launch_bounds__(256) void splitk_fold_kernel(const float* __restrict__ plane, uint16_t* __restrict__ y,
+                                                          size_t count, int splits)
+{
+  for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * VEC; i < count; i += (size_t)gridDim.x * 256 * VEC) {
+    if constexpr (VEC == 4) {
+      floatx4 v = *reinterpret_cast<const floatx4*>(plane + i);
+      for (int s = 1; s < splits; ++s) { v += *reinterpret_cast<const floatx4*>(plane + (size_t)s * count + i); }
+      *reinterpret_cast<uint2*>(y + i) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+    } else {
+      float v = plane[i];
+      for (int s = 1; s < splits; ++s) { v += plane[(size_t)s * count + i]; }
+      y[i] = (uint16_t)f32_to_bf16_bits(v);
+    }
+  }
+}
+
+namespace {
+
+template <int BITS, int GROUP, bool F16>
+hipError_t mid_launch(hipStream_t st, const MidParams& p, int mt, dim3 grid)
+{
+  const dim3 block(kMidWaves * 64);
+  if (mt == 2) { return launch_kernel(qmm_mid_kernel<2, BITS, GROUP, F16>, grid, block, 0, st, p); }
+  if (mt == 3) { return launch_kernel(qmm_mid_kernel<3, BITS, GROUP, F16>, grid, block, 0, st, p); }
+  return launch_kernel(qmm_mid_kernel<4, BITS, GROUP, F16>, grid, block, 0, st, p);
+}
+
+hipError_t mid_launch_as(hipStream_t st, const GemmArgs& a, int mt, int splits, float* plane)
+{
+  if (a.lora_t != nullptr) { return hipErrorInvalidValue; }
+  MidParams p;
+  p.w = a.w; p.scales = a.scales; p.biases = a.biases; p.x = a.x; p.y = a.y;
+  p.K = a.K; p.N = a.N; p.M = a.M;
+  p.gate_act = a.gate_act;
+  p.out_stride = a.out_stride > 0 ? a.out_stride : a.N / 2;
+  p.out_off = a.out_off;
+  p.tiles_m = (a.M + 32 * mt - 1) / (32 * mt);
+  p.tiles_n = (a.N + kMidTileN - 1) / kMidTileN;
+  const int steps = a.K / 64;
+  p.steps_per_split = (steps + splits - 1) / splits;
+  p.ksplit = (steps + p.steps_per_split - 1) / p.steps_per_split;
+  p.plane = plane;
+  const dim3 grid((unsigned)(((long)p.tiles_n * p.ksplit + 7) / 8 * 8 * p.tiles_m));
+  if (a.bits == 8) { return a.group == 64 && !a.f16 ? mid_launch<8, 64, false>(st, p, mt, grid) : hipErrorInvalidValue; }
+  if (a.group == 32) { return a.f16 ? hipErrorInvalidValue : mid_launch<4, 32, false>(st, p, mt, grid); }
+  return a.f16 ? mid_launch<4, 64, true>(st, p, mt, grid) : mid_launch<4, 64, false>(st, p, mt, grid);
+}
+
+// What a GEMM takes, in microseconds; measured on 1024..24576 x 4096..12288 at 80..1024 rows, to about a tenth.  A split
+// writes and reads its planes once more, and folds them in a launch of its own, at about 4 TB/s.
+double planes_us(int N, int M, int splits) { return splits > 1 ? 3.0 + (splits + 0.5) * (double)M * (double)N * 4.0 / 4.0e6 : 0.0; }
+
+// This kernel, per step of 64: a workgroup alone on its CU, and each of several that share one (the busiest CU counts).
+constexpr double kMidAlone[5] = {0, 0, 0.50, 0.57, 0.66}, kMidShared[5] = {0, 0, 0.39, 0.48, 0.61};
+
+double mid_us(int K, int N, int M, int mt, int splits, int cus)
+{
+  const int steps = K / 64, per = (steps + splits - 1) / splits;
+  const long wgs = (long)((M + 32 * mt - 1) / (32 * mt)) * ((N + kMidTileN - 1) / kMidTileN) * splits;
+  const double step = (double)((wgs + cus - 1) / cus) * kMidShared[mt];
+  return 4.0 + per * (step > kMidAlone[mt] ? step : kMidAlone[mt]) + planes_us(N, M, splits);
+}
+
+// Rows of x per workgroup, in 32s: the count that takes least.
+int mid_rows(int K, int N, int M, int splits, int cus)
+{
+  int best = 4;
+  for (int mt = 3; mt >= 2; --mt) {
+    if (mid_us(K, N, M, mt, splits, cus) < mid_us(K, N, M, best, splits, cus)) { best = mt; }
+  }
+  return best;
+}
+
+// The kernels with 256 rows of x a workgroup, one workgroup per CU.  `step` is that of a full chip; the 256 x 128 tiles
+// take 0.89 on a nearly idle one (its clock is higher), 1.1 on a full one, the large tile 1.62 at 256 x 192.
+double tall_us(int K, int N, int M, int width, double step, int splits, int cus)
+{
+  const int steps = K / 64, per = (steps + splits - 1) / splits;
+  const long tiles = (long)((M + 255) / 256) * ((N + width - 1) / width) * splits;
+  const double fill = tiles < cus ? (double)tiles / cus : 1.0;
+  return 4.0 + per * step * (0.8 + 0.2 * fill) * (double)((tiles + cus - 1) / cus) + planes_us(N, M, splits);
+}
+
+constexpr double kTileStep = 1.1;
+
+bool tile_splits_better(int K, int N, int M, int splits, int cus)
+{
+  return tall_us(K, N, M, 128, kTileStep, splits, cus) < mid_us(K, N, M, mid_rows(K, N, M, splits, cus), splits, cus);
+}
+
+// The kernel that takes least without a split of K, and how long.
+GemmKernel choose_unsplit(const GemmArgs& a, double* us)
+{
+  const int cus = a.cu_count > 0 ? a.cu_count : 256;
+  const int tm = (a.M + 255) / 256;
+  double big = 1e30;
+  // below one round of its tiles the large-tile kernel has nothing over the 256 x 128 one
+  if (qmm_big_supports(a)) {
+    const int bn = qmm_big_tile_n(a.N, a.M, cus, a.bits == 8 ? 192 : 256, a.group != 32);
+    if ((long)tm * ((a.N + bn - 1) / bn) >= cus) { big = tall_us(a.K, a.N, a.M, bn, bn == 256 ? 2.05 : bn == 192 ? 1.62 : 1.14, 1, cus); }
+  }
+  const double tile = tall_us(a.K, a.N, a.M, 128, kTileStep, 1, cus);
+  const double mid = a.lora_t != nullptr ? 1e30 : mid_us(a.K, a.N, a.M, mid_rows(a.K, a.N, a.M, 1, cus), 1, cus);
+  const bool takes_big = big < 1e30 && big <= mid, takes_mid = !takes_big && mid <= tile;
+  *us = takes_big ? big : takes_mid ? mid : tile;
+  return takes_big ? GemmKernel::kBig : takes_mid ? GemmKernel::kMid : GemmKernel::kTile;
+}
+
+}  // namespace
+
+GemmKernel qmm_choose(const GemmArgs& a)
+{
+  double us;
+  return choose_unsplit(a, &us);
+}
+
+hipError_t launch_qmm_mid(hipStream_t st, const GemmArgs& a)
+{
+  const int cus = a.cu_count > 0 ? a.cu_count : 256;
+  return mid_launch_as(st, a, mid_rows(a.K, a.N, a.M, 1, cus), 1, nullptr);
+}
+
+// Shares of K that pay for their planes; 1 where the tiles alone fill the chip.
+int qmm_choose_splits(int K, int N, int M, int cu_count)
+{
+  const int cus = cu_count > 0 ? cu_count : 256;
+  const int steps = K / 64;
+  GemmArgs a{};
+  a.K = K; a.N = N; a.M = M; a.cu_count = cus;
+  double best_us;
+  choose_unsplit(a, &best_us);
+  int best = 1;
+  best_us *= 0.95;
+  for (int s = 2; s <= 16 && steps / s >= 4; ++s) {
+    const int per = (steps + s - 1) / s;
+    if ((steps + per - 1) / per != s) { continue; }    // shares would come out uneven: another count covers it
+    const double us = tile_splits_better(K, N, M, s, cus) ? tall_us(K, N, M, 128, kTileStep, s, cus)
+                                                          : mid_us(K, N, M, mid_rows(K, N, M, s, cus), s, cus);
+    if (us < best_us) { best = s; best_us = us; }
+  }
+  return best;
+}
+
+size_t qmm_splitk_workspace_bytes(int K, int N, int M, int cu_count)
+{
+  const int s = qmm_choose_splits(K, N, M, cu_count);
+  return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) : 0;
+}
+
+hipError_t launch_qmm_splitk(hipStream_t st, const GemmArgs& a, int splits, float* plane)
+{
+  const int cus = a.cu_count > 0 ? a.cu_count : 256;
+  const int steps = a.K / 64, per = (steps + splits - 1) / splits;
+  const hipError_t e = tile_splits_better(a.K, a.N, a.M, splits, cus)
+                           ? launch_qmm_tile_planes(st, a, splits, plane)
+                           : mid_launch_as(st, a, mid_rows(a.K, a.N, a.M, splits, cus), splits, plane);
+  if (e != hipSuccess) { return e; }
+  const size_t count = (size_t)a.M * (size_t)a.N;
+  const bool quads = (count & 3) == 0;
+  size_t blocks = (count + (quads ? 1023 : 255)) / (quads ? 1024 : 256);
+  if (blocks > 65536) { blocks = 65536; }
+  const int shares = (steps + per - 1) / per;
+  return quads ? launch_kernel(splitk_fold_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, st, plane, a.y, count, shares)
+               : launch_kernel(splitk_fold_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, st, plane, a.y, count, shares);
+}
+
+}  // namespace vpq

@@ -38,6 +38,7 @@
 
 #include "vpq_device.h"
 #include "vpq_internal.h"
+#include "vpq_tile_dequant.h"
 
 namespace vpq {
 
@@ -82,35 +83,6 @@ struct TileParams {
 };
 
 __device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
-
-// Byte I of a dword as fp32 (selects v_cvt_f32_ubyteI).
-template <int I>
-__device__ __forceinline__ float ubyte_f32(uint32_t v) { return (float)((v >> (8 * I)) & 0xffu); }
-
-// 8 nibbles of one word -> 8 bf16 (F16: IEEE binary16) of fma(s, q, b), as one 16-byte LDS chunk.
-template <bool F16 = false>
-__device__ __forceinline__ uint4 dequant_word(uint32_t word, float s, float b)
-{
-  uint32_t lo = word & 0x0f0f0f0fu;                // q0 q2 q4 q6
-  uint32_t hi = (word >> 4) & 0x0f0f0f0fu;         // q1 q3 q5 q7
-  // No instruction: keeps the masked words as they are, so that each value is one v_cvt_f32_ubyteN
-  // of them (otherwise the mask is folded into a bit-field extract per value, one instruction more).
-  asm volatile("" : "+v"(lo), "+v"(hi));
-  const float v0 = fmaf(s, ubyte_f32<0>(lo), b);
-  const float v1 = fmaf(s, ubyte_f32<0>(hi), b);
-  const float v2 = fmaf(s, ubyte_f32<1>(lo), b);
-  const float v3 = fmaf(s, ubyte_f32<1>(hi), b);
-  const float v4 = fmaf(s, ubyte_f32<2>(lo), b);
-  const float v5 = fmaf(s, ubyte_f32<2>(hi), b);
-  const float v6 = fmaf(s, ubyte_f32<3>(lo), b);
-  const float v7 = fmaf(s, ubyte_f32<3>(hi), b);
-  uint4 o;
-  o.x = pack_elt2<F16>(v0, v1);
-  o.y = pack_elt2<F16>(v2, v3);
-  o.z = pack_elt2<F16>(v4, v5);
-  o.w = pack_elt2<F16>(v6, v7);
-  return o;
-}
 
 // Workgroup barrier without a memory fence: the callers wait on the counters they need.
 // The empty statements keep the compiler from moving LDS accesses across it.
@@ -201,17 +173,6 @@ __device__ __forceinline__ void wait_codes(CodeRegsT<8>& r)
 // The same for the register set of a step (one per producer thread in every form built).
 template <int YOUNGER, int BITS>
 __device__ __forceinline__ void wait_codes(CodeRegsT<BITS> (&r)[1]) { wait_codes<YOUNGER>(r[0]); }
-
-// 8 bytes of two packed words -> 8 bf16 of fma(s, q, b), as one 16-byte LDS chunk (the 8-bit pack).
-__device__ __forceinline__ uint4 dequant_bytes(uint32_t w0, uint32_t w1, float s, float b)
-{
-  uint4 o;
-  o.x = pack_bf16x2(fmaf(s, ubyte_f32<0>(w0), b), fmaf(s, ubyte_f32<1>(w0), b));
-  o.y = pack_bf16x2(fmaf(s, ubyte_f32<2>(w0), b), fmaf(s, ubyte_f32<3>(w0), b));
-  o.z = pack_bf16x2(fmaf(s, ubyte_f32<0>(w1), b), fmaf(s, ubyte_f32<1>(w1), b));
-  o.w = pack_bf16x2(fmaf(s, ubyte_f32<2>(w1), b), fmaf(s, ubyte_f32<3>(w1), b));
-  return o;
-}
 
 }  // namespace
 
@@ -706,50 +667,6 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
   }
 }
 
-// y[i] = bf16(plane[0][i] + plane[1][i] + ... ) in that order, i over M*N.
-__global__ __launch_bounds__(256) void splitk_fold_kernel(const float* __restrict__ plane, uint16_t* __restrict__ y,
-                                                          size_t count, int splits)
-{
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (size_t)gridDim.x * 256) {
-    float v = plane[i];
-    for (int s = 1; s < splits; ++s) { v += plane[(size_t)s * count + i]; }
-    y[i] = (uint16_t)f32_to_bf16_bits(v);
-  }
-}
-
-// Split count by a small cost model (microseconds, from measurements on MI355X): a workgroup costs
-// ~3 us to start and drain plus ~0.9 us per K step; workgroups run one per CU, so the grid takes
-// ceil(workgroups / CUs) rounds; the planes are written and read once more by the fold at ~4 TB/s.
-int qmm_choose_splits(int K, int N, int M, int cu_count)
-{
-  const int tiles = ((M + TM - 1) / TM) * ((N + TN - 1) / TN);
-  const int steps = K / TK;
-  const int cus = cu_count > 0 ? cu_count : 256;
-  if (tiles * 2 > cus) { return 1; }                   // the tiles alone fill at least half of the chip
-  auto cost = [&](int s) {
-    const int per = (steps + s - 1) / s;
-    const int rounds = (tiles * s + cus - 1) / cus;
-    double us = rounds * (3.0 + 0.9 * per);
-    if (s > 1) { us += 3.0 + (s + 0.5) * (double)M * (double)N * 4.0 / 4.0e6; }
-    return us;
-  };
-  int best = 1;
-  double best_us = cost(1);
-  for (int s = 2; s <= 16 && steps / s >= 4; ++s) {
-    const int per = (steps + s - 1) / s;
-    if ((steps + per - 1) / per != s) { continue; }    // shares would come out uneven: another count covers it
-    const double us = cost(s);
-    if (us < 0.9 * best_us) { best = s; best_us = us; }
-  }
-  return best;
-}
-
-size_t qmm_splitk_workspace_bytes(int K, int N, int M, int cu_count)
-{
-  const int s = qmm_choose_splits(K, N, M, cu_count);
-  return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) : 0;
-}
-
 // The scale/bias ring's windows are 16-byte loads of 8 groups: whole windows in every row, aligned.
 static bool sb_ring_ok(const GemmArgs& a)
 {
@@ -757,7 +674,8 @@ static bool sb_ring_ok(const GemmArgs& a)
          (reinterpret_cast<uintptr_t>(a.biases) & 15) == 0;
 }
 
-hipError_t launch_qmm_tile_splitk(hipStream_t st, const GemmArgs& a, int splits, float* plane)
+// The planes of a split over K (no fold).
+hipError_t launch_qmm_tile_planes(hipStream_t st, const GemmArgs& a, int splits, float* plane)
 {
   TileParams p;
   p.w = a.w; p.scales = a.scales; p.biases = a.biases; p.x = a.x; p.y = a.y;
@@ -771,12 +689,7 @@ hipError_t launch_qmm_tile_splitk(hipStream_t st, const GemmArgs& a, int splits,
   p.ksplit = (steps + p.steps_per_split - 1) / p.steps_per_split;
   p.plane = plane;
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * p.ksplit)), block(kThreads);
-  hipError_t e = launch_kernel(qmm_tile_kernel<false>, grid, block, 0, st, p);
-  if (e != hipSuccess) { return e; }
-  const size_t count = (size_t)a.M * (size_t)a.N;
-  size_t blocks = (count + 255) / 256;
-  if (blocks > 65536) { blocks = 65536; }
-  return launch_kernel(splitk_fold_kernel, dim3((unsigned)blocks), dim3(256), 0, st, plane, a.y, count, p.ksplit);
+  return launch_kernel(qmm_tile_kernel<false>, grid, block, 0, st, p);
 }
 
 hipError_t launch_qmm_tile(hipStream_t st, const GemmArgs& a)

@@ -1,4 +1,4 @@
-// QMV for M <= 4: the streaming form of the MFMA kernel in vpq_qmv_mfma.hip.
+// QMV for M <= 4: persistent workgroups that stream items through registers.
 //
 // Same items (16 weight rows x 512 k-values), same arithmetic, but built to keep
 // the VALU work per item near its floor (nibble -> bf16 conversion and the
