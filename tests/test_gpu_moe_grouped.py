@@ -299,3 +299,49 @@ def test_sorted_expert_gemv_rejects_bad_arguments(vpq, dev):
     assert L.vpq_qmv_grouped_down_w4g64_bf16(None, p, p, p, p, p, 60, 8, 2, p, p, 1) == -2            # K % 64
     assert L.vpq_qmv_grouped_down_w4g64_bf16(None, p, p, p, p, p, 64, 8, 2, p, p, 0) == -2            # no expert
     assert L.vpq_qmv_grouped_down_w4g64_bf16(None, p, p, p, p, p, 64, 8, 2, None, p, 1) == -1
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("K,N", [(64, 36), (320, 130), (512, 256)])
+def test_grouped_gemms_at_every_count_of_live_fragments(vpq, dev, D, K, N, bits):
+    # blocks with 1..128 live slots (the edges of 32-row fragments), a full block with one slot behind it, an expert with
+    # none: every live slot is the plain GEMM's row bit for bit, every other slot of gate|up is zero
+    counts = [1, 31, 32, 33, 0, 64, 65, 96, 97, 128, 129]
+    E, B = len(counts), vpq.grouped_block_rows()
+    gen = torch.Generator(device="cpu").manual_seed(5700 + K + bits)
+    w = torch.randint(-2 ** 31, 2 ** 31, (E, N, K * bits // 32), dtype=torch.int32, generator=gen).to(dev)
+    s = (torch.rand((E, N, K // 64), generator=gen) * 0.015 / (16 if bits == 8 else 1) + 0.001).bfloat16().to(dev)
+    b = (-(2 ** (bits - 1)) * s.float()).bfloat16()
+    eid = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(sum(counts), generator=gen)]
+    x = torch.randn((eid.numel(), K), generator=gen).bfloat16().to(dev)
+    t2e, srow, sdst, _ = vpq.moe_sort_pairs(eid.to(torch.int32).to(dev), 1, E)
+    npad = srow.numel()
+    gated = vpq.qmm_grouped_gated_w8g64 if bits == 8 else vpq.qmm_grouped_gated_w4g64
+    down = vpq.qmm_grouped_down_w8g64 if bits == 8 else vpq.qmm_grouped_down_w4g64
+    act = parity.Guarded((npad, N // 2), torch.bfloat16, dev)
+    part = parity.Guarded((eid.numel(), N), torch.bfloat16, dev)
+    act.view.fill_(7.0)
+    part.view.fill_(7.0)
+    xs = x[srow.clamp(min=0).long()].contiguous()
+    xs[srow < 0] = float("nan")                          # a padding slot's x reaches no live row
+    gated(w, s, b, x, K, N, t2e, srow, E, out=act.view)
+    down(w, s, b, xs, K, N, t2e, sdst, E, out=part.view)
+    torch.cuda.synchronize()
+    act.assert_intact()
+    part.assert_intact()
+    owner = t2e.repeat_interleave(B).cpu()
+    live = (srow >= 0).cpu()
+    assert not D.bits(act.view)[((owner >= 0) & ~live).numpy()].any()
+    for e in range(E):
+        slots = torch.nonzero((owner == e) & live).flatten().to(dev)
+        assert slots.numel() == counts[e]
+        if counts[e] == 0:
+            continue
+        xe = x[srow[slots].long()].contiguous()
+        if bits == 8:
+            g, d = (vpq.qmm_w8g64(w[e], s[e], b[e], xe, K, N, counts[e], activation=a) for a in (1, 0))
+        else:
+            g = vpq.qmm_swiglu_w4g64(w[e], s[e], b[e], xe, K, N, counts[e])
+            d = vpq.qmm_w4g64(w[e], s[e], b[e], xe, K, N, counts[e], tile_n=128)
+        assert np.array_equal(D.bits(act.view)[slots.cpu().numpy()], D.bits(g)), "gate|up, expert %d" % e
+        assert np.array_equal(D.bits(part.view)[sdst[slots].cpu().numpy()], D.bits(d)), "down, expert %d" % e

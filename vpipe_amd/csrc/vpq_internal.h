@@ -228,8 +228,8 @@ hipError_t launch_lora_a(hipStream_t st, const uint16_t* x, const uint16_t* a, u
 // 256x128-tile quantized GEMM (+ fused LoRA second factor); a.w must be non-null.
 hipError_t launch_qmm_tile(hipStream_t st, const GemmArgs& a);
 hipError_t launch_qmm_tile_planes(hipStream_t st, const GemmArgs& a, int splits, float* plane);
-// Grouped (expert-sorted) form of the tile kernel at 128 rows per block: a.w/scales/biases are the
-// batched pack [E, N, ...], a.M the padded slot count (a multiple of kGroupedBlockRows); see TileParams.
+// Expert-sorted form (vpq_qmm_mid.hip) in blocks of 128 slots: a.w/scales/biases are the batched pack
+// [E, N, ...], a.M the padded slot count (a multiple of kGroupedBlockRows); see MidParams.
 constexpr int kGroupedBlockRows = 128;
 struct GroupedArgs {
   const int* tile2e;   // [a.M / kGroupedBlockRows]

@@ -48,6 +48,15 @@ struct MidParams {
   int gate_act, out_stride, out_off;          // as in the tile kernel
   int ksplit, steps_per_split;
   float* plane;                               // ksplit > 1: [ksplit][M][N]
+  // Expert-sorted form: slots in blocks of kGroupedBlockRows that each belong to one expert
+  // (gpu-kernels/metal/quant/affine_qmm_steel.metal:1022-1040).  tile2e[block] is the expert whose slab of the batched
+  // pack [E, N, ...] the block multiplies (outside 0..n_experts - 1: nothing to do).  Gated: slot i reads x[srow[i]]
+  // (outside 0..rows_x - 1: a padding slot, whose output is zero) and stores y[i].  Plain: slot i reads x[i] and
+  // stores y[sdst[i]] (outside 0..rows_y - 1: not written).
+  const int* tile2e;
+  const int* srow;
+  const int* sdst;
+  int n_experts, rows_x, rows_y;
 };
 
 __device__ __forceinline__ uint32_t mid_lds(const uint8_t* q)
@@ -75,12 +84,13 @@ __device__ __forceinline__ floatx16 mid_mfma(u32x4 a, u32x4 b, floatx16 c)
   }
 }
 
-}  // namespace
-
-template <int MT, int BITS, int GROUP, bool F16>
-__global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidParams p)
+// A workgroup's tile: rows [m0, m0 + 32 MT) of x (of slots) against weight rows [n0, n0 + 128) of the pack given, over
+// share `ks` of K.
+template <int MT, int BITS, int GROUP, bool F16, bool GROUPED>
+__device__ __forceinline__ void mid_tile(const MidParams& p, uint8_t* x_lds, uint8_t* c_lds, int m0, int n0, int ks,
+                                         const uint32_t* pack_w, const uint16_t* pack_s, const uint16_t* pack_b)
 {
-  constexpr int BM = 32 * MT, BN = kMidTileN;
+  constexpr int BM = 32 * MT;
   constexpr int SPC = 16 / BITS;                    // K steps of 64 per chunk of codes: 4 or 2
   constexpr int SG = SPC * 64 / GROUP;              // groups per chunk
   constexpr int SGW = SG / 2;                       // ... in words of two
@@ -89,41 +99,36 @@ __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidPar
   constexpr int kXStage = BM * kMidRowB;
   constexpr int kSlot = 32 * kMidRowB;
   constexpr int kWords = kMidRowB / 4 / 2;          // words of a weight row's chunk that one lane unpacks
-  __shared__ __attribute__((aligned(16))) uint8_t x_lds[kMidStages * kXStage];
-  __shared__ __attribute__((aligned(16))) uint8_t c_lds[kMidWaves * kSlot];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int frow = lane & 31;                       // row of a 32-row operand
   const int fkh = lane >> 5;                        // which 8 of its 16 k
 
-  // Workgroups go to the XCDs round robin: those that share a weight tile (one per tile of rows of x) are eight apart,
-  // so that the pack is read from HBM once.
-  const int units = p.tiles_n * p.ksplit;
-  const int span = 8 * p.tiles_m;
-  const int uq = (int)blockIdx.x / span, ur = (int)blockIdx.x - uq * span;
-  const int unit = uq * 8 + (ur & 7);
-  if (unit >= units) { return; }
-  const int ks = unit / p.tiles_n;
-  const int m0 = (ur >> 3) * BM, n0 = (unit - ks * p.tiles_n) * BN;
   const int k_first = ks * p.steps_per_split;
   const int k_left = p.K / 64 - k_first;
   const int steps = k_left < p.steps_per_split ? k_left : p.steps_per_split;
   const int chunks = (steps + SPC - 1) / SPC;
 
   // ---- addresses ----
-  const uint8_t* xblk = reinterpret_cast<const uint8_t*>(p.x) + (size_t)m0 * p.K * 2 + (size_t)k_first * 128;
+  const bool gathered = GROUPED && p.srow != nullptr;
+  const uint8_t* xblk = reinterpret_cast<const uint8_t*>(p.x) + (gathered ? (size_t)0 : (size_t)m0 * p.K * 2) +
+                        (size_t)k_first * 128;
   uint32_t x_off[XL];
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
     const int row = (wave * XL + i) * 8 + (lane >> 3);
-    const int rg = m0 + row < p.M ? row : p.M - 1 - m0;
+    int rg = m0 + row < p.M ? row : p.M - 1 - m0;
+    if (gathered) {                                 // a padding slot reads row 0, unused
+      const int src = p.srow[m0 + rg];
+      rg = src >= 0 && src < p.rows_x ? src : 0;
+    }
     x_off[i] = (uint32_t)rg * (uint32_t)p.K * 2u + (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) * 16);
   }
   const int nw = n0 + wave * 32;                    // this wavefront's first weight row
   const uint32_t row_bytes = (uint32_t)p.K * BITS / 8;
   const int row_left = (int)row_bytes - k_first * (8 * BITS);   // bytes of a row from this share's start on
-  const uint8_t* cblk = reinterpret_cast<const uint8_t*>(p.w) + (size_t)(nw < p.N ? nw : p.N - 1) * row_bytes +
+  const uint8_t* cblk = reinterpret_cast<const uint8_t*>(pack_w) + (size_t)(nw < p.N ? nw : p.N - 1) * row_bytes +
                         (size_t)k_first * (8 * BITS);
   const int w_last = nw < p.N ? p.N - 1 - nw : 0;   // rows past the last repeat it
   uint32_t c_row[CL];
@@ -135,8 +140,8 @@ __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidPar
   const uint32_t c_piece = (uint32_t)(((lane & 7) ^ (lane >> 4)) * 16);   // key (row >> 1) & 7, bit 2 by the load
   const int Kg = p.K / GROUP;
   const size_t at = (size_t)((nw < p.N ? nw : p.N - 1) + (frow < w_last ? frow : w_last)) * Kg;
-  const uint16_t* srow = p.scales + at;
-  const uint16_t* brow = p.biases + at;
+  const uint16_t* srow = pack_s + at;
+  const uint16_t* brow = pack_b + at;
   uint8_t* slot = c_lds + wave * kSlot;
 
   auto request_x = [&](int step, int stage) {
@@ -277,16 +282,30 @@ __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidPar
   // ---- store: a lane holds, for row m = lane % 32 of each i, four consecutive n per register quad ----
   const bool quads = (p.N & 3) == 0;
   const bool pairs = ((p.out_stride | p.out_off) & 1) == 0;
+  // rows that a gated block stores: all its slots, zeros past the fragments that were multiplied
+  constexpr int kStored = GROUPED ? kGroupedBlockRows / 32 : MT;
 #pragma unroll
-  for (int i = 0; i < MT; ++i) {
+  for (int i = 0; i < kStored; ++i) {
     const int m = m0 + i * 32 + frow;
-    if (m >= p.M) { continue; }
+    if (m >= p.M || (i >= MT && !p.gate_act)) { continue; }
+    bool pad = i >= MT;                             // act(0) * 0 = +0
+    int mdst = m;
+    if constexpr (GROUPED) {
+      if (p.gate_act) {
+        const int src = p.srow[m];
+        pad = pad || src < 0 || src >= p.rows_x;
+      } else {
+        mdst = p.sdst[m];
+        if (mdst < 0 || mdst >= p.rows_y) { continue; }
+      }
+    }
 #pragma unroll
     for (int rq = 0; rq < 4; ++rq) {
       const int n = nw + rq * 8 + fkh * 4;
       if (n >= p.N) { continue; }
-      const float v[4] = {acc[i][rq * 4], acc[i][rq * 4 + 1], acc[i][rq * 4 + 2], acc[i][rq * 4 + 3]};
-      if (p.ksplit > 1) {
+      const floatx16& ai = acc[i < MT ? i : 0];
+      const float v[4] = {ai[rq * 4], ai[rq * 4 + 1], ai[rq * 4 + 2], ai[rq * 4 + 3]};
+      if (!GROUPED && p.ksplit > 1) {
         float* o = p.plane + ((size_t)ks * p.M + m) * p.N + n;
         if (quads) {
           *reinterpret_cast<floatx4*>(o) = floatx4{v[0], v[1], v[2], v[3]};
@@ -298,7 +317,8 @@ __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidPar
         }
       } else if (p.gate_act) {                    // (gate, up, gate, up)
         uint16_t* o = p.y + (size_t)m * p.out_stride + p.out_off + (n >> 1);
-        const float f0 = gated_f32(p.gate_act, v[0], v[1]), f1 = gated_f32(p.gate_act, v[2], v[3]);
+        const float f0 = GROUPED && pad ? 0.0f : gated_f32(p.gate_act, v[0], v[1]);
+        const float f1 = GROUPED && pad ? 0.0f : gated_f32(p.gate_act, v[2], v[3]);
         if (pairs && n + 3 < p.N) {
           *reinterpret_cast<uint32_t*>(o) = pack_elt2<F16>(f0, f1);
         } else {
@@ -306,7 +326,7 @@ __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidPar
           if (n + 3 < p.N) { o[1] = (uint16_t)f32_to_elt_bits<F16>(f1); }
         }
       } else {
-        uint16_t* o = p.y + (size_t)m * p.N + n;
+        uint16_t* o = p.y + (size_t)mdst * p.N + n;
         if (quads) {
           *reinterpret_cast<uint2*>(o) = make_uint2(pack_elt2<F16>(v[0], v[1]), pack_elt2<F16>(v[2], v[3]));
         } else {
@@ -317,6 +337,69 @@ __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidPar
         }
       }
     }
+  }
+}
+
+}  // namespace
+
+template <int MT, int BITS, int GROUP, bool F16>
+__global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidParams p)
+{
+  constexpr int BM = 32 * MT, BN = kMidTileN;
+  __shared__ __attribute__((aligned(16))) uint8_t x_lds[kMidStages * BM * kMidRowB];
+  __shared__ __attribute__((aligned(16))) uint8_t c_lds[kMidWaves * 32 * kMidRowB];
+
+  // Workgroups go to the XCDs round robin: those that share a weight tile (one per tile of rows of x) are eight apart,
+  // so that the pack is read from HBM once.
+  const int units = p.tiles_n * p.ksplit;
+  const int span = 8 * p.tiles_m;
+  const int uq = (int)blockIdx.x / span, ur = (int)blockIdx.x - uq * span;
+  const int unit = uq * 8 + (ur & 7);
+  if (unit >= units) { return; }
+  const int ks = unit / p.tiles_n;
+  const int m0 = (ur >> 3) * BM, n0 = (unit - ks * p.tiles_n) * BN;
+  mid_tile<MT, BITS, GROUP, F16, false>(p, x_lds, c_lds, m0, n0, ks, p.w, p.scales, p.biases);
+}
+
+// The expert-sorted form.  An expert's last block is mostly padding (16384 pairs of 128 experts: 191 blocks, 63 of them
+// with about ten live slots), and a prompt of some tokens gives each expert a few: a block multiplies as many 32-row
+// fragments as reach its last live slot, each count a K loop of its own, whose loads, LDS reads and MFMAs are those
+// rows' alone.  All weight tiles of a block go to one XCD (eight workgroups apart), whose L2 then holds its rows of x.
+// Bound by the plain tile's step at full blocks, by unpacking and the codes' read at one fragment.  Measured (us, sort +
+// gate|up + down of one layer; before: 128 x 256 tiles with producer wavefronts, every block at full height), 2048 -> 768:
+// 2048 tokens, 8 of 128 experts 370 -> 286; 64 tokens 191 -> 138; 4096 tokens, 8 of 64 experts 557 -> 447, 8 bits 580 -> 498.
+template <int BITS>
+__global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_grouped_kernel(const MidParams p)
+{
+  __shared__ __attribute__((aligned(16))) uint8_t x_lds[kMidStages * kGroupedBlockRows * kMidRowB];
+  __shared__ __attribute__((aligned(16))) uint8_t c_lds[kMidWaves * 32 * kMidRowB];
+  static_assert(kGroupedBlockRows == 128, "two slots per lane, four fragments");
+
+  const int span = 8 * p.tiles_n;
+  const int uq = (int)blockIdx.x / span, ur = (int)blockIdx.x - uq * span;
+  const int tm = uq * 8 + (ur & 7);
+  if (tm >= p.tiles_m) { return; }
+  const int e = p.tile2e[tm];
+  if (e < 0 || e >= p.n_experts) { return; }        // the whole workgroup, before any barrier
+  const int m0 = tm * kGroupedBlockRows, n0 = (ur >> 3) * kMidTileN;
+  const uint32_t* w = p.w + (size_t)e * (size_t)p.N * (size_t)(p.K >> (BITS == 4 ? 3 : 2));
+  const uint16_t* s = p.scales + (size_t)e * (size_t)p.N * (size_t)(p.K >> 6);
+  const uint16_t* b = p.biases + (size_t)e * (size_t)p.N * (size_t)(p.K >> 6);
+
+  const int lane = threadIdx.x & 63;
+  const int* idx = p.gate_act ? p.srow : p.sdst;
+  const int lim = p.gate_act ? p.rows_x : p.rows_y;
+  const int v0 = idx[m0 + lane], v1 = idx[m0 + 64 + lane];
+  const unsigned long long lo = __ballot(v0 >= 0 && v0 < lim), hi = __ballot(v1 >= 0 && v1 < lim);
+  const int live = hi != 0 ? ((hi >> 32) != 0 ? 4 : 3) : (lo >> 32) != 0 ? 2 : 1;
+  if (live == 1) {
+    mid_tile<1, BITS, 64, false, true>(p, x_lds, c_lds, m0, n0, 0, w, s, b);
+  } else if (live == 2) {
+    mid_tile<2, BITS, 64, false, true>(p, x_lds, c_lds, m0, n0, 0, w, s, b);
+  } else if (live == 3) {
+    mid_tile<3, BITS, 64, false, true>(p, x_lds, c_lds, m0, n0, 0, w, s, b);
+  } else {
+    mid_tile<4, BITS, 64, false, true>(p, x_lds, c_lds, m0, n0, 0, w, s, b);
   }
 }
 
@@ -352,7 +435,7 @@ hipError_t mid_launch(hipStream_t st, const MidParams& p, int mt, dim3 grid)
 hipError_t mid_launch_as(hipStream_t st, const GemmArgs& a, int mt, int splits, float* plane)
 {
   if (a.lora_t != nullptr) { return hipErrorInvalidValue; }
-  MidParams p;
+  MidParams p{};
   p.w = a.w; p.scales = a.scales; p.biases = a.biases; p.x = a.x; p.y = a.y;
   p.K = a.K; p.N = a.N; p.M = a.M;
   p.gate_act = a.gate_act;
@@ -442,6 +525,26 @@ hipError_t launch_qmm_mid(hipStream_t st, const GemmArgs& a)
 {
   const int cus = a.cu_count > 0 ? a.cu_count : 256;
   return mid_launch_as(st, a, mid_rows(a.K, a.N, a.M, 1, cus), 1, nullptr);
+}
+
+hipError_t launch_qmm_grouped(hipStream_t st, const GemmArgs& a, const GroupedArgs& g)
+{
+  // gated blocks gather rows of x, plain ones scatter rows of y
+  if ((a.gate_act ? g.srow : g.sdst) == nullptr || (!a.gate_act && g.srow != nullptr)) { return hipErrorInvalidValue; }
+  MidParams p{};
+  p.w = a.w; p.scales = a.scales; p.biases = a.biases; p.x = a.x; p.y = a.y;
+  p.K = a.K; p.N = a.N; p.M = a.M;
+  p.gate_act = a.gate_act;
+  p.out_stride = a.out_stride > 0 ? a.out_stride : a.N / 2;
+  p.out_off = a.out_off;
+  p.tiles_m = a.M / kGroupedBlockRows;              // a.M is a whole number of blocks
+  p.tiles_n = (a.N + kMidTileN - 1) / kMidTileN;
+  p.ksplit = 1; p.steps_per_split = a.K / 64;
+  p.tile2e = g.tile2e; p.srow = g.srow; p.sdst = g.sdst;
+  p.n_experts = g.n_experts; p.rows_x = g.rows_x; p.rows_y = g.rows_y;
+  const dim3 grid((unsigned)((p.tiles_m + 7) / 8 * 8 * p.tiles_n)), block(kMidWaves * 64);
+  return a.bits == 8 ? launch_kernel(qmm_mid_grouped_kernel<8>, grid, block, 0, st, p)
+                     : launch_kernel(qmm_mid_grouped_kernel<4>, grid, block, 0, st, p);
 }
 
 // Shares of K that pay for their planes; 1 where the tiles alone fill the chip.

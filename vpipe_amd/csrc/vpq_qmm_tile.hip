@@ -46,7 +46,7 @@ namespace {
 
 constexpr int TM = 256, TN = 128, TK = 64;
 constexpr int kConsumers = 4;                        // consumer wavefronts: kConsumers/2 along M, 2 along N
-constexpr int kProducers = 4;                        // producer wavefronts (8 in the 128 x 256 grouped form)
+constexpr int kProducers = 4;                        // producer wavefronts
 constexpr int kThreads = (kConsumers + kProducers) * 64;
 constexpr int kStages = 3;
 constexpr int kRowB = TK * 2;                       // 128 bytes per LDS row
@@ -71,15 +71,6 @@ struct TileParams {
   // whatever the split count).
   int ksplit, steps_per_split;
   float* plane;
-  // Grouped (expert-sorted) form, rows in blocks of the tile height that each belong to one expert
-  // (gpu-kernels/metal/quant/affine_qmm_steel.metal:1022-1040): tile2e[block] is the expert whose
-  // slab of the batched pack [E, N, ...] the block multiplies (< 0: nothing to do); with srow, x row
-  // of slot i is x[srow[i]] (< 0: a padding slot, whose output is zero); with sdst, the output row of
-  // slot i goes to y[sdst[i]] (< 0: not written).
-  const int* tile2e = nullptr;
-  const int* srow = nullptr;
-  const int* sdst = nullptr;
-  int n_experts = 0, rows_x = 0, rows_y = 0;
 };
 
 __device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
@@ -127,36 +118,6 @@ __device__ __forceinline__ void request_codes(CodeRegsT<BITS>& r, const uint8_t*
   asm volatile("global_load_ushort %0, %1, off" : "=v"(r.b_bits) : "v"(b) : "memory");
 }
 
-// The codes alone (scale and bias come from the LDS ring, see SBR).
-template <int BITS>
-__device__ __forceinline__ void request_codes_only(CodeRegsT<BITS>& r, const uint8_t* codes)
-{
-  request_code_words(r, codes);
-}
-
-// Scale and bias of one row and step from the ring, as loads the compiler does not track (it would order
-// them after every direct-to-LDS load of the wavefront); the caller's LDS queue is empty before them.
-template <int BITS>
-__device__ __forceinline__ void read_scale_bias(CodeRegsT<BITS>& r, uint32_t s_addr, uint32_t b_addr)
-{
-  asm volatile("ds_read_u16 %0, %1" : "=v"(r.s_bits) : "v"(s_addr) : "memory");
-  asm volatile("ds_read_u16 %0, %1" : "=v"(r.b_bits) : "v"(b_addr) : "memory");
-}
-
-__device__ __forceinline__ uint32_t lds_addr_of(const uint8_t* q)
-{
-  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)q;
-}
-
-// 16 bytes per lane, global -> LDS at lds_dst + 16 * lane, written out by hand for the same reason.
-// The LDS base travels in M0, bound as an operand: the compiler writes it and knows its value, as for the
-// builtin form used elsewhere in this kernel (the s_nop is the wait state between that write and the load).
-__device__ __forceinline__ void dma16_raw(uint32_t lds_dst, const uint8_t* src)
-{
-  const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds_dst);
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "{m0}"(m0v) : "memory");
-}
-
 // Waits until at most YOUNGER vector-memory requests issued after r's are outstanding; the
 // registers pass through the statement so that no use of them can be moved above the wait.
 template <int YOUNGER>
@@ -170,49 +131,32 @@ __device__ __forceinline__ void wait_codes(CodeRegsT<8>& r)
   asm volatile("s_waitcnt vmcnt(%4)" : "+v"(r.codes), "+v"(r.codes2), "+v"(r.s_bits), "+v"(r.b_bits) : "n"(YOUNGER) : "memory");
 }
 
-// The same for the register set of a step (one per producer thread in every form built).
-template <int YOUNGER, int BITS>
-__device__ __forceinline__ void wait_codes(CodeRegsT<BITS> (&r)[1]) { wait_codes<YOUNGER>(r[0]); }
-
 }  // namespace
 
-// TMK x TNK: rows of x and weight rows per workgroup: 256 x 128, or 128 x {128, 256} for the grouped
-// form, whose blocks of rows are 128 tall (the wider tile gives a K step as much work as 256 x 128).
-// P: producer wavefronts.  Where the step is as long as a producer's chain (wait, dequantize, store,
-// wait, barrier) -- the 128-row forms, with half the MFMAs per weight -- 8 producers halve that chain.
-// SBR: scales and biases come through an LDS ring in windows of 8 K steps (16 bytes per row and array),
-// brought in by the CONSUMER wavefronts, whose load counter nothing else uses: a 2-byte load per row, array
-// and step costs a 32-byte sector each, twice the bytes of the codes.  Needs K % 512 == 0, 16-byte
-// aligned scales and biases and no split of K.
 // F16: x, scales, biases, the adapter's factors and y are IEEE binary16 (the reference's VPIPE_ELT = half build): the
 // weight tile is f16_rne(fp32(s*q+b)), the MFMA v_mfma_f32_32x32x16_f16; everything else is the same byte traffic.
-template <bool LORA, int TMK = TM, int TNK = TN, bool GROUPED = false, int P = kProducers, bool SBR = false, int BITS = 4,
-          int GROUP = 64, bool F16 = false>
-__global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const TileParams p)
+template <bool LORA, int BITS = 4, int GROUP = 64, bool F16 = false>
+__global__ __launch_bounds__(kThreads) void qmm_tile_kernel(const TileParams p)
 {
-  static_assert(!F16 || (BITS == 4 && GROUP == 64 && !GROUPED && !SBR), "binary16 elements: the plain 4-bit group-64 tile");
-  static_assert((TMK == 256 && TNK == 128 && P == 4) || (TMK == 128 && !LORA && (TNK == 128 || TNK == 256)), "tiles built");
-  static_assert(TMK % (8 * P) == 0 && TNK % (32 * P) == 0, "whole loads per producer");
-  constexpr int kWStage = TNK * kRowB;             // 16 KB at 128 weight rows
-  constexpr int kWH = TNK / (32 * P);              // weight rows (code requests) per producer thread and step
-  constexpr int kJT = TNK / 64;                    // 32-row W fragments per consumer wavefront
-  constexpr int kCR = ((SBR ? 0 : 2) + BITS / 4) * kWH;   // code (, scale and bias) requests per producer thread and step
-  static_assert(BITS == 4 || (BITS == 8 && kWH == 1 && !LORA), "widths built");
+  static_assert(!F16 || (BITS == 4 && GROUP == 64), "binary16 elements: the plain 4-bit group-64 tile");
+  constexpr int P = kProducers;
+  static_assert(TM % (8 * P) == 0 && TN == 32 * P, "whole loads per producer, one weight row per two of its threads");
+  constexpr int kWStage = TN * kRowB;              // 16 KB
+  constexpr int kJT = TN / 64;                     // 32-row W fragments per consumer wavefront
+  constexpr int kCR = 2 + BITS / 4;                // code, scale and bias requests per producer thread and step
+  static_assert(BITS == 4 || (BITS == 8 && !LORA), "widths built");
   // GROUP: values per scale and bias, 64 or 32 (affine_qmm_steel_w4g32, gpu-kernels/metal/quant/
   // affine_qmm_steel.metal:618-640).  A producer thread's 32 values of a step are one group of 32: it reads
   // the scale of its half.
-  static_assert(GROUP == 64 || (GROUP == 32 && !SBR && !GROUPED && !LORA && BITS == 4), "groups built");
+  static_assert(GROUP == 64 || (GROUP == 32 && !LORA && BITS == 4), "groups built");
   constexpr int kGPS = TK / GROUP;                 // groups per K step
   using CodeRegs = CodeRegsT<BITS>;                // BITS: 4, or 8 (one byte per value: gpu-kernels/metal/quant/affine_qmm_steel.metal:1601-1672)
-  constexpr int kSbSlot = 2 * TNK * 16;            // one window of the ring: scales | biases, 16 bytes per row
-  static_assert(!SBR || kWH == 1, "one row per producer thread");
-  constexpr int kWaveM = TMK / (kConsumers / 2);   // x rows per consumer wavefront
+  constexpr int kWaveM = TM / (kConsumers / 2);    // x rows per consumer wavefront
   constexpr int kIT = kWaveM / 32;                 // 32-row x fragments per consumer wavefront
-  constexpr int kXStage = TMK * kRowB;             // 32 KB at 256 rows
-  constexpr int kXL = TMK / (8 * P);               // x-tile loads per producer wavefront and step
+  constexpr int kXStage = TM * kRowB;              // 32 KB
+  constexpr int kXL = TM / (8 * P);                // x-tile loads per producer wavefront and step
   __shared__ __attribute__((aligned(16))) uint8_t x_lds[kStages * kXStage];   // 96 KB
   __shared__ __attribute__((aligned(16))) uint8_t w_lds[kStages * kWStage];   // 48 KB
-  __shared__ __attribute__((aligned(16))) uint8_t sb_ring[SBR ? 2 * kSbSlot : 16];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -225,17 +169,7 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
   const int tile = (int)blockIdx.x - ks * tiles;
   const int tm = tile % p.tiles_m;
   const int tn = tile / p.tiles_m;
-  const int m0 = tm * TMK, n0 = tn * TNK;
-  const uint32_t* pw_base = p.w;
-  const uint16_t* ps_base = p.scales;
-  const uint16_t* pb_base = p.biases;
-  if constexpr (GROUPED) {
-    const int e = p.tile2e[tm];
-    if (e < 0 || e >= p.n_experts) { return; }        // the whole workgroup, before any barrier
-    pw_base += (size_t)e * (size_t)p.N * (size_t)(p.K >> (BITS == 4 ? 3 : 2));
-    ps_base += (size_t)e * (size_t)p.N * (size_t)(p.K >> 6);
-    pb_base += (size_t)e * (size_t)p.N * (size_t)(p.K >> 6);
-  }
+  const int m0 = tm * TM, n0 = tn * TN;
   // This workgroup's K steps: all of them, or its share of a split.
   const int k_first = ks * p.steps_per_split;
   const int KT = p.ksplit > 1 ? ((p.K / TK - k_first) < p.steps_per_split ? (p.K / TK - k_first) : p.steps_per_split)
@@ -247,37 +181,23 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
     const int pt = tid - kConsumers * 64; // 0..64P-1
     // x tile: 32 direct-to-LDS loads per step, 8 per wavefront.  Load i of wave pw covers tile
     // rows (8 pw + i)*8 .. +8; lane l takes row l/8, LDS position l%8.
-    const bool gathered = GROUPED && p.srow != nullptr;
-    const uint8_t* xblk = reinterpret_cast<const uint8_t*>(p.x) + (gathered ? (size_t)0 : (size_t)m0 * p.K * 2) +
-                          (size_t)k_first * (TK * 2);
+    const uint8_t* xblk = reinterpret_cast<const uint8_t*>(p.x) + (size_t)m0 * p.K * 2 + (size_t)k_first * (TK * 2);
     uint32_t a_off[kXL];
 #pragma unroll
     for (int i = 0; i < kXL; ++i) {
       const int row = (pw * kXL + i) * 8 + (lane >> 3);
       const int chunk = swz(row, lane & 7);
-      int rg = (m0 + row < p.M) ? row : (p.M - 1 - m0);
-      if (gathered) {
-        // A padding slot reads row 0 (any readable row): its output is written as zero.
-        const int src = p.srow[m0 + rg];
-        rg = (src >= 0 && src < p.rows_x) ? src : 0;
-      }
+      const int rg = (m0 + row < p.M) ? row : (p.M - 1 - m0);
       a_off[i] = (uint32_t)rg * (uint32_t)p.K * 2u + (uint32_t)chunk * 16u;
     }
-    // W tile: thread pt dequantizes 32 codes of row pt/2 (k half pt%2) per step, and with kWH = 2 those of
-    // row pt/2 + 32 P as well.
+    // W tile: thread pt dequantizes 32 codes of row pt/2 (k half pt%2) per step.
     const int qrow = pt >> 1, qhalf = pt & 1;
-    const uint8_t* wrow[kWH];
-    const uint16_t* srow[kWH];
-    const uint16_t* brow[kWH];
-#pragma unroll
-    for (int h = 0; h < kWH; ++h) {
-      const int qrg = (n0 + qrow + 32 * P * h < p.N) ? (n0 + qrow + 32 * P * h) : (p.N - 1);
-      wrow[h] = reinterpret_cast<const uint8_t*>(pw_base) + (size_t)qrg * (p.K * BITS / 8) + qhalf * (4 * BITS) +
-                (size_t)k_first * (TK * BITS / 8);
-      srow[h] = ps_base + (size_t)qrg * (p.K / GROUP) + (size_t)k_first * kGPS + (GROUP == 32 ? qhalf : 0);
-      brow[h] = pb_base + (size_t)qrg * (p.K / GROUP) + (size_t)k_first * kGPS + (GROUP == 32 ? qhalf : 0);
-    }
-    int b_dst[4];                          // row + 32 P has the same swizzle: + 32 P rows of bytes
+    const int qrg = (n0 + qrow < p.N) ? (n0 + qrow) : (p.N - 1);
+    const uint8_t* wrow = reinterpret_cast<const uint8_t*>(p.w) + (size_t)qrg * (p.K * BITS / 8) + qhalf * (4 * BITS) +
+                          (size_t)k_first * (TK * BITS / 8);
+    const uint16_t* srow = p.scales + (size_t)qrg * (p.K / GROUP) + (size_t)k_first * kGPS + (GROUP == 32 ? qhalf : 0);
+    const uint16_t* brow = p.biases + (size_t)qrg * (p.K / GROUP) + (size_t)k_first * kGPS + (GROUP == 32 ? qhalf : 0);
+    int b_dst[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) { b_dst[i] = qrow * kRowB + swz(qrow, qhalf * 4 + i) * 16; }
 
@@ -290,66 +210,36 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
                                          (__attribute__((address_space(3))) void*)(dst + i * (8 * kRowB)), 16, 0, 0);
       }
     };
-    auto dequant_to = [&](int stage, const CodeRegs (&r)[kWH]) {
+    auto dequant_to = [&](int stage, const CodeRegs& r) {
+      const float sc = elt_bits_to_f32<F16>(r.s_bits), bi = elt_bits_to_f32<F16>(r.b_bits);
+      uint8_t* nb = w_lds + stage * kWStage;
 #pragma unroll
-      for (int h = 0; h < kWH; ++h) {
-        const float sc = elt_bits_to_f32<F16>(r[h].s_bits), bi = elt_bits_to_f32<F16>(r[h].b_bits);
-        uint8_t* nb = w_lds + stage * kWStage + h * (32 * P * kRowB);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if constexpr (BITS == 4) {
-            *reinterpret_cast<uint4*>(nb + b_dst[i]) = dequant_word<F16>(r[h].codes[i], sc, bi);
-          } else {
-            const u32x4& cw = i < 2 ? r[h].codes : r[h].codes2;
-            *reinterpret_cast<uint4*>(nb + b_dst[i]) = dequant_bytes(cw[2 * (i & 1)], cw[2 * (i & 1) + 1], sc, bi);
-          }
-        }
-      }
-    };
-    auto request = [&](CodeRegs (&r)[kWH], int step) {
-#pragma unroll
-      for (int h = 0; h < kWH; ++h) {
-        if constexpr (SBR) {
-          request_codes_only(r[h], wrow[h] + (size_t)step * (TK * BITS / 8));
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (BITS == 4) {
+          *reinterpret_cast<uint4*>(nb + b_dst[i]) = dequant_word<F16>(r.codes[i], sc, bi);
         } else {
-          request_codes(r[h], wrow[h] + (size_t)step * (TK * BITS / 8), srow[h] + step * kGPS, brow[h] + step * kGPS);
+          const u32x4& cw = i < 2 ? r.codes : r.codes2;
+          *reinterpret_cast<uint4*>(nb + b_dst[i]) = dequant_bytes(cw[2 * (i & 1)], cw[2 * (i & 1) + 1], sc, bi);
         }
       }
     };
-    // SBR: scale and bias of this thread's row for step t, from the window t / 8 of the ring.
-    const uint32_t sb_row = lds_addr_of(sb_ring) + (uint32_t)qrow * 16u;
-    auto fetch_sb = [&](CodeRegs (&r)[kWH], int t) {
-      if constexpr (SBR) {
-        const uint32_t a = sb_row + (uint32_t)((t >> 3) & 1) * kSbSlot + (uint32_t)(t & 7) * 2u;
-        read_scale_bias(r[0], a, a + TNK * 16);
-      }
-    };
-    auto settle_sb = [&](CodeRegs (&r)[kWH]) {
-      if constexpr (SBR) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[0].s_bits), "+v"(r[0].b_bits) : : "memory"); }
+    auto request = [&](CodeRegs& r, int step) {
+      request_codes(r, wrow + (size_t)step * (TK * BITS / 8), srow + step * kGPS, brow + step * kGPS);
     };
 
     // Prologue: steps 0 and 1 complete in stages 0 and 1; codes of steps 2 and 3 requested.
-    CodeRegs ra[kWH], rb[kWH];             // codes of even / odd steps
+    CodeRegs ra, rb;             // codes of even / odd steps
     request(ra, 0);
     request(rb, KT > 1 ? 1 : 0);
     issue_x(0, 0);
     if (KT > 1) { issue_x(1, 1); }
     wait_codes<0>(ra);
     wait_codes<0>(rb);
-    if constexpr (SBR) {
-      wg_barrier();                        // the consumers have brought in the first two windows of the ring
-      fetch_sb(ra, 0);
-      fetch_sb(rb, KT > 1 ? 1 : 0);
-      settle_sb(ra);
-      settle_sb(rb);
-    }
     dequant_to(0, ra);
     if (KT > 1) { dequant_to(1, rb); }
     request(ra, KT > 2 ? 2 : 0);
     request(rb, KT > 3 ? 3 : 0);
-    fetch_sb(ra, 2);                       // step 2's scale and bias (window 0)
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(2 * kCR) : "memory");   // all but the code requests of steps 2, 3
-    settle_sb(ra);
     wg_barrier();
 
     // Steady state, step s fills the stage of step t = s+2.  Requests in issue order, with X = kXL
@@ -359,21 +249,17 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
     // steps ago: X + C + X younger requests may stay in flight while they are awaited (19).
     // Before the barrier x(t-1), the tile of step s+1, must have landed: C + X + C younger requests (14).
     // The first fill follows the prologue, where only codes(3) [C] and x(2) [X] are younger (11).
-    // rn: the other register set, which the next fill uses.  SBR: its scale and bias are read from the ring
-    // here, behind this step's work, and have landed by the wait at the end (not in the chain of the next fill).
-    auto fill = [&](auto younger, int t, int stage, CodeRegs (&r)[kWH], CodeRegs (&rn)[kWH]) {
+    auto fill = [&](auto younger, int t, int stage, CodeRegs& r) {
       issue_x(t, stage);
       wait_codes<decltype(younger)::value>(r);
       dequant_to(stage, r);
       request(r, t + 2 < KT ? t + 2 : t);           // the last two requests are never used
-      fetch_sb(rn, t + 1);
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(kXL + 2 * kCR) : "memory");
-      settle_sb(rn);
     };
     auto next_stage = [](int stage) { return stage == kStages - 1 ? 0 : stage + 1; };
     auto odd_fill = [&](int t, int stage) {
       if (t < KT) {
-        fill(std::integral_constant<int, 2 * kXL + kCR>(), t, stage, rb, ra);
+        fill(std::integral_constant<int, 2 * kXL + kCR>(), t, stage, rb);
       } else {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       }
@@ -381,7 +267,7 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
     int tstage = 2;                        // stage of step s+2
     int s = 0;
     if (KT > 2) {
-      fill(std::integral_constant<int, kXL + kCR>(), 2, tstage, ra, rb);
+      fill(std::integral_constant<int, kXL + kCR>(), 2, tstage, ra);
       wg_barrier();
       tstage = next_stage(tstage);
       odd_fill(3, tstage);
@@ -390,7 +276,7 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
       s = 2;
     }
     for (; s + 2 < KT; s += 2) {
-      fill(std::integral_constant<int, 2 * kXL + kCR>(), s + 2, tstage, ra, rb);   // even step: codes in ra
+      fill(std::integral_constant<int, 2 * kXL + kCR>(), s + 2, tstage, ra);   // even step: codes in ra
       wg_barrier();
       tstage = next_stage(tstage);
       odd_fill(s + 3, tstage);
@@ -459,25 +345,10 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
   const int fkh = lane >> 5;       // which 8 of the 16 k
   int w_rd[kJT], x_rd[kIT];        // stage-relative operand rows
 #pragma unroll
-  for (int jt = 0; jt < kJT; ++jt) { w_rd[jt] = (wn * (TNK / 2) + jt * 32 + frow) * kRowB; }
+  for (int jt = 0; jt < kJT; ++jt) { w_rd[jt] = (wn * (TN / 2) + jt * 32 + frow) * kRowB; }
 #pragma unroll
   for (int it = 0; it < kIT; ++it) { x_rd[it] = (wm * kWaveM + it * 32 + frow) * kRowB; }
   const int f_sw = (frow >> 1) & 7;   // the tile offsets are multiples of 16 rows: same swizzle for all
-  // Grouped form: a 32-row fragment of x whose slots are all padding (the tail of an expert's last block)
-  // is neither read nor multiplied; its accumulators stay zero.
-  bool frag_live[kIT];
-#pragma unroll
-  for (int it = 0; it < kIT; ++it) { frag_live[it] = true; }
-  if constexpr (GROUPED) {
-    static_assert(!GROUPED || kWaveM == 64, "one index per lane covers the wavefront's rows");
-    const int* idx = p.srow != nullptr ? p.srow : p.sdst;
-    const int lim = p.srow != nullptr ? p.rows_x : p.rows_y;
-    const int v = idx[m0 + wm * kWaveM + lane];
-    const unsigned long long mask = __ballot(v >= 0 && v < lim);
-#pragma unroll
-    for (int it = 0; it < kIT; ++it) { frag_live[it] = ((mask >> (32 * it)) & 0xffffffffull) != 0; }
-  }
-
   auto mma_stage = [&](int stage, int ksteps) {
     const uint8_t* xb = x_lds + stage * kXStage;
     const uint8_t* wb = w_lds + stage * kWStage;
@@ -490,20 +361,18 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
         for (int jt = 0; jt < kJT; ++jt) { wf[jt] = *reinterpret_cast<const bf16x8*>(wb + w_rd[jt] + c); }
 #pragma unroll
         for (int it = 0; it < kIT; ++it) {
-          if (!GROUPED || frag_live[it]) { xf[it] = *reinterpret_cast<const bf16x8*>(xb + x_rd[it] + c); }
+          xf[it] = *reinterpret_cast<const bf16x8*>(xb + x_rd[it] + c);
         }
 #pragma unroll
         for (int jt = 0; jt < kJT; ++jt) {
 #pragma unroll
           for (int it = 0; it < kIT; ++it) {
-            if (!GROUPED || frag_live[it]) {
-              if constexpr (F16) {
-                typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
-                acc[jt][it] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, wf[jt]),
-                                                                     __builtin_bit_cast(halfx8, xf[it]), acc[jt][it], 0, 0, 0);
-              } else {
-                acc[jt][it] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[jt], xf[it], acc[jt][it], 0, 0, 0);
-              }
+            if constexpr (F16) {
+              typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+              acc[jt][it] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, wf[jt]),
+                                                                   __builtin_bit_cast(halfx8, xf[it]), acc[jt][it], 0, 0, 0);
+            } else {
+              acc[jt][it] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[jt], xf[it], acc[jt][it], 0, 0, 0);
             }
           }
         }
@@ -511,48 +380,13 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
     }
   };
 
-  // SBR: window wdw of the scales and biases (K steps 8 wdw .. 8 wdw + 7) into its slot of the ring.  The
-  // 2 TNK (array, row) entries of a window are dealt out 64 to a load over the four consumer wavefronts.
-  auto issue_window = [&](int wdw) {
-    if constexpr (SBR) {
-      constexpr int kLoads = 2 * TNK / 64 / kConsumers;        // 1 at 128 rows, 2 at 256
-#pragma unroll
-      for (int j = 0; j < kLoads; ++j) {
-        const int e = (wave * kLoads + j) * 64 + lane;         // entry: array e / TNK, row e % TNK
-        const int arr = e / TNK, row = e % TNK;
-        const int rg = (n0 + row < p.N) ? (n0 + row) : (p.N - 1);
-        const uint16_t* src = (arr ? pb_base : ps_base) + (size_t)rg * (p.K >> 6) + (size_t)wdw * 8;
-        dma16_raw(lds_addr_of(sb_ring) + (uint32_t)(wdw & 1) * kSbSlot + (uint32_t)(wave * kLoads + j) * 1024u,
-                  reinterpret_cast<const uint8_t*>(src));
-      }
-    }
-  };
-  if constexpr (SBR) {
-    issue_window(0);
-    if (KT > 8) { issue_window(1); }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    wg_barrier();                        // the producers read the ring from here on
-  }
   wg_barrier();                          // stages 0 and 1 are ready
   int cstage = 0;
-  if constexpr (SBR) {
-    // The producers fill two steps ahead: window s/8 + 1 is first read in step s + 5 and the slot it
-    // replaces (window s/8 - 1) was last read in step s - 4.  Landed before the barrier of step s + 3.
-    for (int s = 0; s < KT; ++s) {
-      if ((s & 7) == 0 && s > 0 && s + 8 < KT) { issue_window((s >> 3) + 1); }
-      mma_stage(cstage, 4);
-      if ((s & 7) == 3) { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // every operand read of this stage is done
-      wg_barrier();
-      cstage = (cstage == kStages - 1) ? 0 : cstage + 1;
-    }
-  } else {
-    for (int s = 0; s < KT; ++s) {
-      mma_stage(cstage, 4);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // every operand read of this stage is done
-      wg_barrier();
-      cstage = (cstage == kStages - 1) ? 0 : cstage + 1;
-    }
+  for (int s = 0; s < KT; ++s) {
+    mma_stage(cstage, 4);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // every operand read of this stage is done
+    wg_barrier();
+    cstage = (cstage == kStages - 1) ? 0 : cstage + 1;
   }
   if (LORA) {
     const int steps = (p.r + TK - 1) / TK;
@@ -578,7 +412,7 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
       for (int jt = 0; jt < kJT; ++jt) {
 #pragma unroll
         for (int rq = 0; rq < 4; ++rq) {
-          const int n = n0 + wn * (TNK / 2) + jt * 32 + rq * 8 + fkh * 4;
+          const int n = n0 + wn * (TN / 2) + jt * 32 + rq * 8 + fkh * 4;
           if (n >= p.N) { continue; }
           if (vec4 && n + 3 < p.N) {
             floatx4 v = {acc[jt][it][rq * 4 + 0], acc[jt][it][rq * 4 + 1], acc[jt][it][rq * 4 + 2], acc[jt][it][rq * 4 + 3]};
@@ -603,21 +437,14 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
       const int m = m0 + wm * kWaveM + it * 32 + frow;
       if (m >= p.M) { continue; }
       uint16_t* yrow = p.y + (size_t)m * p.out_stride + p.out_off;
-      bool pad_slot = false;                 // a padding slot of the grouped form: x = 0, so act(0) * 0 = +0
-      if constexpr (GROUPED) {
-        if (p.srow != nullptr) {
-          const int src = p.srow[m];
-          pad_slot = src < 0 || src >= p.rows_x;
-        }
-      }
 #pragma unroll
       for (int jt = 0; jt < kJT; ++jt) {
 #pragma unroll
         for (int rq = 0; rq < 4; ++rq) {
-          const int n = n0 + wn * (TNK / 2) + jt * 32 + rq * 8 + fkh * 4;
+          const int n = n0 + wn * (TN / 2) + jt * 32 + rq * 8 + fkh * 4;
           if (n >= p.N) { continue; }
-          const float f0 = pad_slot ? 0.0f : gated_f32(p.gate_act, acc[jt][it][rq * 4 + 0], acc[jt][it][rq * 4 + 1]);
-          const float f1 = pad_slot ? 0.0f : gated_f32(p.gate_act, acc[jt][it][rq * 4 + 2], acc[jt][it][rq * 4 + 3]);
+          const float f0 = gated_f32(p.gate_act, acc[jt][it][rq * 4 + 0], acc[jt][it][rq * 4 + 1]);
+          const float f1 = gated_f32(p.gate_act, acc[jt][it][rq * 4 + 2], acc[jt][it][rq * 4 + 3]);
           if (pair_ok && n + 3 < p.N) {
             *reinterpret_cast<uint32_t*>(yrow + (n >> 1)) = pack_elt2<F16>(f0, f1);
           } else {
@@ -634,19 +461,12 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
   for (int it = 0; it < kIT; ++it) {
     const int m = m0 + wm * kWaveM + it * 32 + frow;
     if (m >= p.M) { continue; }
-    int mdst = m;
-    if constexpr (GROUPED) {
-      if (p.sdst != nullptr) {
-        mdst = p.sdst[m];
-        if (mdst < 0 || mdst >= p.rows_y) { continue; }
-      }
-    }
-    uint16_t* yrow = p.y + (size_t)mdst * p.N;
+    uint16_t* yrow = p.y + (size_t)m * p.N;
 #pragma unroll
     for (int jt = 0; jt < kJT; ++jt) {
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq) {
-        const int n = n0 + wn * (TNK / 2) + jt * 32 + rq * 8 + fkh * 4;
+        const int n = n0 + wn * (TN / 2) + jt * 32 + rq * 8 + fkh * 4;
         if (n >= p.N) { continue; }
         const float v0 = acc[jt][it][rq * 4 + 0], v1 = acc[jt][it][rq * 4 + 1];
         const float v2 = acc[jt][it][rq * 4 + 2], v3 = acc[jt][it][rq * 4 + 3];
@@ -665,13 +485,6 @@ __global__ __launch_bounds__((kConsumers + P) * 64) void qmm_tile_kernel(const T
       }
     }
   }
-}
-
-// The scale/bias ring's windows are 16-byte loads of 8 groups: whole windows in every row, aligned.
-static bool sb_ring_ok(const GemmArgs& a)
-{
-  return (a.K % 512) == 0 && (reinterpret_cast<uintptr_t>(a.scales) & 15) == 0 &&
-         (reinterpret_cast<uintptr_t>(a.biases) & 15) == 0;
 }
 
 // The planes of a split over K (no fold).
@@ -707,51 +520,19 @@ hipError_t launch_qmm_tile(hipStream_t st, const GemmArgs& a)
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block(kThreads);
   if (a.bits == 8) {
     if (a.lora_t != nullptr || a.group != 64 || a.f16) { return hipErrorInvalidValue; }     // no 8-bit form with the adapter
-    return launch_kernel(qmm_tile_kernel<false, TM, TN, false, kProducers, false, 8>, grid, block, 0, st, p);
+    return launch_kernel(qmm_tile_kernel<false, 8>, grid, block, 0, st, p);
   }
   if (a.group == 32) {
     if (a.lora_t != nullptr || a.f16) { return hipErrorInvalidValue; }
-    return launch_kernel(qmm_tile_kernel<false, TM, TN, false, kProducers, false, 4, 32>, grid, block, 0, st, p);
+    return launch_kernel(qmm_tile_kernel<false, 4, 32>, grid, block, 0, st, p);
   }
   if (a.f16) {
     return a.lora_t != nullptr
-               ? launch_kernel(qmm_tile_kernel<true, TM, TN, false, kProducers, false, 4, 64, true>, grid, block, 0, st, p)
-               : launch_kernel(qmm_tile_kernel<false, TM, TN, false, kProducers, false, 4, 64, true>, grid, block, 0, st, p);
+               ? launch_kernel(qmm_tile_kernel<true, 4, 64, true>, grid, block, 0, st, p)
+               : launch_kernel(qmm_tile_kernel<false, 4, 64, true>, grid, block, 0, st, p);
   }
   return a.lora_t != nullptr ? launch_kernel(qmm_tile_kernel<true>, grid, block, 0, st, p)
                              : launch_kernel(qmm_tile_kernel<false>, grid, block, 0, st, p);
-}
-
-hipError_t launch_qmm_grouped(hipStream_t st, const GemmArgs& a, const GroupedArgs& g)
-{
-  TileParams p;
-  p.w = a.w; p.scales = a.scales; p.biases = a.biases; p.x = a.x; p.y = a.y;
-  p.lora_t = nullptr; p.lora_b = nullptr;
-  p.K = a.K; p.N = a.N; p.M = a.M; p.r = 0;
-  p.gate_act = a.gate_act;
-  p.out_stride = a.out_stride > 0 ? a.out_stride : a.N / 2;
-  p.out_off = a.out_off;
-  p.tiles_m = a.M / kGroupedBlockRows;       // a.M is a whole number of blocks
-  const bool wide = a.N > TN;                // 128 x 256 tiles unless one 128-wide tile holds all of N
-  p.tiles_n = wide ? (a.N + 2 * TN - 1) / (2 * TN) : 1;
-  p.ksplit = 1; p.steps_per_split = a.K / TK; p.plane = nullptr;
-  p.tile2e = g.tile2e; p.srow = g.srow; p.sdst = g.sdst;
-  p.n_experts = g.n_experts; p.rows_x = g.rows_x; p.rows_y = g.rows_y;
-  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block(kThreads);
-  if (wide) {
-    const dim3 block12((kConsumers + 8) * 64);
-    if (a.bits == 8) {
-      return sb_ring_ok(a)
-                 ? launch_kernel(qmm_tile_kernel<false, kGroupedBlockRows, 2 * TN, true, 8, true, 8>, grid, block12, 0, st, p)
-                 : launch_kernel(qmm_tile_kernel<false, kGroupedBlockRows, 2 * TN, true, 8, false, 8>, grid, block12, 0, st, p);
-    }
-    return sb_ring_ok(a) ? launch_kernel(qmm_tile_kernel<false, kGroupedBlockRows, 2 * TN, true, 8, true>, grid, block12, 0, st, p)
-                         : launch_kernel(qmm_tile_kernel<false, kGroupedBlockRows, 2 * TN, true, 8>, grid, block12, 0, st, p);
-  }
-  if (a.bits == 8) {
-    return launch_kernel(qmm_tile_kernel<false, kGroupedBlockRows, TN, true, kProducers, false, 8>, grid, block, 0, st, p);
-  }
-  return launch_kernel(qmm_tile_kernel<false, kGroupedBlockRows, TN, true>, grid, block, 0, st, p);
 }
 
 }  // namespace vpq
