@@ -83,3 +83,57 @@ def test_grouped_launch_of_the_batch_kernel(vpq, dev, D, fmt):
     for (w, s, b, N), o in zip(packs, outs):
         o.assert_intact()
         assert torch.equal(o.view, single(w, s, b, xd, K, N, M))
+
+
+def _weight64(fmt, w, s, b, K):
+    """The pack in float64, from its words."""
+    bits, group = (8, 64) if fmt == "w8g64" else (4, 32 if fmt in ("w4g32", "q4_0") else 64)
+    q = (w[:, :, None] >> (np.arange(32 // bits, dtype=np.uint32) * bits)) & np.uint32((1 << bits) - 1)
+    q = q.reshape(w.shape[0], K).astype(np.float64)
+    f = (lambda v: v.view(np.float16).astype(np.float64)) if fmt == "f16" else (lambda v: synth.bf16_bits_to_f32(v).astype(np.float64))
+    return q * np.repeat(f(s), group, 1) + np.repeat(f(b), group, 1)
+
+
+@pytest.mark.parametrize("K", [1344, 4096])
+@pytest.mark.parametrize("fmt", ["w4g64", "w4g32", "q4_0", "w8g64", "f16"])
+def test_rows_of_x_that_are_not_finite(vpq, dev, D, fmt, K):
+    # One infinity in a row gives +-inf by the weight's sign (NaN where the weight is zero), opposite infinities and a NaN
+    # give NaN where the plain sum does, and a row whose values only overflow the kernel's offset sums keeps its finite
+    # results.  The other rows of the batch do not notice.
+    N, M = 70, 9
+    rng = np.random.default_rng(K)
+    if fmt == "f16":
+        w, s, b = f16_pack(N, K, 3)
+        x = rng.standard_normal((M, K)).astype(np.float16)
+    else:
+        w, s, b = {"w4g64": synth.make_weight, "w4g32": synth.make_weight_g32, "w8g64": synth.make_weight8,
+                   "q4_0": lambda N, K, seed: synth.make_weight_g32(N, K, seed, q40=True)}[fmt](N, K, 3)
+        x = synth.bf16_bits_to_f32(synth.make_act(M, K, 4))
+    w.reshape(-1)[::3] &= np.uint32(0xff00ff0f)               # codes of zero too
+    bad = x.copy()
+    bad[1, 5] = np.inf
+    bad[3, K - 1] = -np.inf
+    bad[4, 7], bad[4, K // 2] = np.inf, -np.inf
+    bad[6, 70] = np.nan
+    bad[8] *= 1000 if fmt == "f16" else np.float32(2.0 ** 121)
+    as_dev = (lambda a: torch.from_numpy(a.astype(np.float16)).to(dev)) if fmt == "f16" else (lambda a: torch.from_numpy(a).to(dev).bfloat16())
+    sb = [torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).to(dev).view(torch.float16 if fmt == "f16" else torch.bfloat16) for a in (s, b)]
+    run = {"w4g64": vpq.qmv_w4g64, "w4g32": vpq.qmv_w4g32, "w8g64": vpq.qmv_w8g64, "f16": vpq.qmv_w4g64_f16,
+           "q4_0": lambda w, s, b, *a, **k: vpq.qmv_w4g32(w, s, None, *a, scale_only=True, **k)}[fmt]
+    xb, xg = as_dev(bad), as_dev(x)
+    got = run(D.u32(w, dev), *sb, xb, K, N, M, f32out=True).cpu().double()
+    good = run(D.u32(w, dev), *sb, xg, K, N, M, f32out=True).cpu().double()
+    W = _weight64(fmt, w, s, b, K)
+    with np.errstate(invalid="ignore"):
+        want = torch.from_numpy(np.stack([(r[None] * W).sum(1) for r in xb.cpu().double().numpy()]))
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    inf = torch.isinf(want)
+    assert inf[1].any() and inf[3].any() and torch.equal(got[inf], want[inf]) and not torch.isinf(got[~inf]).any()
+    for m in (0, 2, 5, 7):
+        assert torch.equal(got[m], good[m])
+    parity.check_f32(got[8].numpy(), want[8].numpy())
+    if fmt == "w4g64":
+        gated = vpq.qmv_swiglu_w4g64(D.u32(w, dev), *sb, xb, K, N, M).cpu().double()
+        g, u = got[:, 0::2], got[:, 1::2]
+        ref = (g / (1 + torch.exp(-g)) * u).bfloat16().double()
+        assert torch.equal(torch.isnan(gated), torch.isnan(ref)) and torch.equal(torch.isinf(gated), torch.isinf(ref))

@@ -26,6 +26,8 @@
 // accumulator seeded with -128 * sum(x) of the group; 8-bit codes become q itself (exact in bf16).  The result of a
 // group is sum(x q) exactly to fp32 accumulation, then y += scale * sum(x q) + bias * sum(x) in fp32 -- the factored
 // form of gpu-kernels/metal/quant/affine_qmv.metal:151-174.  The weight is never rounded.
+// An output that this form leaves non-finite (an infinity in x meets the seed's opposite infinity, or a code of zero;
+// finite x from 1e36 on) is summed again as x * fma(scale, q, bias) in fp32: +-inf where the plain sum gives +-inf.
 //
 // No inline-assembly VALU instruction may sit near the MFMAs (the compiler's hazard recogniser cannot see what such a
 // statement writes); the asm here is waits only.
@@ -141,6 +143,34 @@ __device__ __forceinline__ u32x4 batch_permute_x(u32x4 d)
   v[2] = __builtin_amdgcn_perm(d[3], d[1], 0x05040100u);
   v[3] = __builtin_amdgcn_perm(d[3], d[1], 0x07060302u);
   return v;
+}
+
+// sum over k of x[k] * fma(scale, q[k], bias) of one output, by a whole wavefront: 16 bytes of codes per lane and pass,
+// the order of the general kernels (vpq_qmv_simple.hip).
+template <int BITS, int GROUP, bool F16, bool SONLY>
+__device__ float batch_plain_sum(const uint8_t* codes, const uint16_t* scales, const uint16_t* biases, const uint16_t* x, int K)
+{
+  constexpr int kPer = 128 / BITS;                          // values of a lane's 16 bytes
+  float acc = 0.0f;
+  for (int k0 = (int)(threadIdx.x & 63) * kPer; k0 < K; k0 += kWave * kPer) {
+    const uint4 c4 = *reinterpret_cast<const uint4*>(codes + (size_t)k0 * BITS / 8);
+    const uint32_t c[4] = {c4.x, c4.y, c4.z, c4.w};
+    const float s = elt_bits_to_f32<F16>(scales[k0 / GROUP]);
+    const float b = SONLY ? -8.0f * s : elt_bits_to_f32<F16>(biases[k0 / GROUP]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      constexpr int kInWord = 32 / BITS;
+#pragma unroll
+      for (int j = 0; j < kInWord; j += 2) {
+        const uint32_t xd = *reinterpret_cast<const uint32_t*>(x + k0 + i * kInWord + j);
+        const float q0 = (float)((c[i] >> (BITS * j)) & ((1u << BITS) - 1));
+        const float q1 = (float)((c[i] >> (BITS * (j + 1))) & ((1u << BITS) - 1));
+        acc = fmaf(elt_lo_to_f32<F16>(xd), fmaf(s, q0, b), acc);
+        acc = fmaf(elt_hi_to_f32<F16>(xd), fmaf(s, q1, b), acc);
+      }
+    }
+  }
+  return wave_sum(acc);
 }
 
 __device__ __forceinline__ void batch_to_lds(const void* src, void* lds_dst)
@@ -512,6 +542,16 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
     const int n_loc = t * 16 + (l & 15);
     const bool ok = m_loc < rows && n_loc < n_live;
     const int m = m0 + m_loc, n = n0 + n_loc;
+    unsigned long long bad = __ballot(ok && (__float_as_uint(total) & 0x7f800000u) == 0x7f800000u);
+    while (bad != 0) {                                       // one output of the wavefront at a time, all lanes on it
+      const int src = __builtin_ctzll(bad);
+      bad &= bad - 1;
+      const int nb_ = __builtin_amdgcn_readlane(n, src), mb = __builtin_amdgcn_readlane(m, src);
+      const float plain = batch_plain_sum<BITS, GROUP, F16, SONLY>(
+          reinterpret_cast<const uint8_t*>(w_) + (size_t)nb_ * row_bytes, scales_ + (size_t)nb_ * Kg,
+          SONLY ? nullptr : biases_ + (size_t)nb_ * Kg, p.x + (size_t)mb * p.K, p.K);
+      if ((int)(threadIdx.x & 63) == src) { total = plain; }
+    }
     if (p.gate_act) {
       // Lanes 2j and 2j+1 hold the gate and the up sum of one feature (N is even).
       const float up = from_neighbour_lane(total);
