@@ -137,3 +137,26 @@ def test_rows_of_x_that_are_not_finite(vpq, dev, D, fmt, K):
         g, u = got[:, 0::2], got[:, 1::2]
         ref = (g / (1 + torch.exp(-g)) * u).bfloat16().double()
         assert torch.equal(torch.isnan(gated), torch.isnan(ref)) and torch.equal(torch.isinf(gated), torch.isinf(ref))
+
+
+@pytest.mark.parametrize("K", [960, 3840, 9664])
+@pytest.mark.parametrize("fmt", ["w4g64", "w4g32", "q4_0", "w8g64", "f16"])
+def test_fp32_results_are_as_close_as_a_plain_sum(vpq, dev, D, fmt, K):
+    # The fp32 output against float64.  A plain fp32 sum of x * (scale q + bias) over such K is 0.7 to 2.3e-7 away
+    # (2-norm, measured on the one-row-a-wavefront kernel); a sum that cancels against a multiple of sum(x) larger
+    # than the codes is 2 to 6e-7 away.  The bound lies between the two, at four roundings of 2^-24.
+    N, M = 256, 7
+    rng = np.random.default_rng(K)
+    if fmt == "f16":
+        w, s, b = f16_pack(N, K, 3)
+        x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float16)).to(dev)
+    else:
+        w, s, b = {"w4g64": synth.make_weight, "w4g32": synth.make_weight_g32, "w8g64": synth.make_weight8,
+                   "q4_0": lambda N, K, seed: synth.make_weight_g32(N, K, seed, q40=True)}[fmt](N, K, 3)
+        x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(dev).bfloat16()
+    sb = [torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).to(dev).view(x.dtype) for a in (s, b)]
+    run = {"w4g64": vpq.qmv_w4g64, "w4g32": vpq.qmv_w4g32, "w8g64": vpq.qmv_w8g64, "f16": vpq.qmv_w4g64_f16,
+           "q4_0": lambda w, s, b, *a, **k: vpq.qmv_w4g32(w, s, None, *a, scale_only=True, **k)}[fmt]
+    got = run(D.u32(w, dev), *sb, x, K, N, M, f32out=True).cpu().double().numpy()
+    want = x.cpu().double().numpy() @ _weight64(fmt, w, s, b, K).T
+    assert np.linalg.norm(got - want) <= 4 * 2.0 ** -24 * np.linalg.norm(want)

@@ -4,9 +4,9 @@
 // What bounds it: HBM for the pack at few rows, issue of vector instructions from 16 rows on (unpacking costs 14 per
 // 16 x 64 codes, every 16 x 16 outputs 8 multiply-adds per group; the vector ALU is 60-72 % busy at 16..48 rows, the
 // matrix pipe a quarter of that).  Measured (us; before: one-item and ring kernels where K % 512 == 0, one wavefront
-// per weight row elsewhere, slabs of 16 rows above 16): 4096 -> 4096 at 16 / 48 rows 9.3 / 20.4 -> 6.0 / 9.5;
-// 4096 -> 12288 13.3 / 38.6 -> 11.8 / 22.6; 5120 -> 151936 at 8 / 16 rows 102 / 124 -> 97 / 114; 3840 -> 19328 at
-// 4 / 16 rows 51 / 156 -> 13.4 / 16.4.
+// per weight row elsewhere, slabs of 16 rows above 16): 4096 -> 4096 at 16 / 48 rows 9.3 / 20.4 -> 6.3 / 10.0;
+// 4096 -> 12288 13.3 / 38.6 -> 12.2 / 21.0; 5120 -> 151936 at 8 / 16 rows 102 / 124 -> 96 / 114; 3840 -> 19328 at
+// 4 / 16 rows 51 / 156 -> 13.5 / 17.4.
 //
 // Split.  A workgroup of eight wavefronts owns T tiles of 16 weight rows and up to 32 rows of x.  K is cut into chunks
 // of 128 bytes of codes per row (256 values of 4 bits, 128 of 8 bits); chunk c belongs to wavefront c % 8, which
@@ -22,12 +22,15 @@
 // banks.  The scales and biases of the workgroup's rows are two contiguous blocks of the pack and are brought in whole,
 // before anything else.
 //
-// Math.  4-bit codes become (128 + q) in bf16 (16 + q in binary16) by one v_and_or_b32 per pair, against an
-// accumulator seeded with -128 * sum(x) of the group; 8-bit codes become q itself (exact in bf16).  The result of a
-// group is sum(x q) exactly to fp32 accumulation, then y += scale * sum(x q) + bias * sum(x) in fp32 -- the factored
-// form of gpu-kernels/metal/quant/affine_qmv.metal:151-174.  The weight is never rounded.
+// Math.  Codes become q itself in the element type (exact).  4 bits: against an accumulator seeded with -8 sum(x) of the
+// group, then y += scale * sum(x (q - 8)) + (bias + 8 scale) * sum(x) in fp32; 8 bits: y += scale * sum(x q) +
+// bias * sum(x) -- the factored form of gpu-kernels/metal/quant/affine_qmv.metal:151-174.  The weight is never rounded.
+// The error is that of the plain sum of x * fma(scale, q, bias) (2-norm against float64, N(0,1) x, K = 3840 / 9664:
+// 4 bits 0.84 / 1.02e-7 against 0.82 / 1.05, groups of 32 0.87 / 1.06 against 0.81 / 1.04, binary16 0.9 / 1.0 against
+// 1.5 / 2.2, 8 bits 1.2 / 1.4 against 1.3 / 2.0).  With codes as 128 + q by one v_and_or_b32 per pair, as many
+// instructions and 2 to 4 % less time, it was five times that: the sum cancels against 128 sum(x).
 // An output that this form leaves non-finite (an infinity in x meets the seed's opposite infinity, or a code of zero;
-// finite x from 1e36 on) is summed again as x * fma(scale, q, bias) in fp32: +-inf where the plain sum gives +-inf.
+// finite x near the end of the range) is summed again as x * fma(scale, q, bias) in fp32: +-inf where the plain sum gives +-inf.
 //
 // No inline-assembly VALU instruction may sit near the MFMAs (the compiler's hazard recogniser cannot see what such a
 // statement writes); the asm here is waits only.
@@ -100,21 +103,23 @@ __device__ __forceinline__ floatx4 batch_mfma(u32x4 a, u32x4 b, floatx4 c)
   }
 }
 
-// Eight nibbles of a word -> eight elements 128+q (bf16) or 16+q (binary16), order [k0,k4,k1,k5,k2,k6,k3,k7].
+// Eight nibbles of a word -> eight elements q, order [k0,k2,k4,k6,k1,k3,k5,k7].  A byte 0..15 read as fp8 (E4M3) is
+// q * 2^-9 (exponent fields 0 and 1 are one linear range), so the scaled conversion by 2^9 gives q, two a time.
 template <bool F16>
-__device__ __forceinline__ u32x4 batch_nibbles(uint32_t word, uint32_t mask, uint32_t magic)
+__device__ __forceinline__ u32x4 batch_nibbles(uint32_t word, uint32_t mask)
 {
+  const uint32_t even = word & mask, odd = (word >> 4) & mask;
   u32x4 v;
   if constexpr (F16) {
-    v[0] = ((word << 6) & mask) | magic;
-    v[1] = ((word << 2) & mask) | magic;
-    v[2] = ((word >> 2) & mask) | magic;
-    v[3] = ((word >> 6) & mask) | magic;
+    v[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(even, 512.0f, false));
+    v[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(even, 512.0f, true));
+    v[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(odd, 512.0f, false));
+    v[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(odd, 512.0f, true));
   } else {
-    v[0] = (word & mask) | magic;
-    v[1] = ((word >> 4) & mask) | magic;
-    v[2] = ((word >> 8) & mask) | magic;
-    v[3] = ((word >> 12) & mask) | magic;
+    v[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, false));
+    v[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, true));
+    v[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, false));
+    v[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, true));
   }
   return v;
 }
@@ -138,10 +143,10 @@ __device__ __forceinline__ u32x4 batch_bytes(uint32_t w0, uint32_t w1)
 __device__ __forceinline__ u32x4 batch_permute_x(u32x4 d)
 {
   u32x4 v;
-  v[0] = __builtin_amdgcn_perm(d[2], d[0], 0x05040100u);
-  v[1] = __builtin_amdgcn_perm(d[2], d[0], 0x07060302u);
-  v[2] = __builtin_amdgcn_perm(d[3], d[1], 0x05040100u);
-  v[3] = __builtin_amdgcn_perm(d[3], d[1], 0x07060302u);
+  v[0] = __builtin_amdgcn_perm(d[1], d[0], 0x05040100u);
+  v[1] = __builtin_amdgcn_perm(d[3], d[2], 0x05040100u);
+  v[2] = __builtin_amdgcn_perm(d[1], d[0], 0x07060302u);
+  v[3] = __builtin_amdgcn_perm(d[3], d[2], 0x07060302u);
   return v;
 }
 
@@ -285,7 +290,8 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
       if (left >= S::XROWB && (i + 1) * kRowsPerLoad <= rows) {
         batch_to_lds(base + (at + x_row), xbuf + i * 1024);
       } else if (i * kRowsPerLoad < rows) {
-        const int row = lane / kXPieces;
+        int row = lane / kXPieces;
+        asm volatile("" : "+v"(row));                       // (the rare path: nothing of it is held over the loop)
         const int last = rows - 1 - i * kRowsPerLoad;
         batch_to_lds(base + (__umul24((uint32_t)(row < last ? row : last), xb) + ((int)at < left ? at : 0)), xbuf + i * 1024);
       }
@@ -324,23 +330,23 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
     __syncthreads();
   }
 
-  uint32_t magic = F16 ? 0x4c004c00u : 0x43004300u;         // 16.0 (binary16) or 128.0 (bf16) in both halves
-  uint32_t mask = F16 ? 0x03c003c0u : 0x000f000fu;
-  asm volatile("" : "+v"(magic));                           // no instruction: only hides the constants
-  asm volatile("" : "+s"(mask));                            // from constant folding
-  // What x is contracted with for sum(x) of a group: the negated offset of the codes (4 bits), or one.
+  uint32_t mask = 0x0f0f0f0fu;
+  asm volatile("" : "+s"(mask));                            // no instruction: only hides the constant from folding
+  // What x is contracted with for sum(x) of a group: the negated middle code (4 bits), or one.
   u32x4 unit;
-  unit[0] = unit[1] = unit[2] = unit[3] = BITS == 8 ? 0x3f803f80u : F16 ? 0xcc00cc00u : 0xc300c300u;
+  unit[0] = unit[1] = unit[2] = unit[3] = BITS == 8 ? 0x3f803f80u : F16 ? 0xc800c800u : 0xc100c100u;
   asm volatile("" : "+v"(unit));
-  constexpr float kBiasOverUnit = BITS == 8 ? 1.0f : F16 ? -0.0625f : -0.0078125f;
 
-  float acc[T][S::AT][S::RA];
+  // One rounding a 64 values of K in the long sum.  Groups of 64: acc sums scale * sum(x (q - middle)), off the offsets
+  // (bias + middle * scale) * sum(x), small for packs whose zero points lie near the middle code.  Groups of 32: off
+  // holds the first of two groups.
+  float acc[T][S::AT][S::RA], off[T][S::AT][S::RA];
 #pragma unroll
   for (int t = 0; t < T; ++t) {
 #pragma unroll
     for (int a = 0; a < S::AT; ++a) {
 #pragma unroll
-      for (int q = 0; q < S::RA; ++q) { acc[t][a][q] = 0.0f; }
+      for (int q = 0; q < S::RA; ++q) { acc[t][a][q] = off[t][a][q] = 0.0f; }
     }
   }
 
@@ -446,7 +452,7 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
           const int jc = gc * S::MPG + j;                    // MFMA of the chunk
           u32x4 b;
           if constexpr (BITS == 4) {
-            b = batch_nibbles<F16>(cw[t][jc], mask, magic);
+            b = batch_nibbles<F16>(cw[t][jc], mask);
           } else {
             b = batch_bytes(cw[t][2 * jc], cw[t][2 * jc + 1]);
           }
@@ -454,18 +460,30 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
           for (int a = 0; a < S::AT; ++a) { s4[a] = batch_mfma<F16>(xq[a][grp * S::MPG + j], b, s4[a]); }
         }
         const float s = (gc & 1) ? elt_hi_to_f32<F16>(sw[t][gc >> 1]) : elt_lo_to_f32<F16>(sw[t][gc >> 1]);
-        float b2;
-        if constexpr (SONLY) {
-          b2 = s * (-8.0f * kBiasOverUnit);
-        } else {
-          b2 = ((gc & 1) ? elt_hi_to_f32<F16>(bw[t][gc >> 1]) : elt_lo_to_f32<F16>(bw[t][gc >> 1])) * kBiasOverUnit;
+        float b2 = 0.0f;                                     // (bias + 8 scale) / -8; 8 bits: the bias
+        if constexpr (!SONLY) {
+          b2 = (gc & 1) ? elt_hi_to_f32<F16>(bw[t][gc >> 1]) : elt_lo_to_f32<F16>(bw[t][gc >> 1]);
+          if (BITS == 4) { b2 = fmaf(b2, -0.125f, -s); }
         }
 #pragma unroll
         for (int a = 0; a < S::AT; ++a) {
 #pragma unroll
           for (int q = 0; q < S::RA; ++q) {
-            acc[t][a][q] = fmaf(s, s4[a][q], acc[t][a][q]);
-            acc[t][a][q] = fmaf(b2, xs[a][q], acc[t][a][q]);
+            if constexpr (BITS == 8) {
+              acc[t][a][q] = fmaf(s, s4[a][q], acc[t][a][q]);
+              acc[t][a][q] = fmaf(b2, xs[a][q], acc[t][a][q]);
+            } else if constexpr (GROUP == 64) {
+              acc[t][a][q] = fmaf(s, s4[a][q], acc[t][a][q]);
+              off[t][a][q] = fmaf(b2, xs[a][q], off[t][a][q]);
+            } else {
+              float v = (grp & 1) == 0 ? s * s4[a][q] : fmaf(s, s4[a][q], off[t][a][q]);
+              if (!SONLY) { v = fmaf(b2, xs[a][q], v); }
+              if ((grp & 1) == 0 && !(decltype(part_c)::value && grp + 1 >= live)) {
+                off[t][a][q] = v;
+              } else {
+                acc[t][a][q] += v;
+              }
+            }
           }
         }
       }
@@ -522,7 +540,7 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
     for (int a = 0; a < S::AT; ++a) {
 #pragma unroll
       for (int q = 0; q < S::RA; ++q) {
-        sums[(((t * S::AT + a) * S::RA + q) * kBatchWaves + wave) * kWave + lane] = acc[t][a][q];
+        sums[(((t * S::AT + a) * S::RA + q) * kBatchWaves + wave) * kWave + lane] = BITS == 4 && GROUP == 64 ? acc[t][a][q] + off[t][a][q] : acc[t][a][q];
       }
     }
   }
