@@ -196,7 +196,9 @@ int vpq_qmm_tiled_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint1
  * unsplit kernel only by the fp32 reassociation and are bit-reproducible.  No
  * adapter, no gated store.  `ws`: vpq_qmm_workspace_bytes() bytes (0 where the
  * automatic choice is not to split), 256-byte aligned, contents irrelevant.
- * VPQ_ERR_WORKSPACE if it is needed and missing or too small. */
+ * VPQ_ERR_WORKSPACE if it is needed and missing or too small; with `splits` 0 it
+ * is needed where 256 x 128 tiles would fill at most half of the chip and take a
+ * tenth longer unsplit, and elsewhere the call runs unsplit without it. */
 size_t vpq_qmm_workspace_bytes(int K, int N, int M);
 int vpq_qmm_splitk_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
                               const uint16_t* biases, const uint16_t* x, uint16_t* y,

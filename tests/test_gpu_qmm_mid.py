@@ -77,3 +77,20 @@ def test_qmm_mid_uneven_shares(vpq, oracle, dev, D, K, N, M, splits):
     torch.cuda.synchronize()
     out.assert_intact()
     parity.check_bf16(D.bits(out.view), y64, yb)
+
+
+@pytest.mark.parametrize("K,N,M,taken", [(5120, 12288, 333, True), (12288, 5120, 1024, True), (4096, 512, 128, False)])
+def test_automatic_split_without_a_workspace(vpq, dev, K, N, M, taken):
+    # 256 x 128 tiles that fill more than half of the chip by themselves need no workspace: the call runs unsplit;
+    # a few tiles over a long K are refused without it
+    gen = torch.Generator(device=dev).manual_seed(K + M)
+    w = torch.randint(-2 ** 31, 2 ** 31, (N, K // 8), dtype=torch.int32, device=dev, generator=gen)
+    s = torch.empty((N, K // 64), device=dev).uniform_(0.005, 0.02, generator=gen).bfloat16()
+    x = torch.randn((M, K), device=dev, generator=gen).bfloat16()
+    b, y = -8 * s, torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+    L, p = vpq.load(), [t.data_ptr() for t in (w, s, b, x, y)]
+    status = L.vpq_qmm_splitk_w4g64_bf16(torch.cuda.current_stream().cuda_stream, *p, K, N, M, 0, None, 0)
+    torch.cuda.synchronize()
+    assert status == (0 if taken else -4)
+    if taken:
+        assert torch.equal(y, vpq.qmm_w4g64(w, s, b, x, K, N, M))

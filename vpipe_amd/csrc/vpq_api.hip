@@ -608,7 +608,11 @@ int vpq_qmm_splitk_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint
   if (!aligned(x, 16) || !aligned(y, 16) || (ws != nullptr && !aligned(ws, 256))) { return VPQ_ERR_MISALIGNED; }
   st = ensure_init();
   if (st != VPQ_OK) { return st; }
-  if (splits == 0) { splits = vpq::qmm_choose_splits(K, N, M, g_dev.cu_count); }
+  const auto room = [&](int n) { return ws != nullptr && ws_bytes >= (size_t)n * (size_t)M * (size_t)N * sizeof(float); };
+  if (splits == 0) {
+    splits = vpq::qmm_choose_splits(K, N, M, g_dev.cu_count);
+    if (splits > 1 && !room(splits)) { splits = vpq::qmm_required_splits(K, N, M, g_dev.cu_count); }
+  }
   if (splits > K / 64) { splits = K / 64; }
   vpq::GemmArgs g{};
   g.w = w; g.scales = scales; g.biases = biases; g.x = x; g.y = y;
@@ -616,7 +620,7 @@ int vpq_qmm_splitk_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint
   g.cu_count = g_dev.cu_count;
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
   if (splits <= 1) { return gemm_by_size(hs, g); }
-  if (ws == nullptr || ws_bytes < (size_t)splits * (size_t)M * (size_t)N * sizeof(float)) { return VPQ_ERR_WORKSPACE; }
+  if (!room(splits)) { return VPQ_ERR_WORKSPACE; }
   return finish(vpq::launch_qmm_splitk(hs, g, splits, static_cast<float*>(ws)));
 }
 

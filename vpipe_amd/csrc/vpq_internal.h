@@ -257,6 +257,7 @@ GemmKernel qmm_choose(const GemmArgs& a);
 // Split-K (no adapter, no gated store, bf16): `splits` shares of the K steps on that kernel or the 256 x 128 one, fp32
 // planes [splits][M][N] in `plane`, then a fold.  qmm_choose_splits() returns 1 where that does not pay.
 int qmm_choose_splits(int K, int N, int M, int cu_count);
+int qmm_required_splits(int K, int N, int M, int cu_count);   // an automatic split without room for it is refused if > 1
 size_t qmm_splitk_workspace_bytes(int K, int N, int M, int cu_count);
 hipError_t launch_qmm_splitk(hipStream_t st, const GemmArgs& a, int splits, float* plane);
 // y[M,N] = x[M,K] . b[N,K]^T on the large-tile kernel with dense 2-byte weights (bf16, or binary16 with f16;

@@ -569,6 +569,25 @@ int qmm_choose_splits(int K, int N, int M, int cu_count)
   return best;
 }
 
+// The count that an automatic split may not go without room for: two and more where 256 x 128 tiles that fill less than
+// half of the chip would take a tenth longer unsplit (0.9 us a step of 64, 3 us a round, planes at 4 TB/s).  Callers without a workspace
+// are refused there and nowhere else.
+int qmm_required_splits(int K, int N, int M, int cu_count)
+{
+  const int cus = cu_count > 0 ? cu_count : 256;
+  const int steps = K / 64, tiles = ((M + 255) / 256) * ((N + 127) / 128);
+  if (tiles * 2 > cus) { return 1; }
+  int best = 1;
+  double best_us = 3.0 + 0.9 * steps;
+  for (int s = 2; s <= 16 && steps / s >= 4; ++s) {
+    const int per = (steps + s - 1) / s;
+    if ((steps + per - 1) / per != s) { continue; }
+    const double us = (tiles * s + cus - 1) / cus * (3.0 + 0.9 * per) + 3.0 + (s + 0.5) * (double)M * (double)N * 1e-6;
+    if (us < 0.9 * best_us) { best = s; best_us = us; }
+  }
+  return best;
+}
+
 size_t qmm_splitk_workspace_bytes(int K, int N, int M, int cu_count)
 {
   const int s = qmm_choose_splits(K, N, M, cu_count);
