@@ -204,6 +204,15 @@ int vpq_qmm_splitk_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint
                               const uint16_t* biases, const uint16_t* x, uint16_t* y,
                               int K, int N, int M, int splits, void* ws, size_t ws_bytes);
 
+/* Which kernel the fused GEMM entrances of a format (4 or 8 bits, groups of 64 or
+ * 32, binary16 elements, gated store) take for a shape whose pack is 16-byte
+ * aligned, without an adapter: 64, 96 or 128 = 128 weight rows against that many
+ * rows of x per workgroup, 256 = the 256 x 128 tile, -128, -192 or -256 = the large
+ * tile at that width; all give the same bits.  `splits` > 1: of a call that splits K
+ * so.  A negative vpq_status (above -128) for a shape they do not take.  For tests
+ * and measurement; needs no device (256 CUs are assumed without one). */
+int vpq_qmm_plan(int K, int N, int M, int bits, int group, int f16, int gated, int splits);
+
 /* ---- a8: the dequant-once route -------------------------------------------
  * Replaces `gemm_mma_` (generative-models/minimax-h3/metal-minimax-h3-transformer.cc:
  * 2020-2160: `affine_dequant_w4g64` into a scratch, then a dense matrix-unit GEMM,

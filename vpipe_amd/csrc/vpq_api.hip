@@ -513,14 +513,13 @@ int vpq_lora_a_bf16(vpq_stream_t stream, const uint16_t* x, const uint16_t* lora
 
 namespace {
 
-// The fused GEMM by size, for every format: the three kernels give the same bits.  The large-tile kernel from one round
-// of its tiles on (1.02-1.16 against 0.83-0.91 PFLOP/s of the 256 x 128 tiles at M = 16320, 0.98 against 0.78 at
-// 4096 -> 12288 and 0.94 against 0.91 at 12288 -> 4096 with M = 2048), unless the 128-row kernel's tiles fit M better.
+// The fused GEMM by size, for every format: the three kernels give the same bits, so it is the one that a model of
+// their measured times says is fastest (vpq_qmm_mid.hip).
 int gemm_by_size(hipStream_t hs, const vpq::GemmArgs& g)
 {
-  const vpq::GemmKernel k = vpq::qmm_choose(g);
-  if (k == vpq::GemmKernel::kBig) { return finish(vpq::launch_qmm_big(hs, g, 0)); }
-  return finish(k == vpq::GemmKernel::kMid ? vpq::launch_qmm_mid(hs, g) : vpq::launch_qmm_tile(hs, g));
+  const vpq::GemmChoice c = vpq::qmm_choose(g);
+  if (c.kernel == vpq::GemmKernel::kBig) { return finish(vpq::launch_qmm_big(hs, g, c.width)); }
+  return finish(c.kernel == vpq::GemmKernel::kMid ? vpq::launch_qmm_mid(hs, g) : vpq::launch_qmm_tile(hs, g));
 }
 
 // tile: 0 = by size, 128 = the 256 x 128 tile kernel, 192 / 256 = the large-tile kernel at that width,
@@ -595,6 +594,22 @@ size_t vpq_qmm_workspace_bytes(int K, int N, int M)
   if (K <= 0 || N <= 0 || M <= 0 || (K % 64) != 0) { return 0; }
   if (ensure_init() != VPQ_OK) { return 0; }
   return (vpq::qmm_splitk_workspace_bytes(K, N, M, g_dev.cu_count) + 255) / 256 * 256;
+}
+
+int vpq_qmm_plan(int K, int N, int M, int bits, int group, int f16, int gated, int splits)
+{
+  if (K <= 0 || N <= 0 || M <= 0 || (K % 64) != 0 || splits < 0 || splits > 16 || (gated != 0 && (splits > 1 || (N & 1) != 0)) ||
+      !((bits == 4 && (group == 64 || (group == 32 && f16 == 0))) || (bits == 8 && group == 64 && f16 == 0)) ||
+      (splits > 1 && (bits != 4 || group != 64 || f16 != 0))) {
+    return VPQ_ERR_BAD_SHAPE;
+  }
+  (void)ensure_init();                     // (without a device: the plan for 256 CUs)
+  vpq::GemmArgs g{};
+  g.K = K; g.N = N; g.M = M;
+  g.bits = bits; g.group = group; g.f16 = f16 != 0;
+  g.gate_act = gated != 0 ? VPQ_GATE_SWIGLU : 0;
+  g.cu_count = g_dev.cu_count;
+  return vpq::qmm_plan(g, splits);
 }
 
 int vpq_qmm_splitk_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,

@@ -253,7 +253,12 @@ hipError_t launch_qmm_big(hipStream_t st, const GemmArgs& a, int tile_n);
 hipError_t launch_qmm_mid(hipStream_t st, const GemmArgs& a);
 // Which of the three takes least for this call (a rule on sizes, alignment and format).
 enum class GemmKernel { kTile, kBig, kMid };
-GemmKernel qmm_choose(const GemmArgs& a);
+struct GemmChoice {
+  GemmKernel kernel;
+  int width;             // kBig: weight rows per tile
+};
+GemmChoice qmm_choose(const GemmArgs& a);
+int qmm_plan(const GemmArgs& a, int splits);   // as vpq_qmm_plan
 // Split-K (no adapter, no gated store, bf16): `splits` shares of the K steps on that kernel or the 256 x 128 one, fp32
 // planes [splits][M][N] in `plane`, then a fold.  qmm_choose_splits() returns 1 where that does not pay.
 int qmm_choose_splits(int K, int N, int M, int cu_count);

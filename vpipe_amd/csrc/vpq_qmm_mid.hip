@@ -454,78 +454,123 @@ hipError_t mid_launch_as(hipStream_t st, const GemmArgs& a, int mt, int splits, 
   return a.f16 ? mid_launch<4, 64, true>(st, p, mt, grid) : mid_launch<4, 64, false>(st, p, mt, grid);
 }
 
-// What a GEMM takes, in microseconds; measured on 1024..24576 x 4096..12288 at 80..1024 rows, to about a tenth.  A split
-// writes and reads its planes once more, and folds them in a launch of its own, at about 4 TB/s.
-double planes_us(int N, int M, int splits) { return splits > 1 ? 3.0 + (splits + 0.5) * (double)M * (double)N * 4.0 / 4.0e6 : 0.0; }
+// What a GEMM takes, in microseconds: fitted to 36 000 timings of the seven kernels (three heights here, 256 x 128, three
+// large tiles) on 512..17408 x 512..34816 at 65..4096 rows, all four formats and gated stores, which it meets to a
+// twentieth.  Its choice is 0.8 % off the fastest on average.  Against the rule "the large tile from one round of its
+// tiles on, else the 256 x 128 tile" it takes 0.72 of the time, and in 14 of 5500 cases 4 to 8 % more.
+//
+// A split writes and reads its planes once more, and folds them in a launch of its own.
+double planes_us(int N, int M, int splits) { return splits > 1 ? 3.0 + (splits + 0.5) * (double)M * (double)N * 4.0 / 5.0e6 : 0.0; }
 
-// This kernel, per step of 64: a workgroup alone on its CU, and each of several that share one (the busiest CU counts).
-constexpr double kMidAlone[5] = {0, 0, 0.50, 0.57, 0.66}, kMidShared[5] = {0, 0, 0.39, 0.48, 0.61};
+constexpr int kXcds = 8;
 
-double mid_us(int K, int N, int M, int mt, int splits, int cus)
+// Shape of a call, as far as its time goes.
+struct CostShape { int K, N, M, bits; bool gated; };
+
+// This kernel: a round of one workgroup per CU costs `round` (`gated` with that store) and `step` per 64 of K, `alone` if
+// there is only that round.
+// The busiest XCD counts (all workgroups of a weight tile are on one).  Every weight tile reads all of x, at 6.8 TB/s
+// from the shared cache once x outgrows an XCD's L2; that bounds M in the thousands.
+struct MidCost { double fixed, round, gated, step, alone; };
+constexpr MidCost kMidCost[5] = {{}, {}, {5.8, 0.4, 0.8, 0.335, 0.485}, {5.4, 1.2, 1.9, 0.406, 0.556}, {4.3, 2.8, 4.1, 0.468, 0.645}};
+
+double mid_us(const CostShape& s, int mt, int splits, int cus)
 {
-  const int steps = K / 64, per = (steps + splits - 1) / splits;
-  const long wgs = (long)((M + 32 * mt - 1) / (32 * mt)) * ((N + kMidTileN - 1) / kMidTileN) * splits;
-  const double step = (double)((wgs + cus - 1) / cus) * kMidShared[mt];
-  return 4.0 + per * (step > kMidAlone[mt] ? step : kMidAlone[mt]) + planes_us(N, M, splits);
+  const MidCost& c = kMidCost[mt];
+  const int steps = s.K / 64, per = (steps + splits - 1) / splits;
+  const int per_xcd = cus >= kXcds ? cus / kXcds : 1;
+  const long tiles_n = (s.N + kMidTileN - 1) / kMidTileN;
+  const long wgs = (tiles_n * splits + kXcds - 1) / kXcds * ((s.M + 32 * mt - 1) / (32 * mt));
+  const double round = s.gated ? c.gated : c.round;
+  const double busy = (double)((wgs + per_xcd - 1) / per_xcd) * (per * c.step * (s.bits == 8 ? 1.1 : 1.0) + round);
+  const double alone = per * c.alone + round, fetch = (double)tiles_n * (double)s.M * (double)s.K * 2.0 / 6.8e6;
+  const double us = busy > alone ? busy : alone;
+  return c.fixed + (us > fetch ? us : fetch) + planes_us(s.N, s.M, splits);
 }
 
 // Rows of x per workgroup, in 32s: the count that takes least.
-int mid_rows(int K, int N, int M, int splits, int cus)
+int mid_rows(const CostShape& s, int splits, int cus)
 {
   int best = 4;
   for (int mt = 3; mt >= 2; --mt) {
-    if (mid_us(K, N, M, mt, splits, cus) < mid_us(K, N, M, best, splits, cus)) { best = mt; }
+    if (mid_us(s, mt, splits, cus) < mid_us(s, best, splits, cus)) { best = mt; }
   }
   return best;
 }
 
-// The kernels with 256 rows of x a workgroup, one workgroup per CU.  `step` is that of a full chip; the 256 x 128 tiles
-// take 0.89 on a nearly idle one (its clock is higher), 1.1 on a full one, the large tile 1.62 at 256 x 192.
-double tall_us(int K, int N, int M, int width, double step, int splits, int cus)
+// The kernels with 256 rows of x a workgroup, one workgroup per CU: `step` (`step8`: 8-bit codes) and `round` are those
+// of a full chip, a round that leaves CUs idle takes `part` of them and up (the clock rises as the load falls).
+struct TallCost { int width; double fixed, round, gated, step, step8, part; };
+constexpr TallCost kTileCost = {128, 4.1, 6.4, 9.6, 1.04, 1.07, 0.79};
+constexpr TallCost kBigCost[3] = {{256, 5.6, 7.4, 25.4, 1.58, 0.0, 0.70},
+                                  {192, 5.5, 5.8, 16.4, 1.30, 1.35, 0.72},
+                                  {128, 4.6, 3.8, 10.0, 1.03, 0.98, 0.76}};
+
+double tall_us(const TallCost& c, const CostShape& s, int splits, int cus)
 {
-  const int steps = K / 64, per = (steps + splits - 1) / splits;
-  const long tiles = (long)((M + 255) / 256) * ((N + width - 1) / width) * splits;
-  const double fill = tiles < cus ? (double)tiles / cus : 1.0;
-  return 4.0 + per * step * (0.8 + 0.2 * fill) * (double)((tiles + cus - 1) / cus) + planes_us(N, M, splits);
+  const int steps = s.K / 64, per = (steps + splits - 1) / splits;
+  const long tiles = (long)((s.M + 255) / 256) * ((s.N + c.width - 1) / c.width) * splits;
+  const long full = tiles / cus;
+  const double rest = (double)(tiles - full * cus) / cus;
+  const double rounds = (double)full + (rest > 0.0 ? c.part + (1.0 - c.part) * rest * rest : 0.0);
+  return c.fixed + (per * (s.bits == 8 ? c.step8 : c.step) + (s.gated ? c.gated : c.round)) * rounds +
+         planes_us(s.N, s.M, splits);
 }
 
-constexpr double kTileStep = 1.1;
-
-bool tile_splits_better(int K, int N, int M, int splits, int cus)
+bool tile_splits_better(const CostShape& s, int splits, int cus)
 {
-  return tall_us(K, N, M, 128, kTileStep, splits, cus) < mid_us(K, N, M, mid_rows(K, N, M, splits, cus), splits, cus);
+  return tall_us(kTileCost, s, splits, cus) < mid_us(s, mid_rows(s, splits, cus), splits, cus);
 }
 
-// The kernel that takes least without a split of K, and how long.
-GemmKernel choose_unsplit(const GemmArgs& a, double* us)
+CostShape cost_shape(const GemmArgs& a) { return CostShape{a.K, a.N, a.M, a.bits, a.gate_act != 0}; }
+
+// The kernel that takes least without a split of K (for the large tile: its width too), and how long.
+GemmChoice choose_unsplit(const GemmArgs& a, double* us)
 {
   const int cus = a.cu_count > 0 ? a.cu_count : 256;
-  const int tm = (a.M + 255) / 256;
-  double big = 1e30;
-  // below one round of its tiles the large-tile kernel has nothing over the 256 x 128 one
-  if (qmm_big_supports(a)) {
-    const int bn = qmm_big_tile_n(a.N, a.M, cus, a.bits == 8 ? 192 : 256, a.group != 32);
-    if ((long)tm * ((a.N + bn - 1) / bn) >= cus) { big = tall_us(a.K, a.N, a.M, bn, bn == 256 ? 2.05 : bn == 192 ? 1.62 : 1.14, 1, cus); }
+  const CostShape s = cost_shape(a);
+  const long tm = (a.M + 255) / 256;
+  GemmChoice best{GemmKernel::kTile, 0};
+  *us = tall_us(kTileCost, s, 1, cus);
+  if (a.lora_t != nullptr) {                        // with an adapter: the large tile from one round of its tiles on
+    const int bn = qmm_big_tile_n(a.N, a.M, cus);
+    if (qmm_big_supports(a) && tm * ((a.N + bn - 1) / bn) >= cus) { best = {GemmKernel::kBig, bn}; }
+    return best;
   }
-  const double tile = tall_us(a.K, a.N, a.M, 128, kTileStep, 1, cus);
-  const double mid = a.lora_t != nullptr ? 1e30 : mid_us(a.K, a.N, a.M, mid_rows(a.K, a.N, a.M, 1, cus), 1, cus);
-  const bool takes_big = big < 1e30 && big <= mid, takes_mid = !takes_big && mid <= tile;
-  *us = takes_big ? big : takes_mid ? mid : tile;
-  return takes_big ? GemmKernel::kBig : takes_mid ? GemmKernel::kMid : GemmKernel::kTile;
+  const double mid = mid_us(s, mid_rows(s, 1, cus), 1, cus);
+  if (mid <= *us) { best.kernel = GemmKernel::kMid; *us = mid; }
+  if (!qmm_big_supports(a)) { return best; }
+  for (const TallCost& c : kBigCost) {
+    if ((c.width == 256 && a.bits == 8) || (c.width == 192 && a.group == 32)) { continue; }   // (not built)
+    // (with idle CUs the model is less sure of this kernel, and little is to be had)
+    if (tm * ((a.N + c.width - 1) / c.width) * 5 < (long)cus * 4) { continue; }
+    const double big = tall_us(c, s, 1, cus);
+    if (big < *us) { best = {GemmKernel::kBig, c.width}; *us = big; }
+  }
+  return best;
 }
 
 }  // namespace
 
-GemmKernel qmm_choose(const GemmArgs& a)
+GemmChoice qmm_choose(const GemmArgs& a)
 {
   double us;
   return choose_unsplit(a, &us);
 }
 
+int qmm_plan(const GemmArgs& a, int splits)
+{
+  const int cus = a.cu_count > 0 ? a.cu_count : 256;
+  const CostShape s = cost_shape(a);
+  if (splits > 1) { return tile_splits_better(s, splits, cus) ? 256 : 32 * mid_rows(s, splits, cus); }
+  const GemmChoice c = qmm_choose(a);
+  return c.kernel == GemmKernel::kBig ? -c.width : c.kernel == GemmKernel::kTile ? 256 : 32 * mid_rows(s, 1, cus);
+}
+
 hipError_t launch_qmm_mid(hipStream_t st, const GemmArgs& a)
 {
   const int cus = a.cu_count > 0 ? a.cu_count : 256;
-  return mid_launch_as(st, a, mid_rows(a.K, a.N, a.M, 1, cus), 1, nullptr);
+  return mid_launch_as(st, a, mid_rows(cost_shape(a), 1, cus), 1, nullptr);
 }
 
 hipError_t launch_qmm_grouped(hipStream_t st, const GemmArgs& a, const GroupedArgs& g)
@@ -555,6 +600,7 @@ int qmm_choose_splits(int K, int N, int M, int cu_count)
   const int steps = K / 64;
   GemmArgs a{};
   a.K = K; a.N = N; a.M = M; a.cu_count = cus;
+  const CostShape shape = cost_shape(a);
   double best_us;
   choose_unsplit(a, &best_us);
   int best = 1;
@@ -562,8 +608,8 @@ int qmm_choose_splits(int K, int N, int M, int cu_count)
   for (int s = 2; s <= 16 && steps / s >= 4; ++s) {
     const int per = (steps + s - 1) / s;
     if ((steps + per - 1) / per != s) { continue; }    // shares would come out uneven: another count covers it
-    const double us = tile_splits_better(K, N, M, s, cus) ? tall_us(K, N, M, 128, kTileStep, s, cus)
-                                                          : mid_us(K, N, M, mid_rows(K, N, M, s, cus), s, cus);
+    const double us = tile_splits_better(shape, s, cus) ? tall_us(kTileCost, shape, s, cus)
+                                                        : mid_us(shape, mid_rows(shape, s, cus), s, cus);
     if (us < best_us) { best = s; best_us = us; }
   }
   return best;
@@ -598,9 +644,9 @@ hipError_t launch_qmm_splitk(hipStream_t st, const GemmArgs& a, int splits, floa
 {
   const int cus = a.cu_count > 0 ? a.cu_count : 256;
   const int steps = a.K / 64, per = (steps + splits - 1) / splits;
-  const hipError_t e = tile_splits_better(a.K, a.N, a.M, splits, cus)
+  const hipError_t e = tile_splits_better(cost_shape(a), splits, cus)
                            ? launch_qmm_tile_planes(st, a, splits, plane)
-                           : mid_launch_as(st, a, mid_rows(a.K, a.N, a.M, splits, cus), splits, plane);
+                           : mid_launch_as(st, a, mid_rows(cost_shape(a), splits, cus), splits, plane);
   if (e != hipSuccess) { return e; }
   const size_t count = (size_t)a.M * (size_t)a.N;
   const bool quads = (count & 3) == 0;
