@@ -77,9 +77,8 @@ def test_qmv_f16_several_rows_ring_kernel(vpq, oracle, dev, D, K, N, M):
 
 
 @pytest.mark.parametrize("M", [2, 3, 4])
-def test_qmv_f16_lm_head_rows_streaming_kernel(vpq, oracle, dev, D, M):
-    """2..4 rows over an lm_head-sized pack (>= 150 MB of codes) run on the streaming MFMA kernel's binary16 mode.
-    Full-size launch; the oracle evaluates a sample of output rows (first and last tiles included)."""
+def test_qmv_f16_lm_head_rows(vpq, oracle, dev, D, M):
+    """2..4 rows over an lm_head-sized pack (>= 150 MB of codes), on the batch kernel.  Full-size launch; the oracle evaluates a sample of output rows (first and last tiles included)."""
     K, N = 5120, 151936
     w, s, b = f16_pack(N, K, 1200 + M)
     x = np.random.default_rng(1250 + M).standard_normal((M, K)).astype(np.float16).view(np.uint16)
@@ -183,15 +182,17 @@ def test_qmm_f16_dense_route(vpq, oracle, dev, D, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(64, 64, 512), (130, 328, 1024), (257, 136, 512), (300, 520, 1536), (33, 200, 448),
-                                   (513, 130, 1088), (2304, 8192, 512)])
+                                   (513, 130, 1088), (2304, 8192, 512),
+                                   (2048, 12288, 512), (4100, 6144, 512), (4100, 1026, 192)])
 def test_qmm_f16_fused(vpq, oracle, dev, D, M, N, K):
     """The fused GEMM on binary16 elements (weight tile = f16(s q + b), f16 MFMA, fp32 accumulation): against
     the oracle's rounded-weight twin, bit for bit against the dequant-once route (same tiles, same order of
     accumulation), gated stores against the oracle's activations, guard bands intact."""
     w, s, b = f16_pack(N, K, 700 + M)
     x = np.random.default_rng(701 + M).standard_normal((M, K)).astype(np.float16).view(np.uint16)
-    # rows are independent: the shape with enough tiles for the large-tile kernel is checked on a sample of them
-    rows = np.arange(M) if M * N * K < 2e9 else np.r_[0:40, 1000:1024, M - 40:M]
+    # (with 256 CUs: 64 rows of x per workgroup up to (513, 130, 1088), then 96, the large tile 192 and 256 wide, the
+    # 256 x 128 tile.)  Rows are independent: the long shapes are checked on a sample of them
+    rows = np.arange(M) if M < 1000 else np.r_[0:40, 1000:1024, M - 40:M]
     y64, _ = oracle.matmul_f16(w, s, b, x[rows], K, N, len(rows), rounded=True)
     wd, sd, bd, xd = D.u32(w, dev), dev16(s, dev), dev16(b, dev), dev16(x, dev)
     out = parity.Guarded((M, N), torch.float16, dev)

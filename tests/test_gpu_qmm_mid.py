@@ -1,6 +1,8 @@
 """The GEMM with 128-row weight tiles (vpq_qmm_mid.hip) where it can go wrong: K that ends inside a chunk of codes or
-has an odd number of groups, fewer steps of K than x stages, N and M that end inside a tile, each count of rows of x per
-workgroup, split shares of uneven length -- against the oracle and, bit for bit, the 256 x 128 tile kernel."""
+has an odd number of groups, fewer steps of K than x stages, N and M that end inside a tile, split shares of uneven
+length -- against the oracle and, bit for bit, the 256 x 128 tile kernel; then every kernel that the size-based GEMM
+chooses from (each count of rows of x per workgroup here, the 256 x 128 tile, each width of the large tile), in every
+format it is built for, at shapes that take it, with M and N that end inside a tile."""
 import numpy as np
 import pytest
 import torch
@@ -11,7 +13,8 @@ from vpipe_amd import synth
 
 pytestmark = pytest.mark.gpu
 
-# (K, N, M): one step; two; an odd group count and a last chunk of one step; 96- and 128-row tiles with remainders
+# (K, N, M), all with 64 rows of x per workgroup: one step; two; an odd group count and a last chunk of one step; one to
+# five tiles of rows with remainders
 SHAPES = [(64, 130, 65), (128, 2, 17), (320, 258, 33), (1088, 262, 97), (3840, 200, 129), (2112, 1030, 300)]
 
 
@@ -19,6 +22,10 @@ SHAPES = [(64, 130, 65), (128, 2, 17), (320, 258, 33), (1088, 262, 97), (3840, 2
 @pytest.mark.parametrize("act", [0, 1])
 @pytest.mark.parametrize("fmt", ["w4g64", "w4g32", "w8g64", "f16"])
 def test_qmm_mid_edges(vpq, oracle, dev, D, fmt, act, K, N, M):
+    check_gemm(vpq, oracle, dev, D, fmt, act, K, N, M)
+
+
+def check_gemm(vpq, oracle, dev, D, fmt, act, K, N, M):
     seed = K + 3 * N + M
     ms = np.unique(np.r_[0:3, M // 2, M - 3:M])
     if fmt == "f16":
@@ -66,17 +73,47 @@ def test_qmm_mid_edges(vpq, oracle, dev, D, fmt, act, K, N, M):
     assert torch.equal(out.view, run(*args, K, N, M, tile_n=128))
 
 
-@pytest.mark.parametrize("K,N,M,splits", [(1088, 131, 97, 3), (1088, 132, 129, 2), (640, 260, 48, 5)])
-def test_qmm_mid_uneven_shares(vpq, oracle, dev, D, K, N, M, splits):
+ALL = ("w4g64", "w4g32", "w8g64", "f16")
+# kernel (as vpq_qmm_plan), gated store, (K, N, M), formats
+KERNELS = [
+    (96, 0, (192, 24578, 80), ALL), (96, 1, (192, 24578, 80), ALL),
+    (128, 0, (1088, 13314, 385), ("w4g64", "w4g32", "f16")), (128, 1, (1088, 13314, 385), ("w4g64", "w4g32", "f16")),
+    (128, 0, (1088, 1026, 1541), ("w8g64",)), (128, 1, (1088, 1026, 1541), ("w8g64",)),
+    (256, 0, (192, 1026, 4100), ALL), (256, 1, (320, 1026, 4100), ALL),
+    (-128, 0, (512, 13314, 385), ALL), (-128, 1, (1024, 13314, 385), ("w8g64",)), (-128, 1, (4096, 1920, 4096), ("w4g64",)),
+    (-192, 0, (512, 19970, 385), ("w4g64", "w8g64", "f16")),
+    (-192, 1, (1024, 2306, 4100), ("w4g64", "f16")), (-192, 1, (512, 2306, 4100), ("w8g64",)),
+    (-256, 0, (512, 21506, 517), ("w4g64", "w4g32", "f16")), (-256, 1, (1024, 3074, 4100), ("w4g64", "w4g32", "f16")),
+]
+
+
+@pytest.mark.parametrize("want,act,shape,fmt", [k[:3] + (f,) for k in KERNELS for f in k[3]])
+def test_each_gemm_kernel_by_size(vpq, oracle, dev, D, want, act, shape, fmt):
+    bits, group, f16 = {"w4g64": (4, 64, 0), "w4g32": (4, 32, 0), "w8g64": (8, 64, 0), "f16": (4, 64, 1)}[fmt]
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        assert vpq.load().vpq_qmm_plan(*shape, bits, group, f16, act, 1) == want
+    check_gemm(vpq, oracle, dev, D, fmt, act, *shape)
+
+
+# forced counts of shares: 64 rows a workgroup; 96; 128; the 256 x 128 tile (want, as vpq_qmm_plan)
+@pytest.mark.parametrize("K,N,M,splits,want", [(1088, 131, 97, 3, 64), (1088, 132, 129, 2, 64), (640, 260, 48, 5, 64),
+                                               (704, 5122, 129, 2, 96), (1088, 24578, 97, 2, 128),
+                                               (704, 1026, 2049, 2, 256), (1088, 1027, 2049, 2, 256)])
+def test_qmm_mid_uneven_shares(vpq, oracle, dev, D, K, N, M, splits, want):
     # shares that end inside a chunk of codes; a count of outputs that is and is not a multiple of four in the fold
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        assert vpq.load().vpq_qmm_plan(K, N, M, 4, 64, 0, 0, splits) == want
     w, s, b = synth.make_weight(N, K, 40 + M)
     x = synth.make_act(M, K, 41 + M)
-    y64, yb = oracle.qmm(w, s, b, x, K, N, M)
+    ms = np.arange(M) if M < 64 else np.unique(np.r_[0:3, 93:99, 126:130, 255:258, M // 2, M - 3:M] % M)
+    y64, yb = oracle.qmm(w, s, b, x[ms], K, N, len(ms))
+    args = D.u32(w, dev), D.bf16(s, dev), D.bf16(b, dev), D.bf16(x, dev)
     out = parity.Guarded((M, N), torch.bfloat16, dev)
-    vpq.qmm_splitk_w4g64(D.u32(w, dev), D.bf16(s, dev), D.bf16(b, dev), D.bf16(x, dev), K, N, M, splits=splits, out=out.view)
+    vpq.qmm_splitk_w4g64(*args, K, N, M, splits=splits, out=out.view)
     torch.cuda.synchronize()
     out.assert_intact()
-    parity.check_bf16(D.bits(out.view), y64, yb)
+    parity.check_bf16(D.bits(out.view[torch.from_numpy(ms).to(dev)]), y64, yb)
+    assert torch.equal(out.view, vpq.qmm_splitk_w4g64(*args, K, N, M, splits=splits))
 
 
 @pytest.mark.parametrize("K,N,M,taken", [(5120, 12288, 333, True), (12288, 5120, 1024, True), (4096, 512, 128, False)])

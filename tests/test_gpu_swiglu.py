@@ -277,11 +277,14 @@ def test_qmm_and_linear_geglu(vpq, oracle, dev, D, M, F, K):
 
 
 
-# shapes whose tiles fill the CUs, so that the gated store of the large-tile GEMM kernel runs, at each of its
-# tile widths (the library picks 128, 256, 192 for these), ragged M, strided and offset output windows
+# shapes that take the large-tile GEMM kernel with its gated store, at each of its tile widths (256 CUs: 128, 256, 192),
+# and, with 512 of K, smaller tiles; ragged M, strided and offset output windows
 @pytest.mark.parametrize("activation", [capi.VPQ_GATE_SWIGLU, capi.VPQ_GATE_GEGLU])
-@pytest.mark.parametrize("M,F,K,stride,off", [(4100, 2048, 512, 0, 0), (4100, 3072, 512, 3200, 64), (2048, 6144, 512, 6145, 1)])
-def test_qmm_gated_store_of_the_large_tile_kernel(vpq, oracle, dev, D, M, F, K, stride, off, activation):
+@pytest.mark.parametrize("M,F,K,stride,off,want", [(4096, 960, 4096, 0, 0, -128), (4100, 1537, 1024, 1601, 64, -256), (2048, 6144, 2048, 6145, 1, -192),
+                                                   (4100, 2048, 512, 0, 0, 96), (4100, 3072, 512, 3200, 64, 64), (2048, 6144, 512, 6145, 1, 64)])
+def test_qmm_gated_store_of_the_large_tile_kernel(vpq, oracle, dev, D, M, F, K, stride, off, want, activation):
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        assert vpq.load().vpq_qmm_plan(K, 2 * F, M, 4, 64, 0, 1, 1) == want
     _, _, pack = fused_pack(oracle, F, K, 2100 + F)
     x = synth.make_act(M, K, 2101 + M)
     wd, sd, bd, xd = stage(D, dev, pack, x)
