@@ -133,14 +133,14 @@ int qmv_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
   }
   if (variant == VPQ_QMV_RING) {
     if (!mfma_ok || !vpq::qmv_ring_supports(K, N, M)) { return VPQ_ERR_BAD_SHAPE; }
-    return finish(vpq::launch_qmv_ring(hs, a, 0, 1));
+    return finish(vpq::launch_qmv_ring(hs, a, 1));
   }
   if (variant == VPQ_QMV_RING_SPLITK) {
     if (!mfma_ok || !vpq::qmv_ring_supports(K, N, M) || K < 1024) { return VPQ_ERR_BAD_SHAPE; }
     if (ws == nullptr || !aligned(ws, 16)) { return ws == nullptr ? VPQ_ERR_WORKSPACE : VPQ_ERR_MISALIGNED; }
     const int parts = K / 512 < 4 ? K / 512 : 4;
     if (ws_bytes < vpq::qmv_ring_workspace_bytes(K, N, M)) { return VPQ_ERR_WORKSPACE; }
-    return finish(vpq::launch_qmv_ring(hs, a, 0, parts));
+    return finish(vpq::launch_qmv_ring(hs, a, parts));
   }
   if (variant == VPQ_QMV_STREAM) {
     if (!mfma_ok || gate_act != 0 || !vpq::qmv_stream_supports(K, N, M)) { return VPQ_ERR_BAD_SHAPE; }

@@ -88,36 +88,21 @@ static_assert(offsetof(RingParams, y) == kPreloadWords * 4, "y starts the part t
 
 // Eight nibbles of one packed word -> eight bf16 values 128+q, element order
 // [k0,k4,k1,k5,k2,k6,k3,k7].  `mask` and `magic` arrive as opaque register values so that
-// each pair costs a single v_and_or_b32.  F16: binary16 values 16+q instead (the code shifted to
-// mantissa bits 6..9, where a step is 1/64 of 16.0's exponent: exact).
-template <bool F16>
+// each pair costs a single v_and_or_b32.
 __device__ __forceinline__ u32x4 ring_codes_to_elts(uint32_t word, uint32_t mask, uint32_t magic)
 {
   u32x4 v;
-  if constexpr (F16) {
-    v[0] = ((word << 6) & mask) | magic;
-    v[1] = ((word << 2) & mask) | magic;
-    v[2] = ((word >> 2) & mask) | magic;
-    v[3] = ((word >> 6) & mask) | magic;
-  } else {
-    v[0] = (word & mask) | magic;
-    v[1] = ((word >> 4) & mask) | magic;
-    v[2] = ((word >> 8) & mask) | magic;
-    v[3] = ((word >> 12) & mask) | magic;
-  }
+  v[0] = (word & mask) | magic;
+  v[1] = ((word >> 4) & mask) | magic;
+  v[2] = ((word >> 8) & mask) | magic;
+  v[3] = ((word >> 12) & mask) | magic;
   return v;
 }
 
-// D = A (16 x 32) * B (32 x 16) + C on bf16 or binary16 operands, fp32 accumulation.
-template <bool F16>
+// D = A (16 x 32) * B (32 x 16) + C on bf16 operands, fp32 accumulation.
 __device__ __forceinline__ floatx4 ring_mfma(u32x4 a, u32x4 b, floatx4 c)
 {
-  if constexpr (F16) {
-    typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
-  } else {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 // Eight consecutive elements of x -> the element order ring_codes_to_elts produces.
@@ -174,9 +159,7 @@ struct Taken {
 
 // MR: accumulator registers per lane = ceil(M/4).  Row m of x sits in MFMA row 4*(m%4) + m/4,
 // so that output row m is register m/4 of lane group m%4.  MR == 1 (M <= 4) stages x through LDS.
-// F16: x, scales, biases, y and the residual are IEEE binary16 (the reference's VPIPE_ELT = half build); the codes
-// become 16+q and the offset -16*sum(x).
-template <int NW, int MR, bool F32OUT, bool F16 = false>
+template <int NW, int MR, bool F32OUT>
 __global__ __launch_bounds__(NW * 64) void qmv_ring_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<RingParams> tail)
 {
   const RingParams p = preload_assemble<RingParams>(VPQ_PRELOADED_WORD_LIST, tail);
@@ -208,13 +191,13 @@ __global__ __launch_bounds__(NW * 64) void qmv_ring_kernel(VPQ_PRELOADED_WORDS, 
   const int ld_row = lane >> 4;
   const int ld_pos = lane & 15;
 
-  uint32_t magic = F16 ? 0x4c004c00u : 0x43004300u;   // 16.0 (binary16) or 128.0 (bf16) in both halves
-  uint32_t mask = F16 ? 0x03c003c0u : 0x000f000fu;
+  uint32_t magic = 0x43004300u;             // 128.0 in both halves
+  uint32_t mask = 0x000f000fu;
   asm volatile("" : "+v"(magic));           // no instruction: only hides the constants
   asm volatile("" : "+s"(mask));            // from constant folding
-  u32x4 neg128;                             // the offset of the codes, negated: -128.0 (bf16) or -16.0 (binary16)
-  neg128[0] = neg128[1] = neg128[2] = neg128[3] = F16 ? 0xcc00cc00u : 0xc300c300u;
-  constexpr float kBiasOverOffset = F16 ? -0.0625f : -0.0078125f;
+  u32x4 neg128;                             // the offset of the codes, negated
+  neg128[0] = neg128[1] = neg128[2] = neg128[3] = 0xc300c300u;
+  constexpr float kBiasOverOffset = -0.0078125f;
 
   // This wavefront's items: slices s_begin + wave, + NW, ... (rounds) of the workgroup's K part x its tiles.
   const int part = (int)blockIdx.y;
@@ -324,8 +307,8 @@ __global__ __launch_bounds__(NW * 64) void qmv_ring_kernel(VPQ_PRELOADED_WORDS, 
 #pragma unroll
     for (int grp = 0; grp < kG; ++grp) {
       floatx4 xn = {0.f, 0.f, 0.f, 0.f};
-      xn = ring_mfma<F16>(xq[2 * grp], neg128, xn);
-      xn = ring_mfma<F16>(xq[2 * grp + 1], neg128, xn);
+      xn = ring_mfma(xq[2 * grp], neg128, xn);
+      xn = ring_mfma(xq[2 * grp + 1], neg128, xn);
 #pragma unroll
       for (int q = 0; q < MR; ++q) { xneg[grp][q] = xn[q]; }
     }
@@ -346,10 +329,10 @@ __global__ __launch_bounds__(NW * 64) void qmv_ring_kernel(VPQ_PRELOADED_WORDS, 
       floatx4 s4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int q = 0; q < MR; ++q) { s4[q] = xneg[grp][q]; }
-      s4 = ring_mfma<F16>(xq[2 * grp], ring_codes_to_elts<F16>(cw[0], mask, magic), s4);
-      s4 = ring_mfma<F16>(xq[2 * grp + 1], ring_codes_to_elts<F16>(cw[1], mask, magic), s4);
-      const float s = (grp & 1) ? elt_hi_to_f32<F16>(sd[grp >> 1]) : elt_lo_to_f32<F16>(sd[grp >> 1]);
-      const float b = (grp & 1) ? elt_hi_to_f32<F16>(bd[grp >> 1]) : elt_lo_to_f32<F16>(bd[grp >> 1]);
+      s4 = ring_mfma(xq[2 * grp], ring_codes_to_elts(cw[0], mask, magic), s4);
+      s4 = ring_mfma(xq[2 * grp + 1], ring_codes_to_elts(cw[1], mask, magic), s4);
+      const float s = (grp & 1) ? bf16_hi_to_f32(sd[grp >> 1]) : bf16_lo_to_f32(sd[grp >> 1]);
+      const float b = (grp & 1) ? bf16_hi_to_f32(bd[grp >> 1]) : bf16_lo_to_f32(bd[grp >> 1]);
       const float b2 = b * kBiasOverOffset;          // bias * sum(x) = (bias / -offset) * xneg
 #pragma unroll
       for (int q = 0; q < MR; ++q) {
@@ -436,7 +419,7 @@ __global__ __launch_bounds__(NW * 64) void qmv_ring_kernel(VPQ_PRELOADED_WORDS, 
         if (F32OUT) {
           reinterpret_cast<float*>(p.y)[o] = v;
         } else {
-          reinterpret_cast<uint16_t*>(p.y)[o] = (uint16_t)f32_to_elt_bits<F16>(v);
+          reinterpret_cast<uint16_t*>(p.y)[o] = (uint16_t)f32_to_bf16_bits(v);
         }
       }
     } else if (tile < p.tiles && m < p.M && n < p.N) {
@@ -444,9 +427,9 @@ __global__ __launch_bounds__(NW * 64) void qmv_ring_kernel(VPQ_PRELOADED_WORDS, 
       if (F32OUT) {
         reinterpret_cast<float*>(p.y)[o] = total;
       } else {
-        uint32_t v = f32_to_elt_bits<F16>(total);
+        uint32_t v = f32_to_bf16_bits(total);
         if (p.residual != nullptr) {
-          v = f32_to_elt_bits<F16>(elt_bits_to_f32<F16>(v) + elt_bits_to_f32<F16>(p.residual[o]));
+          v = f32_to_bf16_bits(bf16_bits_to_f32(v) + bf16_bits_to_f32(p.residual[o]));
         }
         reinterpret_cast<uint16_t*>(p.y)[o] = (uint16_t)v;
       }
@@ -455,7 +438,7 @@ __global__ __launch_bounds__(NW * 64) void qmv_ring_kernel(VPQ_PRELOADED_WORDS, 
 }
 
 // y = store(plane[0] + plane[1] + ...), the parts added in order: one thread per output element.
-template <bool F32OUT, bool F16>
+template <bool F32OUT>
 __global__ __launch_bounds__(256) void qmv_ring_fold_kernel(const float* __restrict__ plane, void* __restrict__ y,
                                                             const uint16_t* __restrict__ residual, int M, int N, int kparts)
 {
@@ -467,8 +450,8 @@ __global__ __launch_bounds__(256) void qmv_ring_fold_kernel(const float* __restr
   if (F32OUT) {
     reinterpret_cast<float*>(y)[o] = total;
   } else {
-    uint32_t v = f32_to_elt_bits<F16>(total);
-    if (residual != nullptr) { v = f32_to_elt_bits<F16>(elt_bits_to_f32<F16>(v) + elt_bits_to_f32<F16>(residual[o])); }
+    uint32_t v = f32_to_bf16_bits(total);
+    if (residual != nullptr) { v = f32_to_bf16_bits(bf16_bits_to_f32(v) + bf16_bits_to_f32(residual[o])); }
     reinterpret_cast<uint16_t*>(y)[o] = (uint16_t)v;
   }
 }
@@ -487,25 +470,24 @@ size_t qmv_ring_workspace_bytes(int K, int N, int M)
 
 namespace {
 
-template <int NW, bool F16>
+template <int NW>
 hipError_t launch_nw(hipStream_t st, const RingParams& p, int mr, bool f32)
 {
   const dim3 grid((unsigned)((p.tiles + p.tc - 1) / p.tc), (unsigned)p.kparts), block((unsigned)(NW * kWave));
   if (f32) {
-    if (mr == 1) { return launch_preloaded(qmv_ring_kernel<NW, 1, true, F16>, grid, block, 0, st, p); }
-    if (mr == 2) { return launch_preloaded(qmv_ring_kernel<NW, 2, true, F16>, grid, block, 0, st, p); }
-    return launch_preloaded(qmv_ring_kernel<NW, 4, true, F16>, grid, block, 0, st, p);
+    if (mr == 1) { return launch_preloaded(qmv_ring_kernel<NW, 1, true>, grid, block, 0, st, p); }
+    if (mr == 2) { return launch_preloaded(qmv_ring_kernel<NW, 2, true>, grid, block, 0, st, p); }
+    return launch_preloaded(qmv_ring_kernel<NW, 4, true>, grid, block, 0, st, p);
   }
-  if (mr == 1) { return launch_preloaded(qmv_ring_kernel<NW, 1, false, F16>, grid, block, 0, st, p); }
-  if (mr == 2) { return launch_preloaded(qmv_ring_kernel<NW, 2, false, F16>, grid, block, 0, st, p); }
-  return launch_preloaded(qmv_ring_kernel<NW, 4, false, F16>, grid, block, 0, st, p);
+  if (mr == 1) { return launch_preloaded(qmv_ring_kernel<NW, 1, false>, grid, block, 0, st, p); }
+  if (mr == 2) { return launch_preloaded(qmv_ring_kernel<NW, 2, false>, grid, block, 0, st, p); }
+  return launch_preloaded(qmv_ring_kernel<NW, 4, false>, grid, block, 0, st, p);
 }
 
 }  // namespace
 
-// tc_hint > 0 forces the tiles per workgroup (measurement).  splits_hint: 0 = K across workgroups where a.ws has
-// the room and the cost model says it pays, 1 = never, n > 1 = n parts (if a.ws has the room).
-hipError_t launch_qmv_ring(hipStream_t st, const QmvArgs& a, int tc_hint, int splits_hint, bool f16)
+// parts > 1: K in that many parts across workgroups (an error if a.ws has not the room).
+hipError_t launch_qmv_ring(hipStream_t st, const QmvArgs& a, int parts)
 {
   RingParams p;
   p.w = a.w; p.scales = a.scales; p.biases = a.biases; p.x = a.x; p.y = a.y;
@@ -522,12 +504,12 @@ hipError_t launch_qmv_ring(hipStream_t st, const QmvArgs& a, int tc_hint, int sp
   // all of x once.  The count that minimises generations x bytes per workgroup wins; the largest count
   // often does not (9496 tiles at 16 per workgroup: 594 workgroups, a third generation for 82 of them).
   const double tile_bytes = 16.0 * (double)a.K * 9.0 / 16.0, x_bytes = (double)a.M * (double)a.K * 2.0;
-  // cost of a launch with t tiles per workgroup and K in `parts` parts, in bytes a workgroup moves per generation
-  auto plan = [&](int regs, int parts, int& tc_out) {
+  // cost of a launch with t tiles per workgroup and K in `n` parts, in bytes a workgroup moves per generation
+  auto plan = [&](int regs, int n, int& tc_out) {
     double best = 0.0;
     for (int t = 1; t <= max_tc_mr(regs) / regs; ++t) {
-      const int wgs = ((p.tiles + t - 1) / t) * parts;
-      const double cost = (double)((wgs + cus - 1) / cus) * ((double)t * tile_bytes + x_bytes) / (double)parts;
+      const int wgs = ((p.tiles + t - 1) / t) * n;
+      const double cost = (double)((wgs + cus - 1) / cus) * ((double)t * tile_bytes + x_bytes) / (double)n;
       if (t == 1 || cost <= best) { best = cost; tc_out = t; }
     }
     return best;
@@ -541,46 +523,35 @@ hipError_t launch_qmv_ring(hipStream_t st, const QmvArgs& a, int tc_hint, int sp
     const double c2 = plan(2, 1, tc2);
     if (c2 * 1.05 < cost) { mr = 2; tc = tc2; cost = c2; }
   }
-  // K across workgroups where the caller's workspace holds the planes and it pays.  Measured (kernel + fold, us,
-  // unsplit / 4 parts): 17408 -> 5120 at 16 rows 26.3 / 23.5, at 8 rows 21.4 / 20.5, at 4 rows 17.2 / 22.5;
-  // 5120 -> 5120 at 16 rows 11.7 / 14.8; 5120 -> 17408 at 16 rows 19.4 / 31.1; 5120 -> 151936 123.8 / 202.2: the
-  // fold's launch and the shorter K walks cost more than the re-read x except for many rows over a deep K with few
-  // tiles per CU.  Every element of a plane is written by exactly one workgroup before the fold reads it, so the
-  // workspace needs no clearing.
+  // K across workgroups.  Measured (kernel + fold, us, unsplit / 4 parts): 17408 -> 5120 at 16 rows 26.3 / 23.5, at 8
+  // rows 21.4 / 20.5, at 4 rows 17.2 / 22.5; 5120 -> 5120 at 16 rows 11.7 / 14.8; 5120 -> 17408 at 16 rows 19.4 / 31.1;
+  // 5120 -> 151936 123.8 / 202.2: the fold's launch and the shorter K walks cost more than the re-read x except for many
+  // rows over a deep K with few tiles per CU.  Every element of a plane is written by exactly one workgroup before the
+  // fold reads it, so the workspace needs no clearing.
   p.kparts = 1;
   p.part_slices = p.slices;
   p.plane = nullptr;
-  if (splits_hint != 1 && a.ws != nullptr && p.slices >= 2 && a.gate_act == 0) {     // (the gated entry points take no workspace)
-    int parts = splits_hint > 1 ? splits_hint : ((a.M >= 8 && p.slices >= 24 && p.tiles <= 2 * cus) ? 4 : 1);
-    if (parts > p.slices) { parts = p.slices; }
-    if (parts > 1 && (size_t)parts * (size_t)a.M * (size_t)a.N * sizeof(float) <= a.ws_bytes) {
-      p.part_slices = (p.slices + parts - 1) / parts;
-      p.kparts = (p.slices + p.part_slices - 1) / p.part_slices;      // no empty part
-      p.plane = static_cast<float*>(a.ws);
-      int tcp = 1;
-      plan(mr, p.kparts, tcp);
-      tc = tcp;
-    } else if (splits_hint > 1) {
-      return hipErrorInvalidValue;
-    }
+  if (parts > p.slices) { parts = p.slices; }
+  if (parts > 1 && a.gate_act == 0) {                // (the gated entry points take no workspace)
+    if (a.ws == nullptr || (size_t)parts * (size_t)a.M * (size_t)a.N * sizeof(float) > a.ws_bytes) { return hipErrorInvalidValue; }
+    p.part_slices = (p.slices + parts - 1) / parts;
+    p.kparts = (p.slices + p.part_slices - 1) / p.part_slices;      // no empty part
+    p.plane = static_cast<float*>(a.ws);
+    plan(mr, p.kparts, tc);
   }
-  const int tc_max = max_tc_mr(mr) / mr;
-  if (tc_hint > 0) { tc = tc_hint < tc_max ? tc_hint : tc_max; }
   p.tc = tc;
   p.pad_ = 0;
   if (p.kparts > 1) {
-    const hipError_t e = f16 ? launch_nw<8, true>(st, p, mr, a.y_f32) : launch_nw<8, false>(st, p, mr, a.y_f32);
+    const hipError_t e = launch_nw<8>(st, p, mr, a.y_f32);
     if (e != hipSuccess) { return e; }
     const size_t outs = (size_t)a.M * a.N;
     const dim3 fgrid((unsigned)((outs + 255) / 256)), fblock(256);
     if (a.y_f32) {
-      return f16 ? launch_kernel(qmv_ring_fold_kernel<true, true>, fgrid, fblock, 0, st, (const float*)p.plane, a.y, a.residual, a.M, a.N, p.kparts)
-                 : launch_kernel(qmv_ring_fold_kernel<true, false>, fgrid, fblock, 0, st, (const float*)p.plane, a.y, a.residual, a.M, a.N, p.kparts);
+      return launch_kernel(qmv_ring_fold_kernel<true>, fgrid, fblock, 0, st, (const float*)p.plane, a.y, a.residual, a.M, a.N, p.kparts);
     }
-    return f16 ? launch_kernel(qmv_ring_fold_kernel<false, true>, fgrid, fblock, 0, st, (const float*)p.plane, a.y, a.residual, a.M, a.N, p.kparts)
-               : launch_kernel(qmv_ring_fold_kernel<false, false>, fgrid, fblock, 0, st, (const float*)p.plane, a.y, a.residual, a.M, a.N, p.kparts);
+    return launch_kernel(qmv_ring_fold_kernel<false>, fgrid, fblock, 0, st, (const float*)p.plane, a.y, a.residual, a.M, a.N, p.kparts);
   }
-  return f16 ? launch_nw<8, true>(st, p, mr, a.y_f32) : launch_nw<8, false>(st, p, mr, a.y_f32);
+  return launch_nw<8>(st, p, mr, a.y_f32);
 }
 
 }  // namespace vpq
