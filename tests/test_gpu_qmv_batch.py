@@ -7,7 +7,7 @@ import torch
 
 from tests import parity
 from tests.test_oracle_pins import f16_pack
-from vpipe_amd import synth
+from vpipe_amd import capi, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -160,3 +160,28 @@ def test_fp32_results_are_as_close_as_a_plain_sum(vpq, dev, D, fmt, K):
     got = run(D.u32(w, dev), *sb, x, K, N, M, f32out=True).cpu().double().numpy()
     want = x.cpu().double().numpy() @ _weight64(fmt, w, s, b, K).T
     assert np.linalg.norm(got - want) <= 4 * 2.0 ** -24 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("M", [1, 2, 5])
+def test_k_that_is_too_deep_for_the_batch_kernel(vpq, oracle, dev, D, M):
+    # its scales do not fit the LDS: the automatic and the MFMA call, single and grouped, run on the ring kernel
+    K, Ns = 131072, (33, 16)
+    x = synth.make_act(M, K, 7)
+    xd = D.bf16(x, dev)
+    packs, singles = [], []
+    for N in Ns:
+        w, s, b = synth.make_weight(N, K, 8 + N)
+        pack = D.u32(w, dev), D.bf16(s, dev), D.bf16(b, dev)
+        f = vpq.qmv_w4g64(*pack, xd, K, N, M, f32out=True)
+        parity.check_f32(f.cpu().numpy(), oracle.qmv(w, s, b, x, K, N, M)[0])
+        singles.append(vpq.qmv_w4g64(*pack, xd, K, N, M))
+        assert torch.equal(singles[-1], f.bfloat16())
+        for variant in (capi.VPQ_QMV_MFMA, capi.VPQ_QMV_RING):
+            assert torch.equal(vpq.qmv_w4g64(*pack, xd, K, N, M, variant=variant), singles[-1])
+        packs.append(pack + (N,))
+    outs = [parity.Guarded((M, N), torch.bfloat16, dev) for N in Ns]
+    vpq.qmv_group_w4g64(packs, xd, K, M, outs=[o.view for o in outs])
+    torch.cuda.synchronize()
+    for o, one in zip(outs, singles):
+        o.assert_intact()
+        assert torch.equal(o.view, one)

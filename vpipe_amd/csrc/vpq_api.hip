@@ -117,7 +117,8 @@ int qmv_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
 
   const bool batch_ok = vpq::qmv_batch_supports(K, M, vpq::BatchFormat{}) && aligned(scales, 16) && aligned(biases, 16);
-  const bool mfma_ok = batch_ok && (K % 512) == 0;           // what the forced variants of the MFMA kernels take
+  // what the forced variants of the MFMA kernels take
+  const bool mfma_ok = vpq::qmv_ring_supports(K, N, M) && aligned(scales, 16) && aligned(biases, 16);
   const bool flow_ok = vpq::qmv_flow_supports(K, N, M) && aligned(scales, 16) && aligned(biases, 16);
   if (gelu_mul) {        // the two kernels that have this store: the streaming one and the general one
     return finish(flow_ok ? vpq::launch_qmv_flow(hs, a) : vpq::launch_qmv_simple(hs, a));
@@ -132,11 +133,11 @@ int qmv_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
     return finish(vpq::launch_qmv_rows(hs, a, 0));
   }
   if (variant == VPQ_QMV_RING) {
-    if (!mfma_ok || !vpq::qmv_ring_supports(K, N, M)) { return VPQ_ERR_BAD_SHAPE; }
+    if (!mfma_ok) { return VPQ_ERR_BAD_SHAPE; }
     return finish(vpq::launch_qmv_ring(hs, a, 1));
   }
   if (variant == VPQ_QMV_RING_SPLITK) {
-    if (!mfma_ok || !vpq::qmv_ring_supports(K, N, M) || K < 1024) { return VPQ_ERR_BAD_SHAPE; }
+    if (!mfma_ok || K < 1024) { return VPQ_ERR_BAD_SHAPE; }
     if (ws == nullptr || !aligned(ws, 16)) { return ws == nullptr ? VPQ_ERR_WORKSPACE : VPQ_ERR_MISALIGNED; }
     const int parts = K / 512 < 4 ? K / 512 : 4;
     if (ws_bytes < vpq::qmv_ring_workspace_bytes(K, N, M)) { return VPQ_ERR_WORKSPACE; }
@@ -148,14 +149,15 @@ int qmv_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
   }
   if (variant == VPQ_QMV_MFMA) {
     if (!mfma_ok) { return VPQ_ERR_BAD_SHAPE; }
-    return finish(launch_batch(hs, a, vpq::BatchFormat{}));
+    return finish(batch_ok ? launch_batch(hs, a, vpq::BatchFormat{}) : vpq::launch_qmv_ring(hs, a, 1));
   }
   // One row of x: the streaming kernel that requests the whole pack up front.
   if (flow_ok) { return finish(vpq::launch_qmv_flow(hs, a)); }
   // One row over a K that is not a multiple of 512: the row-streaming kernel.
   if (M == 1 && (K % 512) != 0) { return finish(vpq::launch_qmv_rows(hs, a, 0)); }
   if (batch_ok) { return finish(launch_batch(hs, a, vpq::BatchFormat{})); }
-  // Scales or biases off 16-byte alignment, or a K too deep for the batch kernel's LDS.
+  // A K too deep for the batch kernel's LDS (above 114176), or scales or biases off 16-byte alignment.
+  if (mfma_ok) { return finish(vpq::launch_qmv_ring(hs, a, 1)); }
   if (vpq::qmv_rows_supports(K, N, M)) { return finish(vpq::launch_qmv_rows(hs, a, 0)); }
   return finish(vpq::launch_qmv_simple(hs, a));
 }
@@ -1629,20 +1631,21 @@ int vpq_qmv_group_w4g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
 {
   if (w == nullptr || scales == nullptr || biases == nullptr || y == nullptr || N == nullptr) { return VPQ_ERR_NULL_POINTER; }
   if (count < 1 || count > 4) { return VPQ_ERR_BAD_SHAPE; }
-  bool batch = vpq::qmv_batch_supports(K, M, vpq::BatchFormat{});
+  bool wide = true;                                     // 16-byte loads of every pack's scales and biases
   for (int i = 0; i < count; ++i) {
     int st = check_pack(w[i], scales[i], biases[i], K, N[i]);
     if (st != VPQ_OK) { return st; }
     if (y[i] == nullptr) { return VPQ_ERR_NULL_POINTER; }
     if (!aligned(y[i], 2)) { return VPQ_ERR_MISALIGNED; }
-    batch = batch && aligned(scales[i], 16) && aligned(biases[i], 16);
+    wide = wide && aligned(scales[i], 16) && aligned(biases[i], 16);
   }
   if (x == nullptr) { return VPQ_ERR_NULL_POINTER; }
   if (M < 1 || M > 16) { return VPQ_ERR_BAD_SHAPE; }
   if (!aligned(x, 16)) { return VPQ_ERR_MISALIGNED; }
   // The kernels of the single call (qmv_common), each in its grouped form.
+  const bool batch = wide && vpq::qmv_batch_supports(K, M, vpq::BatchFormat{});
   const bool flow = batch && vpq::qmv_flow_supports(K, 1, M);
-  const bool rows = !flow && vpq::qmv_rows_supports(K, 1, M) && (!batch || (M == 1 && (K % 512) != 0));
+  const bool rows = vpq::qmv_rows_supports(K, 1, M) && (!wide || (K % 512) != 0) && (!batch || M == 1);
   if (!flow && !rows && !batch) {
     for (int i = 0; i < count; ++i) {
       const int st = vpq_qmv_w4g64_bf16(stream, w[i], scales[i], biases[i], x, y[i], K, N[i], M, nullptr, nullptr, 0,
