@@ -946,15 +946,7 @@ void ComputeEncoder::dispatch(LaunchDims grid, LaunchDims /*threads_per_threadgr
           M = ival(7);
         }
         if (status == VPQ_OK) {
-          // The split-K scratch is shared by the stream, so concurrent dispatches go without it.
-          void* ws = nullptr;
-          std::size_t ws_bytes = 0;
-          if (!in_scope && K > 0 && N > 0 && M > 0 && M <= 16) {
-            ws_bytes = vpq_qmv_workspace_bytes(K, N, M);
-            ws = s->qmv_workspace(ws_bytes);
-            if (ws == nullptr) { ws_bytes = 0; }
-          }
-          status = vpq_qmv_w4g64_bf16(st, w, sc, bi, x, y, K, N, M, residual, ws, ws_bytes, VPQ_QMV_AUTO);
+          status = vpq_qmv_w4g64_bf16(st, w, sc, bi, x, y, K, N, M, residual, nullptr, 0, VPQ_QMV_AUTO);
         }
       }
     }
@@ -1032,14 +1024,7 @@ void quant_linear_forward(CommandStream& stream, const Linear& lin, const Device
                                 static_cast<const uint16_t*>(lora->b->data()), lora->rank, lora->strength,
                                 static_cast<uint16_t*>(lora_t->data()));
   } else {
-    void* ws = nullptr;
-    std::size_t ws_bytes = 0;
-    if (M <= 16 && M > 0 && lin.K > 0 && lin.N > 0) {
-      ws_bytes = vpq_qmv_workspace_bytes(lin.K, lin.N, M);
-      ws = stream.qmv_workspace(ws_bytes);
-      if (ws == nullptr) { ws_bytes = 0; }
-    }
-    status = vpq_linear_w4g64_bf16(st, w, sc, bi, xp, yp, lin.K, lin.N, M, ws, ws_bytes);
+    status = vpq_linear_w4g64_bf16(st, w, sc, bi, xp, yp, lin.K, lin.N, M, nullptr, 0);
   }
   if (status != VPQ_OK) { stream.record_error(status, "quant_linear_forward"); }
 }
