@@ -103,14 +103,18 @@ int vpq_embed_gather_w4g64_bf16(vpq_stream_t stream, const int32_t* ids, const u
  * QMV arithmetic -- the weight is never rounded to bf16; per (row, group) the
  * kernel forms sum(x*q) and sum(x) in fp32 and combines them as
  * scale*sum(x*q) + bias*sum(x) (affine_qmv.metal:151-174), fp32 accumulate,
- * one bf16 rounding on store.  With `residual` ([M,N] bf16, nullable) the
+ * one bf16 rounding on store.  (At two rows and more as
+ * scale*sum(x*(q-8)) + (bias+8*scale)*sum(x), as close to the exact sum as a
+ * plain fp32 one, about 1e-7; at one row, and in the forced variants other than
+ * MFMA and SIMPLE, sum(x*q) is taken from sum(x*(128+q)): 4 to 9e-7.
+ * An infinity in a row of x makes an output +-inf or NaN as the plain sum would at
+ * two rows and more, NaN at one row.)  With `residual` ([M,N] bf16, nullable) the
  * rounded result is added to it in fp32 and rounded again, as `_add` does
  * (:264-266).
  * Requires K % 64 == 0, N > 0, 1 <= M <= 16.
- * `ws` is scratch for the split of K across workgroups (fp32 planes):
- * vpq_qmv_workspace_bytes() bytes, 16-byte aligned, no initial content
- * needed; it may be NULL, in which case shapes that would have split K run
- * unsplit.
+ * `ws` is scratch for VPQ_QMV_RING_SPLITK's split of K across workgroups (fp32
+ * planes): vpq_qmv_workspace_bytes() bytes, 16-byte aligned, no initial content
+ * needed.  The automatic choice takes none; it may be NULL.
  * `variant`: 0 = automatic; other values select a specific kernel for
  * measurement (see VPQ_QMV_* below). */
 int vpq_qmv_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
@@ -124,8 +128,8 @@ int vpq_qmv_w4g64_f32out(vpq_stream_t stream, const uint32_t* w, const uint16_t*
                          const uint16_t* biases, const uint16_t* x, float* y,
                          int K, int N, int M, void* ws, size_t ws_bytes, int variant);
 
-/* Bytes of split-K scratch the QMV entry points may use for this shape
- * (an upper bound over variants; a multiple of 256). */
+/* Bytes of scratch that VPQ_QMV_RING_SPLITK needs for this shape (a multiple of
+ * 256). */
 size_t vpq_qmv_workspace_bytes(int K, int N, int M);
 
 enum {

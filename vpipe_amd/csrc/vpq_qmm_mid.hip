@@ -11,17 +11,19 @@
 // Loads.  x comes through three LDS stages of 64 values of K (direct-to-LDS, 8 rows x 128 bytes each), requested two
 // steps ahead; one barrier a step.  Codes come 128 bytes per weight row at a time (four steps of 4 bits, two of 8), whole
 // lines into a slot of the wavefront's own, which is copied to registers at the start of those steps and requested
-// again at once.  Scales and biases of those steps are one load of each per lane, a chunk ahead.
+// again at once.  Scales and biases of those steps are one ordinary load of each per lane, requested a chunk ahead.  The
+// wait for them is the compiler's, and falls where they are copied, behind the request of a coming x tile: for 4-bit
+// codes it waits for that tile too, so one step in four starts with an empty queue.
 //
 // With K split over workgroups (few tiles over a long K) a share leaves fp32 planes that splitk_fold adds in order.
 //
 // What bounds it: a step's chain (barrier, operand reads, unpacking, MFMAs) for a workgroup alone on its CU, 0.57 us at
 // 96 rows; several to a CU, the LDS reads of x (4 KB a row fragment and wavefront) and the MFMAs together.  Two 32-row
 // fragments of weights a wavefront halve the LDS reads but leave half the workgroups: slower up to 1024 rows (4096 -> 24576
-// at 128 / 333 rows 73 / 114 us against 52 / 99).  Pinning one MFMA between every seven vector instructions: no gain.
+// at 128 / 333 rows 73 / 114 us against 51 / 92).  Pinning one MFMA between every seven vector instructions: no gain.
 // Measured (us, before: the 256 x 128 tiles, split over K where a workspace allows, and the large tile; after):
-// 4096 -> 24576 gated at 80 / 128 / 333 rows 78 / 78 / 104 -> 44 / 51 / 92; 4096 -> 1024 at 333 rows 22 -> 15;
-// 12288 -> 4096 at 80 / 333 rows 38 / 69 -> 26 / 62; without a workspace 4096 -> 4096 at 80..333 rows 57 -> 37.
+// 4096 -> 24576 gated at 80 / 128 / 333 rows 68 / 69 / 104 -> 45 / 51 / 92; 4096 -> 1024 at 333 rows 24 -> 19;
+// 12288 -> 4096 at 80 / 333 rows 36 / 69 -> 27 / 57; without a workspace 4096 -> 4096 at 80..333 rows 56..63 -> 33..36.
 #include <type_traits>
 
 #include "vpq_device.h"
@@ -230,7 +232,8 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, uint8_t* x_lds, uin
 
   // ---- K loop ----
   // Loads of step t, in order: x(t + 2) [XL], and at a chunk's first step the next chunk's codes [CL] and scales.  The
-  // first step of a chunk waits for everything (its scales are ordinary loads, whose wait is the compiler's); the third
+  // first step of a chunk waits for everything that was requested before it (and, where its scales are copied, the
+  // compiler waits again, for the x of this step's request as well); the third
   // needs x that has the codes and a step of x behind it, the fourth x that has a step of x behind it.  The last steps
   // request the last tile again (never read), so that the counts hold to the end.
   request_codes(0);
@@ -368,7 +371,7 @@ __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidPar
 // Two neighbouring blocks to an XCD, which mostly share an expert's weight tiles: 1 to 2 % slower (2048 tokens 298 -> 305 us).
 // Bound by the plain tile's step at full blocks, by unpacking and the codes' read at one fragment.  Measured (us, sort +
 // gate|up + down of one layer; before: 128 x 256 tiles with producer wavefronts, every block at full height), 2048 -> 768:
-// 2048 tokens, 8 of 128 experts 370 -> 286; 64 tokens 191 -> 138; 4096 tokens, 8 of 64 experts 557 -> 447, 8 bits 580 -> 498.
+// 2048 tokens, 8 of 128 experts 366 -> 300; 64 tokens 191 -> 138; 4096 tokens, 8 of 64 experts 557 -> 447, 8 bits 580 -> 498.
 template <int BITS>
 __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_grouped_kernel(const MidParams p)
 {

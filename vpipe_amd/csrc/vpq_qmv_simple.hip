@@ -1,7 +1,8 @@
 // QMV, general-shape kernel: one wavefront per output row, fp32 VALU.
-// Handles every K % 64 == 0, every N and 1 <= M <= 16; used for shapes the
-// MFMA kernel does not take (K not a multiple of 512, N not a multiple of 16)
-// and as an independent second implementation in the tests.
+// Handles every K % 64 == 0, every N and 1 <= M <= 16; used for what the
+// batch kernel does not take (scales or biases off 16-byte alignment, a K too
+// deep for its LDS, the gelu-mul store) and as an independent second
+// implementation in the tests.
 //
 // Arithmetic: W[n,k] = fma(s, q, b) in fp32 (never rounded to bf16),
 // acc += x * W in fp32, wave reduction, one bf16 rounding on store -- the
