@@ -243,7 +243,7 @@ hipError_t launch_moe_sort(hipStream_t st, const int* pair_eid, int n_pairs, int
                            int max_tiles, int* tile2e, int* srow, int* sdst, int* ntiles, int* ws);
 hipError_t launch_qmm_grouped(hipStream_t st, const GemmArgs& a, const GroupedArgs& g);
 // Large-tile kernel (256 x 256 or 256 x 192 per workgroup, four wavefronts that each load, dequantize
-// and multiply): K % 512 == 0, 16-byte aligned scales / biases, no gated store; same bits as the tile
+// and multiply): K % 512 == 0, 16-byte aligned scales / biases; same bits as the tile
 // kernel.  tile_n 0 = qmm_big_tile_n().
 bool qmm_big_supports(const GemmArgs& a);
 int qmm_big_tile_n(int N, int M, int cu_count, int max_width = 256, bool with_192 = true);

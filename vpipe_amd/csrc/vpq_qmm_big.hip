@@ -870,7 +870,8 @@ bool qmm_big_supports(const GemmArgs& a)
 // rounds, and a round's time grows with the tile width (the MFMA work) over the width's efficiency
 // (measured with whole rounds: 256 wide 1.02, 192 wide 0.98, 128 wide 0.94 PFLOP/s).  4096 -> 12288 at
 // M = 2048: 384 tiles of 256 are one and a half rounds of 256 CUs, 512 tiles of 192 are two;
-// N = 4096 at M = 2048 is exactly one round of 128-wide tiles.
+// N = 4096 at M = 2048 is exactly one round of 128-wide tiles.  (With an adapter, and for dense weights; the width of the
+// other calls comes with the choice of the kernel, qmm_choose.)
 int qmm_big_tile_n(int N, int M, int cu_count, int max_width, bool with_192)
 {
   const int cus = cu_count > 0 ? cu_count : 256;

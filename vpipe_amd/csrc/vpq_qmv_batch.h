@@ -1,9 +1,11 @@
 // QMV for a batch of rows (2..64 rows of x; one row where the one-row kernel does not run), any K that is a multiple
 // of 64 (of 32 for groups of 32): the kernel template of vpq_qmv_batch*.hip.
 //
-// What bounds it: HBM for the pack at few rows, issue of vector instructions from 16 rows on (unpacking costs 14 per
-// 16 x 64 codes, every 16 x 16 outputs 8 multiply-adds per group; the vector ALU is 60-72 % busy at 16..48 rows, the
-// matrix pipe a quarter of that).  Measured (us; before: one-item and ring kernels where K % 512 == 0, one wavefront
+// What bounds it: HBM for the pack at few rows; from 16 rows on no unit alone: the vector ALU is busy half of the cycles
+// (52 % on 4096 -> 24576 at 48 rows, 51 % on 5120 -> 151936 at 16; unpacking costs 14 instructions per 16 x 64 codes,
+// every 16 x 16 outputs 8 multiply-adds per group), the matrix pipe 18 and 13 %, and above 16 rows a wavefront waits for
+// each piece of x, which it has requested one piece ahead.
+// Measured (us; before: one-item and ring kernels where K % 512 == 0, one wavefront
 // per weight row elsewhere, slabs of 16 rows above 16): 4096 -> 4096 at 16 / 48 rows 9.3 / 20.4 -> 6.3 / 10.0;
 // 4096 -> 12288 13.3 / 38.6 -> 12.2 / 21.0; 5120 -> 151936 at 8 / 16 rows 102 / 124 -> 96 / 114; 3840 -> 19328 at
 // 4 / 16 rows 51 / 156 -> 13.5 / 17.4.
