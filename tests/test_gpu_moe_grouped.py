@@ -345,3 +345,45 @@ def test_grouped_gemms_at_every_count_of_live_fragments(vpq, dev, D, K, N, bits)
             d = vpq.qmm_w4g64(w[e], s[e], b[e], xe, K, N, counts[e], tile_n=128)
         assert np.array_equal(D.bits(act.view)[slots.cpu().numpy()], D.bits(g)), "gate|up, expert %d" % e
         assert np.array_equal(D.bits(part.view)[sdst[slots].cpu().numpy()], D.bits(d)), "down, expert %d" % e
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("counts", [[160, 161, 5], [257, 288, 0, 289], [128, 128 + 32, 1]])
+def test_last_block_of_one_fragment_is_multiplied_with_the_block_before(vpq, dev, D, counts, bits):
+    # a last block of 1..32 live slots behind full blocks (the edges of that rule), also at the end of the map, in any slot
+    # order and with a hole in the block before it: the plain GEMM's rows bit for bit, zeros elsewhere
+    K, N, E, B = 320, 264, len(counts), vpq.grouped_block_rows()
+    gen = torch.Generator(device="cpu").manual_seed(5900 + sum(counts) + bits)
+    w = torch.randint(-2 ** 31, 2 ** 31, (E, N, K * bits // 32), dtype=torch.int32, generator=gen).to(dev)
+    s = (torch.rand((E, N, K // 64), generator=gen) * 0.015 / (16 if bits == 8 else 1) + 0.001).bfloat16().to(dev)
+    b = (-(2 ** (bits - 1)) * s.float()).bfloat16()
+    eid = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    x = torch.randn((eid.numel(), K), generator=gen).bfloat16().to(dev)
+    used = sum(-(-c // B) for c in counts)               # the map ends with the last expert's last block
+    t2e, srow, sdst, _ = vpq.moe_sort_pairs(eid.to(torch.int32).to(dev), 1, E)
+    t2e, srow, sdst = t2e[:used], srow[:used * B], sdst[:used * B]
+    srow[3] = sdst[3] = -1                               # the hole
+    gated = vpq.qmm_grouped_gated_w8g64 if bits == 8 else vpq.qmm_grouped_gated_w4g64
+    down = vpq.qmm_grouped_down_w8g64 if bits == 8 else vpq.qmm_grouped_down_w4g64
+    act = parity.Guarded((srow.numel(), N // 2), torch.bfloat16, dev)
+    part = parity.Guarded((eid.numel(), N), torch.bfloat16, dev)
+    act.view.fill_(7.0)
+    part.view.fill_(7.0)
+    gated(w, s, b, x, K, N, t2e, srow, E, out=act.view)
+    down(w, s, b, x[srow.clamp(min=0).long()].contiguous(), K, N, t2e, sdst, E, out=part.view)
+    torch.cuda.synchronize()
+    act.assert_intact()
+    part.assert_intact()
+    owner, live = t2e.repeat_interleave(B).cpu(), (srow >= 0).cpu()
+    assert not D.bits(act.view)[(~live).numpy()].any()
+    for e in range(E):
+        slots = torch.nonzero((owner == e) & live).flatten().to(dev)
+        if slots.numel() == 0:
+            continue
+        xe = x[srow[slots].long()].contiguous()
+        if bits == 8:
+            g, d = (vpq.qmm_w8g64(w[e], s[e], b[e], xe, K, N, slots.numel(), activation=a) for a in (1, 0))
+        else:
+            g, d = vpq.qmm_swiglu_w4g64(w[e], s[e], b[e], xe, K, N, slots.numel()), vpq.qmm_w4g64(w[e], s[e], b[e], xe, K, N, slots.numel())
+        assert np.array_equal(D.bits(act.view)[slots.cpu().numpy()], D.bits(g)), "gate|up, expert %d" % e
+        assert np.array_equal(D.bits(part.view)[sdst[slots].cpu().numpy()], D.bits(d)), "down, expert %d" % e

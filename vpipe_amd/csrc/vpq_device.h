@@ -118,7 +118,8 @@ __device__ __forceinline__ float gated_f32(int act, float gate, float up)
     const float t = tanhf(0.7978845608028654f * (gate + 0.044715f * gate * gate * gate));
     return 0.5f * gate * (1.0f + t) * up;
   }
-  return (gate / (1.0f + __expf(-gate))) * up;
+  const float t = __expf(-fabsf(gate));             // (0, 1]: no overflow, and 1 + t has an exact-to-1-ulp reciprocal
+  return gate * ((gate < 0.0f ? t : 1.0f) * __builtin_amdgcn_rcpf(1.0f + t)) * up;
 }
 
 // The value lane^1 holds (quad_perm [1,0,3,2]).

@@ -8,22 +8,31 @@
 // only thing the wavefronts share is the x tile.  Two workgroups fit a CU and fill each other's waits.  Unpacking costs
 // about 2.9 vector instructions a weight, so a tile shorter than 96 rows would be bound by it.
 //
-// Loads.  x comes through three LDS stages of 64 values of K (direct-to-LDS, 8 rows x 128 bytes each), requested two
-// steps ahead; one barrier a step.  Codes come 128 bytes per weight row at a time (four steps of 4 bits, two of 8), whole
-// lines into a slot of the wavefront's own, which is copied to registers at the start of those steps and requested
-// again at once.  Scales and biases of those steps are one ordinary load of each per lane, requested a chunk ahead.  The
-// wait for them is the compiler's, and falls where they are copied, behind the request of a coming x tile: for 4-bit
-// codes it waits for that tile too, so one step in four starts with an empty queue.
+// Loads.  x comes through three LDS stages of 64 values of K (direct-to-LDS, 8 rows x 128 bytes each), requested two to
+// three steps ahead; one barrier a step.  Codes come 128 bytes per weight row at a time (four steps of 4 bits, two of 8),
+// whole lines into a slot of the wavefront's own, which is copied to registers and requested again at once.  Scales and
+// biases of those steps are one ordinary load of each per lane, requested a chunk ahead.  The wait for them is the
+// compiler's and empties the queue; it stands before the coming tile of x is requested.
+//
+// A step is four quarters of 16 values of K.  While a quarter's MFMAs run, the wavefront reads the next quarter's fragments
+// of x and unpacks its weights, one MFMA between every few vector instructions.  The barrier stands before the fourth
+// quarter: by then every fragment of the step is in registers, and the first reads of the next step run under that
+// quarter's MFMAs.  Read and unpacked in the quarter that uses them: 5 to 12 % slower at 80..333 rows.
 //
 // With K split over workgroups (few tiles over a long K) a share leaves fp32 planes that splitk_fold adds in order.
 //
-// What bounds it: a step's chain (barrier, operand reads, unpacking, MFMAs) for a workgroup alone on its CU, 0.57 us at
-// 96 rows; several to a CU, the LDS reads of x (4 KB a row fragment and wavefront) and the MFMAs together.  Two 32-row
-// fragments of weights a wavefront halve the LDS reads but leave half the workgroups: slower up to 1024 rows (4096 -> 24576
-// at 128 / 333 rows 73 / 114 us against 51 / 92).  Pinning one MFMA between every seven vector instructions: no gain.
-// Measured (us, before: the 256 x 128 tiles, split over K where a workspace allows, and the large tile; after):
-// 4096 -> 24576 gated at 80 / 128 / 333 rows 68 / 69 / 104 -> 45 / 51 / 92; 4096 -> 1024 at 333 rows 24 -> 19;
-// 12288 -> 4096 at 80 / 333 rows 36 / 69 -> 27 / 57; without a workspace 4096 -> 4096 at 80..333 rows 56..63 -> 33..36.
+// What bounds it.  A workgroup alone on its CU: the LDS reads' latency, 230 cycles for a quarter of 130 (0.39 us a step at
+// 64 rows; six stages of x and two slots of codes, without the compiler's wait: no gain).  Several to a CU: LDS (384 cycles
+// of reads and 128 of direct-to-LDS writes a step of 96 rows, 553 taken) and, close behind, a vector ALU that an MFMA
+// shares for half of its 32 cycles (a slot of n instructions lasts 18 + 4 n), at a clock that the power limit holds at
+// 1.5 to 1.8 GHz.  Two 32-row fragments of weights a wavefront halve the LDS reads but leave half the workgroups: 2 % at
+// 2048 tokens of experts, slower below 512 rows.
+// Stores: lanes l and l + 32 exchange quads so that each stores 16 bytes; with four 4-byte pieces and a divide in the
+// activation the store of a 128-row gated tile took 6.9 us of a workgroup's 34.
+// Measured (us, fragments read where they are used, narrow stores; now): 4096 -> 24576 gated at 80 / 128 / 333 rows
+// 47 / 53 / 99 -> 41 / 49 / 91; 4096 -> 4096 at 128 / 333 / 1000 rows 21.4 / 29.3 / 53.7 -> 18.2 / 26.8 / 46.4; groups of
+// 32, 3840 -> 3840 at 333 rows 33.5 -> 30.0.
+#include <atomic>
 #include <type_traits>
 
 #include "vpq_device.h"
@@ -35,7 +44,7 @@ namespace vpq {
 namespace {
 
 constexpr int kMidWaves = 4;
-constexpr int kMidStages = 3;
+constexpr int kMidStages = 3;                 // stages of x
 constexpr int kMidTileN = 32 * kMidWaves;     // weight rows per workgroup
 constexpr int kMidRowB = 128;                 // bytes of an LDS row: 64 elements of x, or a chunk of codes
 
@@ -88,9 +97,12 @@ __device__ __forceinline__ floatx16 mid_mfma(u32x4 a, u32x4 b, floatx16 c)
 
 // A workgroup's tile: rows [m0, m0 + 32 MT) of x (of slots) against weight rows [n0, n0 + 128) of the pack given, over
 // share `ks` of K.
+// GROUPED: `slots` holds the block's srow (gated) or sdst values, lane l of [j] that of slot 64 j + l; `span` slots are
+// the workgroup's.
 template <int MT, int BITS, int GROUP, bool F16, bool GROUPED>
-__device__ __forceinline__ void mid_tile(const MidParams& p, uint8_t* x_lds, uint8_t* c_lds, int m0, int n0, int ks,
-                                         const uint32_t* pack_w, const uint16_t* pack_s, const uint16_t* pack_b)
+__device__ __forceinline__ void mid_tile(const MidParams& p, uint8_t* x_lds, int m0, int n0, int ks,
+                                         const uint32_t* pack_w, const uint16_t* pack_s, const uint16_t* pack_b,
+                                         const int (&slots)[4], int span)
 {
   constexpr int BM = 32 * MT;
   constexpr int SPC = 16 / BITS;                    // K steps of 64 per chunk of codes: 4 or 2
@@ -102,6 +114,7 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, uint8_t* x_lds, uin
   constexpr int kSlot = 32 * kMidRowB;
   constexpr int kWords = kMidRowB / 4 / 2;          // words of a weight row's chunk that one lane unpacks
 
+  uint8_t* c_lds = x_lds + kMidStages * kXStage;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int frow = lane & 31;                       // row of a 32-row operand
@@ -113,37 +126,36 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, uint8_t* x_lds, uin
   const int chunks = (steps + SPC - 1) / SPC;
 
   // ---- addresses ----
-  const bool gathered = GROUPED && p.srow != nullptr;
-  const uint8_t* xblk = reinterpret_cast<const uint8_t*>(p.x) + (gathered ? (size_t)0 : (size_t)m0 * p.K * 2) +
+  const uint8_t* xblk = reinterpret_cast<const uint8_t*>(p.x) + (GROUPED && p.gate_act ? (size_t)0 : (size_t)m0 * p.K * 2) +
                         (size_t)k_first * 128;
   uint32_t x_off[XL];
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
     const int row = (wave * XL + i) * 8 + (lane >> 3);
     int rg = m0 + row < p.M ? row : p.M - 1 - m0;
-    if (gathered) {                                 // a padding slot reads row 0, unused
-      const int src = p.srow[m0 + rg];
-      rg = src >= 0 && src < p.rows_x ? src : 0;
+    if constexpr (GROUPED) {
+      if (p.gate_act) {                             // a padding slot reads row 0, unused
+        const int j = (wave * XL + i) >> 3;         // (8 rows lie in one 64)
+        const int at = j == 0 ? slots[0] : j == 1 ? slots[1] : j == 2 ? slots[2] : slots[3];
+        const int src = __shfl(at, row & 63, kWave);
+        rg = src >= 0 && src < p.rows_x ? src : 0;
+      }
     }
     x_off[i] = (uint32_t)rg * (uint32_t)p.K * 2u + (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) * 16);
   }
-  const int nw = n0 + wave * 32;                    // this wavefront's first weight row
+  const int nw = n0 + wave * 32;                  // this wavefront's first weight row
   const uint32_t row_bytes = (uint32_t)p.K * BITS / 8;
   const int row_left = (int)row_bytes - k_first * (8 * BITS);   // bytes of a row from this share's start on
   const uint8_t* cblk = reinterpret_cast<const uint8_t*>(pack_w) + (size_t)(nw < p.N ? nw : p.N - 1) * row_bytes +
                         (size_t)k_first * (8 * BITS);
   const int w_last = nw < p.N ? p.N - 1 - nw : 0;   // rows past the last repeat it
-  uint32_t c_row[CL];
-#pragma unroll
-  for (int i = 0; i < CL; ++i) {
-    const int row = i * 8 + (lane >> 3);
-    c_row[i] = (uint32_t)(row < w_last ? row : w_last) * row_bytes;
-  }
+  uint32_t c_lane = (uint32_t)(lane >> 3);          // load i of a chunk covers rows 8 i .. 8 i + 7
   const uint32_t c_piece = (uint32_t)(((lane & 7) ^ (lane >> 4)) * 16);   // key (row >> 1) & 7, bit 2 by the load
   const int Kg = p.K / GROUP;
-  const size_t at = (size_t)((nw < p.N ? nw : p.N - 1) + (frow < w_last ? frow : w_last)) * Kg;
-  const uint16_t* srow = pack_s + at;
-  const uint16_t* brow = pack_b + at;
+  const size_t sb_at = (size_t)(nw < p.N ? nw : p.N - 1) * Kg;
+  const uint16_t* sblk = pack_s + sb_at;
+  const uint16_t* bblk = pack_b + sb_at;
+  const uint32_t sb_row = (uint32_t)(frow < w_last ? frow : w_last) * (uint32_t)Kg;
   uint8_t* slot = c_lds + wave * kSlot;
 
   auto request_x = [&](int step, int stage) {
@@ -156,24 +168,26 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, uint8_t* x_lds, uin
     const uint8_t* src = cblk + (size_t)c * 128;
     const int left = row_left - c * 128;            // a piece past the row's end reads the chunk's first, unused
     const uint32_t dst = mid_lds(slot);
+    asm volatile("" : "+v"(c_lane));                // (no register per load is held over the loop)
 #pragma unroll
     for (int i = 0; i < CL; ++i) {
       const uint32_t at = c_piece ^ (uint32_t)((i & 1) * 64);
-      mid_dma16(dst + i * 1024, src, c_row[i] + ((int)at < left ? at : 0u));
+      const uint32_t row = c_lane + 8 * i, live = row < (uint32_t)w_last ? row : (uint32_t)w_last;
+      mid_dma16(dst + i * 1024, src, __umul24(live, row_bytes) + ((int)at < left ? at : 0u));
     }
   };
   uint32_t sn[SGW], bn[SGW];                        // scales and biases of the coming chunk
   auto request_scales = [&](int c) {
     const int g0 = k_first * (64 / GROUP) + c * SG;
     if (g0 + SG <= Kg) {
-      __builtin_memcpy(sn, srow + g0, SG * 2);
-      __builtin_memcpy(bn, brow + g0, SG * 2);
+      __builtin_memcpy(sn, sblk + (sb_row + (uint32_t)g0), SG * 2);
+      __builtin_memcpy(bn, bblk + (sb_row + (uint32_t)g0), SG * 2);
     } else {
 #pragma unroll
       for (int i = 0; i < SGW; ++i) {
-        const int a = g0 + 2 * i < Kg ? g0 + 2 * i : Kg - 1, b = g0 + 2 * i + 1 < Kg ? g0 + 2 * i + 1 : Kg - 1;
-        sn[i] = (uint32_t)srow[a] | ((uint32_t)srow[b] << 16);
-        bn[i] = (uint32_t)brow[a] | ((uint32_t)brow[b] << 16);
+        const int g = g0 + 2 * i < Kg ? g0 + 2 * i : Kg - 1, h = g0 + 2 * i + 1 < Kg ? g0 + 2 * i + 1 : Kg - 1;
+        sn[i] = (uint32_t)sblk[sb_row + (uint32_t)g] | ((uint32_t)sblk[sb_row + (uint32_t)h] << 16);
+        bn[i] = (uint32_t)bblk[sb_row + (uint32_t)g] | ((uint32_t)bblk[sb_row + (uint32_t)h] << 16);
       }
     }
   };
@@ -187,157 +201,270 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, uint8_t* x_lds, uin
   uint32_t cw[kWords], sc[SGW], bi[SGW];
 
   const uint32_t f_sw = (uint32_t)((frow >> 1) & 7);
-  auto take_codes = [&]() {
+  auto take_codes = [&](auto first, auto last) {    // those of the MFMAs [first, last) of a chunk
+    constexpr int lo = decltype(first)::value, hi = decltype(last)::value;
     const uint8_t* rp = slot + frow * kMidRowB;
     if constexpr (BITS == 4) {
 #pragma unroll
-      for (int q = 0; q < 16; ++q) {                // MFMA q of the chunk: word 2q + fkh
+      for (int q = lo; q < hi; ++q) {               // MFMA q: word 2q + fkh
         cw[q] = *reinterpret_cast<const uint32_t*>(rp + (((uint32_t)(q >> 1) ^ f_sw) * 16) + (q & 1) * 8 + fkh * 4);
       }
     } else {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {                 // MFMA q: words 4q + 2 fkh, + 1
+      for (int q = lo; q < hi; ++q) {               // MFMA q: words 4q + 2 fkh, + 1
         const u32x2 v = *reinterpret_cast<const u32x2*>(rp + (((uint32_t)q ^ f_sw) * 16) + fkh * 8);
         cw[2 * q] = v[0];
         cw[2 * q + 1] = v[1];
       }
     }
   };
-  // Step `sub` of the taken chunk against the x tile of `stage`.
-  auto contract = [&](auto sub_c, int stage) {
-    constexpr int sub = decltype(sub_c)::value;
-    const uint8_t* xb = x_lds + stage * kXStage + frow * kMidRowB;
+  // Operands of one quarter step: the MT fragments of x and the unpacked weights, two sets in turn.
+  u32x4 xf[2][MT], wf[2];
+  auto read_x = [&](int stage, auto k_c) {          // quarter k of a step
+    constexpr int k = decltype(k_c)::value;
+    const uint8_t* xb = x_lds + stage * kXStage + frow * kMidRowB + ((uint32_t)(2 * k + fkh) ^ f_sw) * 16;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      u32x4 xf[MT];
-      const uint32_t c = ((uint32_t)(2 * k + fkh) ^ f_sw) * 16;
+    for (int i = 0; i < MT; ++i) { xf[k & 1][i] = *reinterpret_cast<const u32x4*>(xb + i * (32 * kMidRowB)); }
+  };
+  auto unpack = [&](auto q_c) {                     // MFMA q of the taken chunk
+    constexpr int q = decltype(q_c)::value;
+    constexpr int g = q * 16 / GROUP;               // group of the chunk
+    const float s = (g & 1) ? elt_hi_to_f32<F16>(sc[g >> 1]) : elt_lo_to_f32<F16>(sc[g >> 1]);
+    const float b = (g & 1) ? elt_hi_to_f32<F16>(bi[g >> 1]) : elt_lo_to_f32<F16>(bi[g >> 1]);
+    uint4 wv;
+    if constexpr (BITS == 4) {
+      wv = dequant_word_fp8<F16>(cw[q], s, b);
+    } else {
+      wv = dequant_bytes(cw[2 * q], cw[2 * q + 1], s, b);
+    }
+    wf[q & 1] = u32x4{wv.x, wv.y, wv.z, wv.w};
+  };
+  auto keep = [&](auto set_c) {                     // no instruction: the unpacking stays where it is written
+    u32x4& v = wf[decltype(set_c)::value];
+    asm volatile("" : "+v"(v));
+  };
+  auto multiply = [&](auto k_c) {
+    constexpr int k = decltype(k_c)::value;
 #pragma unroll
-      for (int i = 0; i < MT; ++i) { xf[i] = *reinterpret_cast<const u32x4*>(xb + i * (32 * kMidRowB) + c); }
-      constexpr int q0 = sub * 4;
-      const int q = q0 + k;
-      const int g = q * 16 / GROUP;                 // group of the chunk
-      const float s = (g & 1) ? elt_hi_to_f32<F16>(sc[g >> 1]) : elt_lo_to_f32<F16>(sc[g >> 1]);
-      const float b = (g & 1) ? elt_hi_to_f32<F16>(bi[g >> 1]) : elt_lo_to_f32<F16>(bi[g >> 1]);
-      uint4 wv;
-      if constexpr (BITS == 4) {
-        wv = dequant_word<F16>(cw[q], s, b);
-      } else {
-        wv = dequant_bytes(cw[2 * q], cw[2 * q + 1], s, b);
-      }
-      const u32x4 wf = {wv.x, wv.y, wv.z, wv.w};
+    for (int i = 0; i < MT; ++i) { acc[i] = mid_mfma<F16>(wf[k & 1], xf[k & 1][i], acc[i]); }
+  };
+  // What a quarter interleaves: the next quarter's reads of x first, then one MFMA between the unpacking's instructions.
+  auto interleave = [&]() {
+    __builtin_amdgcn_sched_group_barrier(0x100, MT, 0);
 #pragma unroll
-      for (int i = 0; i < MT; ++i) { acc[i] = mid_mfma<F16>(wf, xf[i], acc[i]); }
+    for (int i = 0; i < MT; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 24 / MT, 0);
     }
   };
 
   // ---- K loop ----
-  // Loads of step t, in order: x(t + 2) [XL], and at a chunk's first step the next chunk's codes [CL] and scales.  The
-  // first step of a chunk waits for everything that was requested before it (and, where its scales are copied, the
-  // compiler waits again, for the x of this step's request as well); the third
-  // needs x that has the codes and a step of x behind it, the fourth x that has a step of x behind it.  The last steps
-  // request the last tile again (never read), so that the counts hold to the end.
+  // Stage t % 3 holds x(t); x(t + 3) is requested once every wavefront is past step t.  A chunk of codes is requested once
+  // the one before has been copied to registers.
+  constexpr std::integral_constant<int, 0> kNone{};
+  constexpr std::integral_constant<int, 4> kFour{};
+  constexpr std::integral_constant<int, SPC * 4> kAll{};
+  auto take_scales = [&]() {
+#pragma unroll
+    for (int i = 0; i < SGW; ++i) {
+      sc[i] = sn[i];
+      bi[i] = bn[i];
+      asm volatile("" : "+v"(sc[i]), "+v"(bi[i]));
+    }
+  };
+  auto request_chunk = [&](int c) {                 // (the taken codes are in registers: their slot is free)
+    if (c < chunks) {
+#pragma unroll
+      for (int i = 0; i < kWords; ++i) { asm volatile("" : "+v"(cw[i])); }
+      request_codes(c);
+      request_scales(c);
+    }
+  };
   request_codes(0);
   request_scales(0);
   request_x(0, 0);
-  request_x(steps > 1 ? 1 : 0, 1);
+  for (int t = 1; t < kMidStages && t < steps; ++t) { request_x(t, t); }
+  asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" : : : "memory");
+  take_codes(kNone, kAll);
+  take_scales();
+  asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+  request_chunk(1);
+  read_x(0, kNone);
+  unpack(kNone);
+  keep(kNone);
   int stage = 0;
-  for (int c = 0; c < chunks; ++c) {
-    const bool more = c + 1 < chunks;
-    auto step = [&](auto sub_c) {
-      constexpr int sub = decltype(sub_c)::value;
-      const int t = c * SPC + sub;
-      if (sub > 0 && t >= steps) { return; }
-      if (sub == 0) {
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : : : "memory");
-      } else if (sub == 2 && more) {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(CL + XL) : "memory");
-      } else if (sub >= 2) {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(XL) : "memory");
-      } else {
-        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
-      }
-      __builtin_amdgcn_s_barrier();                 // x(t) is here, and everybody is done with the stage of x(t - 1)
-      asm volatile("" : : : "memory");
-      const int fill = stage == 0 ? 2 : stage - 1;
-      request_x(t + 2 < steps ? t + 2 : steps - 1, fill);
-      if (sub == 0) {
-        take_codes();
-#pragma unroll
-        for (int i = 0; i < SGW; ++i) { sc[i] = sn[i]; bi[i] = bn[i]; }
-        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
-        if (more) {
-          request_codes(c + 1);
-          request_scales(c + 1);
-        }
-      }
-      contract(sub_c, stage);
-      stage = stage == 2 ? 0 : stage + 1;
+  // Step `sub` of chunk c: its first three quarters, then the passage to the next step, under whose cover the fourth runs.
+  auto step = [&](int c, auto sub_c) {
+    constexpr int sub = decltype(sub_c)::value;
+    constexpr int q = sub * 4;
+    const int t = c * SPC + sub;
+    auto quarter = [&](auto k_c) {
+      constexpr int k = decltype(k_c)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      read_x(stage, std::integral_constant<int, k + 1>());
+      multiply(k_c);
+      unpack(std::integral_constant<int, q + k + 1>());
+      interleave();
+      keep(std::integral_constant<int, (k + 1) & 1>());
+      __builtin_amdgcn_sched_barrier(0);
     };
-    step(std::integral_constant<int, 0>());
-    step(std::integral_constant<int, 1>());
+    quarter(std::integral_constant<int, 0>());
+    if (sub == 0 && SPC == 4 && c > 0) { request_chunk(c + 1); }
+    quarter(std::integral_constant<int, 1>());
+    if constexpr (sub == SPC - 1 && SPC == 4) { take_codes(kNone, kFour); }   // (there since the last passage)
+    quarter(std::integral_constant<int, 2>());
+    // The passage needs x(t + 1), requested two passages ago, and at a chunk's end (8 bits) or a step before it the next
+    // codes.  Younger than those are a step of x and, in the first half of a chunk, the codes requested since.
+    if constexpr (sub == SPC - 1) { take_scales(); }          // (the compiler waits for everything)
+    if (t + kMidStages - 1 >= steps) {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : : : "memory");
+    } else if (sub < SPC / 2 && c + 1 < chunks) {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(XL + CL) : "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(XL) : "memory");
+    }
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" : : : "memory");
+    if (t + kMidStages < steps) { request_x(t + kMidStages, stage); }
+    stage = stage == kMidStages - 1 ? 0 : stage + 1;
+    __builtin_amdgcn_sched_barrier(0);
+    read_x(stage, kNone);
+    if constexpr (sub == SPC - 1) {
+      if constexpr (SPC == 4) {
+        take_codes(kFour, kAll);
+      } else {
+        take_codes(kNone, kAll);
+      }
+    }
+    multiply(std::integral_constant<int, 3>());
+    // 8 bits: a chunk is two steps only.  A workgroup alone on its CU wants its codes as early as can be (4096 -> 4096 at
+    // 333 rows 40.4 us, behind the unpacking 41.9); several hide the wait for the copy less well than the unpacking does
+    // (2048 tokens, 128 experts: 303 us, behind it 277)
+    constexpr bool kChunkEnd = sub == 1 && SPC == 2;
+    if constexpr (kChunkEnd && !GROUPED) {
+      __builtin_amdgcn_sched_barrier(0);
+      request_chunk(c + 2);
+    }
+    unpack(std::integral_constant<int, sub + 1 < SPC ? q + 4 : 0>());
+    if (sub + 1 < SPC || SPC == 4) { interleave(); }
+    keep(kNone);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kChunkEnd && GROUPED) { request_chunk(c + 2); }
+  };
+  const int full = steps / SPC;
+  for (int c = 0; c < full; ++c) {
+    step(c, std::integral_constant<int, 0>());
+    step(c, std::integral_constant<int, 1>());
     if constexpr (SPC > 2) {
-      step(std::integral_constant<int, 2>());
-      step(std::integral_constant<int, 3>());
+      step(c, std::integral_constant<int, 2>());
+      step(c, std::integral_constant<int, 3>());
     }
   }
-  asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-
-  // ---- store: a lane holds, for row m = lane % 32 of each i, four consecutive n per register quad ----
-  const bool quads = (p.N & 3) == 0;
-  const bool pairs = ((p.out_stride | p.out_off) & 1) == 0;
-  // rows that a gated block stores: all its slots, zeros past the fragments that were multiplied
-  constexpr int kStored = GROUPED ? kGroupedBlockRows / 32 : MT;
-#pragma unroll
-  for (int i = 0; i < kStored; ++i) {
-    const int m = m0 + i * 32 + frow;
-    if (m >= p.M || (i >= MT && !p.gate_act)) { continue; }
-    bool pad = i >= MT;                             // act(0) * 0 = +0
-    int mdst = m;
-    if constexpr (GROUPED) {
-      if (p.gate_act) {
-        const int src = p.srow[m];
-        pad = pad || src < 0 || src >= p.rows_x;
-      } else {
-        mdst = p.sdst[m];
-        if (mdst < 0 || mdst >= p.rows_y) { continue; }
+  const int rest = steps - full * SPC;
+  if (rest > 0) {
+    step(full, std::integral_constant<int, 0>());
+    if constexpr (SPC > 2) {
+      if (rest > 1) {
+        step(full, std::integral_constant<int, 1>());
+        if (rest > 2) { step(full, std::integral_constant<int, 2>()); }
       }
     }
+  }
+
+  // ---- store: a lane holds, for row m = lane % 32 of each i, four consecutive n per register quad ----
+  if (!GROUPED && p.ksplit > 1) {
 #pragma unroll
-    for (int rq = 0; rq < 4; ++rq) {
-      const int n = nw + rq * 8 + fkh * 4;
-      if (n >= p.N) { continue; }
-      const floatx16& ai = acc[i < MT ? i : 0];
-      const float v[4] = {ai[rq * 4], ai[rq * 4 + 1], ai[rq * 4 + 2], ai[rq * 4 + 3]};
-      if (!GROUPED && p.ksplit > 1) {
+    for (int i = 0; i < MT; ++i) {
+      const int m = m0 + i * 32 + frow;
+      if (m >= p.M) { continue; }
+#pragma unroll
+      for (int ar = 0; ar < 4; ++ar) {
+        const floatx16& v = acc[i];
+        const int n = nw + ar * 8 + fkh * 4;
         float* o = p.plane + ((size_t)ks * p.M + m) * p.N + n;
-        if (quads) {
-          *reinterpret_cast<floatx4*>(o) = floatx4{v[0], v[1], v[2], v[3]};
+        if ((p.N & 3) == 0) {
+          if (n < p.N) { *reinterpret_cast<floatx4*>(o) = floatx4{v[ar * 4], v[ar * 4 + 1], v[ar * 4 + 2], v[ar * 4 + 3]}; }
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            if (n + e < p.N) { o[e] = v[e]; }
+            if (n + e < p.N) { o[e] = v[ar * 4 + e]; }
           }
         }
-      } else if (p.gate_act) {                    // (gate, up, gate, up)
-        uint16_t* o = p.y + (size_t)m * p.out_stride + p.out_off + (n >> 1);
-        const float f0 = GROUPED && pad ? 0.0f : gated_f32(p.gate_act, v[0], v[1]);
-        const float f1 = GROUPED && pad ? 0.0f : gated_f32(p.gate_act, v[2], v[3]);
-        if (pairs && n + 3 < p.N) {
-          *reinterpret_cast<uint32_t*>(o) = pack_elt2<F16>(f0, f1);
+      }
+    }
+    return;
+  }
+  // Lanes l and l + 32 hold alternate quads of one row: they exchange two of their four, and each has 16 consecutive n
+  // (gated: 8 outputs) to store in 16-byte pieces.
+  const uint32_t y_bits = (uint32_t)(uintptr_t)p.y | (uint32_t)(p.gate_act ? p.out_stride | p.out_off : p.N) << 1;
+  const bool wide = (y_bits & 15) == 0, pairs = (y_bits & 3) == 0;
+  auto put = [&](uint16_t* o, u32x4 v, int left) {  // the first `left` of eight elements
+    if (wide && left >= 8) {
+      *reinterpret_cast<u32x4*>(o) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (pairs && left >= 2 * e + 2) {
+          *reinterpret_cast<uint32_t*>(o + 2 * e) = v[e];
         } else {
-          o[0] = (uint16_t)f32_to_elt_bits<F16>(f0);
-          if (n + 3 < p.N) { o[1] = (uint16_t)f32_to_elt_bits<F16>(f1); }
+          if (left > 2 * e) { o[2 * e] = (uint16_t)v[e]; }
+          if (left > 2 * e + 1) { o[2 * e + 1] = (uint16_t)(v[e] >> 16); }
         }
+      }
+    }
+  };
+  auto exchange = [](uint32_t& lo, uint32_t& hi) {  // upper lanes' `lo` for lower lanes' `hi`
+    const auto r = __builtin_amdgcn_permlane32_swap(lo, hi, false, false);
+    lo = r[0];
+    hi = r[1];
+  };
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = m0 + i * 32 + frow;
+    bool pad = false;
+    int mdst = m;
+    if constexpr (GROUPED) {
+      const int at = __shfl(slots[i >> 1], (i & 1) * 32 + frow, kWave);
+      if (p.gate_act) {
+        pad = at < 0 || at >= p.rows_x;
       } else {
-        uint16_t* o = p.y + (size_t)mdst * p.N + n;
-        if (quads) {
-          *reinterpret_cast<uint2*>(o) = make_uint2(pack_elt2<F16>(v[0], v[1]), pack_elt2<F16>(v[2], v[3]));
-        } else {
+        mdst = at;
+        if (at < 0 || at >= p.rows_y) { continue; }
+      }
+    }
+    if (m >= p.M) { continue; }
+    const floatx16& v = acc[i];
+    if (p.gate_act) {                               // (gate, up, gate, up) a quad
+      uint32_t w[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if (n + e < p.N) { o[e] = (uint16_t)f32_to_elt_bits<F16>(v[e]); }
-          }
-        }
+      for (int rq = 0; rq < 4; ++rq) {
+        w[rq] = pad ? 0u : pack_elt2<F16>(gated_f32(p.gate_act, v[rq * 4], v[rq * 4 + 1]), gated_f32(p.gate_act, v[rq * 4 + 2], v[rq * 4 + 3]));
+      }
+      exchange(w[0], w[2]);
+      exchange(w[1], w[3]);
+      const int col = nw / 2 + fkh * 8;
+      put(p.y + (size_t)m * p.out_stride + p.out_off + col, u32x4{w[0], w[2], w[1], w[3]}, p.N / 2 - col);
+    } else {
+      uint32_t w[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) { w[e] = pack_elt2<F16>(v[2 * e], v[2 * e + 1]); }
+      exchange(w[0], w[4]);
+      exchange(w[1], w[5]);
+      exchange(w[2], w[6]);
+      exchange(w[3], w[7]);
+      const int n = nw + fkh * 16;
+      uint16_t* o = p.y + (size_t)mdst * p.N + n;
+      put(o, u32x4{w[0], w[1], w[4], w[5]}, p.N - n);
+      put(o + 8, u32x4{w[2], w[3], w[6], w[7]}, p.N - n - 8);
+    }
+  }
+  if constexpr (GROUPED) {                          // the slots past the fragments that were multiplied: padding, act(0) * 0 = +0
+    if (p.gate_act) {
+      for (int row = BM + frow; row < span; row += 32) {
+        const int col = nw / 2 + fkh * 8;
+        put(p.y + (size_t)(m0 + row) * p.out_stride + p.out_off + col, u32x4{0u, 0u, 0u, 0u}, p.N / 2 - col);
       }
     }
   }
@@ -345,12 +472,13 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, uint8_t* x_lds, uin
 
 }  // namespace
 
+constexpr size_t mid_lds_bytes(int mt) { return (size_t)(kMidStages * 32 * mt + kMidWaves * 32) * kMidRowB; }
+
 template <int MT, int BITS, int GROUP, bool F16>
 __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidParams p)
 {
   constexpr int BM = 32 * MT, BN = kMidTileN;
-  __shared__ __attribute__((aligned(16))) uint8_t x_lds[kMidStages * BM * kMidRowB];
-  __shared__ __attribute__((aligned(16))) uint8_t c_lds[kMidWaves * 32 * kMidRowB];
+  extern __shared__ __attribute__((aligned(16))) uint8_t x_lds[];
 
   // Workgroups go to the XCDs round robin: those that share a weight tile (one per tile of rows of x) are eight apart,
   // so that the pack is read from HBM once.
@@ -361,49 +489,69 @@ __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidPar
   if (unit >= units) { return; }
   const int ks = unit / p.tiles_n;
   const int m0 = (ur >> 3) * BM, n0 = (unit - ks * p.tiles_n) * BN;
-  mid_tile<MT, BITS, GROUP, F16, false>(p, x_lds, c_lds, m0, n0, ks, p.w, p.scales, p.biases);
+  // (the last tile multiplies as many fragments as have rows)
+  const int none[4] = {}, frags = (p.M - m0 + 31) / 32;
+  if (MT > 3 && frags == 3) {
+    mid_tile<3, BITS, GROUP, F16, false>(p, x_lds, m0, n0, ks, p.w, p.scales, p.biases, none, 0);
+  } else if (MT > 2 && frags == 2) {
+    mid_tile<2, BITS, GROUP, F16, false>(p, x_lds, m0, n0, ks, p.w, p.scales, p.biases, none, 0);
+  } else if (frags == 1) {
+    mid_tile<1, BITS, GROUP, F16, false>(p, x_lds, m0, n0, ks, p.w, p.scales, p.biases, none, 0);
+  } else {
+    mid_tile<MT, BITS, GROUP, F16, false>(p, x_lds, m0, n0, ks, p.w, p.scales, p.biases, none, 0);
+  }
 }
 
 // The expert-sorted form.  An expert's last block is mostly padding (16384 pairs of 128 experts: 191 blocks, 63 of them
 // with about ten live slots), and a prompt of some tokens gives each expert a few: a block multiplies as many 32-row
 // fragments as reach its last live slot, each count a K loop of its own, whose loads, LDS reads and MFMAs are those
-// rows' alone.  All weight tiles of a block go to one XCD (eight workgroups apart), whose L2 then holds its rows of x.
+// rows' alone.  A last block of one fragment is multiplied by the block before it as a fifth, so its weights are neither
+// read nor unpacked a second time (two fragments would leave one workgroup per CU).  All weight tiles of a block go to one
+// XCD (eight workgroups apart), whose L2 then holds its rows of x.
 // Two neighbouring blocks to an XCD, which mostly share an expert's weight tiles: 1 to 2 % slower (2048 tokens 298 -> 305 us).
 // Bound by the plain tile's step at full blocks, by unpacking and the codes' read at one fragment.  Measured (us, sort +
-// gate|up + down of one layer; before: 128 x 256 tiles with producer wavefronts, every block at full height), 2048 -> 768:
-// 2048 tokens, 8 of 128 experts 366 -> 300; 64 tokens 191 -> 138; 4096 tokens, 8 of 64 experts 557 -> 447, 8 bits 580 -> 498.
+// gate|up + down of one layer, 2048 -> 768; every block by itself, the plain tile's first form; now): 8 of 128 experts, 2048 /
+// 512 / 64 tokens 299 / 161 / 145 -> 250 / 149 / 135; 8 bits, 2048 tokens 345 -> 290.
 template <int BITS>
 __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_grouped_kernel(const MidParams p)
 {
-  __shared__ __attribute__((aligned(16))) uint8_t x_lds[kMidStages * kGroupedBlockRows * kMidRowB];
-  __shared__ __attribute__((aligned(16))) uint8_t c_lds[kMidWaves * 32 * kMidRowB];
+  extern __shared__ __attribute__((aligned(16))) uint8_t x_lds[];
   static_assert(kGroupedBlockRows == 128, "two slots per lane, four fragments");
 
   const int span = 8 * p.tiles_n;
   const int uq = (int)blockIdx.x / span, ur = (int)blockIdx.x - uq * span;
   const int tm = uq * 8 + (ur & 7);
   if (tm >= p.tiles_m) { return; }
-  const int e = p.tile2e[tm];
-  if (e < 0 || e >= p.n_experts) { return; }        // the whole workgroup, before any barrier
   const int m0 = tm * kGroupedBlockRows, n0 = (ur >> 3) * kMidTileN;
-  const uint32_t* w = p.w + (size_t)e * (size_t)p.N * (size_t)(p.K >> (BITS == 4 ? 3 : 2));
-  const uint16_t* s = p.scales + (size_t)e * (size_t)p.N * (size_t)(p.K >> 6);
-  const uint16_t* b = p.biases + (size_t)e * (size_t)p.N * (size_t)(p.K >> 6);
-
   const int lane = threadIdx.x & 63;
   const int* idx = p.gate_act ? p.srow : p.sdst;
   const int lim = p.gate_act ? p.rows_x : p.rows_y;
-  const int v0 = idx[m0 + lane], v1 = idx[m0 + 64 + lane];
-  const unsigned long long lo = __ballot(v0 >= 0 && v0 < lim), hi = __ballot(v1 >= 0 && v1 < lim);
-  const int live = hi != 0 ? ((hi >> 32) != 0 ? 4 : 3) : (lo >> 32) != 0 ? 2 : 1;
-  if (live == 1) {
-    mid_tile<1, BITS, 64, false, true>(p, x_lds, c_lds, m0, n0, 0, w, s, b);
+  const bool next = tm + 1 < p.tiles_m;
+  const int slots[4] = {idx[m0 + lane], idx[m0 + 64 + lane], next ? idx[m0 + 128 + lane] : -1, next ? idx[m0 + 192 + lane] : -1};
+  const int e = p.tile2e[tm], e_before = tm > 0 ? p.tile2e[tm - 1] : -1;
+  const int e_next = next ? p.tile2e[tm + 1] : -1, e_after = tm + 2 < p.tiles_m ? p.tile2e[tm + 2] : -1;
+  if (e < 0 || e >= p.n_experts) { return; }        // the whole workgroup, before any barrier
+  auto fragments = [&](int v0, int v1) {            // of a block, up to its last live slot
+    const unsigned long long lo = __ballot(v0 >= 0 && v0 < lim), hi = __ballot(v1 >= 0 && v1 < lim);
+    return hi != 0 ? ((hi >> 32) != 0 ? 4 : 3) : (lo >> 32) != 0 ? 2 : 1;
+  };
+  const int live = fragments(slots[0], slots[1]);
+  if (e_before == e && e_next != e && live == 1) { return; }   // the block before multiplies it
+  const bool both = e_next == e && e_after != e && fragments(slots[2], slots[3]) == 1;
+
+  const uint32_t* w = p.w + (size_t)e * (size_t)p.N * (size_t)(p.K >> (BITS == 4 ? 3 : 2));
+  const uint16_t* s = p.scales + (size_t)e * (size_t)p.N * (size_t)(p.K >> 6);
+  const uint16_t* b = p.biases + (size_t)e * (size_t)p.N * (size_t)(p.K >> 6);
+  if (both) {
+    mid_tile<5, BITS, 64, false, true>(p, x_lds, m0, n0, 0, w, s, b, slots, 2 * kGroupedBlockRows);
+  } else if (live == 1) {
+    mid_tile<1, BITS, 64, false, true>(p, x_lds, m0, n0, 0, w, s, b, slots, kGroupedBlockRows);
   } else if (live == 2) {
-    mid_tile<2, BITS, 64, false, true>(p, x_lds, c_lds, m0, n0, 0, w, s, b);
+    mid_tile<2, BITS, 64, false, true>(p, x_lds, m0, n0, 0, w, s, b, slots, kGroupedBlockRows);
   } else if (live == 3) {
-    mid_tile<3, BITS, 64, false, true>(p, x_lds, c_lds, m0, n0, 0, w, s, b);
+    mid_tile<3, BITS, 64, false, true>(p, x_lds, m0, n0, 0, w, s, b, slots, kGroupedBlockRows);
   } else {
-    mid_tile<4, BITS, 64, false, true>(p, x_lds, c_lds, m0, n0, 0, w, s, b);
+    mid_tile<4, BITS, 64, false, true>(p, x_lds, m0, n0, 0, w, s, b, slots, kGroupedBlockRows);
   }
 }
 
@@ -427,13 +575,28 @@ __global__ __launch_bounds__(256) void splitk_fold_kernel(const float* __restric
 
 namespace {
 
+// More LDS than the default limit needs the attribute, set once per kernel (two threads may both set it, which is harmless).
+template <int BITS>
+hipError_t mid_launch_grouped(dim3 grid, dim3 block, size_t lds, hipStream_t st, const MidParams& p)
+{
+  static std::atomic<bool> ready{false};
+  if (!ready.load(std::memory_order_acquire)) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(qmm_mid_grouped_kernel<BITS>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) { return e; }
+    ready.store(true, std::memory_order_release);
+  }
+  return launch_kernel(qmm_mid_grouped_kernel<BITS>, grid, block, lds, st, p);
+}
+
 template <int BITS, int GROUP, bool F16>
 hipError_t mid_launch(hipStream_t st, const MidParams& p, int mt, dim3 grid)
 {
   const dim3 block(kMidWaves * 64);
-  if (mt == 2) { return launch_kernel(qmm_mid_kernel<2, BITS, GROUP, F16>, grid, block, 0, st, p); }
-  if (mt == 3) { return launch_kernel(qmm_mid_kernel<3, BITS, GROUP, F16>, grid, block, 0, st, p); }
-  return launch_kernel(qmm_mid_kernel<4, BITS, GROUP, F16>, grid, block, 0, st, p);
+  const size_t lds = mid_lds_bytes(mt);
+  if (mt == 2) { return launch_kernel(qmm_mid_kernel<2, BITS, GROUP, F16>, grid, block, lds, st, p); }
+  if (mt == 3) { return launch_kernel(qmm_mid_kernel<3, BITS, GROUP, F16>, grid, block, lds, st, p); }
+  return launch_kernel(qmm_mid_kernel<4, BITS, GROUP, F16>, grid, block, lds, st, p);
 }
 
 hipError_t mid_launch_as(hipStream_t st, const GemmArgs& a, int mt, int splits, float* plane)
@@ -457,10 +620,10 @@ hipError_t mid_launch_as(hipStream_t st, const GemmArgs& a, int mt, int splits, 
   return a.f16 ? mid_launch<4, 64, true>(st, p, mt, grid) : mid_launch<4, 64, false>(st, p, mt, grid);
 }
 
-// What a GEMM takes, in microseconds: fitted to 36 000 timings of the seven kernels (three heights here, 256 x 128, three
-// large tiles) on 512..17408 x 512..34816 at 65..4096 rows, all four formats and gated stores, which it meets to a
-// twentieth.  Its choice is 0.8 % off the fastest on average.  Against the rule "the large tile from one round of its
-// tiles on, else the 256 x 128 tile" it takes 0.72 of the time, and in 14 of 5500 cases 4 to 8 % more.
+// What a GEMM takes, in microseconds.  The tall kernels' figures were fitted to 36 000 timings (256 x 128, three large
+// tiles) on 512..17408 x 512..34816 at 65..4096 rows, all four formats and gated stores, which they meet to a twentieth;
+// this kernel's to 160 timings of its three heights in the same ranges (a tenth).  Against the rule "the large tile from
+// one round of its tiles on, else the 256 x 128 tile" the choice takes 0.7 of the time.
 //
 // A split writes and reads its planes once more, and folds them in a launch of its own.
 double planes_us(int N, int M, int splits) { return splits > 1 ? 3.0 + (splits + 0.5) * (double)M * (double)N * 4.0 / 5.0e6 : 0.0; }
@@ -475,7 +638,7 @@ struct CostShape { int K, N, M, bits; bool gated; };
 // The busiest XCD counts (all workgroups of a weight tile are on one).  Every weight tile reads all of x, at 6.8 TB/s
 // from the shared cache once x outgrows an XCD's L2; that bounds M in the thousands.
 struct MidCost { double fixed, round, gated, step, alone; };
-constexpr MidCost kMidCost[5] = {{}, {}, {5.8, 0.4, 0.8, 0.335, 0.485}, {5.4, 1.2, 1.9, 0.406, 0.556}, {4.3, 2.8, 4.1, 0.468, 0.645}};
+constexpr MidCost kMidCost[5] = {{}, {}, {5.7, 0.7, 0.74, 0.328, 0.394}, {5.84, 1.42, 1.94, 0.375, 0.418}, {6.14, 2.02, 3.43, 0.445, 0.371}};
 
 double mid_us(const CostShape& s, int mt, int splits, int cus)
 {
@@ -485,8 +648,8 @@ double mid_us(const CostShape& s, int mt, int splits, int cus)
   const long tiles_n = (s.N + kMidTileN - 1) / kMidTileN;
   const long wgs = (tiles_n * splits + kXcds - 1) / kXcds * ((s.M + 32 * mt - 1) / (32 * mt));
   const double round = s.gated ? c.gated : c.round;
-  const double busy = (double)((wgs + per_xcd - 1) / per_xcd) * (per * c.step * (s.bits == 8 ? 1.1 : 1.0) + round);
-  const double alone = per * c.alone + round, fetch = (double)tiles_n * (double)s.M * (double)s.K * 2.0 / 6.8e6;
+  const double busy = (double)((wgs + per_xcd - 1) / per_xcd) * (per * c.step * (s.bits == 8 ? 1.24 : 1.0) + round);
+  const double alone = per * c.alone * (s.bits == 8 ? 1.22 : 1.0) + round, fetch = (double)tiles_n * (double)s.M * (double)s.K * 2.0 / 6.8e6;
   const double us = busy > alone ? busy : alone;
   return c.fixed + (us > fetch ? us : fetch) + planes_us(s.N, s.M, splits);
 }
@@ -592,8 +755,8 @@ hipError_t launch_qmm_grouped(hipStream_t st, const GemmArgs& a, const GroupedAr
   p.tile2e = g.tile2e; p.srow = g.srow; p.sdst = g.sdst;
   p.n_experts = g.n_experts; p.rows_x = g.rows_x; p.rows_y = g.rows_y;
   const dim3 grid((unsigned)((p.tiles_m + 7) / 8 * 8 * p.tiles_n)), block(kMidWaves * 64);
-  return a.bits == 8 ? launch_kernel(qmm_mid_grouped_kernel<8>, grid, block, 0, st, p)
-                     : launch_kernel(qmm_mid_grouped_kernel<4>, grid, block, 0, st, p);
+  const size_t lds = mid_lds_bytes(kGroupedBlockRows / 32 + 1);
+  return a.bits == 8 ? mid_launch_grouped<8>(grid, block, lds, st, p) : mid_launch_grouped<4>(grid, block, lds, st, p);
 }
 
 // Shares of K that pay for their planes; 1 where the tiles alone fill the chip.

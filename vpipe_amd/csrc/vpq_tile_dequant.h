@@ -37,6 +37,25 @@ __device__ __forceinline__ uint4 dequant_word(uint32_t word, float s, float b)
   return o;
 }
 
+// The same values by fp8 conversions: a byte 0..15 read as E4M3 is q * 2^-9 (exponent fields 0 and 1 are one linear range),
+// so the conversion scaled by 2^9 gives q exactly, two values an instruction.
+template <bool F16 = false>
+__device__ __forceinline__ uint4 dequant_word_fp8(uint32_t word, float s, float b)
+{
+  typedef float floatx2 __attribute__((ext_vector_type(2)));
+  const uint32_t even = word & 0x0f0f0f0fu, odd = (word >> 4) & 0x0f0f0f0fu;
+  const floatx2 e0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(even, 512.0f, false);
+  const floatx2 e1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(even, 512.0f, true);
+  const floatx2 o0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(odd, 512.0f, false);
+  const floatx2 o1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(odd, 512.0f, true);
+  uint4 o;
+  o.x = pack_elt2<F16>(fmaf(s, e0[0], b), fmaf(s, o0[0], b));
+  o.y = pack_elt2<F16>(fmaf(s, e0[1], b), fmaf(s, o0[1], b));
+  o.z = pack_elt2<F16>(fmaf(s, e1[0], b), fmaf(s, o1[0], b));
+  o.w = pack_elt2<F16>(fmaf(s, e1[1], b), fmaf(s, o1[1], b));
+  return o;
+}
+
 // 8 bytes of two packed words -> 8 bf16 of fma(s, q, b), as one 16-byte LDS chunk (the 8-bit pack).
 __device__ __forceinline__ uint4 dequant_bytes(uint32_t w0, uint32_t w1, float s, float b)
 {
