@@ -109,3 +109,48 @@ def test_gather_rejects_bad_arguments(vpq, dev):
     assert L.vpq_gather_qmv_gated_w4g64_bf16(None, p, p, p, p, p, 64, 8, p, 1, 1, 1, 7) == -2                      # activation
     assert L.vpq_gather_down_qmv_w4g64_bf16(None, p, p, p, p, p, 60, 8, p, 1, 1) == -2                             # K % 64
     assert L.vpq_gather_down_qmv_w4g64_bf16(None, p, p, p, p, p, 64, 8, p, 70000, 1) == -2                         # grid limit
+
+
+# one group; half a wavefront's pass and just past it; one pass and two; odd group counts; the deepest that the gather kernel
+# takes and the first that it leaves; N that ends inside a set of rows; enough pairs that a wavefront walks several sets
+@pytest.mark.parametrize("K,N,pairs", [(64, 2, 3), (1024, 130, 2), (1088, 36, 3), (2048, 1026, 40), (2112, 70, 3), (4096, 34, 2), (4160, 34, 2)])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_gathers_have_the_bits_of_the_plain_kernels(vpq, dev, D, bits, K, N, pairs):
+    E, gen = 3, torch.Generator(device="cpu").manual_seed(4800 + K + N + bits)
+    w = torch.randint(-2 ** 31, 2 ** 31, (E, N, K * bits // 32), dtype=torch.int32, generator=gen).to(dev)
+    s = (torch.rand((E, N, K // 64), generator=gen) * 0.015 / (16 if bits == 8 else 1) + 0.001).bfloat16().to(dev)
+    b = (-(2 ** (bits - 1)) * s.float() * 1.03).bfloat16()
+    eid = torch.randint(0, E, (pairs,), dtype=torch.int32, generator=gen)
+    eid[-1] = E                                          # no such expert: zeros
+    x = torch.randn((pairs, K), generator=gen).bfloat16().to(dev)
+    x[0, K // 2] = float("inf")
+    act = parity.Guarded((pairs, N // 2), torch.bfloat16, dev)
+    out = parity.Guarded((pairs, N), torch.bfloat16, dev)
+    gated = vpq.gather_qmv_gated_w8g64 if bits == 8 else vpq.gather_qmv_gated_w4g64
+    down = vpq.gather_down_qmv_w8g64 if bits == 8 else vpq.gather_down_qmv_w4g64
+    gated(w, s, b, x, K, N, eid.to(dev), 1, E, out=act.view)
+    down(w, s, b, x, K, N, eid.to(dev), E, out=out.view)
+    torch.cuda.synchronize()
+    act.assert_intact()
+    out.assert_intact()
+    assert not D.bits(act.view)[-1].any() and not D.bits(out.view)[-1].any()
+    for p in range(0, pairs - 1, max(1, pairs // 5)):
+        pack, xr = [t[int(eid[p])] for t in (w, s, b)], x[p:p + 1]
+        if bits == 8:
+            g = vpq.qmv_gated_w8g64(*pack, xr, K, N, 1, activation=1)
+            d = None
+        else:
+            g = vpq.qmv_swiglu_w4g64(*pack, xr, K, N, 1, variant=capi.VPQ_QMV_ROWS)
+            d = vpq.qmv_w4g64(*pack, xr, K, N, 1, variant=capi.VPQ_QMV_ROWS)
+        assert np.array_equal(D.bits(act.view)[p], D.bits(g)[0])
+        if d is not None:
+            assert np.array_equal(D.bits(out.view)[p], D.bits(d)[0])
+        else:                                            # (no plain entry point has that store: the sums, to their rounding)
+            deq = (s[int(eid[p])].double().repeat_interleave(64, 1) * w[int(eid[p])].view(torch.uint8).view(N, K).double() +
+                   b[int(eid[p])].double().repeat_interleave(64, 1))
+            want = deq @ xr[0].double()
+            got = out.view[p].double()
+            if p == 0:
+                assert not torch.isfinite(got).any()
+            else:                                        # one bf16 rounding, and fp32 sums over K
+                assert ((got - want).norm() / want.norm()).item() < 2.0 ** -8

@@ -304,6 +304,9 @@ static int rows8_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* 
     a.M = rows;
     return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
   }
+  if (gathered && vpq::qmv_gather_supports(K)) {
+    return finish(vpq::launch_qmv_gather(reinterpret_cast<hipStream_t>(stream), a, 8, pair_eid, rows, x_div, n_experts));
+  }
   return finish(vpq::launch_qmv_rows8(reinterpret_cast<hipStream_t>(stream), a, rows, gathered ? pair_eid : nullptr, x_div,
                                       n_experts));
 }
@@ -1050,6 +1053,9 @@ int gather_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales
   a.w = w; a.scales = scales; a.biases = biases; a.x = x; a.y = y;
   a.K = K; a.N = N; a.M = 1; a.y_f32 = false; a.cu_count = g_dev.cu_count;
   a.gate_act = gate_act;
+  if (vpq::qmv_gather_supports(K)) {
+    return finish(vpq::launch_qmv_gather(reinterpret_cast<hipStream_t>(stream), a, 4, pair_eid, npair, x_div, n_experts));
+  }
   return finish(vpq::launch_qmv_rows_gather(reinterpret_cast<hipStream_t>(stream), a, pair_eid, npair, x_div, n_experts));
 }
 

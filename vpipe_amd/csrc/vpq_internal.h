@@ -204,6 +204,9 @@ hipError_t launch_qmv_rows_group(hipStream_t st, const QmvArgs& a, const QmvGrou
 // Gathered (MoE) form, M = 1 per pair: a.w/scales/biases are batches [E, N, ...] of expert slabs,
 // pair p contracts slab pair_eid[p] with x row p / x_div into y row p (zeros for an id outside
 // [0, n_experts)); a.gate_act as in the plain form.
+// The gathers at K <= 4096 (vpq_qmv_gather.hip), with the bits of launch_qmv_rows_gather (8 bits: launch_qmv_rows8).
+bool qmv_gather_supports(int K);
+hipError_t launch_qmv_gather(hipStream_t st, const QmvArgs& a, int bits, const int* pair_eid, int pairs, int x_div, int n_experts);
 hipError_t launch_qmv_rows_gather(hipStream_t st, const QmvArgs& a, const int* pair_eid, int pairs, int x_div,
                                   int n_experts);
 // Sorted pairs, two slots per tile (a.M = 2): expert tile2e[tile], x row srow[slot] (x_from_srow) or the slot.
