@@ -185,3 +185,27 @@ def test_k_that_is_too_deep_for_the_batch_kernel(vpq, oracle, dev, D, M):
     for o, one in zip(outs, singles):
         o.assert_intact()
         assert torch.equal(o.view, one)
+
+
+@pytest.mark.parametrize("K", [6144, 6464, 9664])
+def test_eight_bit_codes_over_a_long_k_have_the_same_bits_in_few_workgroups(vpq, oracle, dev, D, K):
+    # few weight rows over a long K: two or three chunks of a wavefront in flight (every count of x loads, wavefronts with one
+    # chunk more than others, a last chunk that ends early), against many, whose workgroups keep one, and the oracle
+    N, n = 8224, 33
+    w, s, b = synth.make_weight8(n, K, K + 3)
+    gen = torch.Generator(device=dev).manual_seed(K)
+    wd = torch.randint(-2 ** 31, 2 ** 31, (N, K // 4), dtype=torch.int32, device=dev, generator=gen)
+    sd = torch.empty((N, K // 64), device=dev).uniform_(0.0003, 0.0012, generator=gen).bfloat16()
+    bd = -128 * sd
+    wd[:n], sd[:n], bd[:n] = D.u32(w, dev), D.bf16(s, dev), D.bf16(b, dev)
+    x = synth.make_act(21, K, K + 4)
+    xd = D.bf16(x, dev)
+    y64, _ = oracle.matmul8(w, s, b, x, K, n, 21, rounded=False)
+    few = [t[:n].contiguous() for t in (wd, sd, bd)]
+    for M in (2, 3, 4, 5, 6, 7, 8, 9, 16):
+        got = vpq.qmv_w8g64(*few, xd[:M], K, n, M, f32out=True)
+        parity.check_f32(got.cpu().numpy(), y64[:M])
+        assert torch.equal(got, vpq.qmv_w8g64(wd, sd, bd, xd[:M], K, N, M, f32out=True)[:, :n])
+    for M in (17, 21):
+        got = vpq.linear_twin("w8g64", *few, xd[:M], K, n, M)
+        assert torch.equal(got, vpq.linear_twin("w8g64", wd, sd, bd, xd[:M], K, N, M)[:, :n])

@@ -1,10 +1,14 @@
 // QMV for a batch of rows (2..64 rows of x; one row where the one-row kernel does not run), any K that is a multiple
 // of 64 (of 32 for groups of 32): the kernel template of vpq_qmv_batch*.hip.
 //
-// What bounds it: HBM for the pack at few rows; from 16 rows on no unit alone: the vector ALU is busy half of the cycles
-// (52 % on 4096 -> 24576 at 48 rows, 51 % on 5120 -> 151936 at 16; unpacking costs 14 instructions per 16 x 64 codes,
-// every 16 x 16 outputs 8 multiply-adds per group), the matrix pipe 18 and 13 %, and above 16 rows a wavefront waits for
-// each piece of x, which it has requested one piece ahead.
+// What bounds it: a workgroup's life of a request, a wait and a second one (6 to 7 us of 4096 values, two workgroups to a
+// CU), against which neither the arithmetic nor the traffic weighs much up to 32 rows -- 4096 -> 24576 at 4 / 24 rows, us:
+// 15.4 / 24.3; nothing contracted 13.1 / 22.6; no more x requested 15.1 / 20.9; no more codes 13.7 / 23.4; at 48 rows 44, 31,
+// 38 and 41.  Above 32 rows the vector ALU (half busy: unpacking costs 18 instructions per 16 x 64 codes, every 16 x 16
+// outputs 8 multiply-adds per group), the matrix pipe 18 %.  Tried: x in registers and workgroups that walk the tiles (a
+// barrier and a reduction per 16 rows cost more than the second start: 15.4 -> 18.7 at 4 rows; 104 -> 99 on 5120 -> 151936 at
+// 8); all of 33..64 rows in one workgroup, x two pieces ahead (one workgroup per CU: 44 -> 39 at 48 rows, 25 -> 30 at 24);
+// more chunks in flight for 4 bits (the first arrives later: 4096 -> 4096 5.5 -> 6.2).
 // Measured (us; before: one-item and ring kernels where K % 512 == 0, one wavefront
 // per weight row elsewhere, slabs of 16 rows above 16): 4096 -> 4096 at 16 / 48 rows 9.3 / 20.4 -> 6.3 / 10.0;
 // 4096 -> 12288 13.3 / 38.6 -> 12.2 / 21.0; 5120 -> 151936 at 8 / 16 rows 102 / 124 -> 96 / 114; 3840 -> 19328 at
@@ -20,7 +24,8 @@
 // consecutive lanes cover one 128-byte line (an L1 has about 72 requests in flight, so what counts is bytes per
 // request).  A slot is copied to registers (codes, x as MFMA operands, scales, biases), re-requested for the
 // wavefront's next chunk, and only then the copy is contracted: one chunk per wavefront is always in flight and no
-// wait has to be counted.  The 16-byte pieces of a row are XOR-swizzled so that the operand reads do not collide on
+// wait has to be counted.  With 8 bits, one workgroup per CU and a long K (twelve chunks a wavefront at 12288) the wavefront
+// has two or three slots instead: 12288 -> 4096 at 6 rows 17.9 -> 15.6 us.  The 16-byte pieces of a row are XOR-swizzled so that the operand reads do not collide on
 // banks.  The scales and biases of the workgroup's rows are two contiguous blocks of the pack and are brought in whole,
 // before anything else.
 //
@@ -70,13 +75,29 @@ struct BatchParams {
 static_assert(offsetof(BatchParams, y) == kPreloadWords * 4, "y starts the part that is not preloaded");
 
 // BITS: 4 or 8.  GROUP: 64 or 32.
-template <int T, int MR, int BITS, int GROUP>
+// DEEP: one workgroup per CU, which has its LDS to itself: x of a chunk in pieces of 8 KB, and slots for up to three chunks.
+constexpr int batch_x_bytes(int mr, int bits) { return mr * 4 * (128 * 8 / bits) * 2; }
+constexpr int batch_x_piece(int mr, int bits, bool deep)
+{
+  return batch_x_bytes(mr, bits) < (deep ? 8192 : 4096) ? batch_x_bytes(mr, bits) : (deep ? 8192 : 4096);
+}
+constexpr int batch_slot_bytes(int t, int mr, int bits, bool deep) { return t * 2048 + batch_x_piece(mr, bits, deep); }
+constexpr int batch_ring(int t, int mr, int bits, bool deep)
+{
+  return !deep || batch_x_piece(mr, bits, deep) < batch_x_bytes(mr, bits) ? 1
+         : batch_slot_bytes(t, mr, bits, deep) <= 4096                    ? 3
+         : batch_slot_bytes(t, mr, bits, deep) <= 6144                    ? 2
+                                                                          : 1;
+}
+
+template <int T, int MR, int BITS, int GROUP, bool DEEP>
 struct BatchShape {
   static constexpr int CK = 128 * 8 / BITS;                       // values of K per chunk
   static constexpr int AT = MR == 8 ? 2 : 1;                      // MFMA tiles of 16 rows of x
   static constexpr int RA = MR == 8 ? 4 : MR;                     // accumulator registers of one
   // x of a chunk comes in pieces of at most 4 KB: 16 registers of operands per lane, and two workgroups fit a CU
-  static constexpr int XS = MR * 4 * CK * 2 > 4096 ? MR * 4 * CK * 2 / 4096 : 1;
+  static constexpr int XS = batch_x_bytes(MR, BITS) / batch_x_piece(MR, BITS, DEEP);
+  static constexpr int RING = batch_ring(T, MR, BITS, DEEP);      // slots of a wavefront (one where XS > 1)
   static constexpr int SK = CK / XS;                              // values of K per piece
   static constexpr int XROWB = SK * 2;
   static constexpr int XLOADS = MR * 4 * XROWB / 1024;            // direct-to-LDS loads per piece
@@ -88,7 +109,7 @@ struct BatchShape {
 };
 
 // Whether two workgroups may share a CU: at most 128 registers per lane (the build refuses a spill).
-constexpr bool batch_two_per_cu(int t, int mr, int group) { return !(t == 2 && group == 32 && mr == 8); }
+constexpr bool batch_two_per_cu(int t, int mr, int group, bool deep) { return !deep && !(t == 2 && group == 32 && mr == 8); }
 
 inline int batch_scale_bytes(int tiles, int K, int group) { return (tiles * 16 * (K / group) * 2 + 1023) / 1024 * 1024; }
 
@@ -105,23 +126,24 @@ __device__ __forceinline__ floatx4 batch_mfma(u32x4 a, u32x4 b, floatx4 c)
   }
 }
 
-// Eight nibbles of a word -> eight elements q, order [k0,k2,k4,k6,k1,k3,k5,k7].  A byte 0..15 read as fp8 (E4M3) is
-// q * 2^-9 (exponent fields 0 and 1 are one linear range), so the scaled conversion by 2^9 gives q, two a time.
+// Eight nibbles of a word -> eight elements q, in order.  A byte 0..15 read as fp8 (E4M3) is q * 2^-9 (exponent fields 0
+// and 1 are one linear range), so the scaled conversion by 2^9 gives q, two a time.
 template <bool F16>
 __device__ __forceinline__ u32x4 batch_nibbles(uint32_t word, uint32_t mask)
 {
   const uint32_t even = word & mask, odd = (word >> 4) & mask;
+  const uint32_t lo = __builtin_amdgcn_perm(odd, even, 0x05010400u), hi = __builtin_amdgcn_perm(odd, even, 0x07030602u);
   u32x4 v;
   if constexpr (F16) {
-    v[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(even, 512.0f, false));
-    v[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(even, 512.0f, true));
-    v[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(odd, 512.0f, false));
-    v[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(odd, 512.0f, true));
+    v[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.0f, false));
+    v[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.0f, true));
+    v[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.0f, false));
+    v[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.0f, true));
   } else {
-    v[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, false));
-    v[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, true));
-    v[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, false));
-    v[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, true));
+    v[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, false));
+    v[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, true));
+    v[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, false));
+    v[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, true));
   }
   return v;
 }
@@ -138,17 +160,6 @@ __device__ __forceinline__ u32x4 batch_bytes(uint32_t w0, uint32_t w1)
   v[1] = pair((w0 >> 16) & 0xffu, w0 >> 24);
   v[2] = pair(w1 & 0xffu, (w1 >> 8) & 0xffu);
   v[3] = pair((w1 >> 16) & 0xffu, w1 >> 24);
-  return v;
-}
-
-// Eight consecutive elements of x -> the order batch_nibbles produces.
-__device__ __forceinline__ u32x4 batch_permute_x(u32x4 d)
-{
-  u32x4 v;
-  v[0] = __builtin_amdgcn_perm(d[1], d[0], 0x05040100u);
-  v[1] = __builtin_amdgcn_perm(d[3], d[2], 0x05040100u);
-  v[2] = __builtin_amdgcn_perm(d[1], d[0], 0x07060302u);
-  v[3] = __builtin_amdgcn_perm(d[3], d[2], 0x07060302u);
   return v;
 }
 
@@ -180,10 +191,14 @@ __device__ float batch_plain_sum(const uint8_t* codes, const uint16_t* scales, c
   return wave_sum(acc);
 }
 
-__device__ __forceinline__ void batch_to_lds(const void* src, void* lds_dst)
+// 16 bytes per lane, global (base + off) -> LDS at lds_dst + 16 * lane.  Written out by hand: the compiler waits for every
+// such load that it knows about before any later LDS read, whatever the load fills.  The LDS base travels in M0, bound as an
+// operand (the s_nop is the wait state between that write and the load).
+__device__ __forceinline__ void batch_to_lds(const uint8_t* base, uint32_t off, void* lds_dst)
 {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                   (__attribute__((address_space(3))) void*)lds_dst, 16, 0, 0);
+  const uint32_t dst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)(uint8_t*)lds_dst;
+  const uint32_t m0v = __builtin_amdgcn_readfirstlane(dst);
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "{m0}"(m0v) : "memory");
 }
 
 }  // namespace
@@ -191,10 +206,10 @@ __device__ __forceinline__ void batch_to_lds(const void* src, void* lds_dst)
 // MR: accumulator registers per lane and tile, 1 / 2 / 4 / 8 for up to 4 / 8 / 16 / 32 rows of x.  Row m of an MFMA
 // tile of x sits in MFMA row 4*(m%4) + m/4, so that output row m is register m/4 of lane group m%4 and up to four rows
 // need one register.
-template <int T, int MR, int BITS, int GROUP, bool F16, bool SONLY>
-__global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 4 : 2) void qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
+template <int T, int MR, int BITS, int GROUP, bool F16, bool SONLY, bool DEEP>
+__global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP, DEEP) ? 4 : 2) void qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
 {
-  using S = BatchShape<T, MR, BITS, GROUP>;
+  using S = BatchShape<T, MR, BITS, GROUP, DEEP>;
   const BatchParams p = preload_assemble<BatchParams>(VPQ_PRELOADED_WORD_LIST, tail);
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
@@ -236,9 +251,9 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
   const uint32_t row_bytes = (uint32_t)p.K * BITS / 8;
   const int chunks = (p.K + S::CK - 1) / S::CK;
 
-  uint8_t* slot = lds + wave * S::SLOT;
-  uint8_t* xbuf = slot + S::CLOADS * 1024;
-  uint8_t* sblk = lds + kBatchWaves * S::SLOT;
+  uint8_t* const slots = lds + wave * (S::RING * S::SLOT);
+  uint8_t* slot = slots;                                    // of the chunk in hand
+  uint8_t* sblk = lds + kBatchWaves * S::RING * S::SLOT;
   const int sb_bytes = n_live * Kg * 2;
   const int sb_loads = (sb_bytes + 1023) >> 10;
   uint8_t* bblk = sblk + sb_loads * 1024;
@@ -252,7 +267,7 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
   // repeat it.
   uint32_t code_piece = (uint32_t)(((lane & 7) ^ (lane >> 4)) * 16);
   uint32_t code_row = __umul24((uint32_t)(lane >> 3), row_bytes);
-  auto request_codes = [&](int c) {
+  auto request_codes = [&](int c, uint8_t* to) {
     const uint8_t* base = wtile + (size_t)c * 128;
     const int left = (int)row_bytes - c * 128;              // bytes of a row from here on
     uint32_t rb = row_bytes;
@@ -260,7 +275,7 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
     if (left >= 128 && n_live == T * 16) {
 #pragma unroll
       for (int i = 0; i < S::CLOADS; ++i) {
-        batch_to_lds(base + ((code_piece ^ ((i & 1) * 64)) + code_row), slot + i * 1024);
+        batch_to_lds(base, (code_piece ^ ((i & 1) * 64)) + code_row, to + i * 1024);
         base += 8 * (size_t)rb;
       }
     } else {
@@ -268,8 +283,8 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
       for (int i = 0; i < S::CLOADS; ++i) {
         const int row = i * 8 + (lane >> 3);
         const uint32_t at = code_piece ^ ((i & 1) * 64);
-        batch_to_lds(base + (__umul24((uint32_t)(row < n_live ? row : n_live - 1), rb) + ((int)at < left ? at : 0)),
-                     slot + i * 1024);
+        batch_to_lds(base, __umul24((uint32_t)(row < n_live ? row : n_live - 1), rb) + ((int)at < left ? at : 0),
+                     to + i * 1024);
       }
     }
   };
@@ -280,7 +295,7 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
   const uint32_t x_bytes = (uint32_t)p.K * 2u;
   uint32_t x_piece = (uint32_t)(((lane & (kXPieces - 1)) ^ (kXPieces >= 16 ? lane / kXPieces : lane >> 4)) * 16);
   uint32_t x_row = __umul24((uint32_t)(lane / kXPieces), x_bytes);
-  auto request_x = [&](int c, int sub) {
+  auto request_x = [&](int c, int sub, uint8_t* to) {
     const int k0 = c * S::CK + sub * S::SK;
     const int left = (p.K - k0) * 2;
     const uint8_t* base = xtile + (size_t)k0 * 2;
@@ -290,12 +305,12 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
     for (int i = 0; i < S::XLOADS; ++i) {
       const uint32_t at = x_piece ^ (uint32_t)(kXPieces >= 16 ? ((i * kRowsPerLoad) & 15) * 16 : (i & 1) * 64);
       if (left >= S::XROWB && (i + 1) * kRowsPerLoad <= rows) {
-        batch_to_lds(base + (at + x_row), xbuf + i * 1024);
+        batch_to_lds(base, at + x_row, to + (S::CLOADS + i) * 1024);
       } else if (i * kRowsPerLoad < rows) {
         int row = lane / kXPieces;
         asm volatile("" : "+v"(row));                       // (the rare path: nothing of it is held over the loop)
         const int last = rows - 1 - i * kRowsPerLoad;
-        batch_to_lds(base + (__umul24((uint32_t)(row < last ? row : last), xb) + ((int)at < left ? at : 0)), xbuf + i * 1024);
+        batch_to_lds(base, __umul24((uint32_t)(row < last ? row : last), xb) + ((int)at < left ? at : 0), to + (S::CLOADS + i) * 1024);
       }
       base += kRowsPerLoad * (size_t)xb;
     }
@@ -307,7 +322,7 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
       for (int i = wave; i < sb_loads; i += kBatchWaves) {
         int piece = i * 64 + lane;
         if (piece > last) { piece = last; }
-        batch_to_lds(reinterpret_cast<const uint8_t*>(src) + (size_t)piece * 16, dst + i * 1024);
+        batch_to_lds(reinterpret_cast<const uint8_t*>(src), (uint32_t)piece * 16, dst + i * 1024);
       }
     }
   };
@@ -315,9 +330,18 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
   const uint16_t* bi_src = SONLY ? nullptr : biases_ + (size_t)n0 * Kg;
   request_block(sc_src, sblk);
   if (!SONLY) { request_block(bi_src, bblk); }
-  if (wave < chunks) {
-    request_x(wave, 0);
-    request_codes(wave);
+  const int mine = wave < chunks ? (chunks - wave + kBatchWaves - 1) / kBatchWaves : 0;   // chunks of this wavefront
+#pragma unroll
+  for (int i = 0; i < S::RING; ++i) {
+    if (i < mine) {
+      request_x(wave + i * kBatchWaves, 0, slots + i * S::SLOT);
+      request_codes(wave + i * kBatchWaves, slots + i * S::SLOT);
+    }
+  }
+  // the scales: older than every chunk's loads (of x at least one each)
+  if (S::RING > 1 && mine >= S::RING) {
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(S::RING * (S::CLOADS + 1) - 1) : "memory");
+  } else if (mine > 0) {
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(S::CLOADS) : "memory");
   } else {
     asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
@@ -412,7 +436,7 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
     for (int a = 0; a < S::AT; ++a) {
       const int m_real = a * 16 + 4 * (fr & 3) + (fr >> 2);
       const int row = m_real < MR * 4 ? m_real : MR * 4 - 1;   // (MFMA rows past the slot's repeat its last)
-      const uint8_t* rp = xbuf + row * S::XROWB;
+      const uint8_t* rp = slot + S::CLOADS * 1024 + row * S::XROWB;
       const int key = kXPieces >= 16 ? row & 15 : (row >> 1) & 7;
 #pragma unroll
       for (int j = 0; j < kPieceMfmas; ++j) {
@@ -426,13 +450,6 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
   // Contracts piece `sub` of the taken chunk; PART: only its first `live` groups are inside K.
   auto contract_as = [&](auto sub_c, auto part_c, int live) {
     constexpr int kGroups = S::SK / GROUP, kG0 = decltype(sub_c)::value * kGroups;
-    if constexpr (BITS == 4) {
-#pragma unroll
-      for (int a = 0; a < S::AT; ++a) {
-#pragma unroll
-        for (int j = 0; j < kPieceMfmas; ++j) { xq[a][j] = batch_permute_x(xq[a][j]); }
-      }
-    }
 #pragma unroll
     for (int grp = 0; grp < kGroups; ++grp) {
       if (decltype(part_c)::value && grp >= live) { break; }
@@ -502,6 +519,45 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
   // The next chunk's codes are requested behind the piece of x after which they have the longest time that does not
   // make a later piece wait for them (loads return in order).
   constexpr int kCodesAt = S::XS >= 2 ? S::XS - 2 : 0;
+  if constexpr (S::RING > 1) {
+    // Loads return in order: a chunk is there when no more are out than the chunks behind it have.
+    const int x_loads = (rows + kRowsPerLoad - 1) / kRowsPerLoad;
+    auto arrive = [&](int behind) {
+      auto wait = [&](auto x_c) {
+        constexpr int kLoads = S::CLOADS + decltype(x_c)::value;
+        if (S::RING > 2 && behind >= 2) {
+          asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * kLoads) : "memory");
+        } else if (behind >= 1) {
+          asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kLoads) : "memory");
+        } else {
+          asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+        }
+      };
+      if (S::XLOADS > 3 && x_loads > 3) {
+        wait(std::integral_constant<int, 4>());
+      } else if (S::XLOADS > 2 && x_loads == 3) {
+        wait(std::integral_constant<int, 3>());
+      } else if (S::XLOADS > 1 && x_loads == 2) {
+        wait(std::integral_constant<int, 2>());
+      } else {
+        wait(std::integral_constant<int, 1>());
+      }
+    };
+    static_assert(S::XLOADS <= 4, "");
+    for (int i = 0; i < mine; ++i) {
+      const int c = wave + i * kBatchWaves, behind = mine - 1 - i;
+      arrive(behind < S::RING - 1 ? behind : S::RING - 1);
+      take_codes(c);
+      take_x();
+      asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+      if (i + S::RING < mine) {
+        request_x(c + S::RING * kBatchWaves, 0, slot);
+        request_codes(c + S::RING * kBatchWaves, slot);
+      }
+      contract(std::integral_constant<int, 0>(), (p.K - c * S::CK) / GROUP);
+      slot = slot == slots + (S::RING - 1) * S::SLOT ? slots : slot + S::SLOT;
+    }
+  } else
   for (int c = wave; c < chunks; c += kBatchWaves) {
     const int nxt = c + kBatchWaves;
     const bool more = nxt < chunks;                          // (a chunk that ends past K is its wavefront's last)
@@ -518,11 +574,11 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP) ? 
       take_x();
       asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
       if (s + 1 < S::XS) {
-        if (left > S::SK) { request_x(c, s + 1); }
+        if (left > S::SK) { request_x(c, s + 1, slot); }
       } else if (more) {
-        request_x(nxt, 0);
+        request_x(nxt, 0, slot);
       }
-      if (s == kCodesAt && more) { request_codes(nxt); }
+      if (s == kCodesAt && more) { request_codes(nxt, slot); }
       contract(s_c, left / GROUP);
     };
     piece(std::integral_constant<int, 0>());
@@ -603,11 +659,11 @@ constexpr int kLdsOfCu = 160 * 1024;
 
 // One instantiation's launch; the attribute is set once per kernel, whichever thread comes first (two may both set it,
 // which is harmless; neither launches before its own call has returned).
-template <int T, int MR, int BITS, int GROUP, bool F16, bool SONLY>
+template <int T, int MR, int BITS, int GROUP, bool F16, bool SONLY, bool DEEP>
 hipError_t batch_launch_one(hipStream_t st, const BatchParams& p, size_t lds_bytes, int grid)
 {
   static std::atomic<bool> ready{false};
-  auto kern = qmv_batch_kernel<T, MR, BITS, GROUP, F16, SONLY>;
+  auto kern = qmv_batch_kernel<T, MR, BITS, GROUP, F16, SONLY, DEEP>;
   if (!ready.load(std::memory_order_acquire)) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, kLdsOfCu);
@@ -618,18 +674,19 @@ hipError_t batch_launch_one(hipStream_t st, const BatchParams& p, size_t lds_byt
 }
 
 template <int BITS, int GROUP, bool F16, bool SONLY = false>
-hipError_t batch_launch(hipStream_t st, const BatchParams& p, int tiles, int mr, size_t lds_bytes, int grid)
+hipError_t batch_launch(hipStream_t st, const BatchParams& p, int tiles, int mr, bool deep, size_t lds_bytes, int grid)
 {
-#define VPQ_BATCH(T_, MR_) \
-  if (tiles == T_ && mr == MR_) { return batch_launch_one<T_, MR_, BITS, GROUP, F16, SONLY>(st, p, lds_bytes, grid); }
-  VPQ_BATCH(1, 1) VPQ_BATCH(1, 2) VPQ_BATCH(1, 4) VPQ_BATCH(1, 8)
-  VPQ_BATCH(2, 1) VPQ_BATCH(2, 2) VPQ_BATCH(2, 4) VPQ_BATCH(2, 8)
+#define VPQ_BATCH(T_, MR_, DEEP_) \
+  if (tiles == T_ && mr == MR_ && deep == DEEP_) { return batch_launch_one<T_, MR_, BITS, GROUP, F16, SONLY, DEEP_>(st, p, lds_bytes, grid); }
+  VPQ_BATCH(1, 1, false) VPQ_BATCH(1, 2, false) VPQ_BATCH(1, 4, false) VPQ_BATCH(1, 8, false)
+  VPQ_BATCH(2, 1, false) VPQ_BATCH(2, 2, false) VPQ_BATCH(2, 4, false) VPQ_BATCH(2, 8, false)
+  if constexpr (BITS == 8) { VPQ_BATCH(1, 1, true) VPQ_BATCH(1, 2, true) VPQ_BATCH(1, 4, true) VPQ_BATCH(1, 8, true) }
 #undef VPQ_BATCH
   return hipErrorInvalidValue;
 }
 
 // The instantiations of the other formats (vpq_qmv_batch_twins.hip).
-hipError_t launch_qmv_batch_twin(hipStream_t st, const BatchParams& p, int tiles, int mr, size_t lds_bytes, int grid,
+hipError_t launch_qmv_batch_twin(hipStream_t st, const BatchParams& p, int tiles, int mr, bool deep, size_t lds_bytes, int grid,
                                  const BatchFormat& f);
 
 }  // namespace vpq

@@ -8,18 +8,17 @@ namespace vpq {
 
 namespace {
 
-size_t batch_lds_bytes(int tiles, int mr, int K, const BatchFormat& f)
+size_t batch_lds_bytes(int tiles, int mr, int K, const BatchFormat& f, bool deep)
 {
-  const int x_bytes = mr * 4 * (128 * 8 / f.bits) * 2, x_piece = x_bytes > 4096 ? 4096 : x_bytes;
   // (64 more: the unaligned reads of the last row's scales may run past its block)
-  return (size_t)kBatchWaves * (tiles * 2048 + x_piece) + 2 * (size_t)batch_scale_bytes(tiles, K, f.group) + 64;
+  return (size_t)kBatchWaves * batch_ring(tiles, mr, f.bits, deep) * batch_slot_bytes(tiles, mr, f.bits, deep) + 2 * (size_t)batch_scale_bytes(tiles, K, f.group) + 64;
 }
 
 }  // namespace
 
 bool qmv_batch_supports(int K, int M, const BatchFormat& f)
 {
-  return M >= 1 && K >= f.group && K % f.group == 0 && batch_lds_bytes(1, 8, K, f) <= (size_t)kLdsOfCu;
+  return M >= 1 && K >= f.group && K % f.group == 0 && batch_lds_bytes(1, 8, K, f, false) <= (size_t)kLdsOfCu;
 }
 
 hipError_t launch_qmv_batch(hipStream_t st, const QmvArgs& a, const QmvGroup& g, const BatchFormat& f)
@@ -42,8 +41,11 @@ hipError_t launch_qmv_batch(hipStream_t st, const QmvArgs& a, const QmvGroup& g,
   // one workgroup per CU is left.)
   long tiles1 = 0;
   for (int i = 0; i < g.count; ++i) { tiles1 += (g.seg[i].N + 15) / 16; }
-  const int tiles = tiles1 * p.m_tiles <= cus || batch_lds_bytes(2, mr, a.K, f) > (size_t)kLdsOfCu ? 1 : 2;
-  const size_t lds_bytes = batch_lds_bytes(tiles, mr, a.K, f);
+  const int tiles = tiles1 * p.m_tiles <= cus || batch_lds_bytes(2, mr, a.K, f, false) > (size_t)kLdsOfCu ? 1 : 2;
+  // 8 bits, one workgroup per CU, a long K: more chunks in flight.  (us, 12288 -> 4096 at 6 / 16 / 32 rows 17.9 / 19.5 / 24.4 ->
+  // 15.6 / 19.1 / 22.8; 4096 -> 4096, four chunks a wavefront, level; 4 bits, six chunks at 12288: 11.2 -> 11.8 at 4 rows.)
+  const bool deep = f.bits == 8 && a.K >= 6144 && tiles == 1 && tiles1 * p.m_tiles <= cus && batch_lds_bytes(1, mr, a.K, f, true) <= (size_t)kLdsOfCu;
+  const size_t lds_bytes = batch_lds_bytes(tiles, mr, a.K, f, deep);
   int first = 0;
   for (int i = 0; i < g.count; ++i) {
     if (i > 0) {
@@ -54,8 +56,8 @@ hipError_t launch_qmv_batch(hipStream_t st, const QmvArgs& a, const QmvGroup& g,
   }
   p.blocks = first;
   const int grid = p.m_tiles > 1 ? (first + 7) / 8 * 8 * p.m_tiles : first;
-  if (f.bits == 4 && f.group == 64 && !f.f16) { return batch_launch<4, 64, false>(st, p, tiles, mr, lds_bytes, grid); }
-  return launch_qmv_batch_twin(st, p, tiles, mr, lds_bytes, grid, f);
+  if (f.bits == 4 && f.group == 64 && !f.f16) { return batch_launch<4, 64, false>(st, p, tiles, mr, deep, lds_bytes, grid); }
+  return launch_qmv_batch_twin(st, p, tiles, mr, deep, lds_bytes, grid, f);
 }
 
 }  // namespace vpq
