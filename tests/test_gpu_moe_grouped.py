@@ -387,3 +387,16 @@ def test_last_block_of_one_fragment_is_multiplied_with_the_block_before(vpq, dev
             g, d = vpq.qmm_swiglu_w4g64(w[e], s[e], b[e], xe, K, N, slots.numel()), vpq.qmm_w4g64(w[e], s[e], b[e], xe, K, N, slots.numel())
         assert np.array_equal(D.bits(act.view)[slots.cpu().numpy()], D.bits(g)), "gate|up, expert %d" % e
         assert np.array_equal(D.bits(part.view)[sdst[slots].cpu().numpy()], D.bits(d)), "down, expert %d" % e
+
+
+# the one-workgroup form at its edges (one pair; an odd count of slots; pairs that end inside a round of its threads; the most
+# pairs; top_k that is no power of two), and the four launches past them (more pairs; more experts; slots that outgrow the LDS)
+@pytest.mark.parametrize("E,T,top_k,B", [(1, 1, 1, 1), (7, 341, 3, 3), (40, 1025, 1, 32), (64, 5461, 3, 16), (96, 2340, 7, 128),
+                                         (16, 4200, 4, 128), (1025, 300, 2, 8), (1024, 2048, 8, 128)])
+def test_pair_sort_at_the_edges_of_its_forms(vpq, oracle, dev, E, T, top_k, B):
+    eid = routed(E, T, top_k, 6000 + E + T)
+    eid[::17] = E                                        # some pairs without an expert
+    outs = vpq.moe_sort_pairs(torch.from_numpy(eid).to(dev), top_k, E, block_rows=B)
+    torch.cuda.synchronize()
+    t2e, srow, sdst, ntiles = (o.cpu().numpy() for o in outs)
+    check_sort(eid, top_k, E, B, t2e, srow, sdst, ntiles, oracle)
