@@ -400,3 +400,46 @@ def test_pair_sort_at_the_edges_of_its_forms(vpq, oracle, dev, E, T, top_k, B):
     torch.cuda.synchronize()
     t2e, srow, sdst, ntiles = (o.cpu().numpy() for o in outs)
     check_sort(eid, top_k, E, B, t2e, srow, sdst, ntiles, oracle)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("E,K,N", [(128, 128, 516), (100, 320, 700), (600, 64, 100)])
+def test_few_pairs_over_many_experts(vpq, dev, D, E, K, N, bits):
+    # more weight tiles than a round, few pairs each: most blocks of one fragment, the edges of two, and some of three, four
+    # and a block behind; the map with spare blocks at its end
+    counts = [0, 1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 300] + [1 + i * 7 % 11 for i in range(E - 12)]
+    B = vpq.grouped_block_rows()
+    gen = torch.Generator(device="cpu").manual_seed(6100 + K + bits)
+    w = torch.randint(-2 ** 31, 2 ** 31, (E, N, K * bits // 32), dtype=torch.int32, generator=gen).to(dev)
+    s = (torch.rand((E, N, K // 64), generator=gen) * 0.015 / (16 if bits == 8 else 1) + 0.001).bfloat16().to(dev)
+    b = (-(2 ** (bits - 1)) * s.float()).bfloat16()
+    eid = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(sum(counts), generator=gen)]
+    assert -(-eid.numel() // B) * B <= 32 * E
+    x = torch.randn((eid.numel(), K), generator=gen).bfloat16().to(dev)
+    t2e, srow, sdst, ntiles = vpq.moe_sort_pairs(eid.to(torch.int32).to(dev), 1, E)
+    used = int(ntiles.cpu()[0])
+    gated = vpq.qmm_grouped_gated_w8g64 if bits == 8 else vpq.qmm_grouped_gated_w4g64
+    down = vpq.qmm_grouped_down_w8g64 if bits == 8 else vpq.qmm_grouped_down_w4g64
+    act = parity.Guarded((srow.numel(), N // 2), torch.bfloat16, dev)
+    part = parity.Guarded((eid.numel(), N), torch.bfloat16, dev)
+    act.view.fill_(7.0)
+    part.view.fill_(7.0)
+    xs = x[srow.clamp(min=0).long()].contiguous()
+    xs[srow < 0] = float("nan")
+    gated(w, s, b, x, K, N, t2e, srow, E, out=act.view)
+    down(w, s, b, xs, K, N, t2e, sdst, E, out=part.view)
+    torch.cuda.synchronize()
+    act.assert_intact()
+    part.assert_intact()
+    owner, live = t2e.repeat_interleave(B).cpu(), (srow >= 0).cpu()
+    assert not D.bits(act.view)[((owner >= 0) & ~live).numpy()].any()
+    assert (act.view[used * B:] == 7.0).all()
+    for e in list(range(1, 12)) + [E // 2, E - 1]:
+        slots = torch.nonzero((owner == e) & live).flatten().to(dev)
+        xe = x[srow[slots].long()].contiguous()
+        if bits == 8:
+            g, d = (vpq.qmm_w8g64(w[e], s[e], b[e], xe, K, N, counts[e], activation=a) for a in (1, 0))
+        else:
+            g, d = vpq.qmm_swiglu_w4g64(w[e], s[e], b[e], xe, K, N, counts[e]), vpq.qmm_w4g64(w[e], s[e], b[e], xe, K, N, counts[e], tile_n=128)
+        assert np.array_equal(D.bits(act.view)[slots.cpu().numpy()], D.bits(g)), "gate|up, expert %d" % e
+        assert np.array_equal(D.bits(part.view)[sdst[slots].cpu().numpy()], D.bits(d)), "down, expert %d" % e

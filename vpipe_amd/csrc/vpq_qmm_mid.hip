@@ -509,11 +509,14 @@ __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidPar
 // read nor unpacked a second time (two fragments would leave one workgroup per CU).  All weight tiles of a block go to one
 // XCD (eight workgroups apart), whose L2 then holds its rows of x.
 // Two neighbouring blocks to an XCD, which mostly share an expert's weight tiles: 1 to 2 % slower (2048 tokens 298 -> 305 us).
+// WIDE or not is chosen on the host (launch_qmm_grouped).  Not WIDE is for a few tokens, where almost every block has one or
+// two fragments: no loop over more of them, hence registers and LDS for three workgroups per CU instead of two, and the blocks
+// that have more are multiplied half after half.  (A fourth workgroup needs spills and gains 2 % at most.)
 // Bound by the plain tile's step at full blocks, by unpacking and the codes' read at one fragment.  Measured (us, sort +
-// gate|up + down of one layer, 2048 -> 768; every block by itself, the plain tile's first form; now): 8 of 128 experts, 2048 /
-// 512 / 64 tokens 299 / 161 / 145 -> 250 / 149 / 135; 8 bits, 2048 tokens 345 -> 290.
-template <int BITS>
-__global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_grouped_kernel(const MidParams p)
+// gate|up + down of one layer, 2048 -> 768; every block by itself, the plain tile's first form, four launches of the sort;
+// now): 8 of 128 experts, 2048 / 512 / 64 tokens 309 / 163 / 147 -> 262 / 135 / 117; 8 bits, 2048 tokens 357 -> 319.
+template <int BITS, bool WIDE>
+__global__ __launch_bounds__(kMidWaves * 64, WIDE ? 2 : 3) void qmm_mid_grouped_kernel(const MidParams p)
 {
   extern __shared__ __attribute__((aligned(16))) uint8_t x_lds[];
   static_assert(kGroupedBlockRows == 128, "two slots per lane, four fragments");
@@ -536,12 +539,27 @@ __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_grouped_kernel(cons
     return hi != 0 ? ((hi >> 32) != 0 ? 4 : 3) : (lo >> 32) != 0 ? 2 : 1;
   };
   const int live = fragments(slots[0], slots[1]);
-  if (e_before == e && e_next != e && live == 1) { return; }   // the block before multiplies it
+  if (WIDE && e_before == e && e_next != e && live == 1) { return; }   // the block before multiplies it
   const bool both = e_next == e && e_after != e && fragments(slots[2], slots[3]) == 1;
 
   const uint32_t* w = p.w + (size_t)e * (size_t)p.N * (size_t)(p.K >> (BITS == 4 ? 3 : 2));
   const uint16_t* s = p.scales + (size_t)e * (size_t)p.N * (size_t)(p.K >> 6);
   const uint16_t* b = p.biases + (size_t)e * (size_t)p.N * (size_t)(p.K >> 6);
+  if constexpr (!WIDE) {
+    int half[4] = {slots[0], -1, -1, -1};
+    if (live == 1) {
+      mid_tile<1, BITS, 64, false, true>(p, x_lds, m0, n0, 0, w, s, b, half, kGroupedBlockRows);
+      return;
+    }
+    for (int h = 0; h < 2; ++h) {
+      mid_tile<2, BITS, 64, false, true>(p, x_lds, m0 + h * 64, n0, 0, w, s, b, half, live == 2 ? kGroupedBlockRows : 64);
+      if (live == 2) { return; }
+      half[0] = slots[1];
+      __builtin_amdgcn_s_barrier();                 // (nobody reads the first half's x any more)
+      asm volatile("" : : : "memory");
+    }
+    return;
+  }
   if (both) {
     mid_tile<5, BITS, 64, false, true>(p, x_lds, m0, n0, 0, w, s, b, slots, 2 * kGroupedBlockRows);
   } else if (live == 1) {
@@ -576,17 +594,18 @@ __global__ __launch_bounds__(256) void splitk_fold_kernel(const float* __restric
 namespace {
 
 // More LDS than the default limit needs the attribute, set once per kernel (two threads may both set it, which is harmless).
-template <int BITS>
-hipError_t mid_launch_grouped(dim3 grid, dim3 block, size_t lds, hipStream_t st, const MidParams& p)
+template <int BITS, bool WIDE>
+hipError_t mid_launch_grouped(dim3 grid, dim3 block, hipStream_t st, const MidParams& p)
 {
+  constexpr size_t lds = mid_lds_bytes(WIDE ? kGroupedBlockRows / 32 + 1 : 2);
   static std::atomic<bool> ready{false};
   if (!ready.load(std::memory_order_acquire)) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(qmm_mid_grouped_kernel<BITS>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(qmm_mid_grouped_kernel<BITS, WIDE>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) { return e; }
     ready.store(true, std::memory_order_release);
   }
-  return launch_kernel(qmm_mid_grouped_kernel<BITS>, grid, block, lds, st, p);
+  return launch_kernel(qmm_mid_grouped_kernel<BITS, WIDE>, grid, block, lds, st, p);
 }
 
 template <int BITS, int GROUP, bool F16>
@@ -755,8 +774,15 @@ hipError_t launch_qmm_grouped(hipStream_t st, const GemmArgs& a, const GroupedAr
   p.tile2e = g.tile2e; p.srow = g.srow; p.sdst = g.sdst;
   p.n_experts = g.n_experts; p.rows_x = g.rows_x; p.rows_y = g.rows_y;
   const dim3 grid((unsigned)((p.tiles_m + 7) / 8 * 8 * p.tiles_n)), block(kMidWaves * 64);
-  const size_t lds = mid_lds_bytes(kGroupedBlockRows / 32 + 1);
-  return a.bits == 8 ? mid_launch_grouped<8>(grid, block, lds, st, p) : mid_launch_grouped<4>(grid, block, lds, st, p);
+  // Three narrow workgroups per CU instead of two wide ones where the experts' first blocks alone are more than the wide ones'
+  // first round, and up to 32 pairs per expert on average, as far as the count of blocks tells (one an expert and the whole
+  // ones).  Wide against narrow, us of gate|up and down, 2048 -> 768, 8 of 128 experts: 64 tokens (4 pairs an expert) 88 + 38
+  // against 82 + 33, 512 (32) 93 + 44 against 86 + 38, 768 (48) 100 + 51 against 106 + 50, 1024 112 + 55 against 138 + 66;
+  // within one round, 2048 -> 512, 64 experts, 512 tokens, gate|up 29.3 against 30.3.
+  const int cus = a.cu_count > 0 ? a.cu_count : 256;
+  const bool wide = (long)g.n_experts * p.tiles_n <= 2 * cus || ((long)p.tiles_m - g.n_experts) * kGroupedBlockRows > 32L * g.n_experts;
+  if (wide) { return a.bits == 8 ? mid_launch_grouped<8, true>(grid, block, st, p) : mid_launch_grouped<4, true>(grid, block, st, p); }
+  return a.bits == 8 ? mid_launch_grouped<8, false>(grid, block, st, p) : mid_launch_grouped<4, false>(grid, block, st, p);
 }
 
 // Shares of K that pay for their planes; 1 where the tiles alone fill the chip.
