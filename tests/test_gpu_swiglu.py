@@ -339,3 +339,26 @@ def test_qmv_gelu_mul(vpq, oracle, dev, D, K, N):
     p = out.view.data_ptr()
     assert L.vpq_qmv_gelu_mul_w4g64_bf16(None, p, p, p, p, p, K, N, None) == -1
     assert L.vpq_qmv_gelu_mul_w4g64_bf16(None, p, p, p, p, p, K + 8, N, p) == -2
+
+
+@pytest.mark.parametrize("M", [1, 32, 100, 700, 4096])
+def test_silu_over_the_range_of_its_exponential(vpq, dev, M):
+    # y = silu(x[:, 0]) * x[:, 64] through weights of one code each, around the magnitudes where exp overflows, 1 + exp leaves
+    # the reciprocal's range and the quotient is the division's: one bf16 rounding of the product, and what fp32 keeps where it
+    # underflows.  The sums are exact but for one row: its kernel adds 128 * 1.5 and takes it away again, half an ulp of 192 or
+    # 1.6e-5 of 0.5 and more.
+    K, N = 512, 512
+    g = torch.tensor([0.0, 0.5, 1.0, 4.0, 20.0, 63.75, 64.0, 64.5, 87.0, 88.0, 88.5, 89.0, 100.0, 128.0, 200.0])
+    g = torch.cat([g, -g]).bfloat16()
+    for first in (range(g.numel()) if M == 1 else (0,)):
+        x = torch.zeros((M, K), dtype=torch.bfloat16)
+        x[:, 0] = g[(first + torch.arange(M)) % g.numel()]
+        x[:, 64] = 1.5
+        w = torch.zeros((N, K // 8), dtype=torch.int32)
+        w[0::2, 0] = 1
+        w[1::2, 8] = 1
+        s, b = torch.ones((N, K // 64), dtype=torch.bfloat16), torch.zeros((N, K // 64), dtype=torch.bfloat16)
+        y = vpq.linear_swiglu_w4g64(w.to(dev), s.to(dev), b.to(dev), x.to(dev), K, N, M).double().cpu()
+        v = x[:, 0].double()
+        want = (v / (1 + torch.exp(-v)) * 1.5)[:, None].expand(M, N // 2)
+        assert torch.allclose(y, want, rtol=2.0 ** -8, atol=1e-35)

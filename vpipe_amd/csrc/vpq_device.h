@@ -118,8 +118,14 @@ __device__ __forceinline__ float gated_f32(int act, float gate, float up)
     const float t = tanhf(0.7978845608028654f * (gate + 0.044715f * gate * gate * gate));
     return 0.5f * gate * (1.0f + t) * up;
   }
-  const float t = __expf(-fabsf(gate));             // (0, 1]: no overflow, and 1 + t has an exact-to-1-ulp reciprocal
-  return gate * ((gate < 0.0f ? t : 1.0f) * __builtin_amdgcn_rcpf(1.0f + t)) * up;
+  // The division as a reciprocal and one correction of the quotient: 1e-7 at most, like the division (the bare reciprocal
+  // 3e-7), and four instructions in its place (2048 x 4096 -> 24576 gated: 391 -> 387 us).  Past 64 the denominator leaves
+  // the reciprocal's range, or the quotient's correction is inf - inf.
+  const float d = 1.0f + __expf(-gate), r = __builtin_amdgcn_rcpf(d);
+  float q = gate * r;
+  q = fmaf(fmaf(-d, q, gate), r, q);
+  if (__builtin_expect(!(fabsf(gate) < 64.0f), 0)) { q = gate / d; }
+  return q * up;
 }
 
 // The value lane^1 holds (quad_perm [1,0,3,2]).
