@@ -443,3 +443,37 @@ def test_few_pairs_over_many_experts(vpq, dev, D, E, K, N, bits):
             g, d = vpq.qmm_swiglu_w4g64(w[e], s[e], b[e], xe, K, N, counts[e]), vpq.qmm_w4g64(w[e], s[e], b[e], xe, K, N, counts[e], tile_n=128)
         assert np.array_equal(D.bits(act.view)[slots.cpu().numpy()], D.bits(g)), "gate|up, expert %d" % e
         assert np.array_equal(D.bits(part.view)[sdst[slots].cpu().numpy()], D.bits(d)), "down, expert %d" % e
+
+
+@pytest.mark.parametrize("N", [256, 260, 262])
+@pytest.mark.parametrize("off", [0, 4])
+def test_rows_of_y_at_any_alignment_that_the_entrances_take(vpq, dev, D, N, off):
+    # y 16- or 8-byte aligned, its pitch a multiple of 16, 8 or 4 bytes: the stores' pieces and the row's last ones
+    K, E, B = 128, 3, vpq.grouped_block_rows()
+    counts = [5, 130, 64]
+    gen = torch.Generator(device="cpu").manual_seed(6300 + N + off)
+    w = torch.randint(-2 ** 31, 2 ** 31, (E, N, K // 8), dtype=torch.int32, generator=gen).to(dev)
+    s = (torch.rand((E, N, K // 64), generator=gen) * 0.015 + 0.001).bfloat16().to(dev)
+    b = (-8 * s.float()).bfloat16()
+    eid = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    x = torch.randn((eid.numel(), K), generator=gen).bfloat16().to(dev)
+    t2e, srow, sdst, _ = vpq.moe_sort_pairs(eid.to(torch.int32).to(dev), 1, E)
+    act = parity.Guarded((srow.numel() * (N // 2),), torch.bfloat16, dev, guard=4096 + off)
+    part = parity.Guarded((eid.numel() * N,), torch.bfloat16, dev, guard=4096 + off)
+    assert act.view.data_ptr() % 16 == part.view.data_ptr() % 16 == 2 * off
+    act.view.fill_(7.0)
+    ya, yp = act.view.view(-1, N // 2), part.view.view(-1, N)
+    vpq.qmm_grouped_gated_w4g64(w, s, b, x, K, N, t2e, srow, E, out=ya)
+    vpq.qmm_grouped_down_w4g64(w, s, b, x[srow.clamp(min=0).long()].contiguous(), K, N, t2e, sdst, E, out=yp)
+    torch.cuda.synchronize()
+    act.assert_intact()
+    part.assert_intact()
+    owner, live = t2e.repeat_interleave(B), srow >= 0
+    assert not D.bits(ya)[((owner >= 0) & ~live).cpu().numpy()].any()
+    for e in range(E):
+        slots = torch.nonzero((owner == e) & live).flatten()
+        xe = x[srow[slots].long()].contiguous()
+        g = vpq.qmm_swiglu_w4g64(w[e], s[e], b[e], xe, K, N, counts[e])
+        d = vpq.qmm_w4g64(w[e], s[e], b[e], xe, K, N, counts[e], tile_n=128)
+        assert np.array_equal(D.bits(ya)[slots.cpu().numpy()], D.bits(g))
+        assert np.array_equal(D.bits(yp)[sdst[slots].cpu().numpy()], D.bits(d))

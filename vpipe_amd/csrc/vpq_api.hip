@@ -1236,7 +1236,7 @@ int grouped_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scale
   // the kernel addresses rows of x by 32-bit byte offsets
   const long long xrows = srow != nullptr ? rows : npad;
   if (xrows * (long long)K * 2 >= 4000000000LL) { return VPQ_ERR_BAD_SHAPE; }
-  // y rows are stored in 4- and 8-byte pieces
+  // (y rows are stored in 16-byte pieces, at any address)
   if (!aligned(x, 16) || !aligned(y, 8) || !aligned(tile2e, 4) || (srow != nullptr && !aligned(srow, 4)) ||
       (sdst != nullptr && !aligned(sdst, 4))) {
     return VPQ_ERR_MISALIGNED;
