@@ -154,3 +154,43 @@ def test_gathers_have_the_bits_of_the_plain_kernels(vpq, dev, D, bits, K, N, pai
                 assert not torch.isfinite(got).any()
             else:                                        # one bf16 rounding, and fp32 sums over K
                 assert ((got - want).norm() / want.norm()).item() < 2.0 ** -8
+
+
+# enough sets of rows that a wavefront walks several, in every form of the gather kernel (by K and code width), with an N that
+# ends inside a set
+@pytest.mark.parametrize("K,N,pairs", [(768, 2050, 48), (1024, 2050, 96), (2048, 1026, 40), (2112, 1026, 40), (2560, 1026, 40),
+                                       (3072, 1026, 64), (4096, 1026, 40)])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_gathers_whose_wavefronts_walk_several_sets(vpq, dev, D, bits, K, N, pairs):
+    E, gen = 3, torch.Generator(device=dev).manual_seed(4900 + K + N + bits)
+    sets = -(-N // (8 if bits == 4 and K <= 1024 else 4))
+    walked = -(-sets * pairs // (32 * 256))              # sets of a wavefront (256 CUs)
+    assert walked > 1
+    w = torch.randint(-2 ** 31, 2 ** 31, (E, N, K * bits // 32), dtype=torch.int32, device=dev, generator=gen)
+    s = (torch.rand((E, N, K // 64), device=dev, generator=gen) * 0.015 / (16 if bits == 8 else 1) + 0.001).bfloat16()
+    b = (-(2 ** (bits - 1)) * s.float() * 1.03).bfloat16()
+    eid = torch.randint(0, E, (pairs,), dtype=torch.int32, device=dev, generator=gen)
+    x = torch.randn((pairs, K), device=dev, generator=gen).bfloat16()
+    act = parity.Guarded((pairs, N // 2), torch.bfloat16, dev)
+    out = parity.Guarded((pairs, N), torch.bfloat16, dev)
+    gated = vpq.gather_qmv_gated_w8g64 if bits == 8 else vpq.gather_qmv_gated_w4g64
+    down = vpq.gather_down_qmv_w8g64 if bits == 8 else vpq.gather_down_qmv_w4g64
+    gated(w, s, b, x, K, N, eid, 1, E, out=act.view)
+    down(w, s, b, x, K, N, eid, E, out=out.view)
+    torch.cuda.synchronize()
+    act.assert_intact()
+    out.assert_intact()
+    for p in sorted({0, 1, pairs // 2, pairs - 1}):
+        e, xr = int(eid[p]), x[p:p + 1]
+        pack = w[e], s[e], b[e]
+        if bits == 8:
+            g = vpq.qmv_gated_w8g64(*pack, xr, K, N, 1, activation=1)
+        else:
+            g = vpq.qmv_swiglu_w4g64(*pack, xr, K, N, 1, variant=capi.VPQ_QMV_ROWS)
+            assert torch.equal(out.view[p], vpq.qmv_w4g64(*pack, xr, K, N, 1, variant=capi.VPQ_QMV_ROWS)[0])
+        assert torch.equal(act.view[p], g[0])            # every row of the pair, whichever set of its wavefront
+        # the plain store of 8 bits has no entry point of its own: one pair alone, where a wavefront has one set
+        one = vpq.gather_down_qmv_w8g64 if bits == 8 else vpq.gather_down_qmv_w4g64
+        alone = torch.empty((1, N), dtype=torch.bfloat16, device=dev)
+        one(w, s, b, xr, K, N, eid[p:p + 1], E, out=alone)
+        assert torch.equal(out.view[p], alone[0])
