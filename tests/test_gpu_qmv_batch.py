@@ -209,3 +209,63 @@ def test_eight_bit_codes_over_a_long_k_have_the_same_bits_in_few_workgroups(vpq,
     for M in (17, 21):
         got = vpq.linear_twin("w8g64", *few, xd[:M], K, n, M)
         assert torch.equal(got, vpq.linear_twin("w8g64", wd, sd, bd, xd[:M], K, N, M)[:, :n])
+
+
+@pytest.mark.parametrize("K", [6144, 6176, 9664])
+def test_eight_bit_codes_in_groups_of_32_over_a_long_k(vpq, oracle, dev, D, K):
+    # as above, every count of rows of x of the forms that keep two or three chunks in flight
+    N, n = 8224, 33
+    w, s, b = synth.make_weight8(n, K, K + 5, group=32)
+    gen = torch.Generator(device=dev).manual_seed(K)
+    wd = torch.randint(-2 ** 31, 2 ** 31, (N, K // 4), dtype=torch.int32, device=dev, generator=gen)
+    sd = torch.empty((N, K // 32), device=dev).uniform_(0.0003, 0.0012, generator=gen).bfloat16()
+    bd = -128 * sd
+    wd[:n], sd[:n], bd[:n] = D.u32(w, dev), D.bf16(s, dev), D.bf16(b, dev)
+    x = synth.make_act(16, K, K + 6)
+    xd = D.bf16(x, dev)
+    y64, yb = oracle.matmul8(w, s, b, x, K, n, 16, rounded=False, group=32)
+    few = [t[:n].contiguous() for t in (wd, sd, bd)]
+    for M in (2, 3, 4, 5, 6, 7, 8, 9, 13, 16):
+        out = parity.Guarded((M, n), torch.bfloat16, dev)
+        vpq.qmv_w8g32(*few, xd[:M], K, n, M, out=out.view)
+        torch.cuda.synchronize()
+        out.assert_intact()
+        parity.check_bf16(D.bits(out.view), y64[:M], yb[:M])
+        assert torch.equal(out.view, vpq.qmv_w8g32(wd, sd, bd, xd[:M], K, N, M)[:, :n])
+
+
+@pytest.mark.parametrize("K", [6144, 9664])
+@pytest.mark.parametrize("M", [2, 6, 16, 33, 50, 64])
+def test_eight_bit_codes_over_a_long_k_gated_grouped_and_in_two_tiles_of_rows(vpq, dev, K, M):
+    # the same bits from few workgroups, whose wavefronts keep several chunks in flight, as from many
+    N, n = 8224, 34
+    gen = torch.Generator(device=dev).manual_seed(K + M)
+    w = torch.randint(-2 ** 31, 2 ** 31, (N, K // 4), dtype=torch.int32, device=dev, generator=gen)
+    s = torch.empty((N, K // 64), device=dev).uniform_(0.0003, 0.0012, generator=gen).bfloat16()
+    b = -128 * s
+    x = torch.randn((M, K), device=dev, generator=gen).bfloat16()
+    few = [t[:n].contiguous() for t in (w, s, b)]
+    if M > 16:
+        out = parity.Guarded((M, n), torch.bfloat16, dev)
+        vpq.linear_twin("w8g64", *few, x, K, n, M, out=out.view)
+        torch.cuda.synchronize()
+        out.assert_intact()
+        assert torch.equal(out.view, vpq.linear_twin("w8g64", w, s, b, x, K, N, M)[:, :n])
+        return
+    out = parity.Guarded((M, n // 2), torch.bfloat16, dev)
+    vpq.qmv_gated_w8g64(*few, x, K, n, M, out=out.view)
+    many = vpq.qmv_w8g64(w, s, b, x, K, N, M)
+    packs, outs, first = [], [], 0
+    for rows in (17, 130, 48):
+        packs.append(tuple(t[first:first + rows].clone() for t in (w, s, b)) + (rows,))
+        outs.append(parity.Guarded((M, rows), torch.bfloat16, dev))
+        first += rows
+    vpq.qmv_group_w8g64(packs, x, K, M, outs=[o.view for o in outs])
+    torch.cuda.synchronize()
+    out.assert_intact()
+    assert torch.equal(out.view, vpq.qmv_gated_w8g64(w, s, b, x, K, N, M)[:, :n // 2])
+    first = 0
+    for o, p in zip(outs, packs):
+        o.assert_intact()
+        assert torch.equal(o.view, many[:, first:first + p[3]])
+        first += p[3]
