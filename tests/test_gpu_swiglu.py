@@ -362,3 +362,27 @@ def test_silu_over_the_range_of_its_exponential(vpq, dev, M):
         v = x[:, 0].double()
         want = (v / (1 + torch.exp(-v)) * 1.5)[:, None].expand(M, N // 2)
         assert torch.allclose(y, want, rtol=2.0 ** -8, atol=1e-35)
+
+
+def test_silu_of_small_gates_to_fp32(vpq, dev):
+    # silu(g) for 8192 gates of 2^-9 .. 2^-4 in fp32, where the quotient's own error is the largest part: the exponential (one
+    # ulp, and exp / (1 + exp) is a half) 0.6e-7, the denominator's and the quotient's roundings 0.6e-7 each.  A reciprocal in the
+    # division's place adds its ulp and one more rounding, up to 1.8e-7.  The gates are the plain call's sums of the same kernel,
+    # up is 1.
+    K, N, M = 512, 16384, 2
+    gen = torch.Generator(device=dev).manual_seed(77)
+    w = torch.zeros((N, K // 8), dtype=torch.int32, device=dev)
+    w[0::2, 0] = torch.randint(8, 16, (N // 2,), dtype=torch.int32, device=dev, generator=gen)
+    w[1::2, 8] = 1
+    s, b = torch.ones((N, K // 64), dtype=torch.bfloat16, device=dev), torch.zeros((N, K // 64), dtype=torch.bfloat16, device=dev)
+    size = 2.0 ** (-9 - 3 + 4 * torch.rand((N // 2,), device=dev, generator=gen))
+    s[0::2, 0] = (size * (1 - 2 * torch.randint(0, 2, (N // 2,), device=dev, generator=gen))).bfloat16()
+    x = torch.zeros((M, K), dtype=torch.bfloat16, device=dev)
+    x[:, 0] = torch.tensor([1.0, 1.0390625])
+    x[:, 64] = 1.0
+    sums = vpq.qmv_w4g64(w, s, b, x, K, N, M, f32out=True)
+    got = vpq.qmv_swiglu_w4g64(w, s, b, x, K, N, M, f32out=True).double()
+    assert (sums[:, 1::2] == 1.0).all() and sums[:, 0::2].abs().min() > 2.0 ** -10
+    g = sums[:, 0::2].double()
+    want = g / (1 + torch.exp(-g))
+    assert ((got - want).abs() / want.abs()).max().item() < 1.9e-7
