@@ -25,6 +25,29 @@ def test_plan(K, N, M, fmt, gated, want):
     assert vpipe_amd.load().vpq_qmm_plan(K, N, M, *fmt, gated, 1) == want
 
 
+@pytest.mark.parametrize("K,N,M,fmt,gated,want", [
+    # 8 bits: as many 96-row tiles as fill the chip by halves, 183 / 76 / 246 us against 215 / 89 / 267 of 256 x 128 tiles
+    (12288, 3072, 1500, (8, 64, 0), 0, 96),
+    (5120, 3072, 1500, (8, 64, 0), 0, 96),
+    (17408, 3072, 1500, (8, 64, 0), 0, 96),
+    (6144, 4608, 798, (8, 64, 0), 0, 96),            # 86 / 110
+    # less than a round of large tiles over a short K: 21.2 against 27.4 of 256 x 128 large tiles
+    (512, 9664, 1024, (8, 64, 0), 0, -192),
+    (1024, 16832, 768, (4, 64, 0), 0, -256),         # 35 / 45
+    # two thirds of a round of 256-wide tiles against three and a half of 128-row ones: 156 / 191, 192-wide 86 / 105
+    (7168, 2560, 3933, (4, 32, 0), 0, -256),
+    (4096, 2240, 3667, (4, 64, 1), 0, -192),
+    (4096, 6208, 1350, (4, 64, 1), 0, -192),         # 86 / 103
+    # one round and a half of large gated tiles: 207 against 268
+    (2560, 28160, 1212, (8, 64, 0), 1, 128),
+    (512, 3584, 1637, (8, 64, 0), 1, 128),           # 18 / 24
+    # 2.8 rounds of 192-wide tiles, by whose order the busiest XCD has 3.5: 305 against 356
+    (4608, 19456, 1663, (4, 64, 0), 0, 128),
+])
+def test_plan_where_other_kernels_than_the_obvious_one_are_faster(K, N, M, fmt, gated, want):
+    assert vpipe_amd.load().vpq_qmm_plan(K, N, M, *fmt, gated, 1) == want
+
+
 def test_plan_refuses_what_the_entrances_refuse():
     L = vpipe_amd.load()
     for args in [(96, 64, 64, 4, 64, 0, 0, 1), (64, 0, 64, 4, 64, 0, 0, 1), (64, 63, 64, 4, 64, 0, 1, 1), (64, 64, 64, 8, 32, 0, 0, 1),

@@ -204,11 +204,11 @@ hipError_t launch_qmv_rows_group(hipStream_t st, const QmvArgs& a, const QmvGrou
 // Gathered (MoE) form, M = 1 per pair: a.w/scales/biases are batches [E, N, ...] of expert slabs,
 // pair p contracts slab pair_eid[p] with x row p / x_div into y row p (zeros for an id outside
 // [0, n_experts)); a.gate_act as in the plain form.
+hipError_t launch_qmv_rows_gather(hipStream_t st, const QmvArgs& a, const int* pair_eid, int pairs, int x_div,
+                                  int n_experts);
 // The gathers at K <= 4096 (vpq_qmv_gather.hip), with the bits of launch_qmv_rows_gather (8 bits: launch_qmv_rows8).
 bool qmv_gather_supports(int K);
 hipError_t launch_qmv_gather(hipStream_t st, const QmvArgs& a, int bits, const int* pair_eid, int pairs, int x_div, int n_experts);
-hipError_t launch_qmv_rows_gather(hipStream_t st, const QmvArgs& a, const int* pair_eid, int pairs, int x_div,
-                                  int n_experts);
 // Sorted pairs, two slots per tile (a.M = 2): expert tile2e[tile], x row srow[slot] (x_from_srow) or the slot.
 hipError_t launch_qmv_rows_sorted(hipStream_t st, const QmvArgs& a, const int* tile2e, const int* srow, int tiles,
                                   bool x_from_srow, int n_experts);
@@ -250,6 +250,8 @@ hipError_t launch_qmm_grouped(hipStream_t st, const GemmArgs& a, const GroupedAr
 // kernel.  tile_n 0 = qmm_big_tile_n().
 bool qmm_big_supports(const GemmArgs& a);
 int qmm_big_tile_n(int N, int M, int cu_count, int max_width = 256, bool with_192 = true);
+// The tiles that the busiest XCD gets by that kernel's order of tiles, times the eight XCDs.
+long qmm_big_tiles_load(int tiles_m, int tiles_n);
 hipError_t launch_qmm_big(hipStream_t st, const GemmArgs& a, int tile_n);
 // 128 weight rows x {64, 96, 128} rows of x per workgroup, for GEMMs that have few 256-row tiles; every format, gated
 // stores, no adapter; the bits of the other two kernels.

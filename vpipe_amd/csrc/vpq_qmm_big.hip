@@ -912,6 +912,26 @@ unsigned plan_tile_order(BigParams& p)
 
 }  // namespace
 
+long qmm_big_tiles_load(int tiles_m, int tiles_n)
+{
+  BigParams p;
+  p.tiles_m = tiles_m; p.tiles_n = tiles_n;
+  (void)plan_tile_order(p);
+  if (p.bmt == 0) { return (long)tiles_m * tiles_n; }
+  long load[8] = {};                                     // a set's blocks go to the XCDs in turn
+  int xcd = 0;
+  for (int m = 0; m < tiles_m; m += p.bmt) {
+    const int live_m = tiles_m - m < p.bmt ? tiles_m - m : p.bmt;
+    for (int n = 0; n < tiles_n; n += p.bnt) {
+      load[xcd] += (long)live_m * (tiles_n - n < p.bnt ? tiles_n - n : p.bnt);
+      xcd = (xcd + 1) & 7;
+    }
+  }
+  long most = 0;
+  for (long l : load) { most = l > most ? l : most; }
+  return 8 * most;
+}
+
 hipError_t launch_qmm_big(hipStream_t st, const GemmArgs& a, int tile_n)
 {
   const int widest = a.bits == 8 ? 192 : 256;
