@@ -14,9 +14,10 @@
 // expert id lies outside [0, n_experts) gets no slot.
 //
 // Up to 16384 pairs: one workgroup, one launch.  A pair's ticket is an LDS atomic, kept in a register; the slots are put
-// together in LDS as 16-bit pair numbers and written out in order, 16 bytes a lane.  Bound by launch latency at few pairs and by
-// one CU's LDS atomics and stores at many.  Measured against the four launches below (us, in a graph): 512 / 4096 /
-// 16384 pairs of 128 experts 9.7 / 12.0 / 12.6 -> 6.4 / 7.5 / 10.7.
+// together in LDS as 16-bit pair numbers and written out in order, 16 bytes a lane.  Bound by launch latency at few pairs and
+// by one CU's LDS atomics and stores at many.  Measured against the four launches below (us, in a graph): 512 / 4096 /
+// 16384 pairs of 128 experts 9.7 / 12.0 / 12.6 -> 6.4 / 7.5 / 10.7.  The line, in a kernel that takes twice as many: 16384 pairs
+// of 128 / 64 / 8 experts 12.0 / 11.1 / 11.5 -> 11.5 / 10.1 / 11.3, 20480 pairs 12.0 / 11.4 / 11.7 -> 12.4 / 11.0 / 12.8.
 // More pairs, or experts: four launches on the caller's stream (no allocation; ws holds 3 n_experts ints): fill, histogram,
 // offsets by one wavefront (a scan over the experts), scatter.
 #include <atomic>
@@ -144,7 +145,7 @@ __global__ __launch_bounds__(256) void moe_sort_scatter_kernel(const int* __rest
 }
 
 constexpr int kSortOneThreads = 1024;
-constexpr int kSortOneEach = 16;                // pairs per thread, at most (32: 15.9 us against 13.0 of the four launches)
+constexpr int kSortOneEach = 16;                // pairs per thread, at most
 constexpr int kSortOneExperts = 1024;
 constexpr int kSortOneLds = 160 * 1024;
 
@@ -173,7 +174,9 @@ __global__ __launch_bounds__(kSortOneThreads) void moe_sort_one_kernel(const int
 #pragma unroll
   for (int j = 0; j < kSortOneEach; ++j) {
     ticket[j] = 0xffffffffu;
-    if (j * kSortOneThreads < n_pairs && e_of[j] >= 0 && e_of[j] < n_experts) { ticket[j] = ((uint32_t)e_of[j] << 16) | (uint32_t)atomicAdd(count + e_of[j], 1); }
+    if (j * kSortOneThreads < n_pairs && e_of[j] >= 0 && e_of[j] < n_experts) {
+      ticket[j] = ((uint32_t)e_of[j] << 16) | (uint32_t)atomicAdd(count + e_of[j], 1);
+    }
   }
   __syncthreads();
   if (tid < kWave) {                            // one wavefront: lane l owns the experts [l * per, (l + 1) * per)

@@ -25,9 +25,9 @@
 // request).  A slot is copied to registers (codes, x as MFMA operands, scales, biases), re-requested for the
 // wavefront's next chunk, and only then the copy is contracted: one chunk per wavefront is always in flight and no
 // wait has to be counted.  With 8 bits, one workgroup per CU and a long K (twelve chunks a wavefront at 12288) the wavefront
-// has two or three slots instead: 12288 -> 4096 at 6 rows 17.9 -> 15.6 us.  The 16-byte pieces of a row are XOR-swizzled so that the operand reads do not collide on
-// banks.  The scales and biases of the workgroup's rows are two contiguous blocks of the pack and are brought in whole,
-// before anything else.
+// has two or three slots instead: 12288 -> 4096 at 6 rows 17.9 -> 15.6 us.  The 16-byte pieces of a row are XOR-swizzled so
+// that the operand reads do not collide on banks.  The scales and biases of the workgroup's rows are two contiguous blocks of
+// the pack and are brought in whole, before anything else.
 //
 // Math.  Codes become q itself in the element type (exact).  4 bits: against an accumulator seeded with -8 sum(x) of the
 // group, then y += scale * sum(x (q - 8)) + (bias + 8 scale) * sum(x) in fp32; 8 bits: y += scale * sum(x q) +
@@ -207,7 +207,8 @@ __device__ __forceinline__ void batch_to_lds(const uint8_t* base, uint32_t off, 
 // tile of x sits in MFMA row 4*(m%4) + m/4, so that output row m is register m/4 of lane group m%4 and up to four rows
 // need one register.
 template <int T, int MR, int BITS, int GROUP, bool F16, bool SONLY, bool DEEP>
-__global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP, DEEP) ? 4 : 2) void qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
+__global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP, DEEP) ? 4 : 2) void
+qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
 {
   using S = BatchShape<T, MR, BITS, GROUP, DEEP>;
   const BatchParams p = preload_assemble<BatchParams>(VPQ_PRELOADED_WORD_LIST, tail);
@@ -310,7 +311,8 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP, DE
         int row = lane / kXPieces;
         asm volatile("" : "+v"(row));                       // (the rare path: nothing of it is held over the loop)
         const int last = rows - 1 - i * kRowsPerLoad;
-        batch_to_lds(base, __umul24((uint32_t)(row < last ? row : last), xb) + ((int)at < left ? at : 0), to + (S::CLOADS + i) * 1024);
+        batch_to_lds(base, __umul24((uint32_t)(row < last ? row : last), xb) + ((int)at < left ? at : 0),
+                     to + (S::CLOADS + i) * 1024);
       }
       base += kRowsPerLoad * (size_t)xb;
     }
@@ -598,7 +600,8 @@ __global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP, DE
     for (int a = 0; a < S::AT; ++a) {
 #pragma unroll
       for (int q = 0; q < S::RA; ++q) {
-        sums[(((t * S::AT + a) * S::RA + q) * kBatchWaves + wave) * kWave + lane] = BITS == 4 && GROUP == 64 ? acc[t][a][q] + off[t][a][q] : acc[t][a][q];
+        sums[(((t * S::AT + a) * S::RA + q) * kBatchWaves + wave) * kWave + lane] =
+            BITS == 4 && GROUP == 64 ? acc[t][a][q] + off[t][a][q] : acc[t][a][q];
       }
     }
   }
@@ -676,8 +679,10 @@ hipError_t batch_launch_one(hipStream_t st, const BatchParams& p, size_t lds_byt
 template <int BITS, int GROUP, bool F16, bool SONLY = false>
 hipError_t batch_launch(hipStream_t st, const BatchParams& p, int tiles, int mr, bool deep, size_t lds_bytes, int grid)
 {
-#define VPQ_BATCH(T_, MR_, DEEP_) \
-  if (tiles == T_ && mr == MR_ && deep == DEEP_) { return batch_launch_one<T_, MR_, BITS, GROUP, F16, SONLY, DEEP_>(st, p, lds_bytes, grid); }
+#define VPQ_BATCH(T_, MR_, DEEP_)                                                                   \
+  if (tiles == T_ && mr == MR_ && deep == DEEP_) {                                                \
+    return batch_launch_one<T_, MR_, BITS, GROUP, F16, SONLY, DEEP_>(st, p, lds_bytes, grid);     \
+  }
   VPQ_BATCH(1, 1, false) VPQ_BATCH(1, 2, false) VPQ_BATCH(1, 4, false) VPQ_BATCH(1, 8, false)
   VPQ_BATCH(2, 1, false) VPQ_BATCH(2, 2, false) VPQ_BATCH(2, 4, false) VPQ_BATCH(2, 8, false)
   if constexpr (BITS == 8) { VPQ_BATCH(1, 1, true) VPQ_BATCH(1, 2, true) VPQ_BATCH(1, 4, true) VPQ_BATCH(1, 8, true) }

@@ -11,7 +11,8 @@ namespace {
 size_t batch_lds_bytes(int tiles, int mr, int K, const BatchFormat& f, bool deep)
 {
   // (64 more: the unaligned reads of the last row's scales may run past its block)
-  return (size_t)kBatchWaves * batch_ring(tiles, mr, f.bits, deep) * batch_slot_bytes(tiles, mr, f.bits, deep) + 2 * (size_t)batch_scale_bytes(tiles, K, f.group) + 64;
+  return (size_t)kBatchWaves * batch_ring(tiles, mr, f.bits, deep) * batch_slot_bytes(tiles, mr, f.bits, deep) +
+         2 * (size_t)batch_scale_bytes(tiles, K, f.group) + 64;
 }
 
 }  // namespace
@@ -42,10 +43,10 @@ hipError_t launch_qmv_batch(hipStream_t st, const QmvArgs& a, const QmvGroup& g,
   long tiles1 = 0;
   for (int i = 0; i < g.count; ++i) { tiles1 += (g.seg[i].N + 15) / 16; }
   const int tiles = tiles1 * p.m_tiles <= cus || batch_lds_bytes(2, mr, a.K, f, false) > (size_t)kLdsOfCu ? 1 : 2;
-  // 8 bits, one workgroup per CU, a long K: more chunks in flight.  us without / with, groups of 64: 12288 -> 4096 at 4 / 6 / 16 /
-  // 32 rows 16.4 / 15.8 / 17.0 / 23.1 -> 13.1 / 14.4 / 16.9 / 22.0; 6144 -> 4096 at 4 / 32 rows 9.6 / 12.5 -> 8.2 / 12.3, at 12 level
-  // (groups of 32: 9.9 -> 10.1; 6144 -> 2048 9.2 -> 9.5), so 9..16 rows from 7680 on, at 12 rows 11.3 -> 10.8.  4096 -> 4096: 4 rows
-  // 7.4 -> 6.9, 12 rows 8.05 -> 8.5.  4 bits, six chunks at 12288: 11.2 -> 11.8 at 4 rows.
+  // 8 bits, one workgroup per CU, a long K: more chunks in flight.  us without -> with, groups of 64: 12288 -> 4096 at
+  // 4 / 6 / 16 / 32 rows 16.4 / 15.8 / 17.0 / 23.1 -> 13.1 / 14.4 / 16.9 / 22.0; 6144 -> 4096 at 4 / 32 rows 9.6 / 12.5 ->
+  // 8.2 / 12.3, at 12 level (groups of 32: 9.9 -> 10.1; 6144 -> 2048 9.2 -> 9.5), so 9..16 rows from 7680 on, at 12 rows
+  // 11.3 -> 10.8.  4096 -> 4096: 4 rows 7.4 -> 6.9, 12 rows 8.05 -> 8.5.  4 bits, six chunks at 12288: 11.2 -> 11.8 at 4 rows.
   const bool deep = f.bits == 8 && a.K >= (mr == 4 ? 7680 : 6144) && tiles == 1 && tiles1 * p.m_tiles <= cus &&
                     batch_lds_bytes(1, mr, a.K, f, true) <= (size_t)kLdsOfCu;
   const size_t lds_bytes = batch_lds_bytes(tiles, mr, a.K, f, deep);

@@ -247,9 +247,14 @@ hipError_t launch_qmv_gather(hipStream_t st, const QmvArgs& a, int bits, const i
   const int blocks = (int)((sets + 4 * per - 1) / (4 * per));
   const dim3 grid((unsigned)blocks, (unsigned)pairs), block(256);
   uint16_t* y = reinterpret_cast<uint16_t*>(a.y);
-#define VPQ_GATHER(BITS, P, LPR)   launch_kernel(qmv_gather_kernel<BITS, P, LPR>, grid, block, 0, st, a.w, a.scales, a.biases, a.x, pair_eid, a.K, a.N, x_div, n_experts, y, a.gate_act)
+#define VPQ_GATHER(BITS, P, LPR)                                                                                    \
+  launch_kernel(qmv_gather_kernel<BITS, P, LPR>, grid, block, 0, st, a.w, a.scales, a.biases, a.x, pair_eid, a.K, a.N, \
+                x_div, n_experts, y, a.gate_act)
   if (bits == 8) {
-    return a.K <= 1024 ? VPQ_GATHER(8, 1, 64) : a.K <= 2048 ? VPQ_GATHER(8, 2, 64) : a.K <= 3072 ? VPQ_GATHER(8, 3, 64) : VPQ_GATHER(8, 4, 64);
+    return a.K <= 1024   ? VPQ_GATHER(8, 1, 64)
+           : a.K <= 2048 ? VPQ_GATHER(8, 2, 64)
+           : a.K <= 3072 ? VPQ_GATHER(8, 3, 64)
+                         : VPQ_GATHER(8, 4, 64);
   }
   if (half) { return VPQ_GATHER(4, 1, 32); }
   return a.K <= 2048 ? VPQ_GATHER(4, 1, 64) : VPQ_GATHER(4, 2, 64);
