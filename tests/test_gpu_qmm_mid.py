@@ -131,3 +131,23 @@ def test_automatic_split_without_a_workspace(vpq, dev, K, N, M, taken):
     assert status == (0 if taken else -4)
     if taken:
         assert torch.equal(y, vpq.qmm_w4g64(w, s, b, x, K, N, M))
+
+
+# 8 bits: two chunks of codes in LDS in turn, scales read every four steps: every remainder of K, for each count of rows of x
+# per workgroup (want, as vpq_qmm_plan) that takes it
+@pytest.mark.parametrize("want,N,M,steps", [(64, 262, 70, range(1, 14)), (96, 24578, 80, range(1, 10)), (128, 24578, 97, range(6, 14))])
+def test_eight_bit_codes_over_every_remainder_of_k(vpq, dev, want, N, M, steps):
+    gen = torch.Generator(device=dev).manual_seed(want)
+    for K in (64 * t for t in steps):
+        if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+            assert vpq.load().vpq_qmm_plan(K, N, M, 8, 64, 0, 0, 1) == want
+        w = torch.randint(-2 ** 31, 2 ** 31, (N, K // 4), dtype=torch.int32, device=dev, generator=gen)
+        s = torch.empty((N, K // 64), device=dev).uniform_(0.0003, 0.0012, generator=gen).bfloat16()
+        b = -128 * s
+        x = torch.randn((M, K), device=dev, generator=gen).bfloat16()
+        out = parity.Guarded((M, N), torch.bfloat16, dev)
+        vpq.qmm_w8g64(w, s, b, x, K, N, M, out=out.view)
+        torch.cuda.synchronize()
+        out.assert_intact()
+        # (the 256 x 128 tile, which the tests of 8-bit packs compare with the oracle)
+        assert torch.equal(out.view, vpq.qmm_w8g64(w, s, b, x, K, N, M, tile_n=128)), K
