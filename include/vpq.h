@@ -469,8 +469,14 @@ int vpq_qmv_grouped_down_w8g64_bf16(vpq_stream_t stream, const uint32_t* w, cons
  * 128) on that row and that expert's slab.  Requires K % 64 == 0, npad a
  * positive multiple of vpq_qmm_grouped_block_rows(), N even for the gated form,
  * rows * K * 2 < 4e9 for x; w, x 16-byte aligned, y 8-byte aligned (as fast
- * as 16). */
+ * as 16).
+ * vpq_qmm_grouped_plan says how many rows of x a workgroup of them holds (64:
+ * few pairs per expert, else 160; the same bits): rows is rows_x (gated) or
+ * rows_y.  A gated call counts the pairs by its map if that is as the sort
+ * leaves it (npad = max_tiles * block_rows), and takes 8 a token for one cut
+ * down to fewer blocks.  For tests and measurement; needs no device. */
 int vpq_qmm_grouped_block_rows(void);
+int vpq_qmm_grouped_plan(int N, int npad, int n_experts, int rows, int gated);
 size_t vpq_moe_sort_workspace_bytes(int n_experts);
 int vpq_moe_sort_pairs(vpq_stream_t stream, const int32_t* pair_eid, int npair, int top_k, int n_experts,
                        int block_rows, int max_tiles, int32_t* tile2e, int32_t* srow, int32_t* sdst,

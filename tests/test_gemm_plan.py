@@ -53,3 +53,26 @@ def test_plan_refuses_what_the_entrances_refuse():
     for args in [(96, 64, 64, 4, 64, 0, 0, 1), (64, 0, 64, 4, 64, 0, 0, 1), (64, 63, 64, 4, 64, 0, 1, 1), (64, 64, 64, 8, 32, 0, 0, 1),
                  (64, 64, 64, 4, 32, 1, 0, 1), (64, 64, 64, 8, 64, 0, 0, 2), (64, 64, 64, 4, 64, 0, 0, 17)]:
         assert L.vpq_qmm_plan(*args) == -2
+
+
+# Expert-sorted GEMMs: tokens, top_k, experts, blocks of the map (0: as the sort leaves it), rows of x per workgroup.  Times as
+# gate|up + down of 2048 -> 768, 160 rows against 64.
+@pytest.mark.parametrize("tokens,top_k,E,used,want", [
+    (4, 8, 128, 0, 64), (64, 8, 128, 0, 64), (512, 8, 128, 0, 64),     # 93 + 44 / 86 + 38
+    (768, 8, 128, 0, 160), (1024, 8, 128, 0, 160),                     # 112 + 55 / 138 + 66
+    (4096, 1, 128, 0, 64), (512, 16, 128, 0, 160),
+    (64, 8, 128, 126, 64), (512, 8, 128, 128, 64),                     # the map cut down to the blocks in use
+    (1024, 8, 128, 128, 160), (4096, 8, 128, 256, 160),
+])
+def test_expert_sorted_plan(tokens, top_k, E, used, want):
+    L = vpipe_amd.load()
+    pairs, B = tokens * top_k, L.vpq_qmm_grouped_block_rows()
+    npad = B * (used or -(-pairs // B) + min(E, pairs))
+    assert L.vpq_qmm_grouped_plan(1536, npad, E, tokens, 1) == want
+    assert L.vpq_qmm_grouped_plan(2048, npad, E, pairs, 0) == want
+    assert L.vpq_qmm_grouped_plan(512, npad, 64, tokens, 1) == 160     # within one round
+
+
+def test_expert_sorted_plan_refuses_what_the_entrances_refuse():
+    for args in [(0, 128, 8, 4, 0), (64, 100, 8, 4, 0), (64, 128, 0, 4, 0), (64, 128, 8, 0, 0), (63, 128, 8, 4, 1)]:
+        assert vpipe_amd.load().vpq_qmm_grouped_plan(*args) == -2

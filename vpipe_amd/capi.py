@@ -43,6 +43,7 @@ SYMBOLS = [
     ("vpq_gather_qmv_gated_w4g64_bf16", _i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp, _i, _i, _i, _i]),
     ("vpq_gather_down_qmv_w4g64_bf16", _i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp, _i, _i]),
     ("vpq_qmm_grouped_block_rows", _i, []),
+    ("vpq_qmm_grouped_plan", _i, [_i, _i, _i, _i, _i]),
     ("vpq_moe_sort_workspace_bytes", _sz, [_i]),
     ("vpq_moe_sort_pairs", _i, [_vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _sz]),
     ("vpq_qmm_grouped_gated_w4g64_bf16", _i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp, _i, _i, _i]),

@@ -1176,6 +1176,23 @@ int vpq_sample_hist_bf16(vpq_stream_t stream, const uint16_t* logits, int32_t* o
 
 int vpq_qmm_grouped_block_rows(void) { return vpq::kGroupedBlockRows; }
 
+int vpq_qmm_grouped_plan(int N, int npad, int n_experts, int rows, int gated)
+{
+  if (N <= 0 || npad <= 0 || (npad % vpq::kGroupedBlockRows) != 0 || n_experts < 1 || rows < 1 || (gated != 0 && (N & 1) != 0)) {
+    return VPQ_ERR_BAD_SHAPE;
+  }
+  (void)ensure_init();                     // (without a device: the plan for 256 CUs)
+  vpq::GemmArgs g{};
+  g.N = N; g.M = npad;
+  g.gate_act = gated != 0 ? VPQ_GATE_SWIGLU : 0;
+  g.cu_count = g_dev.cu_count;
+  vpq::GroupedArgs ga{};
+  ga.n_experts = n_experts;
+  ga.rows_x = gated != 0 ? rows : npad;
+  ga.rows_y = gated != 0 ? npad : rows;
+  return vpq::qmm_grouped_wide(g, ga) ? 160 : 64;
+}
+
 size_t vpq_moe_sort_workspace_bytes(int n_experts)
 {
   return n_experts > 0 ? (size_t)3 * (size_t)n_experts * sizeof(int32_t) : 0;

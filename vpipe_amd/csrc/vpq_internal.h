@@ -245,6 +245,8 @@ hipError_t launch_moe_scatter_back(hipStream_t st, const uint16_t* dsorted, cons
 hipError_t launch_moe_sort(hipStream_t st, const int* pair_eid, int n_pairs, int top_k, int n_experts, int block_rows,
                            int max_tiles, int* tile2e, int* srow, int* sdst, int* ntiles, int* ws);
 hipError_t launch_qmm_grouped(hipStream_t st, const GemmArgs& a, const GroupedArgs& g);
+// Which of its two forms: five fragments of 32 rows per workgroup, two workgroups a CU; or two, three a CU.
+bool qmm_grouped_wide(const GemmArgs& a, const GroupedArgs& g);
 // Large-tile kernel (256 x 256 or 256 x 192 per workgroup, four wavefronts that each load, dequantize
 // and multiply): K % 512 == 0, 16-byte aligned scales / biases; same bits as the tile
 // kernel.  tile_n 0 = qmm_big_tile_n().

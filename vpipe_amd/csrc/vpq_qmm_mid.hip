@@ -513,7 +513,7 @@ __global__ __launch_bounds__(kMidWaves * 64, 2) void qmm_mid_kernel(const MidPar
 // read nor unpacked a second time (two fragments would leave one workgroup per CU).  All weight tiles of a block go to one
 // XCD (eight workgroups apart), whose L2 then holds its rows of x.
 // Two neighbouring blocks to an XCD, which mostly share an expert's weight tiles: 1 to 2 % slower (2048 tokens 298 -> 305 us).
-// WIDE or not is chosen on the host (launch_qmm_grouped).  Not WIDE is for a few tokens, where almost every block has one or
+// WIDE or not is chosen on the host (qmm_grouped_wide).  Not WIDE is for a few tokens, where almost every block has one or
 // two fragments: no loop over more of them, hence registers and LDS for three workgroups per CU instead of two, and the blocks
 // that have more are multiplied half after half.  (A fourth workgroup needs spills and gains 2 % at most.)
 // Bound by the plain tile's step at full blocks, by unpacking and the codes' read at one fragment.  Measured (us, sort +
@@ -799,6 +799,22 @@ hipError_t launch_qmm_mid(hipStream_t st, const GemmArgs& a)
   return mid_launch_as(st, a, mid_rows(cost_shape(a), 1, cus), 1, nullptr);
 }
 
+// Three narrow workgroups per CU instead of two wide ones where the experts' first blocks alone are more than the wide ones'
+// first round, and up to 32 pairs per expert on average.  Wide against narrow, us of gate|up and down, 2048 -> 768, 8 of 128
+// experts: 64 tokens (4 pairs an expert) 88 + 38 against 82 + 33, 512 (32) 93 + 44 against 86 + 38, 768 (48) 100 + 51 against 106 +
+// 50, 1024 112 + 55 against 138 + 66; within one round, 2048 -> 512, 64 experts, 512 tokens, gate|up 29.3 against 30.3.
+// A down projection knows its pairs (rows_y).  A gated one has its tokens and the map: as the sort leaves it, a block an expert and
+// the whole blocks of all pairs; cut down to the blocks in use it says little, and the pairs are taken to be 8 a token.
+bool qmm_grouped_wide(const GemmArgs& a, const GroupedArgs& g)
+{
+  const long cus = a.cu_count > 0 ? a.cu_count : 256, E = g.n_experts;
+  if (E * ((a.N + kMidTileN - 1) / kMidTileN) <= 2 * cus) { return true; }
+  if (!a.gate_act) { return (long)g.rows_y > 32 * E; }
+  const long blocks = a.M / kGroupedBlockRows, tokens = g.rows_x;
+  const bool whole_map = blocks - E >= (tokens + kGroupedBlockRows - 1) / kGroupedBlockRows;   // (at least a pair a token)
+  return whole_map ? (blocks - E) * kGroupedBlockRows > 32 * E : tokens * 8 > 32 * E;
+}
+
 hipError_t launch_qmm_grouped(hipStream_t st, const GemmArgs& a, const GroupedArgs& g)
 {
   // gated blocks gather rows of x, plain ones scatter rows of y
@@ -815,13 +831,7 @@ hipError_t launch_qmm_grouped(hipStream_t st, const GemmArgs& a, const GroupedAr
   p.tile2e = g.tile2e; p.srow = g.srow; p.sdst = g.sdst;
   p.n_experts = g.n_experts; p.rows_x = g.rows_x; p.rows_y = g.rows_y;
   const dim3 grid((unsigned)((p.tiles_m + 7) / 8 * 8 * p.tiles_n));
-  // Three narrow workgroups per CU instead of two wide ones where the experts' first blocks alone are more than the wide ones'
-  // first round, and up to 32 pairs per expert on average, as far as the count of blocks tells (one an expert and the whole
-  // ones).  Wide against narrow, us of gate|up and down, 2048 -> 768, 8 of 128 experts: 64 tokens (4 pairs an expert) 88 + 38
-  // against 82 + 33, 512 (32) 93 + 44 against 86 + 38, 768 (48) 100 + 51 against 106 + 50, 1024 112 + 55 against 138 + 66;
-  // within one round, 2048 -> 512, 64 experts, 512 tokens, gate|up 29.3 against 30.3.
-  const int cus = a.cu_count > 0 ? a.cu_count : 256;
-  const bool wide = (long)g.n_experts * p.tiles_n <= 2 * cus || ((long)p.tiles_m - g.n_experts) * kGroupedBlockRows > 32L * g.n_experts;
+  const bool wide = qmm_grouped_wide(a, g);
   if (wide) { return a.bits == 8 ? mid_launch_grouped<8, true>(grid, st, p) : mid_launch_grouped<4, true>(grid, st, p); }
   return a.bits == 8 ? mid_launch_grouped<8, false>(grid, st, p) : mid_launch_grouped<4, false>(grid, st, p);
 }
