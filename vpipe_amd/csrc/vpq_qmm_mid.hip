@@ -25,11 +25,12 @@
 // With K split over workgroups (few tiles over a long K) a share leaves fp32 planes that splitk_fold adds in order.
 //
 // What bounds it.  A workgroup alone on its CU: the LDS reads' latency, 230 cycles for a quarter of 130 (0.39 us a step at
-// 64 rows; six stages of x and two slots of codes, without the compiler's wait: no gain).  Several to a CU: LDS (384 cycles
-// of reads and 128 of direct-to-LDS writes a step of 96 rows, 553 taken) and, close behind, a vector ALU that an MFMA
-// shares for half of its 32 cycles (a slot of n instructions lasts 18 + 4 n), at a clock that the power limit holds at
-// 1.5 to 1.8 GHz.  Two 32-row fragments of weights a wavefront halve the LDS reads but leave half the workgroups: 2 % at
-// 2048 tokens of experts, slower below 512 rows.
+// 64 rows; 4 bits with six stages of x and two slots of codes, without the compiler's wait: no gain).  Several to a CU: no unit
+// alone -- on 4096 -> 24576 gated at 333 rows the vector ALU is busy 49 % of the cycles, the matrix pipe 40 %, LDS reads 36 %, a
+// third of that bank conflicts (direct-to-LDS writes are not counted) -- but an MFMA holds the vector ALU for half of its 32
+// cycles (a slot of n instructions lasts 18 + 4 n), at a clock that the power limit holds at 1.5 to 1.8 GHz.  Two 32-row
+// fragments of weights a wavefront halve the LDS reads but leave half the workgroups: 2 % at 2048 tokens of experts, slower
+// below 512 rows.
 // Stores: lanes l and l + 32 exchange quads so that each stores 16 bytes; with four 4-byte pieces and a divide in the
 // activation the store of a 128-row gated tile took 6.9 us of a workgroup's 34.
 // Measured (us, fragments read where they are used, narrow stores; now): 4096 -> 24576 gated at 80 / 128 / 333 rows
@@ -444,7 +445,9 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, uint8_t* x_lds, int
       uint32_t w[4];
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq) {
-        w[rq] = pad ? 0u : pack_elt2<F16>(gated_f32(p.gate_act, v[rq * 4], v[rq * 4 + 1]), gated_f32(p.gate_act, v[rq * 4 + 2], v[rq * 4 + 3]));
+        w[rq] = pad ? 0u
+                    : pack_elt2<F16>(gated_f32(p.gate_act, v[rq * 4], v[rq * 4 + 1]),
+                                     gated_f32(p.gate_act, v[rq * 4 + 2], v[rq * 4 + 3]));
       }
       exchange(w[0], w[2]);
       exchange(w[1], w[3]);
@@ -464,7 +467,7 @@ __device__ __forceinline__ void mid_tile(const MidParams& p, uint8_t* x_lds, int
       put(o + 8, u32x4{w[2], w[3], w[6], w[7]}, p.N - n - 8);
     }
   }
-  if constexpr (GROUPED) {                          // the slots past the fragments that were multiplied: padding, act(0) * 0 = +0
+  if constexpr (GROUPED) {                          // slots past the fragments that were multiplied: padding, act(0) * 0 = +0
     if (p.gate_act) {
       for (int row = BM + frow; row < span; row += 32) {
         const int col = nw / 2 + fkh * 8;
@@ -535,7 +538,8 @@ __global__ __launch_bounds__(kMidWaves * 64, WIDE ? 2 : 3) void qmm_mid_grouped_
   const int* idx = p.gate_act ? p.srow : p.sdst;
   const int lim = p.gate_act ? p.rows_x : p.rows_y;
   const bool next = tm + 1 < p.tiles_m;
-  const int slots[4] = {idx[m0 + lane], idx[m0 + 64 + lane], next ? idx[m0 + 128 + lane] : -1, next ? idx[m0 + 192 + lane] : -1};
+  const int slots[4] = {idx[m0 + lane], idx[m0 + 64 + lane], next ? idx[m0 + 128 + lane] : -1,
+                        next ? idx[m0 + 192 + lane] : -1};
   const int e = p.tile2e[tm], e_before = tm > 0 ? p.tile2e[tm - 1] : -1;
   const int e_next = next ? p.tile2e[tm + 1] : -1, e_after = tm + 2 < p.tiles_m ? p.tile2e[tm + 2] : -1;
   if (e < 0 || e >= p.n_experts) { return; }        // the whole workgroup, before any barrier
@@ -603,7 +607,8 @@ template <typename Kernel>
 hipError_t mid_launch_one(Kernel kern, std::atomic<bool>& ready, size_t lds, dim3 grid, hipStream_t st, const MidParams& p)
 {
   if (!ready.load(std::memory_order_acquire)) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const hipError_t e =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) { return e; }
     ready.store(true, std::memory_order_release);
   }
@@ -739,7 +744,8 @@ double tall_us(const TallCost& c, const CostShape& s, int splits, int cus, long 
 
 double tile_us(const CostShape& s, int splits, int cus)
 {
-  return tall_us(kTileCost, s, splits, cus, (long)((s.M + 255) / 256) * ((s.N + kTileCost.width - 1) / kTileCost.width) * splits);
+  const long tiles = (long)((s.M + 255) / 256) * ((s.N + kTileCost.width - 1) / kTileCost.width);
+  return tall_us(kTileCost, s, splits, cus, tiles * splits);
 }
 
 bool tile_splits_better(const CostShape& s, int splits, int cus)
@@ -749,7 +755,8 @@ bool tile_splits_better(const CostShape& s, int splits, int cus)
 
 CostShape cost_shape(const GemmArgs& a)
 {
-  return CostShape{a.K, a.N, a.M, a.bits == 8 ? kCost8 : a.group == 32 ? kCostG32 : a.f16 ? kCostF16 : kCost4, a.gate_act != 0};
+  const CostFormat f = a.bits == 8 ? kCost8 : a.group == 32 ? kCostG32 : a.f16 ? kCostF16 : kCost4;
+  return CostShape{a.K, a.N, a.M, f, a.gate_act != 0};
 }
 
 // The kernel that takes least without a split of K (for the large tile: its width too), and how long.
@@ -859,8 +866,8 @@ int qmm_choose_splits(int K, int N, int M, int cu_count)
 }
 
 // The count that an automatic split may not go without room for: two and more where 256 x 128 tiles that fill less than
-// half of the chip would take a tenth longer unsplit (0.9 us a step of 64, 3 us a round, planes at 4 TB/s).  Callers without a workspace
-// are refused there and nowhere else.
+// half of the chip would take a tenth longer unsplit (0.9 us a step of 64, 3 us a round, planes at 4 TB/s).  Callers without a
+// workspace are refused there and nowhere else.
 int qmm_required_splits(int K, int N, int M, int cu_count)
 {
   const int cus = cu_count > 0 ? cu_count : 256;
