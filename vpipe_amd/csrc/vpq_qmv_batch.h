@@ -25,7 +25,7 @@
 // request).  A slot is copied to registers (codes, x as MFMA operands, scales, biases), re-requested for the
 // wavefront's next chunk, and only then the copy is contracted: one chunk per wavefront is always in flight and no
 // wait has to be counted.  With 8 bits, one workgroup per CU and a long K (twelve chunks a wavefront at 12288) the wavefront
-// has two or three slots instead: 12288 -> 4096 at 6 rows 17.9 -> 15.6 us.  The 16-byte pieces of a row are XOR-swizzled so
+// has two or three slots instead: 12288 -> 4096 at 6 rows 15.8 -> 14.4 us.  The 16-byte pieces of a row are XOR-swizzled so
 // that the operand reads do not collide on banks.  The scales and biases of the workgroup's rows are two contiguous blocks of
 // the pack and are brought in whole, before anything else.
 //
