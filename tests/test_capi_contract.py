@@ -149,6 +149,28 @@ def test_build_refuses_use_of_a_load_register_before_its_wait():
                                                                                   "v_mov_b32_e32 v20, v4"]))
 
 
+def test_build_refuses_a_load_too_close_behind_its_scalar_base():
+    """A scalar register that a vector instruction wrote may be read by a vector-memory instruction five wait states
+    later; for loads written out by hand only the build's walk over the assembly sees to that."""
+    from vpipe_amd import build
+
+    def kernel(*body):
+        return "_ZN3vpq1kEv:\n%s\n\ts_endpgm\n.Lfunc_end0:\n" % "\n".join("\t" + l for l in body)
+
+    back, load = "v_readlane_b32 s3, v9, 18", "global_load_lds_dwordx4 v1, s[2:3]"
+    for ok in ([back, "s_nop 4", load], [back, "s_mov_b32 m0, s5", "s_add_u32 s8, s8, s9", "s_nop 0x2", load],
+               ["v_readlane_b32 s4, v9, 18", "s_nop 0", load],                       # another register
+               [back, "s_nop 0", "s_add_u32 s10, s2, s4", "v_add_u32_e32 v1, s3, v1"],   # no memory instruction
+               [back, "s_branch .LBB0_2", load, ".LBB0_2:", "s_nop 0"]):             # no path from one to the other
+        build._check_scalar_hazard("x.hip", kernel(*ok))
+    for bad in ([back, "s_nop 3", load], [back, "s_mov_b32 m0, s5", "s_nop 0", load],
+                ["v_cmp_lt_u32_e64 s[2:3], v1, v2", "s_nop 0", load],
+                [back, "s_cbranch_scc1 .LBB0_2", "s_nop 4", ".LBB0_2:", "s_nop 0", load],            # on one of two paths
+                [".LBB0_1:", "s_nop 0", load, "s_nop 0", back, "s_cbranch_scc1 .LBB0_1"]):           # around a loop
+        with pytest.raises(RuntimeError, match="read too soon"):
+            build._check_scalar_hazard("x.hip", kernel(*bad))
+
+
 def test_bench_refuses_more_than_one_gpu():
     # one GPU only: no collectives, no sharding; the benchmark says so instead of starting ranks
     import subprocess

@@ -8,8 +8,10 @@ into one shared library that exports the C ABI declared in include/vpq.h.
 import concurrent.futures
 import os
 import re
+import shutil
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -174,20 +176,84 @@ def _check_inflight(src, asm):
                            % (src, "\n  ".join(bad[:20])))
 
 
+# A scalar register that a vector instruction wrote (a spilled scalar on its way back, v_readlane) may be read by a
+# vector-memory instruction five wait states later at the earliest.  The compiler keeps that distance for its own loads but does
+# not look into assembly statements, so the loads that are written out by hand are checked here, along every path.
+SCALAR_WAIT_STATES = 5
+_SREG = re.compile(r"\bs(\d+)\b|\bs\[(\d+):(\d+)\]|\b(vcc)\b")
+
+
+def _sregs(text):
+    regs = set()
+    for m in _SREG.finditer(text):
+        if m.group(4):
+            regs.add("vcc")
+        elif m.group(1) is not None:
+            regs.add(int(m.group(1)))
+        else:
+            regs.update(range(int(m.group(2)), int(m.group(3)) + 1))
+    return regs
+
+
+def _check_scalar_hazard(src, asm):
+    """Raises if a vector-memory instruction in `asm` reads a scalar register too soon after a vector instruction wrote it."""
+    bad, lines = [], asm.splitlines()
+    for start in (i for i, l in enumerate(lines) if l.startswith("_Z") and _LABEL.match(l)):
+        code, label_at, jumps = [], {}, {}               # instructions; label -> index; label -> indexes that jump there
+        for l in lines[start + 1:]:
+            if l.startswith(".Lfunc_end"):
+                break
+            t = l.split(";")[0].strip()
+            m = _LABEL.match(t)
+            if m:
+                label_at[m.group(1)] = len(code)
+            elif t and not t.startswith("."):
+                if t.startswith(("s_branch", "s_cbranch")):
+                    jumps.setdefault(t.split()[-1], []).append(len(code))
+                code.append(t)
+        into = {}                                         # index -> indexes that jump to it
+        for label, froms in jumps.items():
+            if label in label_at:
+                into.setdefault(label_at[label], []).extend(froms)
+        for i, t in enumerate(code):
+            if not _VMEM.match(t):
+                continue
+            reads = _sregs(t)
+            todo, seen = [(i, 0)], set()
+            while reads and todo:
+                at, states = todo.pop()
+                before = list(into.get(at, []))
+                if at > 0 and not code[at - 1].startswith(("s_branch", "s_endpgm", "s_setpc")):
+                    before.append(at - 1)
+                for j in before:
+                    op = code[j].split()[0]
+                    dst = code[j][len(op):].split(",")[:2 if "_co_" in op else 1]
+                    if op.startswith("v_") and _sregs(",".join(dst)) & reads:
+                        bad.append("%s: `%s` reads what `%s` wrote %d wait states before" % (lines[start][:60], t, code[j], states))
+                    n = states + (int(code[j].split()[1], 0) + 1 if op == "s_nop" else 1)
+                    if n < SCALAR_WAIT_STATES and (j, n) not in seen:
+                        seen.add((j, n))
+                        todo.append((j, n))
+    if bad:
+        raise RuntimeError("%s: scalar register read too soon (see build.py):\n  %s" % (src, "\n  ".join(bad[:20])))
+
+
 def _compile(src):
     obj = os.path.join(CSRC, src.replace(".hip", ".o"))
-    cmd = [HIPCC] + FLAGS + ["-Rpass-analysis=kernel-resource-usage", "-c", os.path.join(CSRC, src), "-o", obj]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        err = "\n".join(l for l in r.stderr.splitlines() if "packed-fp32-ops" not in l and "remark:" not in l)
-        raise RuntimeError("hipcc failed for %s:\n%s" % (src, err))
-    _check_registers(src, r.stderr)
-    if src in ASM_LOAD_SOURCES:
-        a = subprocess.run([HIPCC] + FLAGS + ["-S", "--cuda-device-only", os.path.join(CSRC, src), "-o", "-"],
-                           capture_output=True, text=True)
-        if a.returncode != 0:
-            raise RuntimeError("hipcc -S failed for %s:\n%s" % (src, a.stderr[-2000:]))
-        _check_inflight(src, a.stdout)
+    with tempfile.TemporaryDirectory() as tmp:
+        out = os.path.join(tmp, os.path.basename(obj))
+        cmd = [HIPCC] + FLAGS + ["-Rpass-analysis=kernel-resource-usage", "-save-temps=obj", "-c", os.path.join(CSRC, src), "-o", out]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            err = "\n".join(l for l in r.stderr.splitlines() if "packed-fp32-ops" not in l and "remark:" not in l)
+            raise RuntimeError("hipcc failed for %s:\n%s" % (src, err))
+        _check_registers(src, r.stderr)
+        with open(out.replace(".o", "-hip-amdgcn-amd-amdhsa-gfx950.s")) as f:
+            asm = f.read()
+        if src in ASM_LOAD_SOURCES:
+            _check_inflight(src, asm)
+        _check_scalar_hazard(src, asm)
+        shutil.move(out, obj)
     err = "\n".join(l for l in r.stderr.splitlines()
                     if "packed-fp32-ops" not in l and "remark:" not in l and "-Rpass-analysis" not in l)
     return obj, err

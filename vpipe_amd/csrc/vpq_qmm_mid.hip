@@ -86,11 +86,12 @@ __device__ __forceinline__ uint32_t mid_lds(const uint8_t* q)
 
 // 16 bytes per lane, global -> LDS at lds_dst + 16 * lane.  Written out by hand: the compiler orders every later LDS read
 // after a direct-to-LDS load that it knows about, whatever that load fills.  The LDS base travels in M0, bound as an
-// operand (the s_nop is the wait state between that write and the load).
+// operand (the s_nop is the wait state between that write and the load, and the fifth between a base that comes back from a
+// spill, v_readlane, and the load; the build checks the distance).
 __device__ __forceinline__ void mid_dma16(uint32_t lds_dst, const uint8_t* base, uint32_t lane_off)
 {
   const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds_dst);
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(base), "{m0}"(m0v) : "memory");
+  asm volatile("s_nop 1\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(base), "{m0}"(m0v) : "memory");
 }
 
 template <bool F16>
