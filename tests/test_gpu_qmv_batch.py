@@ -67,6 +67,57 @@ def test_a_row_of_x_has_the_same_bits_in_any_batch(vpq, oracle, dev, D, M, K, N)
         assert torch.equal(vpq.qmv_swiglu_w4g64(wd, sd, bd, part, K, N, n), gated[m0:m0 + n])
 
 
+# The forms of 9 rows and more: K ends inside a piece of x or a chunk, N inside a tile and a quad of outputs.  Three tiles and 48
+# rows, two and 48, two and 64, three and 32 (all rows, two workgroups along M), long pieces of 16 rows with one and two tiles
+# and two to four workgroups along M, four rows a workgroup.
+FORMS = [(320, 8843, 43), (832, 4110, 34), (1088, 6851, 57), (704, 8903, 27), (1856, 4301, 55), (2112, 1067, 27), (4032, 2117, 14),
+         (2560, 4189, 11), (896, 2341, 41), (896, 1813, 61), (1152, 3, 12), (448, 11, 15),
+         (1088, 5443, 32), (512, 3409, 31), (1152, 2579, 62)]      # (8 bits: two and one tile and 32 rows in long pieces)
+
+
+@pytest.mark.parametrize("K,N,M", FORMS)
+@pytest.mark.parametrize("fmt", ["w4g64", "w4g32", "w8g64", "f16"])
+def test_every_form_gives_the_bits_of_few_rows(vpq, dev, D, fmt, K, N, M):
+    # against the same rows in batches of eight, which the oracle checks above
+    bits, group, dtype = {"w4g64": (4, 64, torch.bfloat16), "w4g32": (4, 32, torch.bfloat16), "w8g64": (8, 64, torch.bfloat16),
+                          "f16": (4, 64, torch.float16)}[fmt]
+    def same(a, b):                                           # (a NaN where the infinity meets a weight of zero)
+        return torch.equal(*(torch.nan_to_num(t.float(), nan=1e30, posinf=2e30, neginf=-2e30) for t in (a, b)))
+
+    gen = torch.Generator(device=dev).manual_seed(K + N + M)
+    w = torch.randint(-2 ** 31, 2 ** 31, (N, K * bits // 32), dtype=torch.int32, device=dev, generator=gen)
+    s = torch.empty((N, K // group), device=dev).uniform_(0.005, 0.02, generator=gen).to(dtype)
+    b = (-8 * s.float()).to(dtype)
+    M = min(M, 16) if fmt == "f16" else M
+    firsts = list(range(0, M - 8, 8)) + [M - 8]
+    x = torch.randn((M, K), device=dev, generator=gen).to(dtype)
+    x[M - 1, K - 1] = float("inf")                            # the last row is summed again
+    few = {"w4g64": vpq.qmv_w4g64, "w4g32": vpq.qmv_w4g32, "w8g64": vpq.qmv_w8g64, "f16": vpq.qmv_w4g64_f16}[fmt]
+    out = parity.Guarded((M, N), dtype, dev)
+    if M <= 16:
+        few(w, s, b, x, K, N, M, out=out.view)
+        f32 = few(w, s, b, x, K, N, M, f32out=True)
+        assert same(f32.to(dtype), out.view)
+        res = torch.randn((M, N), device=dev, generator=gen).to(dtype)
+        added = few(w, s, b, x, K, N, M, residual=res)
+        assert same(added, (out.view.float() + res.float()).to(dtype))
+    elif fmt == "w4g64":
+        vpq.linear_w4g64(w, s, b, x, K, N, M, out=out.view)
+        if N % 2 == 0:
+            gated = parity.Guarded((M, N // 2), dtype, dev)
+            vpq.linear_swiglu_w4g64(w, s, b, x, K, N, M, out=gated.view)
+            gated.assert_intact()
+            for m in range(0, M, 8):
+                assert same(vpq.qmv_swiglu_w4g64(w, s, b, x[m:m + 8].contiguous(), K, N, min(8, M - m)), gated.view[m:m + 8])
+    else:
+        vpq.linear_twin(fmt, w, s, b, x, K, N, M, out=out.view)
+    torch.cuda.synchronize()
+    out.assert_intact()
+    assert torch.isinf(out.view[M - 1]).any()
+    for m in firsts:
+        assert same(few(w, s, b, x[m:m + 8].contiguous(), K, N, 8), out.view[m:m + 8])
+
+
 @pytest.mark.parametrize("fmt", ["w4g64", "w4g32", "w8g64"])
 def test_grouped_launch_of_the_batch_kernel(vpq, dev, D, fmt):
     # four packs of different heights, none a multiple of a workgroup's rows: the bits of the separate calls

@@ -1,33 +1,36 @@
 // QMV for a batch of rows (2..64 rows of x; one row where the one-row kernel does not run), any K that is a multiple
 // of 64 (of 32 for groups of 32): the kernel template of vpq_qmv_batch*.hip.
 //
-// What bounds it: a workgroup's life of a request, a wait and a second one (6 to 7 us of 4096 values, two workgroups to a
-// CU), against which neither the arithmetic nor the traffic weighs much up to 32 rows -- 4096 -> 24576 at 4 / 24 rows, us:
-// 15.4 / 24.3; nothing contracted 13.1 / 22.6; no more x requested 15.1 / 20.9; no more codes 13.7 / 23.4; at 48 rows 44, 31,
-// 38 and 41.  Above 32 rows the vector ALU (half busy: unpacking costs 18 instructions per 16 x 64 codes, every 16 x 16
-// outputs 8 multiply-adds per group), the matrix pipe 18 %.  Tried: x in registers and workgroups that walk the tiles (a
-// barrier and a reduction per 16 rows cost more than the second start: 15.4 -> 18.7 at 4 rows; 104 -> 99 on 5120 -> 151936 at
-// 8); all of 33..64 rows in one workgroup, x two pieces ahead (one workgroup per CU: 44 -> 39 at 48 rows, 25 -> 30 at 24);
-// more chunks in flight for 4 bits (the first arrives later: 4096 -> 4096 5.5 -> 6.2).
-// Measured (us; before: one-item and ring kernels where K % 512 == 0, one wavefront
-// per weight row elsewhere, slabs of 16 rows above 16): 4096 -> 4096 at 16 / 48 rows 9.3 / 20.4 -> 6.3 / 10.0;
-// 4096 -> 12288 13.3 / 38.6 -> 12.2 / 21.0; 5120 -> 151936 at 8 / 16 rows 102 / 124 -> 96 / 114; 3840 -> 19328 at
-// 4 / 16 rows 51 / 156 -> 13.5 / 17.4.
+// What bounds it.  Up to 8 rows the pack's read and the start of a launch (4096 -> 24576 at 4 rows 14.6 us, 57 MB).  Above,
+// the instructions and a workgroup's own start and end: of 36 000 cycles of three tiles and 48 rows over K = 4096, 7 800 pass
+// before the first codes are there, 2 500 a piece of 64 values (two wavefronts a SIMD; 1 470 if they only issued: unpacking
+// costs 18 instructions per 16 x 64 codes, every 16 x 16 outputs 8 multiply-adds per group, an MFMA holds the vector ALU for
+// 8 of its 16 cycles), the rest are the end's.  x comes in once per workgroup, so it also counts how many weight rows share
+// it and how many workgroups a CU gets one after the other: batch_plan. Tried: workgroups that walk over the blocks of weight
+// rows and request the next block's codes and scales early (30.5 -> 28.7 us at 48 rows, but level on the mean of 7000 shapes,
+// and scalar registers spill); the next piece of x read from LDS while one is contracted (28.7 -> 30.6); several pieces of x
+// in flight (LDS reads take 450 cycles instead of 200 while they come in: 8 % slower); three tiles in 128 registers, two
+// workgroups to a CU (4 rows 14.6 -> 17.1); x in registers (15.4 -> 18.7 at 4 rows; 104 -> 99 on 5120 -> 151936 at 8); more
+// chunks in flight for 4 bits (the first arrives later: 4096 -> 4096 5.0 -> 5.5). Measured (us, before / now; before: up to
+// 32 rows and two tiles a workgroup): 4096 -> 4096 at 16 / 24 / 48 rows 6.3 / 7.6 / 9.6 -> 6.0 / 7.1 / 9.6; 4096 -> 1024 at
+// 24 / 48 rows 7.3 / 7.5 -> 5.4 / 6.0; 12288 -> 4096 at 16 / 24 rows 13.4 / 17.9 -> 12.1 / 15.6; 4096 -> 24576 at 4 / 48 rows
+// 15.2 / 38.7 -> 14.7 / 30.5; 17408 -> 5120 at 48 / 64 rows 51 / 53 -> 34 / 35.
 //
-// Split.  A workgroup of eight wavefronts owns T tiles of 16 weight rows and up to 32 rows of x.  K is cut into chunks
+// Split.  A workgroup of eight wavefronts owns T tiles of 16 weight rows and up to 64 rows of x.  K is cut into chunks
 // of 128 bytes of codes per row (256 values of 4 bits, 128 of 8 bits); chunk c belongs to wavefront c % 8, which
 // contracts it for all T tiles and all rows of x.  The eight partial results meet in LDS once, at the end, in
 // wavefront order.  So a result depends on K and the format alone -- not on M, N, T or the launch it is part of: a row
 // of x has the same bits in a batch of any size, and a grouped launch the bits of separate ones.
 //
-// Loads.  Codes and x arrive by 128-bit direct-to-LDS loads into one slot per wavefront, laid out so that eight
-// consecutive lanes cover one 128-byte line (an L1 has about 72 requests in flight, so what counts is bytes per
-// request).  A slot is copied to registers (codes, x as MFMA operands, scales, biases), re-requested for the
-// wavefront's next chunk, and only then the copy is contracted: one chunk per wavefront is always in flight and no
-// wait has to be counted.  With 8 bits, one workgroup per CU and a long K (twelve chunks a wavefront at 12288) the wavefront
-// has two or three slots instead: 12288 -> 4096 at 6 rows 15.8 -> 14.4 us.  The 16-byte pieces of a row are XOR-swizzled so
-// that the operand reads do not collide on banks.  The scales and biases of the workgroup's rows are two contiguous blocks of
-// the pack and are brought in whole, before anything else.
+// Loads.  Codes and x arrive by 128-bit direct-to-LDS loads into one slot per wavefront, laid out so that eight consecutive
+// lanes cover one 128-byte line (an L1 has about 72 requests in flight, so what counts is bytes per request).  A slot is
+// copied to registers (codes, x as MFMA operands, scales, biases), re-requested for the wavefront's next chunk, and only then
+// the copy is contracted: one chunk per wavefront is always in flight and no wait has to be counted.  A workgroup with a CU
+// to itself may take pieces of x twice as long (a wait, a read and a start of the contraction fewer: 12288 -> 4096 at 16 rows
+// 13.1 -> 12.1 us) or, with 8 bits and a long K (twelve chunks a wavefront at 12288), two or three slots (12288 -> 4096 at 6
+// rows 15.8 -> 14.4).  The 16-byte pieces of a row are XOR-swizzled so that the operand reads do not collide on banks.  The
+// scales and biases of the workgroup's rows are two contiguous blocks of the pack and are brought in whole, before anything
+// else.
 //
 // Math.  Codes become q itself in the element type (exact).  4 bits: against an accumulator seeded with -8 sum(x) of the
 // group, then y += scale * sum(x (q - 8)) + (bias + 8 scale) * sum(x) in fp32; 8 bits: y += scale * sum(x q) +
@@ -72,32 +75,34 @@ struct BatchParams {
   QmvSeg seg[3];        // the others
   int seg_first[3];     // their first workgroup
 };
+// What a launch runs: tiles of 16 weight rows and rows of x (4 mr at most) of a workgroup, workgroups along M, depth.
+struct BatchPlan {
+  int tiles, mr, m_tiles, depth;
+};
 static_assert(offsetof(BatchParams, y) == kPreloadWords * 4, "y starts the part that is not preloaded");
 
 // BITS: 4 or 8.  GROUP: 64 or 32.
-// DEEP: one workgroup per CU, which has its LDS to itself: x of a chunk in pieces of 8 KB, and slots for up to three chunks.
 constexpr int batch_x_bytes(int mr, int bits) { return mr * 4 * (128 * 8 / bits) * 2; }
-constexpr int batch_x_piece(int mr, int bits, bool deep)
+// DEPTH of one: x of a chunk comes in pieces, of 64 values a row above 16 rows, of at most 4 KB below.  Two and more, where a
+// workgroup has a CU to itself: pieces that many times as long, or, where a chunk is one piece, that many chunks in flight.
+constexpr int batch_x_piece1(int mr, int bits)
 {
-  return batch_x_bytes(mr, bits) < (deep ? 8192 : 4096) ? batch_x_bytes(mr, bits) : (deep ? 8192 : 4096);
+  return mr >= 8 ? mr * 512 : batch_x_bytes(mr, bits) < 4096 ? batch_x_bytes(mr, bits) : 4096;
 }
-constexpr int batch_slot_bytes(int t, int mr, int bits, bool deep) { return t * 2048 + batch_x_piece(mr, bits, deep); }
-constexpr int batch_ring(int t, int mr, int bits, bool deep)
+constexpr int batch_ring(int mr, int bits, int depth) { return batch_x_piece1(mr, bits) == batch_x_bytes(mr, bits) ? depth : 1; }
+constexpr int batch_x_piece(int mr, int bits, int depth)
 {
-  return !deep || batch_x_piece(mr, bits, deep) < batch_x_bytes(mr, bits) ? 1
-         : batch_slot_bytes(t, mr, bits, deep) <= 4096                    ? 3
-         : batch_slot_bytes(t, mr, bits, deep) <= 6144                    ? 2
-                                                                          : 1;
+  return batch_x_piece1(mr, bits) * (depth / batch_ring(mr, bits, depth));
 }
+constexpr int batch_slot_bytes(int t, int mr, int bits, int depth) { return t * 2048 + batch_x_piece(mr, bits, depth); }
 
-template <int T, int MR, int BITS, int GROUP, bool DEEP>
+template <int T, int MR, int BITS, int GROUP, int DEPTH>
 struct BatchShape {
   static constexpr int CK = 128 * 8 / BITS;                       // values of K per chunk
-  static constexpr int AT = MR == 8 ? 2 : 1;                      // MFMA tiles of 16 rows of x
-  static constexpr int RA = MR == 8 ? 4 : MR;                     // accumulator registers of one
-  // x of a chunk comes in pieces of at most 4 KB: 16 registers of operands per lane, and two workgroups fit a CU
-  static constexpr int XS = batch_x_bytes(MR, BITS) / batch_x_piece(MR, BITS, DEEP);
-  static constexpr int RING = batch_ring(T, MR, BITS, DEEP);      // slots of a wavefront (one where XS > 1)
+  static constexpr int AT = MR >= 8 ? MR / 4 : 1;                 // MFMA tiles of 16 rows of x
+  static constexpr int RA = MR >= 8 ? 4 : MR;                     // accumulator registers of one
+  static constexpr int XS = batch_x_bytes(MR, BITS) / batch_x_piece(MR, BITS, DEPTH);   // pieces of x per chunk
+  static constexpr int RING = batch_ring(MR, BITS, DEPTH);        // slots of a wavefront (one where XS > 1)
   static constexpr int SK = CK / XS;                              // values of K per piece
   static constexpr int XROWB = SK * 2;
   static constexpr int XLOADS = MR * 4 * XROWB / 1024;            // direct-to-LDS loads per piece
@@ -106,10 +111,15 @@ struct BatchShape {
   static constexpr int SG = CK / GROUP;                           // groups per chunk
   static constexpr int SGW = SG / 2;                              // their scales of one row, in words
   static constexpr int MPG = GROUP / 32;                          // MFMAs per group
+  static_assert(RING == 1 || XS == 1, "");
+  static_assert(T * AT * RA * kWave * 4 <= RING * SLOT, "the partial results lie over the slots");
 };
 
 // Whether two workgroups may share a CU: at most 128 registers per lane (the build refuses a spill).
-constexpr bool batch_two_per_cu(int t, int mr, int group, bool deep) { return !deep && !(t == 2 && group == 32 && mr == 8); }
+constexpr bool batch_two_per_cu(int t, int mr, int group, int depth)
+{
+  return depth == 1 && t <= 2 && mr <= 8 && !(t == 2 && group == 32 && mr == 8);
+}
 
 inline int batch_scale_bytes(int tiles, int K, int group) { return (tiles * 16 * (K / group) * 2 + 1023) / 1024 * 1024; }
 
@@ -203,14 +213,15 @@ __device__ __forceinline__ void batch_to_lds(const uint8_t* base, uint32_t off, 
 
 }  // namespace
 
-// MR: accumulator registers per lane and tile, 1 / 2 / 4 / 8 for up to 4 / 8 / 16 / 32 rows of x.  Row m of an MFMA
+// MR: accumulator registers per lane and tile, 1 / 2 / 4 / 8 / 12 / 16 for up to 4 / 8 / 16 / 32 / 48 / 64 rows
+// of x.  Row m of an MFMA
 // tile of x sits in MFMA row 4*(m%4) + m/4, so that output row m is register m/4 of lane group m%4 and up to four rows
 // need one register.
-template <int T, int MR, int BITS, int GROUP, bool F16, bool SONLY, bool DEEP>
-__global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP, DEEP) ? 4 : 2) void
+template <int T, int MR, int BITS, int GROUP, bool F16, bool SONLY, int DEPTH>
+__global__ __launch_bounds__(kBatchWaves * 64, batch_two_per_cu(T, MR, GROUP, DEPTH) ? 4 : 2) void
 qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
 {
-  using S = BatchShape<T, MR, BITS, GROUP, DEEP>;
+  using S = BatchShape<T, MR, BITS, GROUP, DEPTH>;
   const BatchParams p = preload_assemble<BatchParams>(VPQ_PRELOADED_WORD_LIST, tail);
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
@@ -301,16 +312,18 @@ qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
     const int left = (p.K - k0) * 2;
     const uint8_t* base = xtile + (size_t)k0 * 2;
     uint32_t xb = x_bytes;
+    int live = rows;
     asm volatile("" : "+v"(x_piece), "+s"(xb));
+    if constexpr (S::XLOADS > 4) { asm volatile("" : "+s"(live)); }   // (no comparison per load is held over the loop)
 #pragma unroll
     for (int i = 0; i < S::XLOADS; ++i) {
       const uint32_t at = x_piece ^ (uint32_t)(kXPieces >= 16 ? ((i * kRowsPerLoad) & 15) * 16 : (i & 1) * 64);
-      if (left >= S::XROWB && (i + 1) * kRowsPerLoad <= rows) {
+      if (left >= S::XROWB && (i + 1) * kRowsPerLoad <= live) {
         batch_to_lds(base, at + x_row, to + (S::CLOADS + i) * 1024);
-      } else if (i * kRowsPerLoad < rows) {
+      } else if (i * kRowsPerLoad < live) {
         int row = lane / kXPieces;
         asm volatile("" : "+v"(row));                       // (the rare path: nothing of it is held over the loop)
-        const int last = rows - 1 - i * kRowsPerLoad;
+        const int last = live - 1 - i * kRowsPerLoad;
         batch_to_lds(base, __umul24((uint32_t)(row < last ? row : last), xb) + ((int)at < left ? at : 0),
                      to + (S::CLOADS + i) * 1024);
       }
@@ -349,6 +362,8 @@ qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
     asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
   }
   asm volatile("s_barrier" : : : "memory");                 // (__syncthreads would wait for the chunks as well)
+  // The arguments that only the store needs are read by here, behind the requests and not when it waits for them.
+  asm volatile("" : : "s"(y_), "s"(p.residual), "s"(p.gate_act), "s"(p.y_f32));
   if ((sb_bytes & 15) != 0) {                               // the last rows of an N that is not a multiple of 8
     const int at = (sb_bytes >> 4) * 8 + (int)threadIdx.x;
     if (at < (sb_bytes >> 1)) {
@@ -380,7 +395,6 @@ qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
 
   // A lane's operands of a chunk.  MFMA j takes from lane (fr, g) the eight values at k = 32j + 8g (groups of 32) or
   // at k = 64(j/2) + 16g + 8(j%2) (groups of 64): any order inside a group is right as long as codes and x agree.
-  constexpr int kMfmas = S::CK / 32;
   constexpr int kPieceMfmas = S::SK / 32;
   uint32_t cw[T][8];
   u32x4 xq[S::AT][kPieceMfmas];
@@ -605,54 +619,142 @@ qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
       }
     }
   }
-  __syncthreads();
-  const int live_waves = chunks < kBatchWaves ? chunks : kBatchWaves;
-  constexpr int kOuts = T * S::AT * S::RA * kWave;
-  for (int o_idx = threadIdx.x; o_idx < kOuts; o_idx += kBatchWaves * kWave) {
-    const int l = o_idx & 63;
-    const int r = o_idx >> 6;                                // (t * AT + a) * RA + q
-    const float* sp = sums + (size_t)r * kBatchWaves * kWave + l;
-    float total = 0.0f;
-    for (int wv = 0; wv < live_waves; ++wv) { total += sp[wv * kWave]; }
-    const int q = r % S::RA;
-    const int a = (r / S::RA) % S::AT;
-    const int t = r / (S::RA * S::AT);
-    const int m_loc = a * 16 + 4 * q + (l >> 4);
-    const int n_loc = t * 16 + (l & 15);
-    const bool ok = m_loc < rows && n_loc < n_live;
-    const int m = m0 + m_loc, n = n0 + n_loc;
-    unsigned long long bad = __ballot(ok && (__float_as_uint(total) & 0x7f800000u) == 0x7f800000u);
-    while (bad != 0) {                                       // one output of the wavefront at a time, all lanes on it
-      const int src = __builtin_ctzll(bad);
-      bad &= bad - 1;
-      const int nb_ = __builtin_amdgcn_readlane(n, src), mb = __builtin_amdgcn_readlane(m, src);
-      const float plain = batch_plain_sum<BITS, GROUP, F16, SONLY>(
-          reinterpret_cast<const uint8_t*>(w_) + (size_t)nb_ * row_bytes, scales_ + (size_t)nb_ * Kg,
-          SONLY ? nullptr : biases_ + (size_t)nb_ * Kg, p.x + (size_t)mb * p.K, p.K);
-      if ((int)(threadIdx.x & 63) == src) { total = plain; }
+  if constexpr (T * S::AT * S::RA <= 16) {
+    // (few: spread over all wavefronts.  As quads 4096 -> 4096 at 16 rows takes 6.9 us for 6.2; more as these 31.0 for 30.5 of
+    // 4096 -> 24576 at 48 rows.)
+    // Wavefront w adds up and stores rows r = w, w + 8, ... of sums (r = (t * AT + a) * RA + q).
+    constexpr int kOuts = T * S::AT * S::RA, kOutsPer = (kOuts + kBatchWaves - 1) / kBatchWaves;
+    auto out_m = [&](int r) { return (r / S::RA) % S::AT * 16 + 4 * (r % S::RA) + g; };
+    auto out_n = [&](int r) { return r / (S::RA * S::AT) * 16 + fr; };
+    // (the residual is on its way while the wavefronts meet)
+    uint16_t res[kOutsPer];
+    if (p.residual != nullptr && p.gate_act == 0) {
+#pragma unroll
+      for (int i = 0; i < kOutsPer; ++i) {
+        const int r = wave + i * kBatchWaves, m = out_m(r), n = out_n(r);
+        res[i] = r < kOuts && m < rows && n < n_live ? p.residual[(size_t)(m0 + m) * N_ + n0 + n] : 0;
+      }
     }
-    if (p.gate_act) {
-      // Lanes 2j and 2j+1 hold the gate and the up sum of one feature (N is even).
-      const float up = from_neighbour_lane(total);
-      if (ok && (l & 1) == 0) {
-        const float v = gated_f32(p.gate_act, total, up);
-        const size_t o = (size_t)m * (N_ >> 1) + (n >> 1);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");   // (__syncthreads would wait for the residual as well)
+    float totals[kOutsPer];
+#pragma unroll
+    for (int i = 0; i < kOutsPer; ++i) {
+      const int r = wave + i * kBatchWaves;
+      const float* sp = sums + (r < kOuts ? r : 0) * (kBatchWaves * kWave) + lane;
+      float part[kBatchWaves];
+#pragma unroll
+      for (int wv = 0; wv < kBatchWaves; ++wv) { part[wv] = sp[wv * kWave]; }
+      totals[i] = 0.0f;
+#pragma unroll
+      for (int wv = 0; wv < kBatchWaves; ++wv) { totals[i] += part[wv]; }     // (wavefronts without a chunk add +0)
+    }
+#pragma unroll
+    for (int i = 0; i < kOutsPer; ++i) {
+      const int r = wave + i * kBatchWaves;
+      if (r >= kOuts) { break; }
+      float total = totals[i];
+      const int m_loc = out_m(r), n_loc = out_n(r);
+      const bool ok = m_loc < rows && n_loc < n_live;
+      const int m = m0 + m_loc, n = n0 + n_loc;
+      unsigned long long bad = __ballot(ok && (__float_as_uint(total) & 0x7f800000u) == 0x7f800000u);
+      while (bad != 0) {                                       // one output of the wavefront at a time, all lanes on it
+        const int src = __builtin_ctzll(bad);
+        bad &= bad - 1;
+        const int row = __builtin_amdgcn_readlane(n_loc, src), mb = __builtin_amdgcn_readlane(m, src);
+        const float plain = batch_plain_sum<BITS, GROUP, F16, SONLY>(
+            wtile + (size_t)row * row_bytes, sc_src + (size_t)row * Kg, SONLY ? nullptr : bi_src + (size_t)row * Kg,
+            p.x + (size_t)mb * p.K, p.K);
+        if (lane == src) { total = plain; }
+      }
+      if (p.gate_act) {
+        // Lanes 2j and 2j+1 hold the gate and the up sum of one feature (N is even).
+        const float up = from_neighbour_lane(total);
+        if (ok && (lane & 1) == 0) {
+          const float v = gated_f32(p.gate_act, total, up);
+          const size_t o = (size_t)m * (N_ >> 1) + (n >> 1);
+          if (p.y_f32) {
+            reinterpret_cast<float*>(y_)[o] = v;
+          } else {
+            reinterpret_cast<uint16_t*>(y_)[o] = (uint16_t)f32_to_elt_bits<F16>(v);
+          }
+        }
+      } else if (ok) {
+        const size_t o = (size_t)m * N_ + n;
         if (p.y_f32) {
-          reinterpret_cast<float*>(y_)[o] = v;
+          reinterpret_cast<float*>(y_)[o] = total;
         } else {
-          reinterpret_cast<uint16_t*>(y_)[o] = (uint16_t)f32_to_elt_bits<F16>(v);
+          uint32_t v = f32_to_elt_bits<F16>(total);
+          if (p.residual != nullptr) {
+            v = f32_to_elt_bits<F16>(elt_bits_to_f32<F16>(v) + elt_bits_to_f32<F16>(res[i]));
+          }
+          reinterpret_cast<uint16_t*>(y_)[o] = (uint16_t)v;
         }
       }
-    } else if (ok) {
-      const size_t o = (size_t)m * N_ + n;
-      if (p.y_f32) {
-        reinterpret_cast<float*>(y_)[o] = total;
-      } else {
-        uint32_t v = f32_to_elt_bits<F16>(total);
-        if (p.residual != nullptr) {
-          v = f32_to_elt_bits<F16>(elt_bits_to_f32<F16>(v) + elt_bits_to_f32<F16>(p.residual[o]));
+    }
+  } else {
+    // A thread adds up and stores quads of outputs, four weight rows of one row of x: quad i is lanes 4 (i % 16) .. + 3 of
+    // register i / 16 = (t * AT + a) * RA + q.
+    constexpr int kThreads = kBatchWaves * kWave, kQuads = T * S::AT * S::RA * 16, kRounds = (kQuads + kThreads - 1) / kThreads;
+    const int tid = (int)threadIdx.x;
+    auto quad_m = [](int i) { return (i >> 4) / S::RA % S::AT * 16 + 4 * ((i >> 4) % S::RA) + ((i >> 2) & 3); };
+    auto quad_n = [](int i) { return (i >> 4) / (S::RA * S::AT) * 16 + (i & 3) * 4; };
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+#pragma unroll
+    for (int j = 0; j < kRounds; ++j) {
+      if (wave * kWave + j * kThreads >= kQuads) { break; }
+      const bool on = tid + j * kThreads < kQuads;             // (all lanes stay: batch_plain_sum needs them)
+      const int i = on ? tid + j * kThreads : 0;
+      floatx4 part[kBatchWaves], total = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int wv = 0; wv < kBatchWaves; ++wv) {
+        part[wv] = *reinterpret_cast<const floatx4*>(sums + ((i >> 4) * kBatchWaves + wv) * kWave + (i & 15) * 4);
+      }
+#pragma unroll
+      for (int wv = 0; wv < kBatchWaves; ++wv) { total += part[wv]; }         // (wavefronts without a chunk add +0)
+      const int m_loc = quad_m(i), n_loc = quad_n(i), left = on && m_loc < rows ? n_live - n_loc : 0;
+      const int m = m0 + m_loc, n = n0 + n_loc;
+      unsigned bad_here = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (e < left && (__float_as_uint(total[e]) & 0x7f800000u) == 0x7f800000u) { bad_here |= 1u << e; }
+      }
+      while (__ballot(bad_here != 0) != 0) {                   // one output of the wavefront at a time, all lanes on it
+        const int src = __builtin_ctzll(__ballot(bad_here != 0));
+        const int e = __builtin_ctz(__builtin_amdgcn_readlane((int)bad_here, src));
+        const int row = __builtin_amdgcn_readlane(n_loc, src) + e, mb = __builtin_amdgcn_readlane(m, src);
+        const float plain = batch_plain_sum<BITS, GROUP, F16, SONLY>(
+            wtile + (size_t)row * row_bytes, sc_src + (size_t)row * Kg, SONLY ? nullptr : bi_src + (size_t)row * Kg,
+            p.x + (size_t)mb * p.K, p.K);
+        if ((tid & 63) == src) {
+          bad_here &= bad_here - 1;
+#pragma unroll
+          for (int f = 0; f < 4; ++f) { total[f] = f == e ? plain : total[f]; }
         }
-        reinterpret_cast<uint16_t*>(y_)[o] = (uint16_t)v;
+      }
+      if (left <= 0) {
+      } else if (p.gate_act) {                                 // (gate, up, gate, up); N is even
+        const float v0 = gated_f32(p.gate_act, total[0], total[1]);
+        const float v1 = gated_f32(p.gate_act, total[2], total[3]);
+        const size_t o = (size_t)m * (N_ >> 1) + (n >> 1);
+        if (left > 2) {
+          const uint32_t v = f32_to_elt_bits<F16>(v0) | f32_to_elt_bits<F16>(v1) << 16;
+          __builtin_memcpy(reinterpret_cast<uint16_t*>(y_) + o, &v, 4);
+        } else {
+          reinterpret_cast<uint16_t*>(y_)[o] = (uint16_t)f32_to_elt_bits<F16>(v0);
+        }
+      } else {
+        uint32_t v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { v[e] = f32_to_elt_bits<F16>(total[e]); }
+        uint16_t* yp = reinterpret_cast<uint16_t*>(y_) + (size_t)m * N_ + n;
+        if (left >= 4) {
+          const u32x2 w = {v[0] | v[1] << 16, v[2] | v[3] << 16};
+          __builtin_memcpy(yp, &w, 8);
+        } else {
+          yp[0] = (uint16_t)v[0];
+          if (left > 1) { yp[1] = (uint16_t)v[1]; }
+          if (left > 2) { yp[2] = (uint16_t)v[2]; }
+        }
       }
     }
   }
@@ -662,11 +764,11 @@ constexpr int kLdsOfCu = 160 * 1024;
 
 // One instantiation's launch; the attribute is set once per kernel, whichever thread comes first (two may both set it,
 // which is harmless; neither launches before its own call has returned).
-template <int T, int MR, int BITS, int GROUP, bool F16, bool SONLY, bool DEEP>
+template <int T, int MR, int BITS, int GROUP, bool F16, bool SONLY, int DEPTH>
 hipError_t batch_launch_one(hipStream_t st, const BatchParams& p, size_t lds_bytes, int grid)
 {
   static std::atomic<bool> ready{false};
-  auto kern = qmv_batch_kernel<T, MR, BITS, GROUP, F16, SONLY, DEEP>;
+  auto kern = qmv_batch_kernel<T, MR, BITS, GROUP, F16, SONLY, DEPTH>;
   if (!ready.load(std::memory_order_acquire)) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, kLdsOfCu);
@@ -677,21 +779,23 @@ hipError_t batch_launch_one(hipStream_t st, const BatchParams& p, size_t lds_byt
 }
 
 template <int BITS, int GROUP, bool F16, bool SONLY = false>
-hipError_t batch_launch(hipStream_t st, const BatchParams& p, int tiles, int mr, bool deep, size_t lds_bytes, int grid)
+hipError_t batch_launch(hipStream_t st, const BatchParams& p, const BatchPlan& plan, size_t lds_bytes, int grid)
 {
-#define VPQ_BATCH(T_, MR_, DEEP_)                                                                   \
-  if (tiles == T_ && mr == MR_ && deep == DEEP_) {                                                \
-    return batch_launch_one<T_, MR_, BITS, GROUP, F16, SONLY, DEEP_>(st, p, lds_bytes, grid);     \
+#define VPQ_BATCH(T_, MR_, DEPTH_)                                                                    \
+  if (plan.tiles == T_ && plan.mr == MR_ && plan.depth == DEPTH_) {                                   \
+    return batch_launch_one<T_, MR_, BITS, GROUP, F16, SONLY, DEPTH_>(st, p, lds_bytes, grid);        \
   }
-  VPQ_BATCH(1, 1, false) VPQ_BATCH(1, 2, false) VPQ_BATCH(1, 4, false) VPQ_BATCH(1, 8, false)
-  VPQ_BATCH(2, 1, false) VPQ_BATCH(2, 2, false) VPQ_BATCH(2, 4, false) VPQ_BATCH(2, 8, false)
-  if constexpr (BITS == 8) { VPQ_BATCH(1, 1, true) VPQ_BATCH(1, 2, true) VPQ_BATCH(1, 4, true) VPQ_BATCH(1, 8, true) }
+  VPQ_BATCH(1, 1, 1) VPQ_BATCH(1, 2, 1) VPQ_BATCH(1, 4, 1) VPQ_BATCH(1, 8, 1) VPQ_BATCH(2, 1, 1) VPQ_BATCH(2, 2, 1)
+  VPQ_BATCH(2, 4, 1) VPQ_BATCH(2, 8, 1) VPQ_BATCH(2, 12, 1) VPQ_BATCH(2, 16, 1) VPQ_BATCH(3, 8, 1) VPQ_BATCH(3, 12, 1)
+  VPQ_BATCH(1, 4, 2)
+  if constexpr (BITS == 4) { VPQ_BATCH(2, 4, 2) }
+  if constexpr (BITS == 8) { VPQ_BATCH(1, 1, 3) VPQ_BATCH(1, 2, 2) VPQ_BATCH(1, 8, 2) VPQ_BATCH(2, 8, 2) }
 #undef VPQ_BATCH
   return hipErrorInvalidValue;
 }
 
 // The instantiations of the other formats (vpq_qmv_batch_twins.hip).
-hipError_t launch_qmv_batch_twin(hipStream_t st, const BatchParams& p, int tiles, int mr, bool deep, size_t lds_bytes, int grid,
+hipError_t launch_qmv_batch_twin(hipStream_t st, const BatchParams& p, const BatchPlan& plan, size_t lds_bytes, int grid,
                                  const BatchFormat& f);
 
 }  // namespace vpq
