@@ -844,7 +844,7 @@ int vpq_sample_topp_bf16(vpq_stream_t stream, const uint16_t* logits, int32_t* o
  * `sample_max_partial_f16`, `sample_max_combine_f16`, `sample_zhist_partial_f16`,
  * `sample_zhist_combine_f16`, `sample_thresh_f16`, `sample_pick_partial_f16`,
  * `sample_pick_combine_f16` (llm_elementwise.metal:3255-3640; its M is n_slabs
- * here) -- seven dispatches there, one call (five launches) here.  Same
+ * here) -- seven dispatches there, one call (four launches) here.  Same
  * pipeline and arguments as vpq_sample_topp_bf16 without n_iter: the
  * vocabulary is cut into n_slabs contiguous slabs of ceil(V / n_slabs) indices,
  * one workgroup each, and top-k / top-p become the low edge of a bin of a
@@ -853,8 +853,8 @@ int vpq_sample_topp_bf16(vpq_stream_t stream, const uint16_t* logits, int32_t* o
  * factor e^(40/1024) = 1.04 below the exact threshold); min-p stays exact.
  * The draw is an exact function of (logits, seen, parameters, seed, n_slabs).
  * `work`: vpq_sample_hist_workspace_bytes(n_slabs) bytes of device scratch
- * (slab maxima, per-slab histograms, their sum, the threshold, per-slab
- * picks), 4-byte aligned; nothing in it needs to be cleared.
+ * (slab maxima, per-slab histograms, the threshold, the best entry of the
+ * draw), 4-byte aligned; nothing in it needs to be cleared.
  * Requires 1 <= V <= 2^24, rep != 0, 1 <= n_slabs <= 1024, ceil(V / n_slabs) <= 65535
  * (the per-slab fixed-point masses); other requirements as above. */
 size_t vpq_sample_hist_workspace_bytes(int n_slabs);

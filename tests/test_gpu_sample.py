@@ -144,6 +144,31 @@ def test_histogram_sampler_matches_the_oracle(vpq, oracle, dev, D, V, n_slabs, s
         assert np.isnan(wk[words:]).all()                     # nothing written past the stated workspace
 
 
+# A thread's entries in flight end (1024, 4096 and one more), slabs past the last entry, slabs in flight of the threshold scan
+# (32, 33 and 1024), the longest slab; logits over so wide a range that the scan walks the upper half of the bins, ties and
+# nothing but one entry kept
+@pytest.mark.parametrize("V,n_slabs", [(1024, 1), (1025, 1), (4096, 1), (4097, 1), (8192, 2), (5000, 32), (20003, 33), (5000, 1024),
+                                       (65535, 1), (100, 60)])
+@pytest.mark.parametrize("kind", ["wide", "ties", "one"])
+def test_histogram_sampler_edges(vpq, oracle, dev, D, V, n_slabs, kind):
+    rng = np.random.default_rng(V + n_slabs)
+    vals = {"wide": -45.0 * rng.random(V), "ties": rng.integers(-4, 4, V) * 0.0, "one": np.where(np.arange(V) == V - 1, 3.0, -np.inf)}[kind]
+    bits = synth.f32_to_bf16_bits(vals.astype(np.float32))
+    seen = (rng.random(V) < 0.1).astype(np.uint8)
+    wt_at = n_slabs + n_slabs * 2049 + 2049
+    for top_p, top_k in ((1.0, 0), (0.9, V - 1), (0.999999, 7)):
+        want, ws_want, seen_want, wt_want = oracle.sample_hist(bits, seen, 1.0, top_p, 9, n_slabs, rep=1.1, top_k=top_k)
+        work = torch.full((vpq.load().vpq_sample_hist_workspace_bytes(n_slabs) // 4,), float("nan"), device=dev)
+        for _ in range(2):                                    # (the second call finds the first one's workspace)
+            seen_d = torch.from_numpy(seen.copy()).to(dev)
+            ws_d = torch.zeros((V,), dtype=torch.bfloat16, device=dev)
+            got = vpq.sample_hist_bf16(D.bf16(bits, dev), seen_d, 1.0, top_p, 9, ws=ws_d, work=work, n_slabs=n_slabs, rep=1.1, top_k=top_k)
+            torch.cuda.synchronize()
+            assert int(got.cpu()[0]) == want
+            assert np.array_equal(D.bits(ws_d), ws_want) and np.array_equal(seen_d.cpu().numpy(), seen_want)
+            assert work[wt_at].item() == np.float32(wt_want)
+
+
 def test_histogram_sampler_rejects_bad_arguments(vpq, dev):
     L = vpq.load()
     buf = torch.zeros(1 << 16, dtype=torch.int32, device=dev)
