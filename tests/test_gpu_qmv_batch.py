@@ -320,3 +320,38 @@ def test_eight_bit_codes_over_a_long_k_gated_grouped_and_in_two_tiles_of_rows(vp
         o.assert_intact()
         assert torch.equal(o.view, many[:, first:first + p[3]])
         first += p[3]
+
+
+# One row (8 bits from K = 2560 on, binary16 where K is no multiple of 512) and two rows of groups of 32: the oracle's sums, the
+# bits of the same rows in a batch of three, a grouped launch the bits of the single ones; chunks in flight end with K
+@pytest.mark.parametrize("fmt,M,K,N", [("w8g64", 1, 2496, 33), ("w8g64", 1, 2560, 33), ("w8g64", 1, 3072, 130), ("w8g64", 1, 9664, 17),
+                                       ("w8g64", 2, 3840, 40), ("w8g64", 7, 3840, 40), ("f16", 1, 64, 3), ("f16", 1, 3840, 130),
+                                       ("w4g32", 2, 96, 5), ("w4g32", 2, 4128, 130), ("w4g32", 1, 4128, 130)])
+def test_one_and_two_rows(vpq, oracle, dev, D, fmt, M, K, N):
+    seed = K + N + M
+    if fmt == "f16":
+        w, s, b = f16_pack(N, K, seed)
+        x = np.random.default_rng(seed).standard_normal((3, K)).astype(np.float16).view(np.uint16)
+        y64, _ = oracle.matmul_f16(w, s, b, x[:M], K, N, M, rounded=False)
+        s, b, xd = (torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).to(dev).view(torch.float16) for a in (s, b, x))
+        run, group = vpq.qmv_w4g64_f16, vpq.qmv_group_w4g64_f16
+    else:
+        w, s, b = (synth.make_weight8 if fmt == "w8g64" else synth.make_weight_g32)(N, K, seed)
+        x = synth.make_act(max(M, 3), K, seed + 1)
+        if fmt == "w8g64":
+            y64, _ = oracle.matmul8(w, s, b, x[:M], K, N, M, rounded=False)
+        else:
+            y64, _ = oracle.qmv_g32(w, s, b, x[:M], K, N, M)
+        s, b, xd = D.bf16(s, dev), D.bf16(b, dev), D.bf16(x, dev)
+        run, group = (vpq.qmv_w8g64, vpq.qmv_group_w8g64) if fmt == "w8g64" else (vpq.qmv_w4g32, vpq.qmv_group_w4g32)
+    w, xm = D.u32(w, dev), xd[:M].contiguous()
+    parity.check_f32(run(w, s, b, xm, K, N, M, f32out=True).cpu().numpy(), y64)
+    out = parity.Guarded((M, N), xd.dtype, dev)
+    run(w, s, b, xm, K, N, M, out=out.view)
+    torch.cuda.synchronize()
+    out.assert_intact()
+    if (fmt, K) != ("w8g64", 2496) and (fmt, M) != ("w4g32", 1):   # (one wavefront per weight row)
+        assert torch.equal(out.view, run(w, s, b, xd[:max(M, 3)], K, N, max(M, 3))[:M])
+    cut = N // 2
+    packs = [tuple(t[i:j].clone() for t in (w, s, b)) + (j - i,) for i, j in ((0, cut), (cut, N))]
+    assert torch.equal(torch.cat(group(packs, xm, K, M), dim=1), out.view)

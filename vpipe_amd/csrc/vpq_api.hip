@@ -82,6 +82,12 @@ int check_pack(const uint32_t* w, const uint16_t* scales, const uint16_t* biases
 // are even on 4096->12288 and the fused kernel is ahead on the N = 4096 shapes).
 constexpr int kDenseRouteMinRows = 8192;
 
+// Rows of x and K from which 8-bit packs run on the batch kernel, below which on one wavefront per weight row.  One row: from the
+// K on from which the batch kernel's error against float64 is the smaller one (fp32 output, 1e-7, K = 2048 / 2560 / 4096 / 12288:
+// 1.02 / 1.13 / 1.36 / 2.20 and 1.05 / 1.12 / 1.17 / 1.51).  us at one row, before / now: 4096 -> 4096 7.7 / 6.8, 12288 -> 4096 18.7 /
+// 13.3, 9664 -> 3840 15.8 / 11.8; q|k|v of 4096 in one launch instead of three 18.1 / 9; 4096 -> 1024 by itself 5.2 / 5.7.
+bool batch_from8(int K, int M) { return M >= 2 || K >= 2560; }
+
 // The batch kernel over one pack.
 hipError_t launch_batch(hipStream_t hs, const vpq::QmvArgs& a, const vpq::BatchFormat& f)
 {
@@ -241,7 +247,7 @@ static int qmv8_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* s
   a.K = K; a.N = N; a.M = M; a.y_f32 = y_f32; a.cu_count = g_dev.cu_count;
   a.gate_act = store;
   const vpq::BatchFormat f{8, 64, false, false};
-  if (M >= 2 && store == 0 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && aligned(biases, 16)) {
+  if (batch_from8(K, M) && store == 0 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && aligned(biases, 16)) {
     return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
   }
   return finish(vpq::launch_qmv_simple8(reinterpret_cast<hipStream_t>(stream), a));
@@ -732,8 +738,10 @@ static int qmv_f16_common(vpq_stream_t stream, const uint32_t* w, const uint16_t
   if (vpq::qmv_flow_supports(K, N, M) && aligned(scales, 16) && aligned(biases, 16)) {
     return finish(vpq::launch_qmv_flow_f16(reinterpret_cast<hipStream_t>(stream), a));
   }
+  // (one row over another K, one wavefront per weight row / now: 3840 -> 19328 17.6 / 13.0 us, 3840 -> 3840 5.8 / 5.1, 9664 -> 3840
+  // 11.3 / 9.4)
   const vpq::BatchFormat f{4, 64, true, false};
-  if (M >= 2 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && aligned(biases, 16)) {
+  if (vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && aligned(biases, 16)) {
     return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
   }
   return finish(vpq::launch_qmv_simple_f16(reinterpret_cast<hipStream_t>(stream), a));
@@ -1443,10 +1451,10 @@ int qmv_g32_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scale
   a.gate_act = gate_act;
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
   if (gelu_mul) { return finish(vpq::launch_qmv_simple_g32(hs, a, scale_only)); }    // the kernel that has this store
-  // up to two rows of x: the row-streaming kernel; more: the batch kernel (4096 -> 12288: 10.5 us at one row, 13.7 at
-  // two, 12.2 at three; two rows on the batch kernel are not measured)
+  // one row of x: the row-streaming kernel; more: the batch kernel (us, rows / batch: one row 4096 -> 24576 16.8 / 17.9, 12288 ->
+  // 4096 9.7 / 11.7; two rows 23.3 / 17.9 and 12.6 / 11.7, 4096 -> 4096 6.9 / 6.0)
   const vpq::BatchFormat f{4, 32, false, scale_only};
-  if (M > 2 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && (scale_only || aligned(biases, 16))) {
+  if (M > 1 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && (scale_only || aligned(biases, 16))) {
     return finish(launch_batch(hs, a, f));
   }
   if (M <= 2) { return finish(vpq::launch_qmv_rows_g32(hs, a, scale_only)); }
@@ -1693,8 +1701,8 @@ int vpq_qmv_group_w4g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
 }
 
 // The fused-QKV GEMV of the format twins (`affine_qmv_qkv_w4g32`, `affine_qmv_qkv_w8g64`,
-// gpu-kernels/metal/quant/affine_qmv.metal:518-559): 1..4 packs that share x.  Group-32 packs at up to two rows of x
-// run as one launch of the row-streaming kernel; otherwise the packs are separate calls, with the same bits.
+// gpu-kernels/metal/quant/affine_qmv.metal:518-559): 1..4 packs that share x, one launch where the kernel of the single
+// call has a grouped form; otherwise the packs are separate calls, with the same bits.
 int vpq_qmv_group_w4g32_bf16(vpq_stream_t stream, int count, const uint32_t* const* w, const uint16_t* const* scales,
                              const uint16_t* const* biases, const uint16_t* x, uint16_t* const* y, int K, const int* N,
                              int M, int scale_only)
@@ -1713,7 +1721,7 @@ int vpq_qmv_group_w4g32_bf16(vpq_stream_t stream, int count, const uint32_t* con
   }
   if (!aligned(x, 16)) { return VPQ_ERR_MISALIGNED; }
   const vpq::BatchFormat f{4, 32, false, scale_only != 0};
-  bool batch = M > 2 && vpq::qmv_batch_supports(K, M, f);
+  bool batch = M > 1 && vpq::qmv_batch_supports(K, M, f);
   for (int i = 0; i < count; ++i) {
     batch = batch && aligned(scales[i], 16) && (scale_only != 0 || aligned(biases[i], 16));
   }
@@ -1743,7 +1751,7 @@ int vpq_qmv_group_w8g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
   if (w == nullptr || scales == nullptr || biases == nullptr || y == nullptr || N == nullptr) { return VPQ_ERR_NULL_POINTER; }
   if (count < 1 || count > 4) { return VPQ_ERR_BAD_SHAPE; }
   const vpq::BatchFormat f{8, 64, false, false};
-  bool batch = M >= 2 && M <= 16 && x != nullptr && aligned(x, 16) && vpq::qmv_batch_supports(K, M, f);
+  bool batch = batch_from8(K, M) && M <= 16 && x != nullptr && aligned(x, 16) && vpq::qmv_batch_supports(K, M, f);
   for (int i = 0; i < count && batch; ++i) {
     batch = check_pack(w[i], scales[i], biases[i], K, N[i]) == VPQ_OK && y[i] != nullptr && aligned(y[i], 2) &&
             aligned(scales[i], 16) && aligned(biases[i], 16);
@@ -1758,7 +1766,7 @@ int vpq_qmv_group_w8g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
     for (int i = 0; i < count; ++i) { g.seg[i] = vpq::QmvSeg{w[i], scales[i], biases[i], y[i], N[i]}; }
     return finish(vpq::launch_qmv_batch(reinterpret_cast<hipStream_t>(stream), a, g, f));
   }
-  // one row, or something to report: the separate calls
+  // one row of a short K, or something to report: the separate calls
   for (int i = 0; i < count; ++i) {
     const int st = vpq_qmv_w8g64_bf16(stream, w[i], scales[i], biases[i], x, y[i], K, N[i], M, nullptr);
     if (st != VPQ_OK) { return st; }
@@ -1806,7 +1814,7 @@ int vpq_qmv_group_w4g64_f16(vpq_stream_t stream, int count, const uint32_t* cons
   if (count < 1 || count > 4) { return VPQ_ERR_BAD_SHAPE; }
   const vpq::BatchFormat f{4, 64, true, false};
   const bool flow = vpq::qmv_flow_supports(K, 1, M);
-  bool one_launch = flow || (M >= 2 && vpq::qmv_batch_supports(K, M, f));
+  bool one_launch = flow || vpq::qmv_batch_supports(K, M, f);
   for (int i = 0; i < count; ++i) {
     int st = check_pack(w[i], scales[i], biases[i], K, N[i]);
     if (st != VPQ_OK) { return st; }

@@ -129,14 +129,15 @@ bool batch_pairs(const BatchPlan& v, int K, const BatchFormat& f)
 // Up to 32 rows of x a workgroup and up to 8 rows of x altogether: two tiles of 16 weight rows share the fetch of x and
 // sum(x); one where the tiles alone do not fill the CUs (us, one / two: 4096 -> 4096 at 2 rows 5.0 / 5.9; 12288 -> 4096 9.6 /
 // 11.7; 5120 -> 17408 19.8 / 17.7; 4096 -> 24576 16.9 / 14.6).  8 bits, one workgroup per CU, a long K: several chunks in
-// flight (12288 -> 4096 at 4 / 6 rows 16.4 / 15.8 -> 13.1 / 14.4; 4096 -> 4096 7.4 -> 6.9 at 4 rows, 12 rows 8.05 -> 8.5; 4
-// bits: 11.2 -> 11.8 at 12288, 4 rows).
+// flight (12288 -> 4096 at 4 / 6 rows 16.4 / 15.8 -> 13.1 / 14.4; 4 rows: 2560 -> 2560 5.1 -> 5.25, 3072 -> 3072 level, 4096 ->
+// 1024 / 4096 6.0 / 7.3 -> 5.7 / 6.8, 5120 -> 4096 8.4 -> 7.7; 7 rows: 3072 -> 3072 and 4096 -> 1024 level, 3840 -> 3840 6.7 ->
+// 6.6, 4096 -> 4096 7.5 -> 7.3, 5120 -> 1280 7.1 -> 6.9; 12 rows: 4096 -> 4096 8.05 -> 8.5; 4 bits: 11.2 -> 11.8 at 12288, 4 rows).
 BatchPlan batch_plan_few(const QmvGroup& g, int K, int M, const BatchFormat& f, int cus)
 {
   const int m_tiles = (M + 31) / 32, mr = batch_mr((M + m_tiles - 1) / m_tiles);
   const bool narrow = batch_blocks(g, 1) * m_tiles <= cus;
   const BatchPlan deep{1, mr, m_tiles, mr == 1 ? 3 : 2};
-  if (f.bits == 8 && narrow && K >= (mr == 4 ? 7680 : 6144) && batch_fits(deep, K, f)) { return deep; }
+  if (f.bits == 8 && narrow && K >= (mr == 1 ? 3072 : mr == 2 ? 3840 : 7680) && batch_fits(deep, K, f)) { return deep; }
   return BatchPlan{narrow || !batch_fits(BatchPlan{2, mr, m_tiles, 1}, K, f) ? 1 : 2, mr, m_tiles, 1};
 }
 
