@@ -141,7 +141,7 @@ enum {
   VPQ_QMV_STREAM = 4,      /* M <= 4: persistent workgroups, x staged in LDS, prefetched items */
   VPQ_QMV_RING = 5,        /* x in registers across a workgroup's tiles, codes through a two-slot LDS ring per wavefront */
   VPQ_QMV_ROWS = 6,        /* M <= 2, any K % 64: a wavefront streams whole rows with full-width loads, packed bf16
-                              dot products, no LDS; what AUTO takes for M = 1 where K is not a multiple of 512 */
+                              dot products, no LDS; what AUTO takes for M = 1 where K < 2048 is not a multiple of 512 */
   VPQ_QMV_FLOW = 7,        /* M = 1, K % 512 == 0, K >= 2048: one wavefront per (row set, K part), every load of the
                               launch requested up front, x in registers, scales / biases staged in LDS; what AUTO
                               takes for M = 1 */

@@ -322,10 +322,10 @@ def test_eight_bit_codes_over_a_long_k_gated_grouped_and_in_two_tiles_of_rows(vp
         first += p[3]
 
 
-# One row (8 bits from K = 2560 on, binary16 where K is no multiple of 512) and two rows of groups of 32: the oracle's sums, the
+# One row (8 bits from K = 2560 on, binary16 below K = 2048) and two rows of groups of 32: the oracle's sums, the
 # bits of the same rows in a batch of three, a grouped launch the bits of the single ones; chunks in flight end with K
 @pytest.mark.parametrize("fmt,M,K,N", [("w8g64", 1, 2496, 33), ("w8g64", 1, 2560, 33), ("w8g64", 1, 3072, 130), ("w8g64", 1, 9664, 17),
-                                       ("w8g64", 2, 3840, 40), ("w8g64", 7, 3840, 40), ("f16", 1, 64, 3), ("f16", 1, 3840, 130),
+                                       ("w8g64", 2, 3840, 40), ("w8g64", 7, 3840, 40), ("f16", 1, 64, 3), ("f16", 1, 1088, 130),
                                        ("w4g32", 2, 96, 5), ("w4g32", 2, 4128, 130), ("w4g32", 1, 4128, 130)])
 def test_one_and_two_rows(vpq, oracle, dev, D, fmt, M, K, N):
     seed = K + N + M
@@ -350,8 +350,57 @@ def test_one_and_two_rows(vpq, oracle, dev, D, fmt, M, K, N):
     run(w, s, b, xm, K, N, M, out=out.view)
     torch.cuda.synchronize()
     out.assert_intact()
-    if (fmt, K) != ("w8g64", 2496) and (fmt, M) != ("w4g32", 1):   # (one wavefront per weight row)
+    if (fmt, K) != ("w8g64", 2496) and (fmt, M) != ("w4g32", 1):   # (kernels of one row)
         assert torch.equal(out.view, run(w, s, b, xd[:max(M, 3)], K, N, max(M, 3))[:M])
     cut = N // 2
     packs = [tuple(t[i:j].clone() for t in (w, s, b)) + (j - i,) for i, j in ((0, cut), (cut, N))]
     assert torch.equal(torch.cat(group(packs, xm, K, M), dim=1), out.view)
+
+
+# One row, scales and biases by 2-byte loads: K one group past a slice of 2048, odd counts of groups, one to four parts of K and
+# the last K that is taken, N that ends inside a wavefront's rows; plain, with a residual, gated, and grouped
+@pytest.mark.parametrize("fmt,N,K", [(f, n, k) for f, n in (("w4g64", 1), ("w4g64", 6), ("w4g32", 3), ("w4g32", 34), ("f16", 10),
+                                                            ("w4g64", 2050))
+                                     for k in (2080, 2112, 3840, 6080, 6208, 17344, 25024, 32704) if k % 64 == 0 or f == "w4g32"])
+def test_one_row_with_narrow_scales(vpq, oracle, dev, D, fmt, N, K):
+    seed = K + N
+    if fmt == "f16":
+        w, s, b = f16_pack(N, K, seed)
+        x = np.random.default_rng(seed).standard_normal((1, K)).astype(np.float16).view(np.uint16)
+        y64, _ = oracle.matmul_f16(w, s, b, x, K, N, 1, rounded=False)
+        s, b, x = (torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).to(dev).view(torch.float16) for a in (s, b, x))
+        run, group = vpq.qmv_w4g64_f16, vpq.qmv_group_w4g64_f16
+    else:
+        w, s, b = (synth.make_weight if fmt == "w4g64" else synth.make_weight_g32)(N, K, seed)
+        x = synth.make_act(1, K, seed + 1)
+        y64, _ = (oracle.qmv if fmt == "w4g64" else oracle.qmv_g32)(w, s, b, x, K, N, 1)
+        s, b, x = D.bf16(s, dev), D.bf16(b, dev), D.bf16(x, dev)
+        run, group = (vpq.qmv_w4g64, vpq.qmv_group_w4g64) if fmt == "w4g64" else (vpq.qmv_w4g32, vpq.qmv_group_w4g32)
+    w = D.u32(w, dev)
+    f = run(w, s, b, x, K, N, 1, f32out=True)
+    parity.check_f32(f.cpu().numpy(), y64)
+    res = torch.randn((1, N), device=dev).to(x.dtype)
+    out, added = parity.Guarded((1, N), x.dtype, dev), parity.Guarded((1, N), x.dtype, dev)
+    run(w, s, b, x, K, N, 1, out=out.view)
+    run(w, s, b, x, K, N, 1, out=added.view, residual=res)
+    torch.cuda.synchronize()
+    out.assert_intact()
+    added.assert_intact()
+    assert torch.equal(out.view, f.to(x.dtype))
+    assert torch.equal(added.view, (out.view.float() + res.float()).to(x.dtype))
+    if N % 2 == 0:
+        gated = parity.Guarded((1, N // 2), x.dtype, dev)
+        if fmt == "w4g64":
+            vpq.qmv_swiglu_w4g64(w, s, b, x, K, N, 1, out=gated.view)
+        else:
+            run(w, s, b, x, K, N, 1, out=gated.view, activation=1)
+        torch.cuda.synchronize()
+        gated.assert_intact()
+        g, u = f.double()[:, 0::2], f.double()[:, 1::2]
+        want = g / (1 + torch.exp(-g)) * u
+        # the result's own rounding (2^-8 bounds it for both elements) and a few steps of fp32 in the activation
+        assert ((gated.view.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-6).all()
+    if N > 1:
+        cuts = sorted({0, N // 3, N // 2, N})
+        packs = [tuple(t[i:j].clone() for t in (w, s, b)) + (j - i,) for i, j in zip(cuts, cuts[1:])]
+        assert torch.equal(torch.cat(group(packs, x, K, 1), dim=1), out.view)

@@ -88,6 +88,12 @@ constexpr int kDenseRouteMinRows = 8192;
 // 13.3, 9664 -> 3840 15.8 / 11.8; q|k|v of 4096 in one launch instead of three 18.1 / 9; 4096 -> 1024 by itself 5.2 / 5.7.
 bool batch_from8(int K, int M) { return M >= 2 || K >= 2560; }
 
+// One row of binary16 whose scales are no whole 16-byte pieces: the one-row kernel from the K on from which its error against
+// float64 is no larger than that of one wavefront per weight row, which ran these (fp32 output, 1e-7, K = 2112 / 3840 / 9664: 1.36 /
+// 1.34 / 1.32 and 1.20 / 1.51 / 2.27; the batch kernel, which takes what is shorter: 0.83 / 0.91 / 1.07).  us, one wavefront per row
+// / batch kernel / now: 3840 -> 3840 5.8 / 5.1 / 3.9, 3840 -> 19328 17.4 / 13.0 / 10.5, 9664 -> 3840 11.3 / 9.4 / 7.8.
+bool flow_narrow_f16(int K, int N, int M) { return K >= 3072 && (K % 512) != 0 && vpq::qmv_flow_narrow_supports(K, N, M, 64); }
+
 // The batch kernel over one pack.
 hipError_t launch_batch(hipStream_t hs, const vpq::QmvArgs& a, const vpq::BatchFormat& f)
 {
@@ -160,7 +166,8 @@ int qmv_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
   // One row of x: the streaming kernel that requests the whole pack up front (measured, this / the batch kernel at one
   // row, us: 4096 -> 4096 3.9 / 5.1, 12288 -> 4096 8.0 / 9.5, 4096 -> 24576 12.5 / 14.3, 5120 -> 151936 75 / 89).
   if (flow_ok) { return finish(vpq::launch_qmv_flow(hs, a)); }
-  // One row over a K that is not a multiple of 512: the row-streaming kernel.
+  // One row over another K: its form with narrow scales, and for a short K the row-streaming kernel.
+  if ((K % 512) != 0 && vpq::qmv_flow_narrow_supports(K, N, M, 64)) { return finish(vpq::launch_qmv_flow_narrow(hs, a, 64)); }
   if (M == 1 && (K % 512) != 0) { return finish(vpq::launch_qmv_rows(hs, a, 0)); }
   if (batch_ok) { return finish(launch_batch(hs, a, vpq::BatchFormat{})); }
   // A K too deep for the batch kernel's LDS (above 114176), or scales or biases off 16-byte alignment.
@@ -738,8 +745,7 @@ static int qmv_f16_common(vpq_stream_t stream, const uint32_t* w, const uint16_t
   if (vpq::qmv_flow_supports(K, N, M) && aligned(scales, 16) && aligned(biases, 16)) {
     return finish(vpq::launch_qmv_flow_f16(reinterpret_cast<hipStream_t>(stream), a));
   }
-  // (one row over another K, one wavefront per weight row / now: 3840 -> 19328 17.6 / 13.0 us, 3840 -> 3840 5.8 / 5.1, 9664 -> 3840
-  // 11.3 / 9.4)
+  if (flow_narrow_f16(K, N, M)) { return finish(vpq::launch_qmv_flow_narrow(reinterpret_cast<hipStream_t>(stream), a, 64, true)); }
   const vpq::BatchFormat f{4, 64, true, false};
   if (vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && aligned(biases, 16)) {
     return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
@@ -1451,12 +1457,14 @@ int qmv_g32_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scale
   a.gate_act = gate_act;
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
   if (gelu_mul) { return finish(vpq::launch_qmv_simple_g32(hs, a, scale_only)); }    // the kernel that has this store
-  // one row of x: the row-streaming kernel; more: the batch kernel (us, rows / batch: one row 4096 -> 24576 16.8 / 17.9, 12288 ->
-  // 4096 9.7 / 11.7; two rows 23.3 / 17.9 and 12.6 / 11.7, 4096 -> 4096 6.9 / 6.0)
+  // one row of x: the one-row kernel, or for a short K (and Q4_0) the row-streaming one; more: the batch kernel (us, row-streaming /
+  // batch / one-row: one row 4096 -> 24576 16.9 / 17.9 / 13.8, 12288 -> 4096 9.7 / 11.7 / 9.1, 4096 -> 4096 5.8 / 6.0 / 4.2; two rows
+  // 23.3 / 17.9, 12.6 / 11.7 and 6.9 / 6.0)
   const vpq::BatchFormat f{4, 32, false, scale_only};
   if (M > 1 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && (scale_only || aligned(biases, 16))) {
     return finish(launch_batch(hs, a, f));
   }
+  if (!scale_only && vpq::qmv_flow_narrow_supports(K, N, M, 32)) { return finish(vpq::launch_qmv_flow_narrow(hs, a, 32)); }
   if (M <= 2) { return finish(vpq::launch_qmv_rows_g32(hs, a, scale_only)); }
   return finish(vpq::launch_qmv_simple_g32(hs, a, scale_only));
 }
@@ -1678,8 +1686,9 @@ int vpq_qmv_group_w4g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
   // The kernels of the single call (qmv_common), each in its grouped form.
   const bool batch = wide && vpq::qmv_batch_supports(K, M, vpq::BatchFormat{});
   const bool flow = batch && vpq::qmv_flow_supports(K, 1, M);
-  const bool rows = vpq::qmv_rows_supports(K, 1, M) && (!wide || (K % 512) != 0) && (!batch || M == 1);
-  if (!flow && !rows && !batch) {
+  const bool narrow = (K % 512) != 0 && vpq::qmv_flow_narrow_supports(K, 1, M, 64);
+  const bool rows = !narrow && vpq::qmv_rows_supports(K, 1, M) && (!wide || (K % 512) != 0) && (!batch || M == 1);
+  if (!flow && !narrow && !rows && !batch) {
     for (int i = 0; i < count; ++i) {
       const int st = vpq_qmv_w4g64_bf16(stream, w[i], scales[i], biases[i], x, y[i], K, N[i], M, nullptr, nullptr, 0,
                                         VPQ_QMV_AUTO);
@@ -1696,6 +1705,7 @@ int vpq_qmv_group_w4g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
   for (int i = 0; i < count; ++i) { g.seg[i] = vpq::QmvSeg{w[i], scales[i], biases[i], y[i], N[i]}; }
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
   if (flow) { return finish(vpq::launch_qmv_flow_group(hs, a, g)); }
+  if (narrow) { return finish(vpq::launch_qmv_flow_narrow_group(hs, a, g, 64)); }
   if (rows) { return finish(vpq::launch_qmv_rows_group(hs, a, g)); }
   return finish(vpq::launch_qmv_batch(hs, a, g, vpq::BatchFormat{}));
 }
@@ -1741,6 +1751,9 @@ int vpq_qmv_group_w4g32_bf16(vpq_stream_t stream, int count, const uint32_t* con
   g.count = count;
   for (int i = 0; i < count; ++i) { g.seg[i] = vpq::QmvSeg{w[i], scales[i], scale_only ? nullptr : biases[i], y[i], N[i]}; }
   if (batch) { return finish(vpq::launch_qmv_batch(reinterpret_cast<hipStream_t>(stream), a, g, f)); }
+  if (scale_only == 0 && vpq::qmv_flow_narrow_supports(K, 1, M, 32)) {
+    return finish(vpq::launch_qmv_flow_narrow_group(reinterpret_cast<hipStream_t>(stream), a, g, 32));
+  }
   return finish(vpq::launch_qmv_rows_group(reinterpret_cast<hipStream_t>(stream), a, g, 32, scale_only != 0));
 }
 
@@ -1813,6 +1826,7 @@ int vpq_qmv_group_w4g64_f16(vpq_stream_t stream, int count, const uint32_t* cons
   if (w == nullptr || scales == nullptr || biases == nullptr || y == nullptr || N == nullptr) { return VPQ_ERR_NULL_POINTER; }
   if (count < 1 || count > 4) { return VPQ_ERR_BAD_SHAPE; }
   const vpq::BatchFormat f{4, 64, true, false};
+  const bool narrow = flow_narrow_f16(K, 1, M);
   const bool flow = vpq::qmv_flow_supports(K, 1, M);
   bool one_launch = flow || vpq::qmv_batch_supports(K, M, f);
   for (int i = 0; i < count; ++i) {
@@ -1825,7 +1839,7 @@ int vpq_qmv_group_w4g64_f16(vpq_stream_t stream, int count, const uint32_t* cons
   if (x == nullptr) { return VPQ_ERR_NULL_POINTER; }
   if (M < 1 || M > 16) { return VPQ_ERR_BAD_SHAPE; }
   if (!aligned(x, 16)) { return VPQ_ERR_MISALIGNED; }
-  if (!one_launch) {
+  if (!one_launch && !narrow) {
     for (int i = 0; i < count; ++i) {
       const int st = vpq_qmv_w4g64_f16(stream, w[i], scales[i], biases[i], x, y[i], K, N[i], M, nullptr);
       if (st != VPQ_OK) { return st; }
@@ -1840,6 +1854,7 @@ int vpq_qmv_group_w4g64_f16(vpq_stream_t stream, int count, const uint32_t* cons
   g.count = count;
   for (int i = 0; i < count; ++i) { g.seg[i] = vpq::QmvSeg{w[i], scales[i], biases[i], y[i], N[i]}; }
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+  if (narrow) { return finish(vpq::launch_qmv_flow_narrow_group(hs, a, g, 64, true)); }
   return finish(flow ? vpq::launch_qmv_flow_group(hs, a, g, true) : vpq::launch_qmv_batch(hs, a, g, f));
 }
 

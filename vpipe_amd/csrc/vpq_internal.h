@@ -188,6 +188,10 @@ bool qmv_flow_supports(int K, int N, int M);
 hipError_t launch_qmv_flow(hipStream_t st, const QmvArgs& a);
 hipError_t launch_qmv_flow_f16(hipStream_t st, const QmvArgs& a);    // IEEE binary16 elements
 hipError_t launch_qmv_flow_group(hipStream_t st, const QmvArgs& a, const QmvGroup& g, bool f16 = false);
+// ... where a row's scales are no whole number of 16-byte pieces, or belong to groups of 32.
+bool qmv_flow_narrow_supports(int K, int N, int M, int group);
+hipError_t launch_qmv_flow_narrow(hipStream_t st, const QmvArgs& a, int group, bool f16 = false);
+hipError_t launch_qmv_flow_narrow_group(hipStream_t st, const QmvArgs& a, const QmvGroup& g, int group, bool f16 = false);
 bool qmv_stream_supports(int K, int N, int M);
 hipError_t launch_qmv_stream(hipStream_t st, const QmvArgs& a);
 bool qmv_ring_supports(int K, int N, int M);

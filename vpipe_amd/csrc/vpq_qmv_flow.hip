@@ -16,7 +16,9 @@
 //   2. the codes, RB * SPW loads of 16 bytes per lane, as soon as their addresses are known:
 //      the time to the first code request is paid by every wavefront of the launch;
 //   3. scales and biases of the wavefront's rows and K range: 16-byte direct-to-LDS loads
-//      (1 KB per instruction, scales and biases in the same instruction where they fit).  They
+//      (1 KB per instruction, scales and biases in the same instruction where they fit), or, where
+//      a row of them is no whole number of 16-byte pieces (K that is no multiple of 512; groups of
+//      32 as well), one 2-byte register load of each per lane, row and slice.  They
 //      are applied to the per-(row, slice) dot products at the end.
 // The loads are inline assembly so that the only waits are the counted ones written here: the
 // compiler would otherwise wait for every outstanding load before the first LDS read.
@@ -78,6 +80,14 @@ __device__ __forceinline__ u32x4v gload16(const void* base, uint32_t voff)
   return r;
 }
 
+// The same with 2 bytes per lane.
+__device__ __forceinline__ uint32_t gload2(const void* base, uint32_t voff)
+{
+  uint32_t r;
+  asm volatile("global_load_ushort %0, %1, %2" : "=&v"(r) : "v"(voff), "s"(base) : "memory");
+  return r;
+}
+
 // 16 bytes per lane, global -> LDS at lds_dst + 16 * lane.  The LDS base travels in M0, bound as an operand: the
 // compiler writes it and knows its value (the s_nop is the wait state between that write and the load).
 __device__ __forceinline__ void dma16(uint32_t lds_dst, const void* src)
@@ -101,6 +111,7 @@ __device__ __forceinline__ void wait_vm_after(float& dep)
 }
 
 __device__ __forceinline__ void touch(u32x4v& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void touch(uint32_t& v) { asm volatile("" : "+v"(v)); }
 
 // Total over the 64 lanes, valid in lane 63.
 __device__ __forceinline__ float wave_total_l63(float v)
@@ -169,15 +180,21 @@ __device__ __forceinline__ void pin_scalar(const T& v) { asm volatile("" : : "s"
 // F16: the elements (x, scales, biases, y, residual) are IEEE binary16 instead of bf16 (the reference's
 // VPIPE_ELT = half build).  The codes then become binary16 pairs 16 + q (the code shifted to mantissa bits 6..9,
 // exact; 1024 + q with the code left in bits 0..3 would cost eight times bf16's cancellation noise).
+// NARROW: 0, or log2 of the group (6, 5) where scales and biases come by 2-byte loads; any K of whole groups.  The sum is then
+// formed as s * (dot - 128 sx) + b * sx, as in the kernel of one wavefront per weight row that ran these K before: the
+// uncancelled 128 s sx adds up over K otherwise (error of the fp32 result 4 to 5e-7, 9e-7 with the other form).
+// Measured (us, that kernel / now): groups of 64, 3840 -> 3840 5.5 / 4.0, 3840 -> 19328 13.6 / 10.7, 9664 -> 3840 8.3 / 7.9; groups of
+// 32, 4096 -> 4096 5.8 / 4.2, 4096 -> 24576 17.0 / 13.8, 12288 -> 4096 9.7 / 9.1.  Where 16-byte pieces fit, both forms are level up to
+// K = 6144, and the pieces 4 to 6 % faster above (12288 -> 4096 8.6 / 8.9).
 // PRELOADED: the arguments are already in scalar registers (nothing to batch; the residual is left to be loaded
 // when the store needs it).
-template <int SPW, int RB, bool F32OUT, int C, bool F16 = false, bool PRELOADED = false>
+template <int SPW, int RB, bool F32OUT, int C, bool F16 = false, bool PRELOADED = false, int NARROW = 0>
 __device__ __forceinline__ void qmv_flow_body(const FlowParams<C>& p)
 {
   constexpr int NL = RB * SPW;                 // code loads of a wavefront
   constexpr int PPR = SPW * 4;                 // 16-byte pieces of scales (or biases) per row and K part
   constexpr int P = RB * PPR;
-  constexpr int NDMA = (2 * P + 63) / 64;
+  constexpr int NDMA = NARROW ? 0 : (2 * P + 63) / 64;
   // LDS: x of the workgroup's K range (wk * SPW slices of 4 KB), one window of scales/biases per wavefront, the
   // row sums of the K parts.
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -226,7 +243,7 @@ __device__ __forceinline__ void qmv_flow_body(const FlowParams<C>& p)
 
   const int rs = (int)((shape >> (3 * wave)) & 7u), part = wave - rs * wk;
   const int W = wk * wr;
-  const int Kg = K >> 6;
+  const int Kg = K >> (NARROW ? NARROW : 6);
   const int row_begin = ((blk - first_block) * wr + rs) * RB;
   const bool active = row_begin < N;           // wave-uniform
   const int slice0 = part * SPW;
@@ -289,8 +306,9 @@ __device__ __forceinline__ void qmv_flow_body(const FlowParams<C>& p)
   float tot[RB];
 
   // codes
-  constexpr int AFTER = NDMA;                  // requests that follow the codes
+  constexpr int AFTER = NARROW ? 2 * NL : NDMA;   // requests that follow the codes
   u32x4v c[RB][SPW];
+  uint32_t sreg[NARROW ? RB : 1][SPW], breg[NARROW ? RB : 1][SPW];
   {
     const uint8_t* wbase = reinterpret_cast<const uint8_t*>(wq) + (size_t)row_begin * (size_t)(K >> 1);
 #pragma unroll
@@ -303,7 +321,22 @@ __device__ __forceinline__ void qmv_flow_body(const FlowParams<C>& p)
         c[r][s] = gload16(wrow, koff);
       }
     }
-    request_scales_biases();
+    if constexpr (NARROW) {
+      static_for<0, RB>([&](auto rc) {
+        constexpr int r = decltype(rc)::value;
+        const int rr = (row_begin + r < N) ? r : (N - 1 - row_begin);
+        const uint16_t* srow = sq + (size_t)(row_begin + rr) * Kg;
+        const uint16_t* brow = bq + (size_t)(row_begin + rr) * Kg;
+        static_for<0, SPW>([&](auto sc_) {
+          constexpr int s = decltype(sc_)::value;
+          const uint32_t at = kvalid[s] ? (uint32_t)(((slice0 + s) * kSlice + lane * 32) >> NARROW) * 2u : 0u;
+          sreg[r][s] = gload2(srow, at);
+          breg[r][s] = gload2(brow, at);
+        });
+      });
+    } else {
+      request_scales_biases();
+    }
     wait_vm<NL + AFTER>();                       // this wavefront's share of x has landed
   }
   __syncthreads();                               // ... and everybody else's share
@@ -361,6 +394,19 @@ __device__ __forceinline__ void qmv_flow_body(const FlowParams<C>& p)
     });
     wait_vm_after<0>(chain);
     float acc[RB];
+    if constexpr (NARROW) {
+      static_for<0, RB>([&](auto rc) {
+        constexpr int r = decltype(rc)::value;
+        acc[r] = 0.0f;
+        static_for<0, SPW>([&](auto sc_) {
+          constexpr int s = decltype(sc_)::value;
+          touch(sreg[r][s]);
+          touch(breg[r][s]);
+          acc[r] = fmaf(elt_bits_to_f32<F16>(sreg[r][s]), fmaf(kOffset, sx[s], dots[r][s]), acc[r]);
+          acc[r] = fmaf(elt_bits_to_f32<F16>(breg[r][s]), sx[s], acc[r]);
+        });
+      });
+    } else {
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
       acc[r] = 0.0f;
@@ -372,6 +418,7 @@ __device__ __forceinline__ void qmv_flow_body(const FlowParams<C>& p)
         acc[r] = fmaf(sc, dots[r][s], acc[r]);
         acc[r] = fmaf(fmaf(kOffset, sc, bi), sx[s], acc[r]);
       }
+    }
     }
 #pragma unroll
     for (int r = 0; r < RB; ++r) { tot[r] = wave_total_l63(acc[r]); }
@@ -436,7 +483,7 @@ __device__ __forceinline__ void qmv_flow_body(const FlowParams<C>& p)
 // kernel-argument preloading, which delivers the first sixteen words in scalar registers when a wavefront starts,
 // so a wavefront's first requests do not wait for a load of the argument buffer (an aggregate argument is not
 // preloaded).
-template <int SPW, int RB, bool F32OUT, bool F16 = false>
+template <int SPW, int RB, bool F32OUT, bool F16, int NARROW>
 __global__ __launch_bounds__(64 * kMaxWavesPerWg) void qmv_flow_kernel_1(
     const uint16_t* x, const uint32_t* w, const uint16_t* scales, const uint16_t* biases, void* y, int K, uint32_t shape,
     int N, const uint16_t* residual)
@@ -446,7 +493,7 @@ __global__ __launch_bounds__(64 * kMaxWavesPerWg) void qmv_flow_kernel_1(
   FlowParams<1> p;
   p.h.x = x; p.h.residual = residual; p.h.K = K; p.h.shape = shape;
   p.w[0] = w; p.scales[0] = scales; p.biases[0] = biases; p.y[0] = y; p.N[0] = N; p.first_block[0] = 0;
-  qmv_flow_body<SPW, RB, F32OUT, 1, F16, true>(p);
+  qmv_flow_body<SPW, RB, F32OUT, 1, F16, true, NARROW>(p);
 }
 
 // The grouped form (2..4 packs sharing x) with preloaded arguments: the fourteen preloaded words hold what every
@@ -462,7 +509,7 @@ struct FlowRest {
   int N[C - 1];
 };
 
-template <int SPW, int RB, bool F32OUT, int C, bool F16 = false>
+template <int SPW, int RB, bool F32OUT, int C, bool F16, int NARROW>
 __global__ __launch_bounds__(64 * kMaxWavesPerWg) void qmv_flow_kernel_g(
     const uint16_t* x, int K, uint32_t shape, int N0, int fb1, int fb2, int fb3, const uint32_t* w0,
     const uint16_t* scales0, const uint16_t* biases0, const FlowRest<C> rest)
@@ -476,7 +523,7 @@ __global__ __launch_bounds__(64 * kMaxWavesPerWg) void qmv_flow_kernel_g(
     p.w[i] = rest.w[i - 1]; p.scales[i] = rest.scales[i - 1]; p.biases[i] = rest.biases[i - 1]; p.y[i] = rest.y[i - 1];
     p.N[i] = rest.N[i - 1]; p.first_block[i] = fb[i - 1];
   }
-  qmv_flow_body<SPW, RB, F32OUT, C, F16, true>(p);
+  qmv_flow_body<SPW, RB, F32OUT, C, F16, true, NARROW>(p);
 }
 
 namespace {
@@ -484,6 +531,8 @@ namespace {
 struct FlowPlan {
   int spw, wk, wr, rb;
 };
+// Elements, and how scales and biases come (qmv_flow_body's NARROW).
+enum class FlowForm { kWide, kF16, kNarrow64, kNarrow32, kNarrowF16 };
 
 // Slices per wavefront and K parts, from measurements on MI355X with HBM-cold packs: up to three slices (K <= 6144)
 // a wavefront walks the whole K; longer rows are split between 2 to 4 wavefronts of the workgroup (12288->4096:
@@ -513,13 +562,13 @@ FlowPlan flow_plan(int K, double pack_bytes)
   return pl;
 }
 
-template <int S, int R, bool F32, int C, bool F16 = false>
+template <int S, int R, bool F32, int C, bool F16, int NARROW>
 hipError_t launch_flow_kernel(dim3 grid, dim3 block, size_t lds_bytes, hipStream_t st, const FlowParams<C>& p)
 {
   static std::once_flag once;          // one per instantiation
   static hipError_t attr_status = hipSuccess;
   if constexpr (C == 1) {
-    const auto kern = qmv_flow_kernel_1<S, R, F32, F16>;
+    const auto kern = qmv_flow_kernel_1<S, R, F32, F16, NARROW>;
     std::call_once(once, [&] {
       attr_status = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                         kMaxLdsBytes);
@@ -529,7 +578,7 @@ hipError_t launch_flow_kernel(dim3 grid, dim3 block, size_t lds_bytes, hipStream
                          p.h.shape, p.N[0], p.h.residual);
   } else {
     // a grouped launch has no residual
-    const auto kern = qmv_flow_kernel_g<S, R, F32, C, F16>;
+    const auto kern = qmv_flow_kernel_g<S, R, F32, C, F16, NARROW>;
     std::call_once(once, [&] {
       attr_status = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                         kMaxLdsBytes);
@@ -551,7 +600,7 @@ hipError_t launch_flow_kernel(dim3 grid, dim3 block, size_t lds_bytes, hipStream
 
 template <int C>
 hipError_t dispatch_flow(const FlowPlan& pl, bool y_f32, const FlowHead& h, const FlowSeg* segs, int rows_per_block,
-                         dim3 block, size_t lds_bytes, hipStream_t st, bool f16)
+                         dim3 block, size_t lds_bytes, hipStream_t st, FlowForm form)
 {
   FlowParams<C> p;
   p.h = h;
@@ -564,16 +613,23 @@ hipError_t dispatch_flow(const FlowPlan& pl, bool y_f32, const FlowHead& h, cons
   const dim3 grid((unsigned)blocks);
   // grouped launches store the element type
   if (C > 1 && y_f32) { return hipErrorInvalidValue; }
+  const auto launch = [&](auto s_c, auto r_c, auto f32_c) {
+    constexpr int S = decltype(s_c)::value, R = decltype(r_c)::value;
+    constexpr bool kF32 = decltype(f32_c)::value;
+    if (form == FlowForm::kF16) { return launch_flow_kernel<S, R, kF32, C, true, 0>(grid, block, lds_bytes, st, p); }
+    if (form == FlowForm::kNarrow64) { return launch_flow_kernel<S, R, kF32, C, false, 6>(grid, block, lds_bytes, st, p); }
+    if (form == FlowForm::kNarrow32) { return launch_flow_kernel<S, R, kF32, C, false, 5>(grid, block, lds_bytes, st, p); }
+    if (form == FlowForm::kNarrowF16) { return launch_flow_kernel<S, R, kF32, C, true, 6>(grid, block, lds_bytes, st, p); }
+    return launch_flow_kernel<S, R, kF32, C, false, 0>(grid, block, lds_bytes, st, p);
+  };
 #define VPQ_FLOW(S, R)                                                                                    \
   if (pl.spw == S && pl.rb == R) {                                                                        \
+    const std::integral_constant<int, S> s_c{};                                                           \
+    const std::integral_constant<int, R> r_c{};                                                           \
     if constexpr (C == 1) {                                                                               \
-      if (y_f32) {                                                                                        \
-        return f16 ? launch_flow_kernel<S, R, true, 1, true>(grid, block, lds_bytes, st, p)               \
-                   : launch_flow_kernel<S, R, true, 1, false>(grid, block, lds_bytes, st, p);             \
-      }                                                                                                   \
+      if (y_f32) { return launch(s_c, r_c, std::true_type()); }                                           \
     }                                                                                                     \
-    return f16 ? launch_flow_kernel<S, R, false, C, true>(grid, block, lds_bytes, st, p)                  \
-               : launch_flow_kernel<S, R, false, C, false>(grid, block, lds_bytes, st, p);                \
+    return launch(s_c, r_c, std::false_type());                                                           \
   }
   // every (slices per wavefront, rows per wavefront) that flow_plan can return
   VPQ_FLOW(1, 2) VPQ_FLOW(2, 2) VPQ_FLOW(3, 2) VPQ_FLOW(4, 2)
@@ -584,7 +640,7 @@ hipError_t dispatch_flow(const FlowPlan& pl, bool y_f32, const FlowHead& h, cons
 
 // segs[0 .. count): the packs; count == 1 takes the one-line argument form.
 hipError_t launch_flow(hipStream_t st, const FlowSeg* segs, int count, const QmvArgs& a, double pack_bytes,
-                       bool f16 = false)
+                       FlowForm form)
 {
   const FlowPlan pl = flow_plan(a.K, pack_bytes);
   if (pl.spw == 0 || pl.wk < 1 || pl.wk > 4 || pl.wr < 1 || pl.wk * pl.wr > kMaxWavesPerWg ||
@@ -599,16 +655,17 @@ hipError_t launch_flow(hipStream_t st, const FlowSeg* segs, int count, const Qmv
   for (int wv = 0; wv < pl.wk * pl.wr; ++wv) { h.shape |= (uint32_t)(wv / pl.wk) << (3 * wv); }
   const int rows_per_block = pl.wr * pl.rb;
   const int W = pl.wk * pl.wr;
-  const int ndma = (2 * pl.rb * pl.spw * 4 + 63) / 64;
+  const bool windows = form == FlowForm::kWide || form == FlowForm::kF16;
+  const int ndma = windows ? (2 * pl.rb * pl.spw * 4 + 63) / 64 : 0;
   const size_t lds_bytes = (size_t)pl.wk * pl.spw * (kSlice * 2) + (size_t)W * ndma * 1024 +
                            (size_t)W * pl.rb * sizeof(float);
   if (lds_bytes > (size_t)kMaxLdsBytes) { return hipErrorInvalidValue; }
   const dim3 block((unsigned)(64 * W));
   switch (count) {
-    case 1: return dispatch_flow<1>(pl, a.y_f32, h, segs, rows_per_block, block, lds_bytes, st, f16);
-    case 2: return dispatch_flow<2>(pl, a.y_f32, h, segs, rows_per_block, block, lds_bytes, st, f16);
-    case 3: return dispatch_flow<3>(pl, a.y_f32, h, segs, rows_per_block, block, lds_bytes, st, f16);
-    case 4: return dispatch_flow<4>(pl, a.y_f32, h, segs, rows_per_block, block, lds_bytes, st, f16);
+    case 1: return dispatch_flow<1>(pl, a.y_f32, h, segs, rows_per_block, block, lds_bytes, st, form);
+    case 2: return dispatch_flow<2>(pl, a.y_f32, h, segs, rows_per_block, block, lds_bytes, st, form);
+    case 3: return dispatch_flow<3>(pl, a.y_f32, h, segs, rows_per_block, block, lds_bytes, st, form);
+    case 4: return dispatch_flow<4>(pl, a.y_f32, h, segs, rows_per_block, block, lds_bytes, st, form);
     default: return hipErrorInvalidValue;
   }
 }
@@ -620,31 +677,62 @@ bool qmv_flow_supports(int K, int N, int M)
   return M == 1 && N >= 1 && K >= kSlice && K % 512 == 0 && K <= 32768;
 }
 
-hipError_t launch_qmv_flow(hipStream_t st, const QmvArgs& a)
+bool qmv_flow_narrow_supports(int K, int N, int M, int group)
+{
+  return M == 1 && N >= 1 && K >= kSlice && K % group == 0 && K <= 32768;
+}
+
+namespace {
+
+FlowForm flow_narrow(int group, bool f16)
+{
+  return f16 ? FlowForm::kNarrowF16 : group == 32 ? FlowForm::kNarrow32 : FlowForm::kNarrow64;
+}
+
+hipError_t launch_flow_one(hipStream_t st, const QmvArgs& a, double bytes_per_weight, FlowForm form)
 {
   const FlowSeg seg{a.w, a.scales, a.biases, a.y, a.N};
-  return launch_flow(st, &seg, 1, a, (double)a.N * (double)a.K * 9.0 / 16.0);
+  return launch_flow(st, &seg, 1, a, (double)a.N * (double)a.K * bytes_per_weight, form);
 }
+
+}  // namespace
+
+hipError_t launch_qmv_flow(hipStream_t st, const QmvArgs& a) { return launch_flow_one(st, a, 9.0 / 16.0, FlowForm::kWide); }
 
 // The same kernel over IEEE binary16 elements (x, scales, biases, y, residual).
-hipError_t launch_qmv_flow_f16(hipStream_t st, const QmvArgs& a)
+hipError_t launch_qmv_flow_f16(hipStream_t st, const QmvArgs& a) { return launch_flow_one(st, a, 9.0 / 16.0, FlowForm::kF16); }
+
+hipError_t launch_qmv_flow_narrow(hipStream_t st, const QmvArgs& a, int group, bool f16)
 {
-  const FlowSeg seg{a.w, a.scales, a.biases, a.y, a.N};
-  return launch_flow(st, &seg, 1, a, (double)a.N * (double)a.K * 9.0 / 16.0, true);
+  return launch_flow_one(st, a, group == 32 ? 5.0 / 8.0 : 9.0 / 16.0, flow_narrow(group, f16));
 }
 
-hipError_t launch_qmv_flow_group(hipStream_t st, const QmvArgs& a, const QmvGroup& g, bool f16)
+namespace {
+
+hipError_t launch_flow_group(hipStream_t st, const QmvArgs& a, const QmvGroup& g, double bytes_per_weight, FlowForm form)
 {
   FlowSeg segs[4];
   double bytes = 0.0;
   for (int i = 0; i < g.count; ++i) {
     segs[i] = FlowSeg{g.seg[i].w, g.seg[i].scales, g.seg[i].biases, g.seg[i].y, g.seg[i].N};
-    bytes += (double)g.seg[i].N * (double)a.K * 9.0 / 16.0;
+    bytes += (double)g.seg[i].N * (double)a.K * bytes_per_weight;
   }
   QmvArgs b = a;
   b.residual = nullptr;
   b.gate_act = 0;
-  return launch_flow(st, segs, g.count, b, bytes, f16);
+  return launch_flow(st, segs, g.count, b, bytes, form);
+}
+
+}  // namespace
+
+hipError_t launch_qmv_flow_group(hipStream_t st, const QmvArgs& a, const QmvGroup& g, bool f16)
+{
+  return launch_flow_group(st, a, g, 9.0 / 16.0, f16 ? FlowForm::kF16 : FlowForm::kWide);
+}
+
+hipError_t launch_qmv_flow_narrow_group(hipStream_t st, const QmvArgs& a, const QmvGroup& g, int group, bool f16)
+{
+  return launch_flow_group(st, a, g, group == 32 ? 5.0 / 8.0 : 9.0 / 16.0, flow_narrow(group, f16));
 }
 
 }  // namespace vpq
