@@ -194,3 +194,24 @@ def test_gathers_whose_wavefronts_walk_several_sets(vpq, dev, D, bits, K, N, pai
         alone = torch.empty((1, N), dtype=torch.bfloat16, device=dev)
         one(w, s, b, xr, K, N, eid[p:p + 1], E, out=alone)
         assert torch.equal(out.view[p], alone[0])
+
+
+# One row of a gated 8-bit pack runs on the gathers' kernel: one to five passes over K and the first K past them, N that ends
+# inside a set, wavefronts with several sets; against the oracle and the bits of the sorted form, which is another kernel
+@pytest.mark.parametrize("K,N", [(64, 2), (1024, 10), (1088, 34), (2112, 70), (3136, 6), (4160, 130), (5120, 18), (5184, 18), (128, 65538)])
+def test_one_gated_row_of_eight_bits(vpq, oracle, dev, D, K, N):
+    w, s, b = synth.make_weight8(N, K, K + N)
+    x = synth.make_act(1, K, K + N + 1)
+    wd, sd, bd, xd = D.u32(w, dev), D.bf16(s, dev), D.bf16(b, dev), D.bf16(x, dev)
+    out = parity.Guarded((1, N // 2), torch.bfloat16, dev)
+    vpq.qmv_gated_w8g64(wd, sd, bd, xd, K, N, 1, out=out.view, activation=1)
+    tile = torch.zeros((1,), dtype=torch.int32, device=dev)
+    srow = torch.tensor([0, -1], dtype=torch.int32, device=dev)
+    both = torch.empty((2, N // 2), dtype=torch.bfloat16, device=dev)
+    vpq.qmv_grouped_gated_w8g64(wd[None], sd[None], bd[None], xd, K, N, tile, srow, 1, both)
+    torch.cuda.synchronize()
+    out.assert_intact()
+    assert torch.equal(out.view[0], both[0])
+    y64, _ = oracle.matmul8(w, s, b, x, K, N, 1, rounded=False)
+    g64, gb = oracle.swiglu(np.asarray(y64).reshape(1, N))
+    parity.check_bf16(D.bits(out.view), g64, gb)

@@ -317,8 +317,11 @@ static int rows8_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* 
     a.M = rows;
     return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
   }
-  if (gathered && vpq::qmv_gather_supports(K)) {
-    return finish(vpq::launch_qmv_gather(reinterpret_cast<hipStream_t>(stream), a, 8, pair_eid, rows, x_div, n_experts));
+  // (one row of one pack: the row kernel's bits; gated 4096 -> 24576 29.9 -> 25.0 us, 3840 -> 19328 26.3 -> 19.1, 5120 -> 34816 49.3 ->
+  // 41.0)
+  if ((gathered || rows == 1) && vpq::qmv_gather_supports(K, 8)) {
+    return finish(vpq::launch_qmv_gather(reinterpret_cast<hipStream_t>(stream), a, 8, gathered ? pair_eid : nullptr, rows, x_div,
+                                         n_experts));
   }
   return finish(vpq::launch_qmv_rows8(reinterpret_cast<hipStream_t>(stream), a, rows, gathered ? pair_eid : nullptr, x_div,
                                       n_experts));
@@ -1067,7 +1070,7 @@ int gather_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales
   a.w = w; a.scales = scales; a.biases = biases; a.x = x; a.y = y;
   a.K = K; a.N = N; a.M = 1; a.y_f32 = false; a.cu_count = g_dev.cu_count;
   a.gate_act = gate_act;
-  if (vpq::qmv_gather_supports(K)) {
+  if (vpq::qmv_gather_supports(K, 4)) {
     return finish(vpq::launch_qmv_gather(reinterpret_cast<hipStream_t>(stream), a, 4, pair_eid, npair, x_div, n_experts));
   }
   return finish(vpq::launch_qmv_rows_gather(reinterpret_cast<hipStream_t>(stream), a, pair_eid, npair, x_div, n_experts));

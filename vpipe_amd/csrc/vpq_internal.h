@@ -211,7 +211,7 @@ hipError_t launch_qmv_rows_group(hipStream_t st, const QmvArgs& a, const QmvGrou
 hipError_t launch_qmv_rows_gather(hipStream_t st, const QmvArgs& a, const int* pair_eid, int pairs, int x_div,
                                   int n_experts);
 // The gathers at K <= 4096 (vpq_qmv_gather.hip), with the bits of launch_qmv_rows_gather (8 bits: launch_qmv_rows8).
-bool qmv_gather_supports(int K);
+bool qmv_gather_supports(int K, int bits);
 hipError_t launch_qmv_gather(hipStream_t st, const QmvArgs& a, int bits, const int* pair_eid, int pairs, int x_div, int n_experts);
 // Sorted pairs, two slots per tile (a.M = 2): expert tile2e[tile], x row srow[slot] (x_from_srow) or the slot.
 hipError_t launch_qmv_rows_sorted(hipStream_t st, const QmvArgs& a, const int* tile2e, const int* srow, int tiles,

@@ -1,4 +1,5 @@
-// Gathered expert projections of an MoE block at decode (groups of 64, K up to 4096): each (token, expert) pair's row of x
+// Gathered expert projections of an MoE block at decode (groups of 64, K up to 4096, 8 bits 5120), and one row of a gated 8-bit
+// pack (no pair_eid): each (token, expert) pair's row of x
 // against that expert's slab, one launch for all pairs (gpu-kernels/metal/quant/affine_qmv.metal:908-962, 1262-1292).  Per
 // row of weights the arithmetic and the order of every sum are those of the kernels of one wavefront per weight row
 // (vpq_qmv_rows.hip, qmv_rows8_kernel), so a pair has the bits of the plain call on its slab.
@@ -87,7 +88,7 @@ __global__ __launch_bounds__(256) void qmv_gather_kernel(const uint32_t* __restr
 #pragma unroll
     for (int t = 0; t < kX; ++t) { xd[c][t] = k0 < K ? *reinterpret_cast<const uint4*>(x + k0 + 8 * t) : make_uint4(0u, 0u, 0u, 0u); }
   }
-  int e = pair_eid[p];
+  int e = pair_eid != nullptr ? pair_eid[p] : 0;    // (none: one pack, one row)
   const bool expert_ok = e >= 0 && e < n_experts;
   e = expert_ok ? e : 0;
   const uint32_t* w = w_ + (size_t)e * (size_t)N * Kw;
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(256) void qmv_gather_kernel(const uint32_t* __restr
   }
 }
 
-bool qmv_gather_supports(int K) { return K % 64 == 0 && K <= 4096; }
+bool qmv_gather_supports(int K, int bits) { return K % 64 == 0 && K <= (bits == 8 ? 5120 : 4096); }
 
 hipError_t launch_qmv_gather(hipStream_t st, const QmvArgs& a, int bits, const int* pair_eid, int pairs, int x_div, int n_experts)
 {
@@ -254,7 +255,8 @@ hipError_t launch_qmv_gather(hipStream_t st, const QmvArgs& a, int bits, const i
     return a.K <= 1024   ? VPQ_GATHER(8, 1, 64)
            : a.K <= 2048 ? VPQ_GATHER(8, 2, 64)
            : a.K <= 3072 ? VPQ_GATHER(8, 3, 64)
-                         : VPQ_GATHER(8, 4, 64);
+           : a.K <= 4096 ? VPQ_GATHER(8, 4, 64)
+                         : VPQ_GATHER(8, 5, 64);
   }
   if (half) { return VPQ_GATHER(4, 1, 32); }
   return a.K <= 2048 ? VPQ_GATHER(4, 1, 64) : VPQ_GATHER(4, 2, 64);
