@@ -171,6 +171,16 @@ def test_build_refuses_a_load_too_close_behind_its_scalar_base():
             build._check_scalar_hazard("x.hip", kernel(*bad))
 
 
+def test_build_gives_the_same_object_for_the_same_source(tmp_path):
+    """The hash of libvpq.so names the library that a profile was taken on: it may depend on the sources alone."""
+    from vpipe_amd import build
+    objs = []
+    for i in range(2):
+        build._compile("vpq_norm.hip", str(tmp_path / ("%d.o" % i)))
+        objs.append((tmp_path / ("%d.o" % i)).read_bytes())
+    assert objs[0] == objs[1]
+
+
 def test_bench_refuses_more_than_one_gpu():
     # one GPU only: no collectives, no sharding; the benchmark says so instead of starting ranks
     import subprocess

@@ -238,11 +238,14 @@ def _check_scalar_hazard(src, asm):
         raise RuntimeError("%s: scalar register read too soon (see build.py):\n  %s" % (src, "\n  ".join(bad[:20])))
 
 
-def _compile(src):
-    obj = os.path.join(CSRC, src.replace(".hip", ".o"))
+def _compile(src, obj=None):
+    obj = obj or os.path.join(CSRC, src.replace(".hip", ".o"))
     with tempfile.TemporaryDirectory() as tmp:
-        out = os.path.join(tmp, os.path.basename(obj))
-        cmd = [HIPCC] + FLAGS + ["-Rpass-analysis=kernel-resource-usage", "-save-temps=obj", "-c", os.path.join(CSRC, src), "-o", out]
+        out = os.path.join(tmp, src.replace(".hip", ".o"))
+        # The unit's id goes into symbol names; by default it is a hash over the command, the temporary folder's name with it.  By
+        # the source's name, equal sources give equal objects, so that the library's hash names a state of the sources.
+        cmd = [HIPCC] + FLAGS + ["-cuid=" + os.path.splitext(src)[0], "-Rpass-analysis=kernel-resource-usage", "-save-temps=obj",
+                                 "-c", os.path.join(CSRC, src), "-o", out]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             err = "\n".join(l for l in r.stderr.splitlines() if "packed-fp32-ops" not in l and "remark:" not in l)
