@@ -594,7 +594,8 @@ int vpq_argmax_combine(vpq_stream_t stream, const float* partials, int32_t* out_
  *   vpq_gather_down_qmv_w8g64_bf16   replaces `affine_gather_down_qmv_w8g64` (:1295-1322): the MoE
  *                                    gathers over a batched 8-bit pack [E, N, K/4], arguments and
  *                                    conventions of the 4-bit vpq_gather_* entries; a pair is
- *                                    bit-identical to the plain 8-bit call on that expert's slab.
+ *                                    bit-identical to the one-row 8-bit call (gated / plain, at any K)
+ *                                    on that expert's slab.
  *   vpq_qmm_w8g64_bf16, vpq_qmm_gated_w8g64_bf16   the fused kernels with byte codes (the large-tile kernel
  *                                    once its tiles fill the CUs, else the 256 x 128 tile kernel; same bits): replace
  *                                    `affine_qmm_steel_w8g64[_bm64|_bm128]` (affine_qmm_steel.metal:1601-1672)
@@ -758,7 +759,8 @@ int vpq_qmm_dense_route_w4g64_f16(vpq_stream_t stream, const uint32_t* w, const 
 /* The grouped launch of the format twins (`affine_qmv_qkv_w4g32`, `affine_qmv_qkv_w8g64`, affine_qmv.metal:518-559):
  * arguments as vpq_qmv_group_w4g64_bf16 (w uint32 [N_i, K/8] with scales / biases [N_i, K/32], resp. w uint32
  * [N_i, K/4] with [N_i, K/64]); bit-identical to `count` calls of vpq_qmv_w4g32_bf16 / vpq_qmv_w8g64_bf16.  One launch,
- * but for one row of 8-bit codes with K < 2560 and for packs whose scales or biases are not 16-byte aligned. */
+ * but for one row of 8-bit codes with K < 2560, and at two rows and more for packs whose scales or biases are not 16-byte
+ * aligned. */
 int vpq_qmv_group_w4g32_bf16(vpq_stream_t stream, int count, const uint32_t* const* w,
                              const uint16_t* const* scales, const uint16_t* const* biases,
                              const uint16_t* x, uint16_t* const* y, int K, const int* N, int M, int scale_only);

@@ -142,6 +142,54 @@ def test_gathered_expert_projections_w8(vpq, oracle, dev, D, activation):
     parity.check_bf16(gotd, d64, dbits)
 
 
+# K: where one row leaves the general kernel (2560), a last pass of one group, where the gathers' kernel ends (5120); N: no
+# whole set of four rows, one row more than a set for every wavefront of the chip
+@pytest.mark.parametrize("K,N", [(2496, 21), (2560, 1133), (3136, 70), (4096, 1030), (4160, 5), (4608, 32773), (5120, 1041),
+                                 (5184, 23), (12288, 1539)])
+def test_one_row_w8_has_the_bits_of_a_gathered_pair(vpq, dev, D, K, N):
+    gen = torch.Generator(device=dev).manual_seed(K + N)
+
+    # The second half of K nearly cancels the first, so that another order of additions shows in the stored elements.
+    half = K // 128 * 64
+
+    def pack(n):
+        w = torch.randint(-2 ** 31, 2 ** 31, (n, K // 4), dtype=torch.int32, device=dev, generator=gen)
+        s = torch.empty((n, K // 64), device=dev).uniform_(0.0003, 0.0012, generator=gen).bfloat16()
+        b = (s.float() * (-128 + 4 * torch.randn(s.shape, device=dev, generator=gen))).bfloat16()
+        for t, per in ((w, 4), (s, 64), (b, 64)):
+            t[:, half // per:2 * half // per] = t[:, :half // per]
+        return w, s, b
+
+    packs = [pack(n) for n in (N, 1, 18)]
+    x = torch.randn((1, K), device=dev, generator=gen)
+    x[:, half:2 * half] = -x[:, :half] * (1 + torch.randn((1, half), device=dev, generator=gen) / 64)
+    x[:, 2 * half:] /= 64
+    x = x.bfloat16()
+    zero = torch.zeros((1,), dtype=torch.int32, device=dev)
+    out = parity.Guarded((1, N), torch.bfloat16, dev)
+    vpq.qmv_w8g64(*packs[0], x, K, N, 1, out=out.view)
+    torch.cuda.synchronize()
+    out.assert_intact()
+    assert torch.equal(out.view, vpq.gather_down_qmv_w8g64(*(t[None] for t in packs[0]), x, K, N, zero, 1))
+    f32 = vpq.qmv_w8g64(*packs[0], x, K, N, 1, f32out=True)
+    assert torch.equal(f32.bfloat16(), out.view)
+    w, s, b = (t[:64] for t in packs[0])
+    q = torch.stack([(w >> 8 * i) & 255 for i in range(4)], -1).reshape(-1, K).double()
+    W = q * s.double().repeat_interleave(64, 1) + b.double().repeat_interleave(64, 1)
+    exact, terms = W @ x[0].double(), W.abs() @ x[0].double().abs()
+    # (a lane's K / 64 multiply-adds, six additions between lanes, the weight's own: half a unit in the last place each)
+    assert ((f32[0, :64].double() - exact).abs() <= (K / 64 + 8) * 2.0 ** -24 * terms).all()
+    res = torch.randn((1, N), device=dev, generator=gen).bfloat16()
+    added = vpq.qmv_w8g64(*packs[0], x, K, N, 1, residual=res)
+    assert torch.equal(added, (out.view.float() + res.float()).bfloat16())
+    outs = [parity.Guarded((1, t[0].shape[0]), torch.bfloat16, dev) for t in packs]
+    vpq.qmv_group_w8g64([t + (t[0].shape[0],) for t in packs], x, K, 1, outs=[o.view for o in outs])
+    torch.cuda.synchronize()
+    for t, o in zip(packs, outs):
+        o.assert_intact()
+        assert torch.equal(o.view, vpq.qmv_w8g64(*t, x, K, t[0].shape[0], 1))
+
+
 def test_w8_gather_ids_out_of_range_and_bad_arguments(vpq, dev, D):
     K, inner, E = 256, 8, 3
     w, s, b = (np.stack([p[i] for p in [interleaved8(inner, K, 2800 + e) for e in range(E)]]) for i in range(3))

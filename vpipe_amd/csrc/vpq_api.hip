@@ -82,11 +82,16 @@ int check_pack(const uint32_t* w, const uint16_t* scales, const uint16_t* biases
 // are even on 4096->12288 and the fused kernel is ahead on the N = 4096 shapes).
 constexpr int kDenseRouteMinRows = 8192;
 
-// Rows of x and K from which 8-bit packs run on the batch kernel, below which on one wavefront per weight row.  One row: from the
-// K on from which the batch kernel's error against float64 is the smaller one (fp32 output, 1e-7, K = 2048 / 2560 / 4096 / 12288:
-// 1.02 / 1.13 / 1.36 / 2.20 and 1.05 / 1.12 / 1.17 / 1.51).  us at one row, before / now: 4096 -> 4096 7.7 / 6.8, 12288 -> 4096 18.7 /
-// 13.3, 9664 -> 3840 15.8 / 11.8; q|k|v of 4096 in one launch instead of three 18.1 / 9; 4096 -> 1024 by itself 5.2 / 5.7.
-bool batch_from8(int K, int M) { return M >= 2 || K >= 2560; }
+// One row of 8-bit codes: below this K the general kernel, a launch a pack; from it on launch_row8, the same bits.  us: 2048 ->
+// 512 3.0 / 3.3, 2560 -> 640 4.2 / 4.2, 2560 -> 2560 5.5 / 4.8, 4096 -> 4096 7.8 / 7.2, 12288 -> 4096 19.8 / 15.2; q|k|v of 4096
+// in three launches 18.3, in one 9.5.
+constexpr int kRow8MinK = 2560;
+
+// One row of x against the 8-bit packs of g, each with the bits that it has as an expert's slab of a gather.
+hipError_t launch_row8(hipStream_t hs, const vpq::QmvArgs& a, const vpq::QmvGroup& g)
+{
+  return vpq::qmv_gather_supports(a.K, 8) ? vpq::launch_qmv_gather_row8(hs, a, g) : vpq::launch_qmv_row8(hs, a, g);
+}
 
 // One row of binary16 whose scales are no whole 16-byte pieces: the one-row kernel from the K on from which its error against
 // float64 is no larger than that of one wavefront per weight row, which ran these (fp32 output, 1e-7, K = 2112 / 3840 / 9664: 1.36 /
@@ -254,8 +259,11 @@ static int qmv8_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* s
   a.K = K; a.N = N; a.M = M; a.y_f32 = y_f32; a.cu_count = g_dev.cu_count;
   a.gate_act = store;
   const vpq::BatchFormat f{8, 64, false, false};
-  if (batch_from8(K, M) && store == 0 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && aligned(biases, 16)) {
+  if (M >= 2 && store == 0 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && aligned(biases, 16)) {
     return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
+  }
+  if (M == 1 && store == 0 && K >= kRow8MinK) {
+    return finish(launch_row8(reinterpret_cast<hipStream_t>(stream), a, vpq::QmvGroup{1, {{w, scales, biases, y, N}}}));
   }
   return finish(vpq::launch_qmv_simple8(reinterpret_cast<hipStream_t>(stream), a));
 }
@@ -317,11 +325,10 @@ static int rows8_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* 
     a.M = rows;
     return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
   }
-  // (one row of one pack: the row kernel's bits; gated 4096 -> 24576 29.9 -> 25.0 us, 3840 -> 19328 26.3 -> 19.1, 5120 -> 34816 49.3 ->
-  // 41.0)
-  if ((gathered || rows == 1) && vpq::qmv_gather_supports(K, 8)) {
-    return finish(vpq::launch_qmv_gather(reinterpret_cast<hipStream_t>(stream), a, 8, gathered ? pair_eid : nullptr, rows, x_div,
-                                         n_experts));
+  if (vpq::qmv_gather_supports(K, 8)) {
+    hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+    if (gathered) { return finish(vpq::launch_qmv_gather(hs, a, 8, pair_eid, rows, x_div, n_experts)); }
+    if (rows == 1) { return finish(vpq::launch_qmv_gather_row8(hs, a, vpq::QmvGroup{1, {{w, scales, biases, y, N}}})); }
   }
   return finish(vpq::launch_qmv_rows8(reinterpret_cast<hipStream_t>(stream), a, rows, gathered ? pair_eid : nullptr, x_div,
                                       n_experts));
@@ -1767,12 +1774,13 @@ int vpq_qmv_group_w8g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
   if (w == nullptr || scales == nullptr || biases == nullptr || y == nullptr || N == nullptr) { return VPQ_ERR_NULL_POINTER; }
   if (count < 1 || count > 4) { return VPQ_ERR_BAD_SHAPE; }
   const vpq::BatchFormat f{8, 64, false, false};
-  bool batch = batch_from8(K, M) && M <= 16 && x != nullptr && aligned(x, 16) && vpq::qmv_batch_supports(K, M, f);
-  for (int i = 0; i < count && batch; ++i) {
-    batch = check_pack(w[i], scales[i], biases[i], K, N[i]) == VPQ_OK && y[i] != nullptr && aligned(y[i], 2) &&
-            aligned(scales[i], 16) && aligned(biases[i], 16);
+  const bool row = M == 1 && K >= kRow8MinK;
+  bool one_launch = x != nullptr && aligned(x, 16) && (row || (M >= 2 && M <= 16 && vpq::qmv_batch_supports(K, M, f)));
+  for (int i = 0; i < count && one_launch; ++i) {
+    one_launch = check_pack(w[i], scales[i], biases[i], K, N[i]) == VPQ_OK && y[i] != nullptr && aligned(y[i], 2) &&
+                 (row || (aligned(scales[i], 16) && aligned(biases[i], 16)));
   }
-  if (batch) {
+  if (one_launch) {
     const int st = ensure_init();
     if (st != VPQ_OK) { return st; }
     vpq::QmvArgs a{};
@@ -1780,9 +1788,10 @@ int vpq_qmv_group_w8g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
     vpq::QmvGroup g;
     g.count = count;
     for (int i = 0; i < count; ++i) { g.seg[i] = vpq::QmvSeg{w[i], scales[i], biases[i], y[i], N[i]}; }
-    return finish(vpq::launch_qmv_batch(reinterpret_cast<hipStream_t>(stream), a, g, f));
+    hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+    return finish(row ? launch_row8(hs, a, g) : vpq::launch_qmv_batch(hs, a, g, f));
   }
-  // one row of a short K, or something to report: the separate calls
+  // one row of a short K, packs that the batch kernel does not take, or something to report: the separate calls
   for (int i = 0; i < count; ++i) {
     const int st = vpq_qmv_w8g64_bf16(stream, w[i], scales[i], biases[i], x, y[i], K, N[i], M, nullptr);
     if (st != VPQ_OK) { return st; }

@@ -158,6 +158,10 @@ hipError_t launch_qmv_split_gate_up(hipStream_t st, const SplitGateUp& a);
 // 8-bit gated / gathered QMV, one wavefront per output and row (a.gate_act: interleaved gate|up pack);
 // rows = rows of x, or with pair_eid the (token, expert) pairs over a batched pack.
 hipError_t launch_qmv_rows8(hipStream_t st, const QmvArgs& a, int rows, const int* pair_eid, int x_div, int n_experts);
+// One row of x, up to four 8-bit packs in one launch (a.w / scales / biases / y / N are ignored, the segments give them; residual
+// and fp32 store with a single one), with the bits of launch_qmv_rows8.
+struct QmvGroup;
+hipError_t launch_qmv_row8(hipStream_t st, const QmvArgs& a, const QmvGroup& g);
 // Two-slot expert-sorted GEMV over a batched 8-bit pack (a.gate_act != 0: x rows gathered through srow).
 hipError_t launch_qmv_rows8_sorted(hipStream_t st, const QmvArgs& a, const int* tile2e, const int* srow, int tiles,
                                    int n_experts);
@@ -210,8 +214,10 @@ hipError_t launch_qmv_rows_group(hipStream_t st, const QmvArgs& a, const QmvGrou
 // [0, n_experts)); a.gate_act as in the plain form.
 hipError_t launch_qmv_rows_gather(hipStream_t st, const QmvArgs& a, const int* pair_eid, int pairs, int x_div,
                                   int n_experts);
-// The gathers at K <= 4096 (vpq_qmv_gather.hip), with the bits of launch_qmv_rows_gather (8 bits: launch_qmv_rows8).
+// The gathers up to a K of 4096, 8 bits 5120 (vpq_qmv_gather.hip), with the bits of launch_qmv_rows_gather (8 bits:
+// launch_qmv_rows8); launch_qmv_gather_row8: launch_qmv_row8, gated too.
 bool qmv_gather_supports(int K, int bits);
+hipError_t launch_qmv_gather_row8(hipStream_t st, const QmvArgs& a, const QmvGroup& g);
 hipError_t launch_qmv_gather(hipStream_t st, const QmvArgs& a, int bits, const int* pair_eid, int pairs, int x_div, int n_experts);
 // Sorted pairs, two slots per tile (a.M = 2): expert tile2e[tile], x row srow[slot] (x_from_srow) or the slot.
 hipError_t launch_qmv_rows_sorted(hipStream_t st, const QmvArgs& a, const int* tile2e, const int* srow, int tiles,

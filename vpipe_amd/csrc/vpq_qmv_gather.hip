@@ -1,8 +1,8 @@
-// Gathered expert projections of an MoE block at decode (groups of 64, K up to 4096, 8 bits 5120), and one row of a gated 8-bit
-// pack (no pair_eid): each (token, expert) pair's row of x
-// against that expert's slab, one launch for all pairs (gpu-kernels/metal/quant/affine_qmv.metal:908-962, 1262-1292).  Per
-// row of weights the arithmetic and the order of every sum are those of the kernels of one wavefront per weight row
-// (vpq_qmv_rows.hip, qmv_rows8_kernel), so a pair has the bits of the plain call on its slab.
+// Gathered expert projections of an MoE block at decode (groups of 64, K up to 4096, 8 bits 5120): each (token, expert) pair's
+// row of x against that expert's slab, one launch for all pairs (gpu-kernels/metal/quant/affine_qmv.metal:908-962, 1262-1292);
+// and one row of x against up to four 8-bit packs.  Per row of weights the arithmetic and the order of every sum are those of
+// the kernels of one wavefront per weight row (vpq_qmv_rows.hip, qmv_rows8_kernel), so a pair has the bits of that row's call on
+// its slab.
 //
 // What bounds it: the slabs' read from HBM, a few megabytes a pair; the row-streaming kernel, one or two rows a wavefront,
 // was bound by the vector ALU instead -- of its 140 instructions a row of 2048 values, 50 unpack and contract, the others
@@ -58,13 +58,17 @@ __device__ __forceinline__ float row_sum(float v)
 
 }  // namespace
 
+namespace {
+
 // P: passes over K of LPR lanes by 32 values of 4 bits, 16 of 8 bits.  LPR: lanes per weight row (32: two row groups a
-// wavefront, 4 bits and K up to 1024).
-template <int BITS, int P, int LPR>
-__global__ __launch_bounds__(256) void qmv_gather_kernel(const uint32_t* __restrict__ w_, const uint16_t* __restrict__ scales_,
-                                                         const uint16_t* __restrict__ biases_, const uint16_t* __restrict__ x_,
-                                                         const int* __restrict__ pair_eid, int K, int N, int x_div, int n_experts,
-                                                         uint16_t* __restrict__ y_, int gate_act)
+// wavefront, 4 bits and K up to 1024).  block, blocks: this workgroup among those of the pair, or of the pack (ONE: one row of
+// x, pair_eid unread; residual and fp32 stores).
+template <int BITS, int P, int LPR, bool ONE>
+__device__ __forceinline__ void gather_body(const uint32_t* __restrict__ w_, const uint16_t* __restrict__ scales_,
+                                            const uint16_t* __restrict__ biases_, const uint16_t* __restrict__ x_,
+                                            const int* __restrict__ pair_eid, int K, int N, int x_div, int n_experts,
+                                            void* __restrict__ y_, int gate_act, int block, int blocks,
+                                            const uint16_t* __restrict__ residual, int y_f32)
 {
   static_assert(LPR == 64 || (LPR == 32 && BITS == 4), "");
   constexpr int R = 4;                              // rows of a set and row group (the reduction below)
@@ -74,11 +78,11 @@ __global__ __launch_bounds__(256) void qmv_gather_kernel(const uint32_t* __restr
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = lane / LPR, ll = lane % LPR;
-  const int sets = (N + kRows - 1) / kRows, stride = (int)gridDim.x * 4;
-  int set = (int)blockIdx.x * 4 + wave;
+  const int sets = (N + kRows - 1) / kRows, stride = blocks * 4;
+  int set = block * 4 + wave;
   if (set >= sets) { return; }                      // (no barrier in this kernel)
 
-  const int p = (int)blockIdx.y;
+  const int p = ONE ? 0 : (int)blockIdx.y;
   const uint16_t* x = x_ + (size_t)(p / x_div) * K;
   const int Kw = K * BITS / 32, Kg = K >> 6;
   uint4 xd[P][kX];
@@ -88,13 +92,13 @@ __global__ __launch_bounds__(256) void qmv_gather_kernel(const uint32_t* __restr
 #pragma unroll
     for (int t = 0; t < kX; ++t) { xd[c][t] = k0 < K ? *reinterpret_cast<const uint4*>(x + k0 + 8 * t) : make_uint4(0u, 0u, 0u, 0u); }
   }
-  int e = pair_eid != nullptr ? pair_eid[p] : 0;    // (none: one pack, one row)
-  const bool expert_ok = e >= 0 && e < n_experts;
+  int e = ONE ? 0 : pair_eid[p];
+  const bool expert_ok = ONE || (e >= 0 && e < n_experts);
   e = expert_ok ? e : 0;
   const uint32_t* w = w_ + (size_t)e * (size_t)N * Kw;
   const uint16_t* scales = scales_ + (size_t)e * (size_t)N * Kg;
   const uint16_t* biases = biases_ + (size_t)e * (size_t)N * Kg;
-  uint16_t* y = y_ + (size_t)p * (size_t)(gate_act ? (N >> 1) : N);
+  uint16_t* y = static_cast<uint16_t*>(y_) + (size_t)p * (size_t)(gate_act ? (N >> 1) : N);
 
   struct Pass {
     uint4 c[R];
@@ -207,7 +211,13 @@ __global__ __launch_bounds__(256) void qmv_gather_kernel(const uint32_t* __restr
           y[n >> 1] = (uint16_t)f32_to_bf16_bits(gated_f32(gate_act, total, __uint_as_float(o[1])));
         }
       } else if ((lane & 15) == 0 && n < N) {
-        y[n] = (uint16_t)f32_to_bf16_bits(total);
+        if (ONE && y_f32) {
+          static_cast<float*>(y_)[n] = total;
+        } else {
+          uint32_t v16 = f32_to_bf16_bits(total);
+          if (ONE && residual != nullptr) { v16 = f32_to_bf16_bits(bf16_bits_to_f32(v16) + bf16_bits_to_f32(residual[n])); }
+          y[n] = (uint16_t)v16;
+        }
       }
     } else {
       // even rows of 16 lanes: rows 0 (a) and 2 (b) of the half's four; odd ones: 1 and 3
@@ -234,17 +244,86 @@ __global__ __launch_bounds__(256) void qmv_gather_kernel(const uint32_t* __restr
   }
 }
 
+// One row of x against up to four packs: the workgroups of pack i start at first[i].
+struct GatherRow {
+  const uint16_t* x;
+  const uint16_t* residual;   // (of a single pack)
+  int K, gate_act, y_f32, nseg;
+  QmvSeg seg[4];
+  int first[5];
+};
+
+}  // namespace
+
+template <int BITS, int P, int LPR>
+__global__ __launch_bounds__(256) void qmv_gather_kernel(const uint32_t* __restrict__ w, const uint16_t* __restrict__ scales,
+                                                         const uint16_t* __restrict__ biases, const uint16_t* __restrict__ x,
+                                                         const int* __restrict__ pair_eid, int K, int N, int x_div, int n_experts,
+                                                         uint16_t* __restrict__ y, int gate_act)
+{
+  gather_body<BITS, P, LPR, false>(w, scales, biases, x, pair_eid, K, N, x_div, n_experts, y, gate_act, (int)blockIdx.x,
+                                   (int)gridDim.x, nullptr, 0);
+}
+
+template <int P>
+__global__ __launch_bounds__(256) void qmv_gather_row8_kernel(const GatherRow p)
+{
+  const int at = (int)blockIdx.x;
+  QmvSeg seg = p.seg[0];
+  int first = 0, end = p.first[1];                          // (constant indexes: a variable one would put p into scratch)
+  if (p.nseg > 1 && at >= p.first[1]) { seg = p.seg[1]; first = p.first[1]; end = p.first[2]; }
+  if (p.nseg > 2 && at >= p.first[2]) { seg = p.seg[2]; first = p.first[2]; end = p.first[3]; }
+  if (p.nseg > 3 && at >= p.first[3]) { seg = p.seg[3]; first = p.first[3]; end = p.first[4]; }
+  gather_body<8, P, 64, true>(seg.w, seg.scales, seg.biases, p.x, nullptr, p.K, seg.N, 1, 1, seg.y, p.gate_act, at - first,
+                              end - first, p.residual, p.y_f32);
+}
+
 bool qmv_gather_supports(int K, int bits) { return K % 64 == 0 && K <= (bits == 8 ? 5120 : 4096); }
+
+namespace {
+
+// Wavefronts of about two rounds (32 a CU), each with as many sets of its pair or pack as that leaves.  With 16 / 32 a CU, 2048 ->
+// 2 x 768 at 4 tokens of 8 experts 14.6 / 13.3 us, 768 -> 2048 at 16 tokens 23.9 / 22.2.
+long gather_sets_per_wave(long sets, int cus)
+{
+  const long room = 32L * cus;
+  return (sets + room - 1) / room;
+}
+
+}  // namespace
+
+// One row of x, up to four 8-bit packs.  Measured (us, the general kernel / now): 4096 -> 1024 5.2 / 5.3, 4096 -> 4096 7.8 / 7.2,
+// 4096 -> 12288 16.6 / 14.2, 5120 -> 151936 182 / 145; gated, by qmv_rows8_kernel / now: 4096 -> 24576 29.9 / 25.0, 3840 -> 19328
+// 26.3 / 19.1, 5120 -> 34816 49.3 / 40.
+hipError_t launch_qmv_gather_row8(hipStream_t st, const QmvArgs& a, const QmvGroup& g)
+{
+  const int cus = a.cu_count > 0 ? a.cu_count : 256;
+  GatherRow p{};
+  p.x = a.x; p.residual = a.residual; p.K = a.K; p.gate_act = a.gate_act; p.y_f32 = a.y_f32 ? 1 : 0; p.nseg = g.count;
+  long sets = 0;
+  for (int i = 0; i < g.count; ++i) { sets += (g.seg[i].N + 3) / 4; }
+  const long per = gather_sets_per_wave(sets, cus);
+  for (int i = 0; i < g.count; ++i) {
+    p.seg[i] = g.seg[i];
+    p.first[i + 1] = p.first[i] + (int)(((g.seg[i].N + 3) / 4 + 4 * per - 1) / (4 * per));
+  }
+  const dim3 grid((unsigned)p.first[g.count]), block(256);
+  switch ((a.K + 1023) / 1024) {
+    case 1: return launch_kernel(qmv_gather_row8_kernel<1>, grid, block, 0, st, p);
+    case 2: return launch_kernel(qmv_gather_row8_kernel<2>, grid, block, 0, st, p);
+    case 3: return launch_kernel(qmv_gather_row8_kernel<3>, grid, block, 0, st, p);
+    case 4: return launch_kernel(qmv_gather_row8_kernel<4>, grid, block, 0, st, p);
+    case 5: return launch_kernel(qmv_gather_row8_kernel<5>, grid, block, 0, st, p);
+    default: return hipErrorInvalidValue;
+  }
+}
 
 hipError_t launch_qmv_gather(hipStream_t st, const QmvArgs& a, int bits, const int* pair_eid, int pairs, int x_div, int n_experts)
 {
   const int cus = a.cu_count > 0 ? a.cu_count : 256;
   const bool half = bits == 4 && a.K <= 1024;
   const int rows = half ? 8 : 4, sets = (a.N + rows - 1) / rows;
-  // Wavefronts of about two rounds (32 a CU), each with as many sets of its pair as that leaves.  With 16 / 32 a CU, 2048 -> 2 x
-  // 768 at 4 tokens of 8 experts 14.6 / 13.3 us, 768 -> 2048 at 16 tokens 23.9 / 22.2.
-  const long room = 32L * cus;
-  const long per = ((long)sets * pairs + room - 1) / room;
+  const long per = gather_sets_per_wave((long)sets * pairs, cus);
   const int blocks = (int)((sets + 4 * per - 1) / (4 * per));
   const dim3 grid((unsigned)blocks, (unsigned)pairs), block(256);
   uint16_t* y = reinterpret_cast<uint16_t*>(a.y);

@@ -221,6 +221,53 @@ __global__ __launch_bounds__(256) void qmv_simple8_kernel(
   }
 }
 
+namespace {
+
+// The sums of R consecutive weight rows of an 8-bit pack with one row of x, by a wavefront.
+template <int R>
+__device__ __forceinline__ void rows8_sums(const uint32_t* __restrict__ w, const uint16_t* __restrict__ scales,
+                                           const uint16_t* __restrict__ biases, const uint16_t* __restrict__ xr, int n0, int K,
+                                           float (&acc)[R])
+{
+  const int lane = threadIdx.x & 63;
+  const int Kw = K >> 2, Kg = K >> 6;
+#pragma unroll
+  for (int r = 0; r < R; ++r) { acc[r] = 0.0f; }
+  for (int k0 = lane * 16; k0 < K; k0 += kWave * 16) {
+    const uint4* xp = reinterpret_cast<const uint4*>(xr + k0);
+    float xv[16];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint4 x4 = xp[h];
+      const uint32_t xd[4] = {x4.x, x4.y, x4.z, x4.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        xv[8 * h + 2 * j] = bf16_lo_to_f32(xd[j]);
+        xv[8 * h + 2 * j + 1] = bf16_hi_to_f32(xd[j]);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const size_t n = (size_t)(n0 + r);
+      const uint4 c4 = *reinterpret_cast<const uint4*>(w + n * Kw + (k0 >> 2));
+      const uint32_t codes[4] = {c4.x, c4.y, c4.z, c4.w};
+      const float s = bf16_bits_to_f32(scales[n * Kg + (k0 >> 6)]);
+      const float b = bf16_bits_to_f32(biases[n * Kg + (k0 >> 6)]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          acc[r] = fmaf(xv[4 * i + j], fmaf(s, (float)((codes[i] >> (8 * j)) & 0xffu), b), acc[r]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) { acc[r] = wave_sum(acc[r]); }
+}
+
+}  // namespace
+
 // 8-bit gated and gathered forms (affine_qmv_swiglu_w8g64 / affine_qmv_geglu_w8g64,
 // gpu-kernels/metal/quant/affine_qmv.metal:3140-3178; affine_gather_qmv_swiglu_w8g64 :962-990,
 // affine_gather_qmv_geglu_w8g64 :1524-1552, affine_gather_down_qmv_w8g64 :1295-1322).  One wavefront
@@ -257,44 +304,57 @@ __global__ __launch_bounds__(256) void qmv_rows8_kernel(
   constexpr int R = GATED ? 2 : 1;
   const int n0 = GATED ? 2 * o : o;
   float acc[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) { acc[r] = 0.0f; }
-  for (int k0 = lane * 16; k0 < K; k0 += kWave * 16) {
-    const uint4* xp = reinterpret_cast<const uint4*>(xr + k0);
-    float xv[16];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint4 x4 = xp[h];
-      const uint32_t xd[4] = {x4.x, x4.y, x4.z, x4.w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        xv[8 * h + 2 * j] = bf16_lo_to_f32(xd[j]);
-        xv[8 * h + 2 * j + 1] = bf16_hi_to_f32(xd[j]);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const size_t n = (size_t)(n0 + r);
-      const uint4 c4 = *reinterpret_cast<const uint4*>(w + n * Kw + (k0 >> 2));
-      const uint32_t codes[4] = {c4.x, c4.y, c4.z, c4.w};
-      const float s = bf16_bits_to_f32(scales[n * Kg + (k0 >> 6)]);
-      const float b = bf16_bits_to_f32(biases[n * Kg + (k0 >> 6)]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          acc[r] = fmaf(xv[4 * i + j], fmaf(s, (float)((codes[i] >> (8 * j)) & 0xffu), b), acc[r]);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < R; ++r) { acc[r] = wave_sum(acc[r]); }
+  rows8_sums<R>(w, scales, biases, xr, n0, K, acc);
   if (lane == 0) {
     const float v = GATED ? gated_f32(gate_act, acc[0], acc[R - 1])
                           : (gate_act == kStoreSigmoid ? 1.0f / (1.0f + __expf(-acc[0])) : acc[0]);
     y[(size_t)m * outs + o] = (uint16_t)f32_to_bf16_bits(v);
   }
+}
+
+// One row of x against up to four 8-bit packs (q|k|v, or one with a residual or an fp32 store), one wavefront per weight row:
+// where vpq_qmv_gather.hip does not run.  The workgroups of pack i start at first[i].
+struct Row8Params {
+  const uint16_t* x;
+  const uint16_t* residual;
+  int K, y_f32, nseg;
+  QmvSeg seg[4];
+  int first[4];
+};
+
+__global__ __launch_bounds__(256) void qmv_row8_kernel(const Row8Params p)
+{
+  const int at = (int)blockIdx.x;
+  QmvSeg seg = p.seg[0];
+  int first = 0;                                            // (constant indexes: a variable one would put p into scratch)
+  if (p.nseg > 1 && at >= p.first[1]) { seg = p.seg[1]; first = p.first[1]; }
+  if (p.nseg > 2 && at >= p.first[2]) { seg = p.seg[2]; first = p.first[2]; }
+  if (p.nseg > 3 && at >= p.first[3]) { seg = p.seg[3]; first = p.first[3]; }
+  const int n = (at - first) * 4 + (int)(threadIdx.x >> 6);
+  if (n >= seg.N) { return; }  // wave-uniform; no barrier in this kernel
+  float acc[1];
+  rows8_sums<1>(seg.w, seg.scales, seg.biases, p.x, n, p.K, acc);
+  if ((threadIdx.x & 63) != 0) { return; }
+  if (p.y_f32) {
+    static_cast<float*>(seg.y)[n] = acc[0];
+  } else {
+    uint32_t v = f32_to_bf16_bits(acc[0]);
+    if (p.residual != nullptr) { v = f32_to_bf16_bits(bf16_bits_to_f32(v) + bf16_bits_to_f32(p.residual[n])); }
+    static_cast<uint16_t*>(seg.y)[n] = (uint16_t)v;
+  }
+}
+
+hipError_t launch_qmv_row8(hipStream_t st, const QmvArgs& a, const QmvGroup& g)
+{
+  Row8Params p{};
+  p.x = a.x; p.residual = a.residual; p.K = a.K; p.y_f32 = a.y_f32 ? 1 : 0; p.nseg = g.count;
+  int blocks = 0;
+  for (int i = 0; i < g.count; ++i) {
+    p.seg[i] = g.seg[i];
+    p.first[i] = blocks;
+    blocks += (g.seg[i].N + 3) / 4;
+  }
+  return launch_kernel(qmv_row8_kernel, dim3((unsigned)blocks), dim3(256), 0, st, p);
 }
 
 hipError_t launch_qmv_rows8(hipStream_t st, const QmvArgs& a, int rows, const int* pair_eid, int x_div, int n_experts)
