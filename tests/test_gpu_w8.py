@@ -190,6 +190,25 @@ def test_one_row_w8_has_the_bits_of_a_gathered_pair(vpq, dev, D, K, N):
         assert torch.equal(o.view, vpq.qmv_w8g64(*t, x, K, t[0].shape[0], 1))
 
 
+@pytest.mark.parametrize("K,N,npair", [(4160, 1365, 24), (4160, 1366, 24), (5120, 40, 3), (5184, 40, 3)])
+def test_gathered_pairs_w8_over_a_long_k(vpq, dev, D, K, N, npair):
+    # few pairs and many on either side of the 32768 rows (of 256 CUs) where the kernel changes: the bits of the one-row call
+    E, gen = 5, torch.Generator(device=dev).manual_seed(K + N)
+    w = torch.randint(-2 ** 31, 2 ** 31, (E, N, K // 4), dtype=torch.int32, device=dev, generator=gen)
+    s = torch.empty((E, N, K // 64), device=dev).uniform_(0.0003, 0.0012, generator=gen).bfloat16()
+    b = (-128 * s.float()).bfloat16()
+    x = torch.randn((npair, K), device=dev, generator=gen).bfloat16()
+    eid = torch.randint(0, E, (npair,), dtype=torch.int32, device=dev, generator=gen)
+    eid[1] = -1
+    out = parity.Guarded((npair, N), torch.bfloat16, dev)
+    vpq.gather_down_qmv_w8g64(w, s, b, x, K, N, eid, E, out=out.view)
+    torch.cuda.synchronize()
+    out.assert_intact()
+    for p, e in enumerate(eid.tolist()):
+        want = vpq.qmv_w8g64(w[e], s[e], b[e], x[p:p + 1], K, N, 1)[0] if e >= 0 else torch.zeros_like(out.view[p])
+        assert torch.equal(out.view[p], want)
+
+
 def test_w8_gather_ids_out_of_range_and_bad_arguments(vpq, dev, D):
     K, inner, E = 256, 8, 3
     w, s, b = (np.stack([p[i] for p in [interleaved8(inner, K, 2800 + e) for e in range(E)]]) for i in range(3))

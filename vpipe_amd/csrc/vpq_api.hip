@@ -87,10 +87,22 @@ constexpr int kDenseRouteMinRows = 8192;
 // in three launches 18.3, in one 9.5.
 constexpr int kRow8MinK = 2560;
 
-// One row of x against the 8-bit packs of g, each with the bits that it has as an expert's slab of a gather.
+// Whether `rows` weight rows of 8-bit codes (of all pairs together) are worth the gathers' kernel.  In its fifth pass over K, from
+// 4096 on, it holds x in so many registers that a CU has eight wavefronts; one wavefront per weight row, sixteen and more a CU, is
+// ahead where the former would have no more than one set of four rows each (us, that / the gathers' kernel, pairs of K -> N:
+// one of 5120 -> 5120 8.7 / 10.0; 4 of 5120 -> 3072 15.7 / 17.3; 8 of 4160 -> 1536 13.1 / 15.1; 24 of 4160 -> 1536, 9216 sets,
+// 33.5 / 33.0; 32 of it 44.6 / 40.2; 8 of 4608 -> 5120, 10240 sets, 38.1 / 37.2; 32 of it 141 / 123).  Gated, where the other
+// kernel reads two rows a wavefront, the gathers' kernel always is (one token of 4 experts, 4608 -> 1536: 11.6 / 9.5).
+bool gather8_takes(int K, long rows, bool gated)
+{
+  return vpq::qmv_gather_supports(K, 8) && (K <= 4096 || gated || rows > 4 * 32L * g_dev.cu_count);
+}
+
+// One row of x against the 8-bit packs of g, each with the bits that it has as an expert's slab of a gather.  (Several packs: a
+// wavefront of one row would pay for the choice among them; q|k|v of 5120 13.1 us, on the gathers' kernel 11.8.)
 hipError_t launch_row8(hipStream_t hs, const vpq::QmvArgs& a, const vpq::QmvGroup& g)
 {
-  return vpq::qmv_gather_supports(a.K, 8) ? vpq::launch_qmv_gather_row8(hs, a, g) : vpq::launch_qmv_row8(hs, a, g);
+  return gather8_takes(a.K, g.seg[0].N, g.count > 1) ? vpq::launch_qmv_gather_row8(hs, a, g) : vpq::launch_qmv_row8(hs, a, g);
 }
 
 // One row of binary16 whose scales are no whole 16-byte pieces: the one-row kernel from the K on from which its error against
@@ -325,7 +337,7 @@ static int rows8_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* 
     a.M = rows;
     return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
   }
-  if (vpq::qmv_gather_supports(K, 8)) {
+  if (gather8_takes(K, (long)N * rows, gate_act != 0)) {
     hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
     if (gathered) { return finish(vpq::launch_qmv_gather(hs, a, 8, pair_eid, rows, x_div, n_experts)); }
     if (rows == 1) { return finish(vpq::launch_qmv_gather_row8(hs, a, vpq::QmvGroup{1, {{w, scales, biases, y, N}}})); }
