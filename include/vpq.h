@@ -500,7 +500,8 @@ int vpq_qmm_grouped_down_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, cons
  *                                    `affine_qmv_w4g32[_add]_q40` (:327-342, 387-403): the bias is
  *                                    -8 * scale computed in registers and `biases` is never read
  *                                    (may be NULL) -- bit-identical to the affine form on a pack
- *                                    whose stored bias is -8 * scale, 10 % fewer bytes.
+ *                                    whose stored bias is -8 * scale (at two rows and more: with
+ *                                    scales and biases 16-byte aligned), 10 % fewer bytes.
  *                                    QMV arithmetic, 1 <= M <= 16.
  *   vpq_qmv_gated_w4g32_bf16         replaces `affine_qmv_geglu_w4g32[_q40]` (:1451-1490) and the
  *                                    SwiGLU twin over an interleaved gate|up pack; y [M, N/2].

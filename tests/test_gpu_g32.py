@@ -68,6 +68,33 @@ def test_qmv_g32_scale_only_is_the_affine_form_on_a_q40_pack(vpq, oracle, dev, D
     parity.check_f32(vpq.qmv_w4g32(wd, sd, None, xd, K, N, M, f32out=True, scale_only=True).cpu().numpy(), y64)
 
 
+# below, at and above the one-row kernel's first K, every number of slices of 2048 and of parts of K, two rows and more
+@pytest.mark.parametrize("K,N,M", [(1504, 70, 1), (2048, 70, 1), (2080, 130, 1), (5120, 1030, 1), (6176, 70, 1), (12288, 515, 1),
+                                   (17408, 33, 1), (32768, 5, 1), (2080, 130, 2), (5120, 515, 2), (4096, 95, 8)])
+def test_qmv_g32_scale_only_has_the_affine_sums(vpq, dev, D, K, N, M):
+    # the fp32 sums, which a stored element seldom shows; single, with a residual, gated and grouped
+    packs = []
+    for i, n in enumerate((N, 18, 1)):
+        w, s, b = synth.make_weight_g32(n, K, 6350 + K + n + i, q40=True)
+        packs.append((*stage(D, dev, w, s, b), n))
+    w, s, b, _ = packs[0]
+    x = D.bf16(synth.make_act(M, K, 6450 + K + M), dev)
+    only = vpq.qmv_w4g32(w, s, None, x, K, N, M, f32out=True, scale_only=True)
+    assert torch.equal(only, vpq.qmv_w4g32(w, s, b, x, K, N, M, f32out=True))
+    res = D.bf16(synth.make_act(M, N, 6460), dev)
+    added = vpq.qmv_w4g32(w, s, None, x, K, N, M, residual=res, scale_only=True)
+    assert torch.equal(added, (only.bfloat16().float() + res.float()).bfloat16())
+    F = N // 2 * 2
+    gated = vpq.qmv_w4g32(w[:F], s[:F], None, x, K, F, M, activation=1, scale_only=True)
+    assert torch.equal(gated, vpq.qmv_w4g32(w[:F], s[:F], b[:F], x, K, F, M, activation=1))
+    outs = [parity.Guarded((M, p[3]), torch.bfloat16, dev) for p in packs]
+    vpq.qmv_group_w4g32([(p[0], p[1], p[1], p[3]) for p in packs], x, K, M, outs=[o.view for o in outs], scale_only=True)
+    torch.cuda.synchronize()
+    for p, o in zip(packs, outs):
+        o.assert_intact()
+        assert torch.equal(o.view, vpq.qmv_w4g32(p[0], p[1], None, x, K, p[3], M, scale_only=True))
+
+
 @pytest.mark.parametrize("scale_only", [False, True])
 @pytest.mark.parametrize("activation", [capi.VPQ_GATE_SWIGLU, capi.VPQ_GATE_GEGLU])
 @pytest.mark.parametrize("K,F,M", [(96, 17, 1), (2048, 64, 2), (2592, 40, 5), (4096, 128, 16)])

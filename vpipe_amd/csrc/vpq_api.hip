@@ -184,7 +184,7 @@ int qmv_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scales,
   // row, us: 4096 -> 4096 3.9 / 5.1, 12288 -> 4096 8.0 / 9.5, 4096 -> 24576 12.5 / 14.3, 5120 -> 151936 75 / 89).
   if (flow_ok) { return finish(vpq::launch_qmv_flow(hs, a)); }
   // One row over another K: its form with narrow scales, and for a short K the row-streaming kernel.
-  if ((K % 512) != 0 && vpq::qmv_flow_narrow_supports(K, N, M, 64)) { return finish(vpq::launch_qmv_flow_narrow(hs, a, 64)); }
+  if ((K % 512) != 0 && vpq::qmv_flow_narrow_supports(K, N, M, 64)) { return finish(vpq::launch_qmv_flow_narrow(hs, a, vpq::BatchFormat{})); }
   if (M == 1 && (K % 512) != 0) { return finish(vpq::launch_qmv_rows(hs, a, 0)); }
   if (batch_ok) { return finish(launch_batch(hs, a, vpq::BatchFormat{})); }
   // A K too deep for the batch kernel's LDS (above 114176), or scales or biases off 16-byte alignment.
@@ -767,8 +767,8 @@ static int qmv_f16_common(vpq_stream_t stream, const uint32_t* w, const uint16_t
   if (vpq::qmv_flow_supports(K, N, M) && aligned(scales, 16) && aligned(biases, 16)) {
     return finish(vpq::launch_qmv_flow_f16(reinterpret_cast<hipStream_t>(stream), a));
   }
-  if (flow_narrow_f16(K, N, M)) { return finish(vpq::launch_qmv_flow_narrow(reinterpret_cast<hipStream_t>(stream), a, 64, true)); }
   const vpq::BatchFormat f{4, 64, true, false};
+  if (flow_narrow_f16(K, N, M)) { return finish(vpq::launch_qmv_flow_narrow(reinterpret_cast<hipStream_t>(stream), a, f)); }
   if (vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && aligned(biases, 16)) {
     return finish(launch_batch(reinterpret_cast<hipStream_t>(stream), a, f));
   }
@@ -1479,14 +1479,14 @@ int qmv_g32_common(vpq_stream_t stream, const uint32_t* w, const uint16_t* scale
   a.gate_act = gate_act;
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
   if (gelu_mul) { return finish(vpq::launch_qmv_simple_g32(hs, a, scale_only)); }    // the kernel that has this store
-  // one row of x: the one-row kernel, or for a short K (and Q4_0) the row-streaming one; more: the batch kernel (us, row-streaming /
-  // batch / one-row: one row 4096 -> 24576 16.9 / 17.9 / 13.8, 12288 -> 4096 9.7 / 11.7 / 9.1, 4096 -> 4096 5.8 / 6.0 / 4.2; two rows
-  // 23.3 / 17.9, 12.6 / 11.7 and 6.9 / 6.0)
+  // one row of x: the one-row kernel, or for a short K the row-streaming one; more: the batch kernel.  Each takes packs with and
+  // without biases, and gives both the same bits.  (us, row-streaming / batch / one-row: one row 4096 -> 24576 16.9 / 17.9 / 13.8,
+  // 12288 -> 4096 9.7 / 11.7 / 9.1, 4096 -> 4096 5.8 / 6.0 / 4.2; two rows 23.3 / 17.9, 12.6 / 11.7 and 6.9 / 6.0)
   const vpq::BatchFormat f{4, 32, false, scale_only};
   if (M > 1 && vpq::qmv_batch_supports(K, M, f) && aligned(scales, 16) && (scale_only || aligned(biases, 16))) {
     return finish(launch_batch(hs, a, f));
   }
-  if (!scale_only && vpq::qmv_flow_narrow_supports(K, N, M, 32)) { return finish(vpq::launch_qmv_flow_narrow(hs, a, 32)); }
+  if (vpq::qmv_flow_narrow_supports(K, N, M, 32)) { return finish(vpq::launch_qmv_flow_narrow(hs, a, f)); }
   if (M <= 2) { return finish(vpq::launch_qmv_rows_g32(hs, a, scale_only)); }
   return finish(vpq::launch_qmv_simple_g32(hs, a, scale_only));
 }
@@ -1727,7 +1727,7 @@ int vpq_qmv_group_w4g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
   for (int i = 0; i < count; ++i) { g.seg[i] = vpq::QmvSeg{w[i], scales[i], biases[i], y[i], N[i]}; }
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
   if (flow) { return finish(vpq::launch_qmv_flow_group(hs, a, g)); }
-  if (narrow) { return finish(vpq::launch_qmv_flow_narrow_group(hs, a, g, 64)); }
+  if (narrow) { return finish(vpq::launch_qmv_flow_narrow_group(hs, a, g, vpq::BatchFormat{})); }
   if (rows) { return finish(vpq::launch_qmv_rows_group(hs, a, g)); }
   return finish(vpq::launch_qmv_batch(hs, a, g, vpq::BatchFormat{}));
 }
@@ -1773,8 +1773,8 @@ int vpq_qmv_group_w4g32_bf16(vpq_stream_t stream, int count, const uint32_t* con
   g.count = count;
   for (int i = 0; i < count; ++i) { g.seg[i] = vpq::QmvSeg{w[i], scales[i], scale_only ? nullptr : biases[i], y[i], N[i]}; }
   if (batch) { return finish(vpq::launch_qmv_batch(reinterpret_cast<hipStream_t>(stream), a, g, f)); }
-  if (scale_only == 0 && vpq::qmv_flow_narrow_supports(K, 1, M, 32)) {
-    return finish(vpq::launch_qmv_flow_narrow_group(reinterpret_cast<hipStream_t>(stream), a, g, 32));
+  if (vpq::qmv_flow_narrow_supports(K, 1, M, 32)) {
+    return finish(vpq::launch_qmv_flow_narrow_group(reinterpret_cast<hipStream_t>(stream), a, g, f));
   }
   return finish(vpq::launch_qmv_rows_group(reinterpret_cast<hipStream_t>(stream), a, g, 32, scale_only != 0));
 }
@@ -1878,7 +1878,7 @@ int vpq_qmv_group_w4g64_f16(vpq_stream_t stream, int count, const uint32_t* cons
   g.count = count;
   for (int i = 0; i < count; ++i) { g.seg[i] = vpq::QmvSeg{w[i], scales[i], biases[i], y[i], N[i]}; }
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
-  if (narrow) { return finish(vpq::launch_qmv_flow_narrow_group(hs, a, g, 64, true)); }
+  if (narrow) { return finish(vpq::launch_qmv_flow_narrow_group(hs, a, g, f)); }
   return finish(flow ? vpq::launch_qmv_flow_group(hs, a, g, true) : vpq::launch_qmv_batch(hs, a, g, f));
 }
 

@@ -194,8 +194,8 @@ hipError_t launch_qmv_flow_f16(hipStream_t st, const QmvArgs& a);    // IEEE bin
 hipError_t launch_qmv_flow_group(hipStream_t st, const QmvArgs& a, const QmvGroup& g, bool f16 = false);
 // ... where a row's scales are no whole number of 16-byte pieces, or belong to groups of 32.
 bool qmv_flow_narrow_supports(int K, int N, int M, int group);
-hipError_t launch_qmv_flow_narrow(hipStream_t st, const QmvArgs& a, int group, bool f16 = false);
-hipError_t launch_qmv_flow_narrow_group(hipStream_t st, const QmvArgs& a, const QmvGroup& g, int group, bool f16 = false);
+hipError_t launch_qmv_flow_narrow(hipStream_t st, const QmvArgs& a, const BatchFormat& f);
+hipError_t launch_qmv_flow_narrow_group(hipStream_t st, const QmvArgs& a, const QmvGroup& g, const BatchFormat& f);
 bool qmv_stream_supports(int K, int N, int M);
 hipError_t launch_qmv_stream(hipStream_t st, const QmvArgs& a);
 bool qmv_ring_supports(int K, int N, int M);

@@ -511,6 +511,9 @@ qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
               acc[t][a][q] = fmaf(s, s4[a][q], acc[t][a][q]);
               off[t][a][q] = fmaf(b2, xs[a][q], off[t][a][q]);
             } else {
+              // (not contracted: the product of a last, single group would join its addition without the bias between them, and
+              // a Q4_0 pack not have the bits of one that stores its biases)
+#pragma clang fp contract(off)
               float v = (grp & 1) == 0 ? s * s4[a][q] : fmaf(s, s4[a][q], off[t][a][q]);
               if (!SONLY) { v = fmaf(b2, xs[a][q], v); }
               if ((grp & 1) == 0 && !(decltype(part_c)::value && grp + 1 >= live)) {

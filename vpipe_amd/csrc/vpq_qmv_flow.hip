@@ -18,7 +18,7 @@
 //   3. scales and biases of the wavefront's rows and K range: 16-byte direct-to-LDS loads
 //      (1 KB per instruction, scales and biases in the same instruction where they fit), or, where
 //      a row of them is no whole number of 16-byte pieces (K that is no multiple of 512; groups of
-//      32 as well), one 2-byte register load of each per lane, row and slice.  They
+//      32 as well), one 2-byte register load of each (Q4_0: of the scale) per lane, row and slice.  They
 //      are applied to the per-(row, slice) dot products at the end.
 // The loads are inline assembly so that the only waits are the counted ones written here: the
 // compiler would otherwise wait for every outstanding load before the first LDS read.
@@ -186,9 +186,10 @@ __device__ __forceinline__ void pin_scalar(const T& v) { asm volatile("" : : "s"
 // Measured (us, that kernel / now): groups of 64, 3840 -> 3840 5.5 / 4.0, 3840 -> 19328 13.6 / 10.7, 9664 -> 3840 8.3 / 7.9; groups of
 // 32, 4096 -> 4096 5.8 / 4.2, 4096 -> 24576 17.0 / 13.8, 12288 -> 4096 9.7 / 9.1.  Where 16-byte pieces fit, both forms are level up to
 // K = 6144, and the pieces 4 to 6 % faster above (12288 -> 4096 8.6 / 8.9).
+// SONLY (groups of 32): a Q4_0 pack, b = -8 s and no biases are read; the bits of a pack that stores them.
 // PRELOADED: the arguments are already in scalar registers (nothing to batch; the residual is left to be loaded
 // when the store needs it).
-template <int SPW, int RB, bool F32OUT, int C, bool F16 = false, bool PRELOADED = false, int NARROW = 0>
+template <int SPW, int RB, bool F32OUT, int C, bool F16 = false, bool PRELOADED = false, int NARROW = 0, bool SONLY = false>
 __device__ __forceinline__ void qmv_flow_body(const FlowParams<C>& p)
 {
   constexpr int NL = RB * SPW;                 // code loads of a wavefront
@@ -306,9 +307,10 @@ __device__ __forceinline__ void qmv_flow_body(const FlowParams<C>& p)
   float tot[RB];
 
   // codes
-  constexpr int AFTER = NARROW ? 2 * NL : NDMA;   // requests that follow the codes
+  constexpr int AFTER = NARROW ? (SONLY ? NL : 2 * NL) : NDMA;   // requests that follow the codes
   u32x4v c[RB][SPW];
-  uint32_t sreg[NARROW ? RB : 1][SPW], breg[NARROW ? RB : 1][SPW];
+  static_assert(NARROW == 5 || !SONLY, "");
+  uint32_t sreg[NARROW ? RB : 1][SPW], breg[NARROW && !SONLY ? RB : 1][SPW];
   {
     const uint8_t* wbase = reinterpret_cast<const uint8_t*>(wq) + (size_t)row_begin * (size_t)(K >> 1);
 #pragma unroll
@@ -326,12 +328,12 @@ __device__ __forceinline__ void qmv_flow_body(const FlowParams<C>& p)
         constexpr int r = decltype(rc)::value;
         const int rr = (row_begin + r < N) ? r : (N - 1 - row_begin);
         const uint16_t* srow = sq + (size_t)(row_begin + rr) * Kg;
-        const uint16_t* brow = bq + (size_t)(row_begin + rr) * Kg;
+        const uint16_t* brow = SONLY ? nullptr : bq + (size_t)(row_begin + rr) * Kg;
         static_for<0, SPW>([&](auto sc_) {
           constexpr int s = decltype(sc_)::value;
           const uint32_t at = kvalid[s] ? (uint32_t)(((slice0 + s) * kSlice + lane * 32) >> NARROW) * 2u : 0u;
           sreg[r][s] = gload2(srow, at);
-          breg[r][s] = gload2(brow, at);
+          if constexpr (!SONLY) { breg[r][s] = gload2(brow, at); }
         });
       });
     } else {
@@ -401,9 +403,14 @@ __device__ __forceinline__ void qmv_flow_body(const FlowParams<C>& p)
         static_for<0, SPW>([&](auto sc_) {
           constexpr int s = decltype(sc_)::value;
           touch(sreg[r][s]);
-          touch(breg[r][s]);
-          acc[r] = fmaf(elt_bits_to_f32<F16>(sreg[r][s]), fmaf(kOffset, sx[s], dots[r][s]), acc[r]);
-          acc[r] = fmaf(elt_bits_to_f32<F16>(breg[r][s]), sx[s], acc[r]);
+          const float sc = elt_bits_to_f32<F16>(sreg[r][s]);
+          float bi = -8.0f * sc;
+          if constexpr (!SONLY) {
+            touch(breg[r][s]);
+            bi = elt_bits_to_f32<F16>(breg[r][s]);
+          }
+          acc[r] = fmaf(sc, fmaf(kOffset, sx[s], dots[r][s]), acc[r]);
+          acc[r] = fmaf(bi, sx[s], acc[r]);
         });
       });
     } else {
@@ -483,7 +490,7 @@ __device__ __forceinline__ void qmv_flow_body(const FlowParams<C>& p)
 // kernel-argument preloading, which delivers the first sixteen words in scalar registers when a wavefront starts,
 // so a wavefront's first requests do not wait for a load of the argument buffer (an aggregate argument is not
 // preloaded).
-template <int SPW, int RB, bool F32OUT, bool F16, int NARROW>
+template <int SPW, int RB, bool F32OUT, bool F16, int NARROW, bool SONLY>
 __global__ __launch_bounds__(64 * kMaxWavesPerWg) void qmv_flow_kernel_1(
     const uint16_t* x, const uint32_t* w, const uint16_t* scales, const uint16_t* biases, void* y, int K, uint32_t shape,
     int N, const uint16_t* residual)
@@ -493,7 +500,7 @@ __global__ __launch_bounds__(64 * kMaxWavesPerWg) void qmv_flow_kernel_1(
   FlowParams<1> p;
   p.h.x = x; p.h.residual = residual; p.h.K = K; p.h.shape = shape;
   p.w[0] = w; p.scales[0] = scales; p.biases[0] = biases; p.y[0] = y; p.N[0] = N; p.first_block[0] = 0;
-  qmv_flow_body<SPW, RB, F32OUT, 1, F16, true, NARROW>(p);
+  qmv_flow_body<SPW, RB, F32OUT, 1, F16, true, NARROW, SONLY>(p);
 }
 
 // The grouped form (2..4 packs sharing x) with preloaded arguments: the fourteen preloaded words hold what every
@@ -509,7 +516,7 @@ struct FlowRest {
   int N[C - 1];
 };
 
-template <int SPW, int RB, bool F32OUT, int C, bool F16, int NARROW>
+template <int SPW, int RB, bool F32OUT, int C, bool F16, int NARROW, bool SONLY>
 __global__ __launch_bounds__(64 * kMaxWavesPerWg) void qmv_flow_kernel_g(
     const uint16_t* x, int K, uint32_t shape, int N0, int fb1, int fb2, int fb3, const uint32_t* w0,
     const uint16_t* scales0, const uint16_t* biases0, const FlowRest<C> rest)
@@ -523,7 +530,7 @@ __global__ __launch_bounds__(64 * kMaxWavesPerWg) void qmv_flow_kernel_g(
     p.w[i] = rest.w[i - 1]; p.scales[i] = rest.scales[i - 1]; p.biases[i] = rest.biases[i - 1]; p.y[i] = rest.y[i - 1];
     p.N[i] = rest.N[i - 1]; p.first_block[i] = fb[i - 1];
   }
-  qmv_flow_body<SPW, RB, F32OUT, C, F16, true, NARROW>(p);
+  qmv_flow_body<SPW, RB, F32OUT, C, F16, true, NARROW, SONLY>(p);
 }
 
 namespace {
@@ -531,8 +538,8 @@ namespace {
 struct FlowPlan {
   int spw, wk, wr, rb;
 };
-// Elements, and how scales and biases come (qmv_flow_body's NARROW).
-enum class FlowForm { kWide, kF16, kNarrow64, kNarrow32, kNarrowF16 };
+// Elements, and how scales and biases come (qmv_flow_body's NARROW and SONLY).
+enum class FlowForm { kWide, kF16, kNarrow64, kNarrow32, kNarrowQ40, kNarrowF16 };
 
 // Slices per wavefront and K parts, from measurements on MI355X with HBM-cold packs: up to three slices (K <= 6144)
 // a wavefront walks the whole K; longer rows are split between 2 to 4 wavefronts of the workgroup (12288->4096:
@@ -562,13 +569,13 @@ FlowPlan flow_plan(int K, double pack_bytes)
   return pl;
 }
 
-template <int S, int R, bool F32, int C, bool F16, int NARROW>
+template <int S, int R, bool F32, int C, bool F16, int NARROW, bool SONLY = false>
 hipError_t launch_flow_kernel(dim3 grid, dim3 block, size_t lds_bytes, hipStream_t st, const FlowParams<C>& p)
 {
   static std::once_flag once;          // one per instantiation
   static hipError_t attr_status = hipSuccess;
   if constexpr (C == 1) {
-    const auto kern = qmv_flow_kernel_1<S, R, F32, F16, NARROW>;
+    const auto kern = qmv_flow_kernel_1<S, R, F32, F16, NARROW, SONLY>;
     std::call_once(once, [&] {
       attr_status = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                         kMaxLdsBytes);
@@ -578,7 +585,7 @@ hipError_t launch_flow_kernel(dim3 grid, dim3 block, size_t lds_bytes, hipStream
                          p.h.shape, p.N[0], p.h.residual);
   } else {
     // a grouped launch has no residual
-    const auto kern = qmv_flow_kernel_g<S, R, F32, C, F16, NARROW>;
+    const auto kern = qmv_flow_kernel_g<S, R, F32, C, F16, NARROW, SONLY>;
     std::call_once(once, [&] {
       attr_status = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                         kMaxLdsBytes);
@@ -619,6 +626,7 @@ hipError_t dispatch_flow(const FlowPlan& pl, bool y_f32, const FlowHead& h, cons
     if (form == FlowForm::kF16) { return launch_flow_kernel<S, R, kF32, C, true, 0>(grid, block, lds_bytes, st, p); }
     if (form == FlowForm::kNarrow64) { return launch_flow_kernel<S, R, kF32, C, false, 6>(grid, block, lds_bytes, st, p); }
     if (form == FlowForm::kNarrow32) { return launch_flow_kernel<S, R, kF32, C, false, 5>(grid, block, lds_bytes, st, p); }
+    if (form == FlowForm::kNarrowQ40) { return launch_flow_kernel<S, R, kF32, C, false, 5, true>(grid, block, lds_bytes, st, p); }
     if (form == FlowForm::kNarrowF16) { return launch_flow_kernel<S, R, kF32, C, true, 6>(grid, block, lds_bytes, st, p); }
     return launch_flow_kernel<S, R, kF32, C, false, 0>(grid, block, lds_bytes, st, p);
   };
@@ -684,10 +692,12 @@ bool qmv_flow_narrow_supports(int K, int N, int M, int group)
 
 namespace {
 
-FlowForm flow_narrow(int group, bool f16)
+FlowForm flow_narrow(const BatchFormat& f)
 {
-  return f16 ? FlowForm::kNarrowF16 : group == 32 ? FlowForm::kNarrow32 : FlowForm::kNarrow64;
+  return f.f16 ? FlowForm::kNarrowF16 : f.scale_only ? FlowForm::kNarrowQ40 : f.group == 32 ? FlowForm::kNarrow32 : FlowForm::kNarrow64;
 }
+
+double flow_narrow_bytes(const BatchFormat& f) { return f.group == 64 || f.scale_only ? 9.0 / 16.0 : 5.0 / 8.0; }   // per weight
 
 hipError_t launch_flow_one(hipStream_t st, const QmvArgs& a, double bytes_per_weight, FlowForm form)
 {
@@ -702,9 +712,9 @@ hipError_t launch_qmv_flow(hipStream_t st, const QmvArgs& a) { return launch_flo
 // The same kernel over IEEE binary16 elements (x, scales, biases, y, residual).
 hipError_t launch_qmv_flow_f16(hipStream_t st, const QmvArgs& a) { return launch_flow_one(st, a, 9.0 / 16.0, FlowForm::kF16); }
 
-hipError_t launch_qmv_flow_narrow(hipStream_t st, const QmvArgs& a, int group, bool f16)
+hipError_t launch_qmv_flow_narrow(hipStream_t st, const QmvArgs& a, const BatchFormat& f)
 {
-  return launch_flow_one(st, a, group == 32 ? 5.0 / 8.0 : 9.0 / 16.0, flow_narrow(group, f16));
+  return launch_flow_one(st, a, flow_narrow_bytes(f), flow_narrow(f));
 }
 
 namespace {
@@ -730,9 +740,9 @@ hipError_t launch_qmv_flow_group(hipStream_t st, const QmvArgs& a, const QmvGrou
   return launch_flow_group(st, a, g, 9.0 / 16.0, f16 ? FlowForm::kF16 : FlowForm::kWide);
 }
 
-hipError_t launch_qmv_flow_narrow_group(hipStream_t st, const QmvArgs& a, const QmvGroup& g, int group, bool f16)
+hipError_t launch_qmv_flow_narrow_group(hipStream_t st, const QmvArgs& a, const QmvGroup& g, const BatchFormat& f)
 {
-  return launch_flow_group(st, a, g, group == 32 ? 5.0 / 8.0 : 9.0 / 16.0, flow_narrow(group, f16));
+  return launch_flow_group(st, a, g, flow_narrow_bytes(f), flow_narrow(f));
 }
 
 }  // namespace vpq
