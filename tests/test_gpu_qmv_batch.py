@@ -136,6 +136,41 @@ def test_grouped_launch_of_the_batch_kernel(vpq, dev, D, fmt):
         assert torch.equal(o.view, single(w, s, b, xd, K, N, M))
 
 
+# the K of the one-row kernel in 16-byte pieces, of its narrow form, of neither
+@pytest.mark.parametrize("K,M", [(4096, 1), (2560, 2), (4096, 3), (2112, 1), (2112, 2), (1024, 1), (1344, 1), (1344, 2), (1344, 5)])
+@pytest.mark.parametrize("fmt", ["w4g32", "q4_0", "w8g64", "f16"])
+def test_grouped_launch_with_a_pack_off_alignment(vpq, dev, fmt, K, M):
+    # one pack with scales two bytes off a 16-byte boundary: every pack has the bits of its own call.  The second half of K
+    # nearly cancels the first, so that another order of additions shows in the stored elements.
+    bits, group, dtype = {"w4g64": (4, 64, torch.bfloat16), "w8g64": (8, 64, torch.bfloat16), "f16": (4, 64, torch.float16)}.get(
+        fmt, (4, 32, torch.bfloat16))
+    half = K // 128 * 64
+    gen = torch.Generator(device=dev).manual_seed(K + M)
+    packs = []
+    for i, N in enumerate((1030, 610, 40)):
+        w = torch.randint(-2 ** 31, 2 ** 31, (N, K * bits // 32), dtype=torch.int32, device=dev, generator=gen)
+        s = torch.empty((N, K // group), device=dev).uniform_(0.005, 0.02, generator=gen).to(dtype)
+        for t, per in ((w, 32 // bits), (s, group)):
+            t[:, half // per:2 * half // per] = t[:, :half // per]
+        if i == 1:
+            s = torch.cat([s.new_zeros(1), s.view(-1)])[1:].view(s.shape)
+            assert s.data_ptr() % 16 == 2
+        packs.append((w, s, (-8 * s.float()).to(dtype), N))
+    x = torch.randn((M, K), device=dev, generator=gen)
+    x[:, half:2 * half] = -x[:, :half] * (1 + torch.randn((M, half), device=dev, generator=gen) / 64)
+    x[:, 2 * half:] /= 64
+    x = x.to(dtype)
+    outs = [parity.Guarded((M, p[3]), dtype, dev) for p in packs]
+    so = {"scale_only": True} if fmt == "q4_0" else {}
+    run, single = {"w4g64": (vpq.qmv_group_w4g64, vpq.qmv_w4g64), "w8g64": (vpq.qmv_group_w8g64, vpq.qmv_w8g64),
+                   "f16": (vpq.qmv_group_w4g64_f16, vpq.qmv_w4g64_f16)}.get(fmt, (vpq.qmv_group_w4g32, vpq.qmv_w4g32))
+    run(packs, x, K, M, outs=[o.view for o in outs], **so)
+    torch.cuda.synchronize()
+    for (w, s, b, N), o in zip(packs, outs):
+        o.assert_intact()
+        assert torch.equal(o.view, single(w, s, b, x, K, N, M, **so))
+
+
 def _weight64(fmt, w, s, b, K):
     """The pack in float64, from its words."""
     bits, group = (8, 64) if fmt == "w8g64" else (4, 32 if fmt in ("w4g32", "q4_0") else 64)

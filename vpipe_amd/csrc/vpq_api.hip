@@ -1757,7 +1757,7 @@ int vpq_qmv_group_w4g32_bf16(vpq_stream_t stream, int count, const uint32_t* con
   for (int i = 0; i < count; ++i) {
     batch = batch && aligned(scales[i], 16) && (scale_only != 0 || aligned(biases[i], 16));
   }
-  if (M > 2 && !batch) {
+  if (M > 1 && !batch) {                                // (a pack's own alignment chooses its kernel)
     for (int i = 0; i < count; ++i) {
       const int st = vpq_qmv_w4g32_bf16(stream, w[i], scales[i], scale_only ? nullptr : biases[i], x, y[i], K, N[i], M,
                                         nullptr, scale_only);
