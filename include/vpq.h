@@ -284,7 +284,8 @@ int vpq_linear_w4g64_bf16(vpq_stream_t stream, const uint32_t* w, const uint16_t
  * vpq_qmv_w4g64_bf16 per pack (no residual); results are bit-identical to
  * `count` separate calls of it (VPQ_QMV_AUTO).  The pointer tables are host
  * arrays, read before the call returns.  Packs whose scales or biases are not
- * 16-byte aligned run as separate launches at M > 2. */
+ * 16-byte aligned run as separate launches at M > 2, and so do packs of which
+ * some are aligned and others not (but for one row with K % 512 != 0). */
 int vpq_qmv_group_w4g64_bf16(vpq_stream_t stream, int count, const uint32_t* const* w,
                              const uint16_t* const* scales, const uint16_t* const* biases,
                              const uint16_t* x, uint16_t* const* y, int K, const int* N, int M);

@@ -138,7 +138,7 @@ def test_grouped_launch_of_the_batch_kernel(vpq, dev, D, fmt):
 
 # the K of the one-row kernel in 16-byte pieces, of its narrow form, of neither
 @pytest.mark.parametrize("K,M", [(4096, 1), (2560, 2), (4096, 3), (2112, 1), (2112, 2), (1024, 1), (1344, 1), (1344, 2), (1344, 5)])
-@pytest.mark.parametrize("fmt", ["w4g32", "q4_0", "w8g64", "f16"])
+@pytest.mark.parametrize("fmt", ["w4g64", "w4g32", "q4_0", "w8g64", "f16"])
 def test_grouped_launch_with_a_pack_off_alignment(vpq, dev, fmt, K, M):
     # one pack with scales two bytes off a 16-byte boundary: every pack has the bits of its own call.  The second half of K
     # nearly cancels the first, so that another order of additions shows in the stored elements.

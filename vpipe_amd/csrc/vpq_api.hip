@@ -1694,22 +1694,24 @@ int vpq_qmv_group_w4g64_bf16(vpq_stream_t stream, int count, const uint32_t* con
 {
   if (w == nullptr || scales == nullptr || biases == nullptr || y == nullptr || N == nullptr) { return VPQ_ERR_NULL_POINTER; }
   if (count < 1 || count > 4) { return VPQ_ERR_BAD_SHAPE; }
-  bool wide = true;                                     // 16-byte loads of every pack's scales and biases
+  int wides = 0;                                        // packs whose scales and biases allow 16-byte loads
   for (int i = 0; i < count; ++i) {
     int st = check_pack(w[i], scales[i], biases[i], K, N[i]);
     if (st != VPQ_OK) { return st; }
     if (y[i] == nullptr) { return VPQ_ERR_NULL_POINTER; }
     if (!aligned(y[i], 2)) { return VPQ_ERR_MISALIGNED; }
-    wide = wide && aligned(scales[i], 16) && aligned(biases[i], 16);
+    wides += aligned(scales[i], 16) && aligned(biases[i], 16) ? 1 : 0;
   }
   if (x == nullptr) { return VPQ_ERR_NULL_POINTER; }
   if (M < 1 || M > 16) { return VPQ_ERR_BAD_SHAPE; }
   if (!aligned(x, 16)) { return VPQ_ERR_MISALIGNED; }
-  // The kernels of the single call (qmv_common), each in its grouped form.
+  // The kernels of the single call (qmv_common), each in its grouped form.  Packs of both kinds have the same one only at one row
+  // of a K that is no multiple of 512.
+  const bool wide = wides == count, mixed = wides != 0 && !wide && !(M == 1 && (K % 512) != 0);
   const bool batch = wide && vpq::qmv_batch_supports(K, M, vpq::BatchFormat{});
   const bool flow = batch && vpq::qmv_flow_supports(K, 1, M);
   const bool narrow = (K % 512) != 0 && vpq::qmv_flow_narrow_supports(K, 1, M, 64);
-  const bool rows = !narrow && vpq::qmv_rows_supports(K, 1, M) && (!wide || (K % 512) != 0) && (!batch || M == 1);
+  const bool rows = !narrow && !mixed && vpq::qmv_rows_supports(K, 1, M) && (!wide || (K % 512) != 0) && (!batch || M == 1);
   if (!flow && !narrow && !rows && !batch) {
     for (int i = 0; i < count; ++i) {
       const int st = vpq_qmv_w4g64_bf16(stream, w[i], scales[i], biases[i], x, y[i], K, N[i], M, nullptr, nullptr, 0,
