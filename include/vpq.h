@@ -702,13 +702,13 @@ int vpq_qmm_dense_route_w8g64_bf16(vpq_stream_t stream, const uint32_t* w, const
  * and half: apple-silicon/metal-compute/CMakeLists.txt:71-72, 159-162; the
  * metallibs without the `_bf16` suffix).  These entries are the f16 forms of
  * the 4-bit group-64 functions: scales, biases, x, y, residual and w_deq are
- * IEEE binary16 bit patterns, the packed codes are the same.  One row of x on
- * K % 512 == 0, K >= 2048 with 16-byte aligned scales and biases takes the
- * streaming decode kernel of the bf16 entry on binary16 arithmetic (same
- * speed), 2..16 rows on K % 512 == 0 the ring kernel (VPQ_QMV_RING) or, for 2..4
- * rows over 150 MB of codes and more, the streaming kernel (VPQ_QMV_STREAM) on
- * binary16 arithmetic; every other QMV shape takes a general path (one wavefront per
- * output row); the QMM is expansion + the dense GEMM:
+ * IEEE binary16 bit patterns, the packed codes are the same.  The QMV runs the
+ * kernels of the bf16 entry on binary16 arithmetic: the one-row kernel where
+ * K % 512 == 0, K >= 2048 with 16-byte aligned scales and biases and, in its form
+ * with narrow loads, for any other K >= 3072; the batch kernel for every other
+ * aligned pack, one wavefront per output row for the rest.  An infinity in a row of
+ * x gives +-inf or NaN as the plain sum would; in the first of these forms NaN.
+ * The QMM is expansion + the dense GEMM:
  *   vpq_dequant_w4g64_f16         `affine_dequant_w4g64` (affine_dequant.metal:25-58), bit-exact:
  *                                 f16_rne(fp32(s) * q + fp32(b)).
  *   vpq_qmv_w4g64_f16 / _f32out   `affine_qmv_w4g64[_add]` (affine_qmv.metal:286-301, 347-363),
@@ -751,7 +751,8 @@ int vpq_qmm_lora_w4g64_f16(vpq_stream_t stream, const uint32_t* w, const uint16_
                            uint16_t* lora_t_ws);
 /* The grouped launch on binary16 elements (`affine_qmv_qkv_w4g64` of the half build, affine_qmv.metal:497-516):
  * arguments and results as vpq_qmv_group_w4g64_bf16 -- bit-identical to `count` calls of vpq_qmv_w4g64_f16; one
- * launch at M = 1 on K % 512 == 0, K >= 2048 with 16-byte aligned scales / biases, separate calls otherwise. */
+ * launch where every pack's scales and biases are 16-byte aligned, or M = 1, K >= 3072 and K % 512 != 0; separate calls
+ * otherwise. */
 int vpq_qmv_group_w4g64_f16(vpq_stream_t stream, int count, const uint32_t* const* w,
                             const uint16_t* const* scales, const uint16_t* const* biases,
                             const uint16_t* x, uint16_t* const* y, int K, const int* N, int M);

@@ -225,6 +225,35 @@ def test_rows_of_x_that_are_not_finite(vpq, dev, D, fmt, K):
         assert torch.equal(torch.isnan(gated), torch.isnan(ref)) and torch.equal(torch.isinf(gated), torch.isinf(ref))
 
 
+# K on either side of where one row leaves the batch kernel, in one part and in several, of two and of four weight rows a wavefront
+@pytest.mark.parametrize("K,N", [(2112, 70), (3136, 70), (3136, 23001), (9664, 69), (17472, 2400)])
+def test_one_row_of_binary16_that_is_not_finite(vpq, dev, K, N):
+    # an infinity in x gives +-inf by the weight's sign, NaN where the weight is zero or infinities meet; a NaN gives NaN
+    gen = torch.Generator(device=dev).manual_seed(K + N)
+    w = torch.randint(-2 ** 31, 2 ** 31, (N, K // 8), dtype=torch.int32, device=dev, generator=gen)
+    s = torch.empty((N, K // 64), device=dev).uniform_(0.005, 0.02, generator=gen).half()
+    b = (-8 * s.float()).half()
+    q = torch.stack([(w[:, [0, K // 16, K // 8 - 1]] >> 4 * i) & 15 for i in range(8)], -1).float()     # codes of three words
+    W = q * s[:, [0, K // 128, K // 64 - 1], None].float() + b[:, [0, K // 128, K // 64 - 1], None].float()
+    x = torch.randn((K,), device=dev, generator=gen).half()
+    for at, inf in (((0, 5),), (1.0,)), (((2, 7),), (-1.0,)), (((0, 5), (1, 3)), (1.0, -1.0)):
+        bad = x.clone()
+        want = torch.zeros((N,), device=dev)
+        for (word, i), sign in zip(at, inf):
+            bad[[0, K // 2, K - 8][word] + i] = sign * float("inf")
+            want = want + sign * float("inf") * W[:, word, i]
+        assert torch.isinf(want).any() and torch.isnan(want).any()
+        got = vpq.qmv_w4g64_f16(w, s, b, bad[None], K, N, 1, f32out=True)[0]
+        assert torch.equal(torch.nan_to_num(got, nan=7.0), torch.nan_to_num(want, nan=7.0))
+        out = vpq.qmv_w4g64_f16(w, s, b, bad[None], K, N, 1, residual=x[None, :1].expand(1, N).contiguous())[0]
+        assert torch.equal(torch.nan_to_num(out.float(), nan=7.0, posinf=1e9, neginf=-1e9), torch.nan_to_num(want, nan=7.0, posinf=1e9, neginf=-1e9))
+        outs = vpq.qmv_group_w4g64_f16([(w[:40], s[:40], b[:40], 40), (w[40:], s[40:], b[40:], N - 40)], bad[None], K, 1)
+        assert torch.equal(torch.nan_to_num(torch.cat(outs, 1)[0].float(), nan=7.0), torch.nan_to_num(want.half().float(), nan=7.0))
+    bad = x.clone()
+    bad[70] = float("nan")
+    assert torch.isnan(vpq.qmv_w4g64_f16(w, s, b, bad[None], K, N, 1)).all()
+
+
 @pytest.mark.parametrize("K", [960, 3840, 9664])
 @pytest.mark.parametrize("fmt", ["w4g64", "w4g32", "q4_0", "w8g64", "f16"])
 def test_fp32_results_are_as_close_as_a_plain_sum(vpq, dev, D, fmt, K):

@@ -142,4 +142,32 @@ __device__ __forceinline__ float wave_sum(float v)
   return v;
 }
 
+// sum over k of x[k] * fma(scale, q[k], bias) of one output, by a whole wavefront: 16 bytes of codes per lane and pass,
+// the order of the general kernels (vpq_qmv_simple.hip).
+template <int BITS, int GROUP, bool F16, bool SONLY>
+__device__ float plain_sum(const uint8_t* codes, const uint16_t* scales, const uint16_t* biases, const uint16_t* x, int K)
+{
+  constexpr int kPer = 128 / BITS;                          // values of a lane's 16 bytes
+  float acc = 0.0f;
+  for (int k0 = (int)(threadIdx.x & 63) * kPer; k0 < K; k0 += kWave * kPer) {
+    const uint4 c4 = *reinterpret_cast<const uint4*>(codes + (size_t)k0 * BITS / 8);
+    const uint32_t c[4] = {c4.x, c4.y, c4.z, c4.w};
+    const float s = elt_bits_to_f32<F16>(scales[k0 / GROUP]);
+    const float b = SONLY ? -8.0f * s : elt_bits_to_f32<F16>(biases[k0 / GROUP]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      constexpr int kInWord = 32 / BITS;
+#pragma unroll
+      for (int j = 0; j < kInWord; j += 2) {
+        const uint32_t xd = *reinterpret_cast<const uint32_t*>(x + k0 + i * kInWord + j);
+        const float q0 = (float)((c[i] >> (BITS * j)) & ((1u << BITS) - 1));
+        const float q1 = (float)((c[i] >> (BITS * (j + 1))) & ((1u << BITS) - 1));
+        acc = fmaf(elt_lo_to_f32<F16>(xd), fmaf(s, q0, b), acc);
+        acc = fmaf(elt_hi_to_f32<F16>(xd), fmaf(s, q1, b), acc);
+      }
+    }
+  }
+  return wave_sum(acc);
+}
+
 }  // namespace vpq

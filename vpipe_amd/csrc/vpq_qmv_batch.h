@@ -173,34 +173,6 @@ __device__ __forceinline__ u32x4 batch_bytes(uint32_t w0, uint32_t w1)
   return v;
 }
 
-// sum over k of x[k] * fma(scale, q[k], bias) of one output, by a whole wavefront: 16 bytes of codes per lane and pass,
-// the order of the general kernels (vpq_qmv_simple.hip).
-template <int BITS, int GROUP, bool F16, bool SONLY>
-__device__ float batch_plain_sum(const uint8_t* codes, const uint16_t* scales, const uint16_t* biases, const uint16_t* x, int K)
-{
-  constexpr int kPer = 128 / BITS;                          // values of a lane's 16 bytes
-  float acc = 0.0f;
-  for (int k0 = (int)(threadIdx.x & 63) * kPer; k0 < K; k0 += kWave * kPer) {
-    const uint4 c4 = *reinterpret_cast<const uint4*>(codes + (size_t)k0 * BITS / 8);
-    const uint32_t c[4] = {c4.x, c4.y, c4.z, c4.w};
-    const float s = elt_bits_to_f32<F16>(scales[k0 / GROUP]);
-    const float b = SONLY ? -8.0f * s : elt_bits_to_f32<F16>(biases[k0 / GROUP]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      constexpr int kInWord = 32 / BITS;
-#pragma unroll
-      for (int j = 0; j < kInWord; j += 2) {
-        const uint32_t xd = *reinterpret_cast<const uint32_t*>(x + k0 + i * kInWord + j);
-        const float q0 = (float)((c[i] >> (BITS * j)) & ((1u << BITS) - 1));
-        const float q1 = (float)((c[i] >> (BITS * (j + 1))) & ((1u << BITS) - 1));
-        acc = fmaf(elt_lo_to_f32<F16>(xd), fmaf(s, q0, b), acc);
-        acc = fmaf(elt_hi_to_f32<F16>(xd), fmaf(s, q1, b), acc);
-      }
-    }
-  }
-  return wave_sum(acc);
-}
-
 // 16 bytes per lane, global (base + off) -> LDS at lds_dst + 16 * lane.  Written out by hand: the compiler waits for every
 // such load that it knows about before any later LDS read, whatever the load fills.  The LDS base travels in M0, bound as an
 // operand (the s_nop is the wait state between that write and the load).
@@ -664,7 +636,7 @@ qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
         const int src = __builtin_ctzll(bad);
         bad &= bad - 1;
         const int row = __builtin_amdgcn_readlane(n_loc, src), mb = __builtin_amdgcn_readlane(m, src);
-        const float plain = batch_plain_sum<BITS, GROUP, F16, SONLY>(
+        const float plain = plain_sum<BITS, GROUP, F16, SONLY>(
             wtile + (size_t)row * row_bytes, sc_src + (size_t)row * Kg, SONLY ? nullptr : bi_src + (size_t)row * Kg,
             p.x + (size_t)mb * p.K, p.K);
         if (lane == src) { total = plain; }
@@ -705,7 +677,7 @@ qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
 #pragma unroll
     for (int j = 0; j < kRounds; ++j) {
       if (wave * kWave + j * kThreads >= kQuads) { break; }
-      const bool on = tid + j * kThreads < kQuads;             // (all lanes stay: batch_plain_sum needs them)
+      const bool on = tid + j * kThreads < kQuads;             // (all lanes stay: plain_sum needs them)
       const int i = on ? tid + j * kThreads : 0;
       floatx4 part[kBatchWaves], total = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -725,7 +697,7 @@ qmv_batch_kernel(VPQ_PRELOADED_WORDS, const PreloadTail<BatchParams> tail)
         const int src = __builtin_ctzll(__ballot(bad_here != 0));
         const int e = __builtin_ctz(__builtin_amdgcn_readlane((int)bad_here, src));
         const int row = __builtin_amdgcn_readlane(n_loc, src) + e, mb = __builtin_amdgcn_readlane(m, src);
-        const float plain = batch_plain_sum<BITS, GROUP, F16, SONLY>(
+        const float plain = plain_sum<BITS, GROUP, F16, SONLY>(
             wtile + (size_t)row * row_bytes, sc_src + (size_t)row * Kg, SONLY ? nullptr : bi_src + (size_t)row * Kg,
             p.x + (size_t)mb * p.K, p.K);
         if ((tid & 63) == src) {
