@@ -73,6 +73,16 @@ def test_argmax_partial_and_combine_for_any_slab_count(vpq, oracle, dev, D, part
     assert int(out.item()) == int(oracle.argmax(bits)[0])
 
 
+@pytest.mark.parametrize("two_stage", [False, True])
+def test_argmax_of_the_longest_row(vpq, dev, two_stage):
+    # every step of the scan past the end would wrap a signed index
+    V = 2 ** 31 - 1
+    logits = torch.zeros((1, V), dtype=torch.bfloat16, device=dev)
+    for at in (V - 1, V - 2040):
+        logits[0, at] = 1.0
+        assert vpq.argmax_bf16(logits, two_stage=two_stage).tolist() == [at]
+
+
 def test_argmax_rejects_bad_arguments(vpq, dev):
     L = vpq.load()
     t = torch.zeros(64, dtype=torch.int32, device=dev)

@@ -35,19 +35,19 @@ __device__ __forceinline__ void take_better(float& best, int& bi, float v, int i
 }
 
 // Entries [i, i + 8) of a row, up to `hi`: one 16-byte load, at whatever address (the row's start need not be aligned).  One entry a
-// load: 6.5 us over 8 rows of 151936, now 4.9.
-__device__ __forceinline__ void take_eight(float& best, int& bi, const uint16_t* src, int i, int hi)
+// load: 6.5 us over 8 rows of 151936, now 4.9.  (Unsigned: a step past the end of the longest row is no wrap to its front.)
+__device__ __forceinline__ void take_eight(float& best, int& bi, const uint16_t* src, uint32_t i, uint32_t hi)
 {
   if (i + 8 <= hi) {
     uint32_t v[4];
     __builtin_memcpy(v, src + i, 16);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      take_better(best, bi, bf16_bits_to_f32((uint16_t)v[j]), i + 2 * j);
-      take_better(best, bi, bf16_bits_to_f32((uint16_t)(v[j] >> 16)), i + 2 * j + 1);
+      take_better(best, bi, bf16_bits_to_f32((uint16_t)v[j]), (int)i + 2 * j);
+      take_better(best, bi, bf16_bits_to_f32((uint16_t)(v[j] >> 16)), (int)i + 2 * j + 1);
     }
   } else {
-    for (; i < hi; ++i) { take_better(best, bi, bf16_bits_to_f32(src[i]), i); }
+    for (; i < hi; ++i) { take_better(best, bi, bf16_bits_to_f32(src[i]), (int)i); }
   }
 }
 
@@ -78,12 +78,12 @@ __global__ __launch_bounds__(256) void argmax_partial_kernel(const uint16_t* __r
 {
   const int row = blockIdx.y;
   const uint16_t* src = logits + (size_t)row * V;
-  const int slab = (V + parts - 1) / parts;
-  const int lo = blockIdx.x * slab;
-  const int hi = lo + slab < V ? lo + slab : V;
+  const uint32_t slab = ((uint32_t)V + (uint32_t)parts - 1) / (uint32_t)parts;
+  const uint32_t lo = blockIdx.x * slab;
+  const uint32_t hi = lo + slab < (uint32_t)V ? lo + slab : (uint32_t)V;
   float best = -INFINITY;
   int bi = kNoIndex;
-  for (int i = lo + (int)threadIdx.x * 8; i < hi; i += 256 * 8) { take_eight(best, bi, src, i, hi); }
+  for (uint32_t i = lo + threadIdx.x * 8; i < hi; i += 256 * 8) { take_eight(best, bi, src, i, hi); }
   block_argmax(best, bi);
   if (threadIdx.x == 0) {
     float* slot = partials + 2 * ((size_t)row * parts + blockIdx.x);
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void argmax_row_kernel(const uint16_t* __restr
   const uint16_t* src = logits + (size_t)row * V;
   float best = -INFINITY;
   int bi = kNoIndex;
-  for (int i = (int)threadIdx.x * 8; i < V; i += 256 * 8) { take_eight(best, bi, src, i, V); }
+  for (uint32_t i = threadIdx.x * 8; i < (uint32_t)V; i += 256 * 8) { take_eight(best, bi, src, i, (uint32_t)V); }
   block_argmax(best, bi);
   if (threadIdx.x == 0) { out_id[row] = bi == kNoIndex ? 0 : bi; }
 }
@@ -124,8 +124,8 @@ __global__ __launch_bounds__(256) void argmax_row_kernel(const uint16_t* __restr
 int argmax_parts(int V)
 {
   // about 2048 entries per slab, at most 256 slabs (one combine pass of 256 threads)
-  const int p = (V + 2047) / 2048;
-  return p < 1 ? 1 : (p > 256 ? 256 : p);
+  const uint32_t p = ((uint32_t)V + 2047) / 2048;
+  return p < 1 ? 1 : (p > 256 ? 256 : (int)p);
 }
 
 hipError_t argmax_static_scratch(float** out)
