@@ -753,6 +753,7 @@ hipError_t batch_launch_one(hipStream_t st, const BatchParams& p, size_t lds_byt
   return launch_preloaded(kern, dim3((unsigned)grid), dim3(kBatchWaves * kWave), lds_bytes, st, p);
 }
 
+// The formats whose entrances end at 16 rows of x (binary16, 8 bits in groups of 32, Q4_0) have no forms for more.
 template <int BITS, int GROUP, bool F16, bool SONLY = false>
 hipError_t batch_launch(hipStream_t st, const BatchParams& p, const BatchPlan& plan, size_t lds_bytes, int grid)
 {
@@ -760,11 +761,15 @@ hipError_t batch_launch(hipStream_t st, const BatchParams& p, const BatchPlan& p
   if (plan.tiles == T_ && plan.mr == MR_ && plan.depth == DEPTH_) {                                   \
     return batch_launch_one<T_, MR_, BITS, GROUP, F16, SONLY, DEPTH_>(st, p, lds_bytes, grid);        \
   }
-  VPQ_BATCH(1, 1, 1) VPQ_BATCH(1, 2, 1) VPQ_BATCH(1, 4, 1) VPQ_BATCH(1, 8, 1) VPQ_BATCH(2, 1, 1) VPQ_BATCH(2, 2, 1)
-  VPQ_BATCH(2, 4, 1) VPQ_BATCH(2, 8, 1) VPQ_BATCH(2, 12, 1) VPQ_BATCH(2, 16, 1) VPQ_BATCH(3, 8, 1) VPQ_BATCH(3, 12, 1)
+  constexpr bool kMoreRows = !F16 && !SONLY && !(BITS == 8 && GROUP == 32);
+  VPQ_BATCH(1, 1, 1) VPQ_BATCH(1, 2, 1) VPQ_BATCH(1, 4, 1) VPQ_BATCH(2, 1, 1) VPQ_BATCH(2, 2, 1) VPQ_BATCH(2, 4, 1)
   VPQ_BATCH(1, 4, 2)
   if constexpr (BITS == 4) { VPQ_BATCH(2, 4, 2) }
-  if constexpr (BITS == 8) { VPQ_BATCH(1, 1, 3) VPQ_BATCH(1, 2, 2) VPQ_BATCH(1, 8, 2) VPQ_BATCH(2, 8, 2) }
+  if constexpr (BITS == 8) { VPQ_BATCH(1, 1, 3) VPQ_BATCH(1, 2, 2) }
+  if constexpr (kMoreRows) {
+    VPQ_BATCH(1, 8, 1) VPQ_BATCH(2, 8, 1) VPQ_BATCH(2, 12, 1) VPQ_BATCH(2, 16, 1) VPQ_BATCH(3, 8, 1) VPQ_BATCH(3, 12, 1)
+    if constexpr (BITS == 8) { VPQ_BATCH(1, 8, 2) VPQ_BATCH(2, 8, 2) }
+  }
 #undef VPQ_BATCH
   return hipErrorInvalidValue;
 }

@@ -642,10 +642,15 @@ hipError_t dispatch_flow(const FlowPlan& pl, bool y_f32, const FlowHead& h, cons
     constexpr int S = decltype(s_c)::value, R = decltype(r_c)::value;
     constexpr bool kF32 = decltype(f32_c)::value;
     if (form == FlowForm::kF16) { return launch_flow_kernel<S, R, kF32, C, true, 0>(grid, block, lds_bytes, st, p); }
-    if (form == FlowForm::kNarrow64) { return launch_flow_kernel<S, R, kF32, C, false, 6>(grid, block, lds_bytes, st, p); }
     if (form == FlowForm::kNarrow32) { return launch_flow_kernel<S, R, kF32, C, false, 5>(grid, block, lds_bytes, st, p); }
     if (form == FlowForm::kNarrowQ40) { return launch_flow_kernel<S, R, kF32, C, false, 5, true>(grid, block, lds_bytes, st, p); }
-    if (form == FlowForm::kNarrowF16) { return launch_flow_kernel<S, R, kF32, C, true, 6>(grid, block, lds_bytes, st, p); }
+    if (form == FlowForm::kNarrow64 || form == FlowForm::kNarrowF16) {
+      if constexpr (S > 1) {                   // (a K above 2048: the ones of groups of 64 are no multiple of 512)
+        return form == FlowForm::kNarrow64 ? launch_flow_kernel<S, R, kF32, C, false, 6>(grid, block, lds_bytes, st, p)
+                                           : launch_flow_kernel<S, R, kF32, C, true, 6>(grid, block, lds_bytes, st, p);
+      }
+      return hipErrorInvalidValue;
+    }
     return launch_flow_kernel<S, R, kF32, C, false, 0>(grid, block, lds_bytes, st, p);
   };
 #define VPQ_FLOW(S, R)                                                                                    \
