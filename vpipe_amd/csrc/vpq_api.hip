@@ -106,9 +106,12 @@ hipError_t launch_row8(hipStream_t hs, const vpq::QmvArgs& a, const vpq::QmvGrou
 }
 
 // One row of binary16 whose scales are no whole 16-byte pieces: the one-row kernel from the K on from which its error against
-// float64 is no larger than that of one wavefront per weight row, which ran these (fp32 output, 1e-7, K = 2112 / 3840 / 9664: 1.36 /
-// 1.34 / 1.32 and 1.20 / 1.51 / 2.27; the batch kernel, which takes what is shorter: 0.83 / 0.91 / 1.07).  us, one wavefront per row
-// / batch kernel / now: 3840 -> 3840 5.8 / 5.1 / 3.9, 3840 -> 19328 17.4 / 13.0 / 10.5, 9664 -> 3840 11.3 / 9.4 / 7.8.
+// float64 is no larger than that of one wavefront per weight row, which ran these (fp32 output, 1e-7, K = 2112 / 3840 / 9664:
+// 1.36 / 1.34 / 1.32 and 1.20 / 1.51 / 2.27; the batch kernel, which takes what is shorter: 0.83 / 0.91 / 1.07).  us, one
+// wavefront per row / batch kernel / now: 3840 -> 3840 5.8 / 5.1 / 3.9, 3840 -> 19328 17.4 / 13.0 / 10.5, 9664 -> 3840 11.3 / 9.4 /
+// 7.8.  What is shorter, one wavefront per row / batch kernel: 1280 -> 4096 3.8 / 3.7, 1280 -> 16384 8.6 / 6.2, 2496 -> 4096 5.7 /
+// 5.1, 2496 -> 16384 14.4 / 9.3, but 1280 -> 1024 2.9 / 3.4 and 2496 -> 1024 3.5 / 4.2: the line may not depend on N, or a narrow
+// k or v would have other bits in a launch with q, and the three together gain (2496 -> 2496 | 640 | 640 12.1 / 5.1).
 bool flow_narrow_f16(int K, int N, int M) { return K >= 3072 && (K % 512) != 0 && vpq::qmv_flow_narrow_supports(K, N, M, 64); }
 
 // The batch kernel over one pack.

@@ -37,7 +37,9 @@ long batch_blocks(const QmvGroup& g, int tiles)
 // shapes (512..36000 x 2048..17408, packs from HBM; 4 bits, 4 bits in groups of 32, 8 bits), first to the times (met to 5..9
 // %), then to the time of what is chosen: on average 0.2..0.6 % above the fastest plan's.  Over the rule for few rows at
 // 9..16 / 17..32 / 33..48 / 49..64 rows: 4 bits 1.08 / 1.16 / 1.25 / 1.13 times as fast, groups of 32 1.09 / 1.19 / 1.34 /
-// 1.17, 8 bits 1.05 / 1.13 / 1.22 / 1.12.
+// 1.17, 8 bits 1.05 / 1.13 / 1.22 / 1.12.  Binary16 and Q4_0 take the figures of 4 bits in groups of 64 and of 32, 8 bits in
+// groups of 32 those of 8 bits: on 30 drawn shapes at 9..16 rows 1.12, 1.12 and 1.06 times as fast as the kernel before with the
+// rule for few rows, the slowest 1.00, 0.97 and 0.98.
 struct BatchCost {
   int tiles, mr, depth;
   bool pairs;
