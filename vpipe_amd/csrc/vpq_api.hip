@@ -83,23 +83,23 @@ int check_pack(const uint32_t* w, const uint16_t* scales, const uint16_t* biases
 constexpr int kDenseRouteMinRows = 8192;
 
 // One row of 8-bit codes: below this K the general kernel, a launch a pack; from it on launch_row8, the same bits.  us: 2048 ->
-// 512 3.0 / 3.3, 2560 -> 640 4.2 / 4.2, 2560 -> 2560 5.5 / 4.8, 4096 -> 4096 7.8 / 7.2, 12288 -> 4096 19.8 / 15.2; q|k|v of 4096
-// in three launches 18.3, in one 9.5.
+// 512 3.0 / 3.3, 2560 -> 640 4.2 / 4.2, 2560 -> 2560 5.5 / 4.9, 4096 -> 4096 7.8 / 6.8, 12288 -> 4096 19.8 / 15.1; q|k|v of 4096
+// in three launches 18.3, in one 9.1.
 constexpr int kRow8MinK = 2560;
 
 // Whether `rows` weight rows of 8-bit codes (of all pairs together) are worth the gathers' kernel.  In its fifth pass over K, from
-// 4096 on, it holds x in so many registers that a CU has eight wavefronts; one wavefront per weight row, sixteen and more a CU, is
-// ahead where the former would have no more than one set of four rows each (us, that / the gathers' kernel, pairs of K -> N:
-// one of 5120 -> 5120 8.7 / 10.0; 4 of 5120 -> 3072 15.7 / 17.3; 8 of 4160 -> 1536 13.1 / 15.1; 24 of 4160 -> 1536, 9216 sets,
-// 33.5 / 33.0; 32 of it 44.6 / 40.2; 8 of 4608 -> 5120, 10240 sets, 38.1 / 37.2; 32 of it 141 / 123).  Gated, where the other
-// kernel reads two rows a wavefront, the gathers' kernel always is (one token of 4 experts, 4608 -> 1536: 11.6 / 9.5).
+// 4096 on, it holds x in so many registers that a CU has eight wavefronts, of four rows each; one wavefront per weight row, sixteen
+// and more a CU, is ahead up to about twelve sets of four rows a CU (us, that / the gathers' kernel, pairs of K -> N: one of 5120
+// -> 5120 8.7 / 9.5, 4 of 4160 -> 1536 8.3 / 9.2, 8 of it, twelve sets a CU, 13.0 / 13.6; 8 of 4608 -> 2048 17.7 / 16.9, 8 of 5120
+// -> 3072 26.5 / 24.9, 48 of it 142 / 123).  Gated, where the other kernel reads two rows a wavefront, the gathers' kernel always is
+// (one token of 4 experts, 4608 -> 1536: 11.6 / 9.5).
 bool gather8_takes(int K, long rows, bool gated)
 {
-  return vpq::qmv_gather_supports(K, 8) && (K <= 4096 || gated || rows > 4 * 32L * g_dev.cu_count);
+  return vpq::qmv_gather_supports(K, 8) && (K <= 4096 || gated || rows > 4 * 12L * g_dev.cu_count);
 }
 
 // One row of x against the 8-bit packs of g, each with the bits that it has as an expert's slab of a gather.  (Several packs: a
-// wavefront of one row would pay for the choice among them; q|k|v of 5120 13.1 us, on the gathers' kernel 11.8.)
+// wavefront of one row would pay for the choice among them; q|k|v of 5120 13.1 us, on the gathers' kernel 11.1.)
 hipError_t launch_row8(hipStream_t hs, const vpq::QmvArgs& a, const vpq::QmvGroup& g)
 {
   return gather8_takes(a.K, g.seg[0].N, g.count > 1) ? vpq::launch_qmv_gather_row8(hs, a, g) : vpq::launch_qmv_row8(hs, a, g);

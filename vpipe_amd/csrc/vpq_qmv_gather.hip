@@ -85,12 +85,14 @@ __device__ __forceinline__ void gather_body(const uint32_t* __restrict__ w_, con
   const int p = ONE ? 0 : (int)blockIdx.y;
   const uint16_t* x = x_ + (size_t)(p / x_div) * K;
   const int Kw = K * BITS / 32, Kg = K >> 6;
+  // (lanes past K, which contract nothing, take the row's start: under a condition a load waited for the one before it, 4 tokens
+  // of 8 of 128 experts 25.9 -> 25.0 us a layer)
   uint4 xd[P][kX];
 #pragma unroll
   for (int c = 0; c < P; ++c) {
-    const int k0 = (c * LPR + ll) * kVals;
+    const int k = (c * LPR + ll) * kVals, k0 = k < K ? k : 0;
 #pragma unroll
-    for (int t = 0; t < kX; ++t) { xd[c][t] = k0 < K ? *reinterpret_cast<const uint4*>(x + k0 + 8 * t) : make_uint4(0u, 0u, 0u, 0u); }
+    for (int t = 0; t < kX; ++t) { xd[c][t] = *reinterpret_cast<const uint4*>(x + k0 + 8 * t); }
   }
   int e = ONE ? 0 : pair_eid[p];
   const bool expert_ok = ONE || (e >= 0 && e < n_experts);
@@ -292,9 +294,9 @@ long gather_sets_per_wave(long sets, int cus)
 
 }  // namespace
 
-// One row of x, up to four 8-bit packs.  Measured (us, the general kernel / now): 4096 -> 1024 5.2 / 5.3, 4096 -> 4096 7.8 / 7.2,
-// 4096 -> 12288 16.6 / 14.2, 5120 -> 151936 182 / 145; gated, by qmv_rows8_kernel / now: 4096 -> 24576 29.9 / 25.0, 3840 -> 19328
-// 26.3 / 19.1, 5120 -> 34816 49.3 / 40.
+// One row of x, up to four 8-bit packs.  Measured (us, the general kernel / now): 4096 -> 1024 5.2 / 5.1, 4096 -> 4096 7.8 / 6.8,
+// 4096 -> 12288 16.6 / 14.1, 5120 -> 151936 182 / 146; gated, by qmv_rows8_kernel / now: 4096 -> 24576 29.9 / 23.9, 5120 -> 34816
+// 49.3 / 38.8.
 hipError_t launch_qmv_gather_row8(hipStream_t st, const QmvArgs& a, const QmvGroup& g)
 {
   const int cus = a.cu_count > 0 ? a.cu_count : 256;
