@@ -108,7 +108,8 @@ int vpq_embed_gather_w4g64_bf16(vpq_stream_t stream, const int32_t* ids, const u
  * plain fp32 one, about 1e-7; at one row, and in the forced variants other than
  * MFMA and SIMPLE, sum(x*q) is taken from sum(x*(128+q)): 4 to 9e-7.
  * An infinity in a row of x makes an output +-inf or NaN as the plain sum would at
- * two rows and more, NaN at one row.)  With `residual` ([M,N] bf16, nullable) the
+ * two rows and more, and at one row of a K < 2048 that is a multiple of 512; NaN at
+ * one row of any other K.)  With `residual` ([M,N] bf16, nullable) the
  * rounded result is added to it in fp32 and rounded again, as `_add` does
  * (:264-266).
  * Requires K % 64 == 0, N > 0, 1 <= M <= 16.
@@ -576,13 +577,12 @@ int vpq_argmax_combine(vpq_stream_t stream, const float* partials, int32_t* out_
 /* ---- 8-bit group-64 twins (w8g64) -------------------------------------------
  * The same affine format with one BYTE per value: w uint32 [N, K/4],
  * q[n, 4j+i] = (w[n,j] >> 8i) & 0xFF; scales, biases bf16 [N, K/64]
- * (gpu-kernels/metal/quant/affine_dequant.metal:60-97).  A first, general path for
- * the 8-bit checkpoints and the 8-bit linears of mixed-precision ones; not tuned
- * like the 4-bit kernels:
+ * (gpu-kernels/metal/quant/affine_dequant.metal:60-97).  For the 8-bit checkpoints
+ * and the 8-bit linears of mixed-precision ones:
  *   vpq_dequant_w8g64_bf16           replaces `affine_dequant_w8g64` (:68-97), bit-exact.
  *   vpq_qmv_w8g64_bf16 / _f32out     replace `affine_qmv_w8g64[_add]`
  *                                    (affine_qmv.metal:3034-3050, 3122-3140): QMV arithmetic,
- *                                    1 <= M <= 16, one wavefront per output row.
+ *                                    1 <= M <= 16.
  *   vpq_qmm_dense_route_w8g64_bf16   the dequant-once route for any M (replaces
  *                                    `affine_qmm_steel_w8g64`, affine_qmm_steel.metal:1601-1672,
  *                                    by the reference's own second route): expansion into

@@ -29,8 +29,8 @@ def test_dequant_g32_bit_exact(vpq, oracle, dev, D, N, K):
     out.assert_intact()
 
 
-# both kernels (up to two rows of x: row-streaming; more: one wavefront per row), K below / at / above a
-# 2048-wide pass and not a multiple of 64, ragged N
+# every kernel (one row of x: row-streaming below K = 2048, else the one-row kernel; more: the batch kernel), K below / at / above
+# a 2048-wide pass and not a multiple of 64, ragged N
 QMV_SHAPES = [(32, 5, 1), (96, 33, 2), (1024, 48, 3), (2080, 130, 1), (3872, 64, 2), (4096, 95, 8), (2560, 64, 16),
               (5120, 4096, 1)]
 
@@ -214,7 +214,7 @@ def test_qmm_g32_gated_store(vpq, oracle, dev, D, activation):
 def test_qmv_group_g32_is_the_separate_calls(vpq, dev, D, K, M, rows):
     """affine_qmv_qkv_w4g32 (gpu-kernels/metal/quant/affine_qmv.metal:518-538): the row-concatenated q|k|v pack as one
     call; every output has the bits of its own vpq_qmv_w4g32_bf16 call (whose parity test_qmv_g32 holds), guard bands
-    intact.  M <= 2 is one launch of the row-streaming kernel, more rows are separate launches."""
+    intact.  One launch of the kernel of the single call."""
     N = sum(rows)
     w, s, b = synth.make_weight_g32(N, K, 6800 + K + N)
     x = synth.make_act(M, K, 6900 + K + M)

@@ -138,14 +138,13 @@ def test_gathers_have_the_bits_of_the_plain_kernels(vpq, dev, D, bits, K, N, pai
         pack, xr = [t[int(eid[p])] for t in (w, s, b)], x[p:p + 1]
         if bits == 8:
             g = vpq.qmv_gated_w8g64(*pack, xr, K, N, 1, activation=1)
-            d = None
+            d = vpq.qmv_w8g64(*pack, xr, K, N, 1)
         else:
             g = vpq.qmv_swiglu_w4g64(*pack, xr, K, N, 1, variant=capi.VPQ_QMV_ROWS)
             d = vpq.qmv_w4g64(*pack, xr, K, N, 1, variant=capi.VPQ_QMV_ROWS)
         assert np.array_equal(D.bits(act.view)[p], D.bits(g)[0])
-        if d is not None:
-            assert np.array_equal(D.bits(out.view)[p], D.bits(d)[0])
-        else:                                            # (no plain entry point has that store: the sums, to their rounding)
+        assert np.array_equal(D.bits(out.view)[p], D.bits(d)[0])
+        if bits == 8:                                    # (and the sums, to their rounding)
             deq = (s[int(eid[p])].double().repeat_interleave(64, 1) * w[int(eid[p])].view(torch.uint8).view(N, K).double() +
                    b[int(eid[p])].double().repeat_interleave(64, 1))
             want = deq @ xr[0].double()
